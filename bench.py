@@ -62,13 +62,13 @@ def weight_and_packed(K, N, sparsity, seed, device):
 
 
 def kernel_source_hash():
-    """sha256 over the sources the headline's three kernels and their launcher are built from (the row-parallel
-    kernels' translation unit, what it shares with the others, the blob builder, the shared constants): a traffic
+    """sha256 over the sources the headline's kernel and its launcher are built from (the matrix-core
+    kernel's translation unit, what it shares with the others, the blob builder, the shared constants): a traffic
     figure recorded for other sources is not reported."""
     import hashlib
     h = hashlib.sha256()
     csrc = os.path.join(ROOT, "ternaryllm_amd", "csrc")
-    for name in ("tl_rows.hip", "tl_device.h", "tl_layout.cpp", "tl_common.h"):
+    for name in ("tl_matrix.hip", "tl_matrix.h", "tl_device.h", "tl_layout.cpp", "tl_common.h"):
         with open(os.path.join(csrc, name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()[:16]
@@ -527,15 +527,14 @@ def main():
         "ms_per_step": round(wall_ms, 5), "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f16 in / f32 accumulate / f16 out", "data": "synthetic",
         "config": {"workload": "Llama-2-7B ternary MLP gate projection SpMM: M=1024 (8x128 tokens), K=4096, N=11008, "
-                               "80% sparsity, fp16 activations, per-output fp16 scale, u8 tile-local indices",
+                               "80% sparsity, fp16 activations, per-output fp16 scale, two-bit weight codes (u8 tile-local indices beside them)",
                    "M": M, "K": K, "N": N, "sparsity": sparsity, "nnz": int(nnz), "algorithmic_bytes": int(B),
                    "x_layout": "row-major [M][K]", "max_rel_err": max_rel},
         "pct_hbm_peak": round(100 * gbs / HBM_PEAK_GBS, 3),
         "tokens_per_s": round(M / (wall_ms * 1e-3), 1),
         "roofline": {"bound": "hbm", "achieved": round(B / (ev_ms * 1e-3) / 1e9, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(B / (ev_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 5), "traffic": traffic, "traffic_note": traffic_note,
-                     "kernel": "tl_relayout_rows_h + tl_spmm_rows<__half, 4, 8, 16, false, false> + tl_rows_fixup<__half, 4, 8, 16, false, false> "
-                               "(the three launches of one tl_spmm call on row-major activations)",
+                     "kernel": "tl_matrix_rows<1, 2, 4, 4, 2, 4, 0> (the one launch of a tl_spmm call on row-major activations)",
                      "kernel_ms": round(ev_ms, 5)},
     }
     extra = {

@@ -64,7 +64,7 @@ const char* tl_last_error(void);
 int tl_version(void);
 
 /* The launchers' tuning knobs (environment variables TL_SMALL_LDS, TL_TILE_GROUP, TL_QUAD_SHARE, TL_LW,
- * TL_SPMV_SHARE, TL_SPMV_WIDE, TL_SPMV_TILES, TL_SMALL_MT, TL_SPMV_DIRECT, TL_BLOCK_SET, TL_ROWS_SPLIT,
+ * TL_SPMV_SHARE, TL_SPMV_WIDE, TL_SPMV_TILES, TL_SMALL_MT, TL_SPMV_DIRECT, TL_BLOCK_SET,
  * TL_OCTET, TL_QUAD_WIDE, TL_RES16; unset = the launcher's own choice) are read once per process.  This
  * reads them again -- for tests and tuning runs that change them between calls. */
 int tl_reload_options(void);
@@ -139,12 +139,23 @@ int tl_tiled_mcsc_to_dense(const void* merged_row, int index_width, int64_t n_in
 /*   - the stream is block-major: all tiles of block 0, then block 1, ...;  */
 /*     chunkstart[block * T + tile] is the dword where a chunk begins       */
 /*     (one extra entry marks the end).                                     */
+/*   - codes: the same matrix once more, two bits an entry, in the order    */
+/*     in which a wave of the matrix-core kernels wants it.  One 1-KB unit  */
+/*     holds 16 columns x 256 rows: lane l of the wave owns bytes 16l ..    */
+/*     16l + 15, which are column l % 16 and, in dword d, the rows          */
+/*     64d + 32h + 8(l / 16) + 2i + j (h, j in {0, 1}, i in 0 .. 3): bits   */
+/*     15 - 2(4h + i) (sign) and 14 - 2(4h + i) (non-zero) of the low (j=0) */
+/*     or high (j=1) half.  Units run codes[block][plane][unit]; rows past  */
+/*     K and columns past N are zero.                                       */
 /* The blob starts with a tl_layout_header (256 bytes).                     */
 /* ======================================================================== */
 
 #define TL_LAYOUT_MAGIC 0x35474C54u /* "TLG5" */
-#define TL_LAYOUT_VERSION 5
+#define TL_LAYOUT_VERSION 6
+#define TL_LAYOUT_VERSION_NO_CODES 5 /* the same without the two-bit codes: still read, multiplied by a slow general kernel */
 #define TL_BLOCK_COLUMNS 16
+#define TL_CODE_UNIT_ROWS 256
+#define TL_CODE_UNIT_BYTES 1024
 
 typedef struct tl_layout_header {
     uint32_t magic;
@@ -164,12 +175,19 @@ typedef struct tl_layout_header {
     uint32_t max_run_dwords; /* largest (+1 run dwords + -1 run dwords) of any (column, tile)             */
     uint32_t mean_run_dwords_x16; /* mean of the same, times 16, rounded up                               */
     uint64_t checksum;       /* FNV-1a (64-bit, one step per dword) over the chunk table, then the stream */
-    uint32_t reserved[40];   /* zero */
+    uint64_t off_codes;      /* byte offset of the two-bit codes, 0 = none                                */
+    uint32_t code_units;     /* ceil(K / TL_CODE_UNIT_ROWS)                                               */
+    uint32_t code_planes;    /* ternary matrices the codes hold: W is their sum (1 unless rows repeat)    */
+    uint32_t reserved[36];   /* zero */
 } tl_layout_header;
 
 /* Bytes of the blob that tl_layout_build will write for these tiled-CSC arrays
  * (as produced by tl_convert_to_ter_tiled_csc with tile height tile_k).
- * tile_rows = 0 picks the default (the largest balanced height <= 255). */
+ * tile_rows = 0 picks the default (the largest balanced height <= 255).
+ * The offsets do not say whether a column names a row twice: arrays that do want
+ * room for code_planes - 1 further planes of codes (the largest |entry| of the matrix
+ * less one, times n_blocks * code_units * TL_CODE_UNIT_BYTES); with less room the blob is
+ * built without codes. */
 int tl_layout_size(const int32_t* neg_off_tiled, const int32_t* pos_off_tiled,
                    int columns, int inners, int tile_k, int tile_rows, int64_t* blob_bytes);
 
@@ -200,7 +218,11 @@ int tl_layout_from_mcsc(const void* merged_row, int index_width, int64_t n_index
                         const int32_t* merged_off, int columns, int inners, int tile_k,
                         int uniformed, int tile_rows, void* blob, int64_t* blob_bytes);
 
-/* Validates a host copy of a blob (header, bounds, monotone offsets, row range, sentinel use, checksum). */
+/* Copies a blob of TL_LAYOUT_VERSION_NO_CODES (or any other) to `out` with its codes made anew.
+ * Call with out == NULL to get out_bytes only. */
+int tl_layout_add_codes(const void* blob, int64_t blob_bytes, void* out, int64_t* out_bytes);
+
+/* Validates a host copy of a blob (header, bounds, monotone offsets, row range, sentinel use, checksum, codes). */
 int tl_layout_validate(const void* blob, int64_t blob_bytes);
 
 /* Decodes a host blob back to dense int32 [inners][columns] (round-trip check): an entry is the

@@ -43,7 +43,8 @@ class LayoutHeader(ctypes.Structure):
         ("off_chunkstart", ctypes.c_uint64), ("off_stream", ctypes.c_uint64),
         ("stream_bytes", ctypes.c_uint64), ("total_bytes", ctypes.c_uint64),
         ("max_run_dwords", ctypes.c_uint32), ("mean_run_dwords_x16", ctypes.c_uint32),
-        ("checksum", ctypes.c_uint64), ("reserved", ctypes.c_uint32 * 40),
+        ("checksum", ctypes.c_uint64), ("off_codes", ctypes.c_uint64), ("code_units", ctypes.c_uint32), ("code_planes", ctypes.c_uint32),
+        ("reserved", ctypes.c_uint32 * 36),
     ]
 
 
@@ -71,6 +72,7 @@ SIGNATURES = {
     "tl_layout_build": (_INT, [_I32P, _I32P, _I32P, _I32P, _INT, _INT, _INT, _INT, _VP, _I64]),
     "tl_layout_from_dense": (_INT, [_I32P, _INT, _INT, _INT, _VP, _I64P]),
     "tl_layout_from_mcsc": (_INT, [_VP, _INT, _I64, _I32P, _INT, _INT, _INT, _INT, _INT, _VP, _I64P]),
+    "tl_layout_add_codes": (_INT, [_VP, _I64, _VP, _I64P]),
     "tl_layout_validate": (_INT, [_VP, _I64]),
     "tl_layout_to_dense": (_INT, [_VP, _I64, _I32P]),
     "tl_spmm_workspace": (_INT, [_HDRP, _I64, _INT, _INT, _I64P]),

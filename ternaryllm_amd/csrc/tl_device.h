@@ -1,7 +1,7 @@
 // What the translation units of libternary_spmm's device code share: the argument block of the kernels, the
 // device helpers every kernel family uses, and the host helpers of the launchers (knobs, device facts, checks).
 //   tl_small_m.hip  the kernels for 1 to 48 activation rows and their launchers
-//   tl_rows.hip     the row-parallel kernel (more than 48 rows), its re-layout and fix-up kernels and launchers
+//   tl_matrix.hip   the matrix-core kernel for more than 48 rows, the image of its activations, their launcher
 //   tl_kernels.hip  the entry points, the checks in front of them, the knobs, the measurement helpers
 #pragma once
 #include <hip/hip_fp16.h>
@@ -29,6 +29,7 @@ __device__ __forceinline__ const_u32_ptr as_const(const uint32_t* p) { return (c
 struct WeightPtrs {
     const uint32_t* chunkstart;  // [NB * T + 1], dword offsets into stream
     const uint32_t* stream;      // chunks: 64 descriptors + runs of four 8-bit rows per dword
+    const unsigned char* codes;  // two-bit codes [NB][planes][units], 1 KB each, or null
     const void* scale;           // per-column factor or null
 };
 
@@ -48,10 +49,6 @@ struct KernelArgs {
     unsigned vpt_magic;   // small-M kernel, row-copy staging: ceil(2^32 / (tile_rows / values per vector))
     unsigned tile_magic;  // ceil(2^32 / tile_rows): k / tile_rows == (k * tile_magic) >> 32 for every k < 2^24
     long long x_sm, x_sk; // small-M kernel: element strides of the activations along M and along K
-    long long split_steps;  // row kernel: 0, or the number of (output tile, K tile) steps shared out among the workgroups
-    int whole_units;        // row kernel: output tiles every workgroup works through on its own first
-    int split_first_unit;   // row kernel: first output tile of those whose steps are shared out
-    float* partial;         // row kernel: partial sums of output tiles whose K tiles were shared out
     float one;  // 1.0f, passed in so that the fp16 -> fp32 accumulate stays a single mixed-precision fma
     // single-row kernel with a fused producer of its input (tl_spmv_fused)
     const void* X2;       // second summand of the residual add, or null
@@ -73,6 +70,12 @@ struct KernelArgs {
     float* chain_sq_out;      // [NB][16]
     const float* chain_sq_in; // [chain_sq_blocks][16] sums of squares of the rows X was made from: the product is multiplied by rsqrt(sum / K + eps), row by row
     int chain_sq_blocks;
+    // matrix-core kernels
+    int units, planes;        // code units along K; ternary matrices the codes hold
+    const void* image;        // the activations they multiply: row-major, 16-byte pieces along K ...
+    long long image_ld;       // ... elements between rows
+    long long image_plane;    // ... and, for fp32 activations in three bf16 parts, between parts
+    int vector_out;           // four neighbouring outputs of a row may be stored as one piece
 };
 
 // rsqrt(mean square + eps) of the rows behind a chained product.  Called by the first 64 threads of a workgroup (one
@@ -145,19 +148,14 @@ __device__ __forceinline__ int run_neg_dwords(uint32_t d) { return (int)((((d >>
 // ---------------------------------------------------------------------------
 // Host side, shared by the launchers.
 // ---------------------------------------------------------------------------
-constexpr int kSmallMaxM = 48;       // above this the row-parallel kernel takes over
-constexpr int kRowsWaves = 16;
-constexpr int kRowsCols = 4;       // columns per wave of the fused gate/up kernel (two accumulator sets)
-constexpr int kRowsColsPlain = 8;  // columns per wave of the plain kernel: an activation tile then serves 128 columns
+constexpr int kSmallMaxM = 48;       // above this the product runs on the matrix cores
 constexpr int kMaxComputeUnits = 256;
 constexpr int kMaxChunkBytes = (TL_BLOCK_COLUMNS + TL_BLOCK_COLUMNS * 128) * 4;  // a chunk of all-non-zero columns
-
-inline int rows_mtile(int x_dtype) { return x_dtype == TL_F16 ? 256 : 128; }
 
 // Tuning knobs (environment variables of the same names).  They are read once, at the first launch of the
 // process; tl_reload_options() reads them again.  A knob that is not set leaves the launcher's own choice.
 enum Knob { TL_SMALL_LDS, TL_TILE_GROUP, TL_QUAD_SHARE, TL_LW, TL_SPMV_SHARE, TL_SPMV_WIDE, TL_SMALL_MT, TL_SPMV_DIRECT,
-            TL_BLOCK_SET, TL_ROWS_SPLIT, TL_OCTET, TL_QUAD_WIDE, TL_SPMV_TILES, TL_RES16, kKnobCount };
+            TL_BLOCK_SET, TL_OCTET, TL_QUAD_WIDE, TL_SPMV_TILES, TL_RES16, kKnobCount };
 int knob(Knob which, int fallback);   // tl_kernels.hip
 int compute_units();                  // of the current device, read once per device
 int check_header(const tl_layout_header* h);
@@ -182,14 +180,13 @@ inline int64_t small_kmajor_bytes(const tl_layout_header* h, int64_t M, int x_dt
 }
 int launch_small(KernelArgs a, const tl_layout_header* h, int x_dtype, void* workspace, int64_t workspace_bytes, hipStream_t st);
 
-// tl_rows.hip
-// Bytes of partial sums the row kernel may leave when K tiles are shared out (both weight sets of the
-// fused gate/up kernel): two slots per workgroup of a one-workgroup-per-compute-unit launch.
-constexpr int64_t kRowsPartialBytes = (int64_t)kMaxComputeUnits * 2 * 2 * kRowsWaves * kRowsCols * 4 * 64 * sizeof(float);
-inline int64_t rows_relayout_bytes(int64_t K, int64_t M, int x_dtype)
+// tl_matrix.hip
+// The row-major image of the activations where the kernel does not read them as they lie: two bytes a value, for fp32
+// three times two.
+inline int64_t matrix_image_bytes(int64_t K, int64_t M, int x_dtype)
 {
-    return round_up(K * round_up(M, rows_mtile(x_dtype)) * (x_dtype == TL_F16 ? 2 : 4), 256);
+    return round_up(M, 256) * round_up(K, 8) * 2 * (x_dtype == TL_F16 ? 1 : 3) + 256;
 }
-int launch_rows(KernelArgs a, int x_dtype, void* workspace, int64_t workspace_bytes, bool gated, hipStream_t st);
+int launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t workspace_bytes, bool two_weights, hipStream_t st);
 
 }  // namespace tl

@@ -1,5 +1,5 @@
 // Entry points of libternary_spmm's device code (include/ternary_spmm.h): the checks in front of every launch, the
-// choice between the kernels for few rows (tl_small_m.hip) and the row-parallel kernel (tl_rows.hip), the tuning
+// choice between the kernels for few rows (tl_small_m.hip) and the matrix-core kernel (tl_matrix.hip), the tuning
 // knobs, the scratch of the entry point that allocates nothing, and the measurement helpers.
 #include "tl_device.h"
 
@@ -12,7 +12,7 @@ namespace tl {
 int check_header(const tl_layout_header* h)
 {
     if (!h) return fail(TL_ERR_ARG, "layout header is null");
-    if (h->magic != TL_LAYOUT_MAGIC || h->version != TL_LAYOUT_VERSION) return fail(TL_ERR_FORMAT, "bad layout magic/version");
+    if (h->magic != TL_LAYOUT_MAGIC || (h->version != TL_LAYOUT_VERSION && h->version != TL_LAYOUT_VERSION_NO_CODES)) return fail(TL_ERR_FORMAT, "bad layout magic/version");
     if (h->tile_rows == 0 || h->tile_rows > (uint32_t)kMaxTileRows || h->n_tiles != (uint32_t)ceil_div(h->inners, h->tile_rows) ||
         h->n_blocks != (uint32_t)ceil_div(h->columns, TL_BLOCK_COLUMNS) || h->max_chunk_dwords < TL_BLOCK_COLUMNS ||
         (int64_t)h->max_chunk_dwords * 4 > kMaxChunkBytes + 16)
@@ -27,7 +27,7 @@ int check_dtype(int d, const char* what)
 }
 
 const char* const kKnobNames[kKnobCount] = {"TL_SMALL_LDS", "TL_TILE_GROUP", "TL_QUAD_SHARE", "TL_LW", "TL_SPMV_SHARE", "TL_SPMV_WIDE",
-                                            "TL_SMALL_MT", "TL_SPMV_DIRECT", "TL_BLOCK_SET", "TL_ROWS_SPLIT", "TL_OCTET", "TL_QUAD_WIDE", "TL_SPMV_TILES", "TL_RES16"};
+                                            "TL_SMALL_MT", "TL_SPMV_DIRECT", "TL_BLOCK_SET", "TL_OCTET", "TL_QUAD_WIDE", "TL_SPMV_TILES", "TL_RES16"};
 struct Knobs {
     bool set[kKnobCount];
     int value[kKnobCount];
@@ -56,8 +56,7 @@ int knob(Knob which, int fallback)
     return k->set[which] ? k->value[which] : fallback;
 }
 
-// Compute units of the current device, asked once per device.  Launch shapes are sized by it; the row
-// kernel's one-workgroup-per-unit launch is capped at kMaxComputeUnits, which sizes its partial-sum area.
+// Compute units of the current device, asked once per device.  Launch shapes are sized by it.
 int compute_units()
 {
     static std::atomic<int> cached[64];
@@ -77,6 +76,7 @@ WeightPtrs weight_ptrs(const tl_layout_header* h, const void* blob_dev, const vo
     WeightPtrs w;
     w.chunkstart = reinterpret_cast<const uint32_t*>(b + h->off_chunkstart);
     w.stream = reinterpret_cast<const uint32_t*>(b + h->off_stream);
+    w.codes = h->off_codes ? b + h->off_codes : nullptr;
     w.scale = scale;
     return w;
 }
@@ -126,8 +126,7 @@ extern "C" int tl_spmm_workspace(const tl_layout_header* header, int64_t M, int 
         *workspace_bytes = small_kmajor_bytes(header, M, x_dtype);
         return TL_OK;
     }
-    // the K-major image of the activations, then room for the partial sums of shared-out output tiles
-    *workspace_bytes = rows_relayout_bytes(header->inners, M, x_dtype) + kRowsPartialBytes;
+    *workspace_bytes = matrix_image_bytes(header->inners, M, x_dtype);
     return TL_OK;
 }
 
@@ -175,12 +174,12 @@ int spmm_call(const tl_layout_header* header, const void* blob_dev, const void* 
     a.X = X; a.Y = Y;
     a.ldx = ldx; a.ldy = ldy;
     a.M = (int)M; a.N = (int)header->columns; a.K = (int)header->inners; a.T = (int)header->n_tiles; a.tile_rows = (int)header->tile_rows;
-    a.NB = (int)header->n_blocks;
+    a.NB = (int)header->n_blocks; a.units = (int)header->code_units; a.planes = (int)header->code_planes;
     a.x_f16 = x_dtype == TL_F16; a.x_kmajor = x_layout == TL_X_K_MAJOR; a.y_f16 = y_dtype == TL_F16; a.scale_f16 = scale_dtype == TL_F16;
     a.one = 1.0f;
     hipStream_t st = static_cast<hipStream_t>(stream);
     int rc = (M <= kSmallMaxM) ? launch_small(a, header, x_dtype, workspace, workspace_bytes, st)
-                               : launch_rows(a, x_dtype, workspace, workspace_bytes, false, st);
+                               : launch_matrix_rows(a, x_dtype, workspace, workspace_bytes, false, st);
     if (rc) return rc;
     return finish_launch();
 }
@@ -214,9 +213,43 @@ extern "C" int tl_spmm_gated(const tl_layout_header* header, const void* blob_de
     return spmm_call(header, blob_dev, X, x_dtype, x_layout, ldx, M, Y, y_dtype, ldy, y_layout, scale, scale_dtype, workspace, workspace_bytes, stream);
 }
 
+extern "C" int tl_mlp_gate_up(const tl_layout_header* gate_header, const void* gate_blob_dev,
+                              const tl_layout_header* up_header, const void* up_blob_dev,
+                              const void* X, int x_dtype, int x_layout, int64_t ldx, int64_t M,
+                              void* H, int h_dtype, int64_t ldh,
+                              const void* gate_scale, const void* up_scale, int scale_dtype,
+                              int activation,
+                              void* workspace, int64_t workspace_bytes, void* stream)
+{
+    if (int rc = check_header(gate_header)) return rc;
+    if (int rc = check_header(up_header)) return rc;
+    if (gate_header->inners != up_header->inners || gate_header->columns != up_header->columns ||
+        gate_header->tile_rows != up_header->tile_rows || gate_header->code_planes != up_header->code_planes)
+        return fail(TL_ERR_SHAPE, "gate and up weights must share K, N, tile height and code planes");
+    if (activation != TL_ACT_SILU_GATE) return fail(TL_ERR_UNSUPPORTED, "activation code %d (only TL_ACT_SILU_GATE)", activation);
+    if (!up_blob_dev || reinterpret_cast<uintptr_t>(up_blob_dev) % 256) return fail(TL_ERR_ALIGN, "up blob null or not 256-byte aligned");
+    if (int rc = check_io(gate_blob_dev, X, H, x_dtype, x_layout, ldx, M, h_dtype, ldh, gate_scale, scale_dtype, gate_header)) return rc;
+    if ((gate_scale == nullptr) != (up_scale == nullptr)) return fail(TL_ERR_ARG, "pass both scales or neither");
+    if (M <= kSmallMaxM) return fail(TL_ERR_UNSUPPORTED, "fused gate/up needs M > %d; use two tl_spmm calls below that", kSmallMaxM);
+    KernelArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.w0 = weight_ptrs(gate_header, gate_blob_dev, gate_scale);
+    a.w1 = weight_ptrs(up_header, up_blob_dev, up_scale);
+    a.X = X; a.Y = H;
+    a.ldx = ldx; a.ldy = ldh;
+    a.NB = (int)gate_header->n_blocks; a.units = (int)gate_header->code_units; a.planes = (int)gate_header->code_planes;
+    a.M = (int)M; a.N = (int)gate_header->columns; a.K = (int)gate_header->inners; a.T = (int)gate_header->n_tiles;
+    a.tile_rows = (int)gate_header->tile_rows;
+    a.x_f16 = x_dtype == TL_F16; a.x_kmajor = x_layout == TL_X_K_MAJOR; a.y_f16 = h_dtype == TL_F16; a.scale_f16 = scale_dtype == TL_F16;
+    a.one = 1.0f;
+    if (int rc = launch_matrix_rows(a, x_dtype, workspace, workspace_bytes, true, static_cast<hipStream_t>(stream))) return rc;
+    return finish_launch();
+}
+
+
 // Scratch of tl_spmm_noalloc: device memory that belongs to the library's code object, one copy per GPU,
 // there from the moment the library is loaded on a device until the process ends.
-constexpr int64_t kStaticScratchBytes = 32ll << 20;
+constexpr int64_t kStaticScratchBytes = 48ll << 20;  // (fp32 rows of 32 MiB are 48 MiB in three bf16 parts)
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 namespace {
@@ -249,9 +282,8 @@ extern "C" int tl_spmm_noalloc(const tl_layout_header* header, const void* blob_
     if (int rc = check_header(header)) return rc;
     if (int rc = check_dtype(x_dtype, "x")) return rc;
     if (M <= 0) return fail(TL_ERR_SHAPE, "M=%lld must be positive", (long long)M);
-    // what the kernels stage in the scratch: the K-major image of the activations (none for 4 rows and fewer).
-    // Room for partial sums is not offered, so the row kernel gives every output tile a workgroup of its own.
-    const int64_t need = M <= kSmallMaxM ? small_kmajor_bytes(header, M, x_dtype) : rows_relayout_bytes(header->inners, M, x_dtype);
+    // what the kernels stage in the scratch: the image of the activations (none for 4 rows and fewer)
+    const int64_t need = M <= kSmallMaxM ? small_kmajor_bytes(header, M, x_dtype) : matrix_image_bytes(header->inners, M, x_dtype);
     if (need > kStaticScratchBytes)
         return fail(TL_ERR_SIZE, "M=%lld rows of K=%u need %lld bytes of scratch; tl_spmm_noalloc has %lld (use tl_spmm with a workspace)",
                     (long long)M, header->inners, (long long)need, (long long)kStaticScratchBytes);

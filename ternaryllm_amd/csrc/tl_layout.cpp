@@ -55,17 +55,25 @@ constexpr int64_t kStreamSpareBytes = 1024;
 static_assert(kStreamSpareBytes >= kSparePrefetchDwords * 4, "the spare must cover the index prefetch");
 
 struct Sections {
-    int64_t off_chunkstart, off_stream, total;
+    int64_t off_chunkstart, off_stream, off_codes, total;
 };
 
-Sections place_sections(const Geometry& g, int64_t stream_bytes)
+// Bytes of the two-bit codes of `planes` ternary matrices.
+int64_t code_bytes(int n_blocks, int inners, int planes)
+{
+    return (int64_t)n_blocks * planes * ceil_div(inners, TL_CODE_UNIT_ROWS) * TL_CODE_UNIT_BYTES;
+}
+
+Sections place_sections(const Geometry& g, int inners, int64_t stream_bytes, int planes)
 {
     Sections s;
     s.off_chunkstart = 256;
     s.off_stream = s.off_chunkstart + round_up(((int64_t)g.n_tiles * g.n_blocks + 1) * 4, 256);
-    // Spare bytes behind the stream: the row kernel requests a wave's first kSparePrefetchDwords index
+    // Spare bytes behind the stream: a kernel may request a wave's first kSparePrefetchDwords index
     // dwords from wherever its piece starts, also when the piece is the stream's last and shorter.
-    s.total = s.off_stream + round_up(stream_bytes, 256) + kStreamSpareBytes;
+    s.off_codes = s.off_stream + round_up(stream_bytes, 256) + kStreamSpareBytes;
+    s.total = s.off_codes + code_bytes(g.n_blocks, inners, planes);
+    if (planes == 0) s.off_codes = 0;
     return s;
 }
 
@@ -306,8 +314,8 @@ uint64_t content_checksum(const uint32_t* chunkstart, size_t n_table, const uint
     return h;
 }
 
-// Threads for the row-ordering pass of one tl_layout_build call: TL_PACK_THREADS if set, else the machine's hardware
-// threads up to 8, shared among the calls that are in that pass at the moment (callers that pack many weights on
+// Threads for a pass of one tl_layout_build call: TL_PACK_THREADS if set, else the machine's hardware
+// threads up to 8, shared among the calls that are in such a pass at the moment (callers that pack many weights on
 // threads of their own then get one each).  The caller gives its count back when its pass is over.
 std::atomic<int> g_builds_running{0};
 
@@ -318,6 +326,71 @@ int pack_workers(int n_blocks)
     if (cap <= 0) cap = (int)std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
     const int running = g_builds_running.fetch_add(1) + 1;
     return std::max(1, std::min(cap / running, n_blocks));
+}
+
+// work(block) for every block, shared out among pack_workers() threads.
+template <typename Work>
+void for_each_block(int n_blocks, const Work& work)
+{
+    const int workers = pack_workers(n_blocks);
+    std::atomic<int> next{0};
+    auto take = [&]() {
+        for (int nb = next.fetch_add(1); nb < n_blocks; nb = next.fetch_add(1)) work(nb);
+    };
+    std::vector<std::thread> pool;
+    for (int i = 1; i < workers; ++i) pool.emplace_back(take);
+    take();
+    for (auto& th : pool) th.join();
+    g_builds_running.fetch_sub(1);
+}
+
+// The codes of column `y`, whose entry in row k is value[k], into their units (zero before the call).
+void put_codes(uint8_t* codes, int y, int inners, int planes, const int16_t* value)
+{
+    const int units = (int)ceil_div(inners, TL_CODE_UNIT_ROWS);
+    for (int k = 0; k < inners; ++k) {
+        const int v = value[k];
+        if (v == 0) continue;
+        const int r = k % TL_CODE_UNIT_ROWS, lane = y % kBlock + 16 * ((r % 32) / 8);
+        const int pair = ((r / 32) & 1) * 4 + (r % 8) / 2, half = r & 1;
+        const uint32_t code = (v < 0 ? 3u : 1u) << (14 - 2 * pair + 16 * half);
+        for (int p = 0; p < std::abs(v); ++p) {
+            uint8_t* unit = codes + (((size_t)(y / kBlock) * planes + p) * units + k / TL_CODE_UNIT_ROWS) * TL_CODE_UNIT_BYTES;
+            reinterpret_cast<uint32_t*>(unit + lane * 16)[r / 64] |= code;
+        }
+    }
+}
+
+// Column y of the matrix that the index stream encodes, an entry being its +1 minus its -1 mentions.
+void column_values(const uint32_t* chunkstart, const uint32_t* stream, int n_tiles, int tile_rows, int y, int16_t* value)
+{
+    for (int t = 0; t < n_tiles; ++t) {
+        const uint32_t* chunk = stream + chunkstart[(size_t)(y / kBlock) * n_tiles + t];
+        const uint32_t d = chunk[y % kBlock], p = d & 0xff, n = (d >> 8) & 0xff;
+        const uint8_t* run = reinterpret_cast<const uint8_t*>(chunk + (d >> 16));
+        int16_t* v = value + (size_t)t * tile_rows;
+        for (uint32_t i = 0; i < p; ++i) ++v[run[i]];
+        run += ((p + 3) / 4) * 4;
+        for (uint32_t i = 0; i < n; ++i) --v[run[i]];
+    }
+}
+
+// The largest |entry| of the matrix that tiled-CSC row lists encode: 1 unless a column names a row more than once.
+int largest_entry(const int32_t* neg_row, const int32_t* neg_off, const int32_t* pos_row, const int32_t* pos_off, int columns, int inners, int tile_k)
+{
+    const int Ta = (int)ceil_div(inners, tile_k);
+    std::vector<int16_t> value((size_t)Ta * tile_k, 0);
+    int most = 1;
+    for (int y = 0; y < columns; ++y)
+        for (int t = 0; t < Ta; ++t) {
+            int16_t* v = value.data() + (size_t)t * tile_k;
+            const size_t c = ((size_t)y * Ta + t) * 2;
+            for (int32_t i = pos_off[c]; i < pos_off[c + 1]; ++i) ++v[pos_row[i]];
+            for (int32_t i = neg_off[c]; i < neg_off[c + 1]; ++i) --v[neg_row[i]];
+            for (int32_t i = pos_off[c]; i < pos_off[c + 1]; ++i) { most = std::max(most, std::abs((int)v[pos_row[i]])); v[pos_row[i]] = 0; }
+            for (int32_t i = neg_off[c]; i < neg_off[c + 1]; ++i) { most = std::max(most, std::abs((int)v[neg_row[i]])); v[neg_row[i]] = 0; }
+        }
+    return most;
 }
 
 // Last "end" entry of a tiled-CSC offset array = number of stored rows of that sign.
@@ -337,7 +410,7 @@ extern "C" int tl_layout_size(const int32_t* neg_off_tiled, const int32_t* pos_o
     Geometry g;
     if (int rc = pick_geometry(columns, inners, tile_rows, &g)) return rc;
     const int64_t nnz = stream_length(neg_off_tiled, columns, inners, tile_k) + stream_length(pos_off_tiled, columns, inners, tile_k);
-    *blob_bytes = place_sections(g, stream_upper_bound(nnz, columns, g)).total;
+    *blob_bytes = place_sections(g, inners, stream_upper_bound(nnz, columns, g), 1).total;
     return TL_OK;
 }
 
@@ -364,7 +437,7 @@ extern "C" int tl_layout_build(const int32_t* neg_row, const int32_t* neg_off_ti
     const int T = g.n_tiles, NB = g.n_blocks;
     const int Ta = (int)ceil_div(inners, tile_k);
     const int64_t reserve = stream_upper_bound(n_pos + n_neg, columns, g);
-    const Sections s = place_sections(g, reserve);
+    const Sections s = place_sections(g, inners, reserve, 0);
     std::memset(blob, 0, (size_t)blob_bytes);
     uint8_t* base = static_cast<uint8_t*>(blob);
     uint32_t* chunkstart = reinterpret_cast<uint32_t*>(base + s.off_chunkstart);
@@ -452,24 +525,35 @@ extern "C" int tl_layout_build(const int32_t* neg_row, const int32_t* neg_off_ti
             }
         }
     };
-    {
-        const int workers = pack_workers(NB);
-        std::atomic<int> next{0};
-        auto work = [&]() {
-            for (int nb = next.fetch_add(1); nb < NB; nb = next.fetch_add(1)) order_block(nb);
-        };
-        std::vector<std::thread> pool;
-        for (int i = 1; i < workers; ++i) pool.emplace_back(work);
-        work();
-        for (auto& th : pool) th.join();
-        g_builds_running.fetch_sub(1);
+    for_each_block(NB, order_block);
+
+    // Pass 4: the codes, behind the stream as it has come out (its reserve was an upper bound), blocks shared out among
+    // threads again.  Arrays that name a row more than once need a plane for each mention.
+    const int most = largest_entry(neg_row, neg_off_tiled, pos_row, pos_off_tiled, columns, inners, tile_k);
+    int planes = most;
+    Sections fin = place_sections(g, inners, (int64_t)dwords * 4, planes);
+    if (fin.total > blob_bytes) {
+        planes = 0;
+        fin = place_sections(g, inners, (int64_t)dwords * 4, 0);
+    } else {
+        for_each_block(NB, [&](int nb) {
+            std::vector<int16_t> value((size_t)T * g.tile_rows);
+            for (int y = nb * kBlock; y < std::min(columns, (nb + 1) * kBlock); ++y) {
+                std::fill(value.begin(), value.end(), (int16_t)0);
+                column_values(chunkstart, stream, T, g.tile_rows, y, value.data());
+                put_codes(base + fin.off_codes, y, inners, planes, value.data());
+            }
+        });
     }
 
     tl_layout_header h;
     std::memset(&h, 0, sizeof(h));
     static_assert(sizeof(tl_layout_header) == 256, "header must stay 256 bytes");
     h.magic = TL_LAYOUT_MAGIC;
-    h.version = TL_LAYOUT_VERSION;
+    h.version = planes ? TL_LAYOUT_VERSION : TL_LAYOUT_VERSION_NO_CODES;
+    h.off_codes = (uint64_t)fin.off_codes;
+    h.code_units = planes ? (uint32_t)ceil_div(inners, TL_CODE_UNIT_ROWS) : 0;
+    h.code_planes = (uint32_t)planes;
     h.inners = (uint32_t)inners;
     h.columns = (uint32_t)columns;
     h.tile_rows = (uint32_t)g.tile_rows;
@@ -482,7 +566,7 @@ extern "C" int tl_layout_build(const int32_t* neg_row, const int32_t* neg_off_ti
     h.off_stream = (uint64_t)s.off_stream;
     h.stream_bytes = dwords * 4;
     // The blob handed in is sized by an upper bound; what the format occupies is smaller.
-    h.total_bytes = (uint64_t)place_sections(g, (int64_t)dwords * 4).total;
+    h.total_bytes = (uint64_t)fin.total;
     h.max_run_dwords = run_max;
     h.mean_run_dwords_x16 = (uint32_t)ceil_div((int64_t)run_sum * 16, (int64_t)columns * T);
     h.checksum = content_checksum(chunkstart, (size_t)NB * T + 1, stream, (size_t)dwords);
@@ -557,6 +641,8 @@ extern "C" int tl_layout_from_mcsc(const void* merged_row, int index_width, int6
         }
     int64_t need = 0;
     if (int rc = tl_layout_size(neg_off.data(), pos_off.data(), columns, inners, tile_k, tile_rows, &need)) return rc;
+    const int planes = largest_entry(neg_row.data(), neg_off.data(), pos_row.data(), pos_off.data(), columns, inners, tile_k);
+    need += code_bytes((int)ceil_div(columns, kBlock), inners, planes - 1);
     if (!blob) {
         *blob_bytes = need;
         return TL_OK;
@@ -574,13 +660,16 @@ extern "C" int tl_layout_validate(const void* blob, int64_t blob_bytes)
     if (blob_bytes < (int64_t)sizeof(tl_layout_header)) return fail(TL_ERR_FORMAT, "blob shorter than its header");
     tl_layout_header h;
     std::memcpy(&h, blob, sizeof(h));
-    if (h.magic != TL_LAYOUT_MAGIC || h.version != TL_LAYOUT_VERSION) return fail(TL_ERR_FORMAT, "bad magic/version %08x/%u", h.magic, h.version);
+    if (h.magic != TL_LAYOUT_MAGIC || (h.version != TL_LAYOUT_VERSION && h.version != TL_LAYOUT_VERSION_NO_CODES)) return fail(TL_ERR_FORMAT, "bad magic/version %08x/%u", h.magic, h.version);
     if (h.tile_rows == 0 || h.tile_rows > (uint32_t)kMaxTileRows || h.columns == 0 || h.inners == 0 ||
         h.n_tiles != (uint32_t)ceil_div(h.inners, h.tile_rows) || h.n_blocks != (uint32_t)ceil_div(h.columns, kBlock))
         return fail(TL_ERR_FORMAT, "inconsistent geometry K=%u N=%u rows=%u tiles=%u blocks=%u", h.inners, h.columns,
                     h.tile_rows, h.n_tiles, h.n_blocks);
     Geometry g{(int)h.tile_rows, (int)h.n_tiles, (int)h.n_blocks};
-    const Sections s = place_sections(g, (int64_t)h.stream_bytes);
+    const Sections s = place_sections(g, (int)h.inners, (int64_t)h.stream_bytes, (int)h.code_planes);
+    const uint32_t units = h.code_planes ? (uint32_t)ceil_div(h.inners, TL_CODE_UNIT_ROWS) : 0;
+    if (h.code_planes > 255 || h.code_units != units || (h.code_planes != 0) != (h.version == TL_LAYOUT_VERSION) || h.off_codes != (uint64_t)s.off_codes)
+        return fail(TL_ERR_FORMAT, "the code section does not match the header");
     if (h.off_chunkstart != (uint64_t)s.off_chunkstart || h.off_stream != (uint64_t)s.off_stream ||
         h.total_bytes != (uint64_t)s.total || h.total_bytes > (uint64_t)blob_bytes || (h.stream_bytes & 15))
         return fail(TL_ERR_FORMAT, "section table does not match the geometry");
@@ -635,6 +724,63 @@ extern "C" int tl_layout_validate(const void* blob, int64_t blob_bytes)
         return fail(TL_ERR_FORMAT, "header totals do not match the streams");
     if (content_checksum(chunkstart, (size_t)T * NB + 1, stream, (size_t)expect_start) != h.checksum)
         return fail(TL_ERR_FORMAT, "checksum of the chunk table and the stream does not match the header");
+    if (h.code_planes) {  // what the codes must be follows from the stream
+        const size_t block_bytes = (size_t)h.code_planes * units * TL_CODE_UNIT_BYTES;
+        std::atomic<int> bad{-1};
+        for_each_block((int)NB, [&](int nb) {
+            std::vector<int16_t> value((size_t)T * h.tile_rows);
+            std::vector<uint32_t> want(block_bytes / 4, 0);
+            for (int y = nb * kBlock; y < std::min((int)h.columns, (nb + 1) * kBlock); ++y) {
+                std::fill(value.begin(), value.end(), (int16_t)0);
+                column_values(chunkstart, stream, (int)T, (int)h.tile_rows, y, value.data());
+                for (int16_t v : value)
+                    if (std::abs((int)v) > (int)h.code_planes) { bad = nb; return; }
+                put_codes(reinterpret_cast<uint8_t*>(want.data()), y % kBlock, (int)h.inners, (int)h.code_planes, value.data());
+            }
+            if (std::memcmp(want.data(), base + h.off_codes + (size_t)nb * block_bytes, block_bytes) != 0) bad = nb;
+        });
+        if (bad >= 0) return fail(TL_ERR_FORMAT, "block %d: codes and index stream are not the same matrix", bad.load());
+    }
+    return TL_OK;
+}
+
+extern "C" int tl_layout_add_codes(const void* blob, int64_t blob_bytes, void* out, int64_t* out_bytes)
+{
+    if (!out_bytes) return fail(TL_ERR_ARG, "out_bytes is null");
+    if (int rc = tl_layout_validate(blob, blob_bytes)) return rc;
+    tl_layout_header h;
+    std::memcpy(&h, blob, sizeof(h));
+    const uint8_t* from = static_cast<const uint8_t*>(blob);
+    const uint32_t* chunkstart = reinterpret_cast<const uint32_t*>(from + h.off_chunkstart);
+    const uint32_t* stream = reinterpret_cast<const uint32_t*>(from + h.off_stream);
+    std::vector<int16_t> value((size_t)h.n_tiles * h.tile_rows);
+    int planes = 1;
+    for (int y = 0; y < (int)h.columns; ++y) {
+        std::fill(value.begin(), value.end(), (int16_t)0);
+        column_values(chunkstart, stream, (int)h.n_tiles, (int)h.tile_rows, y, value.data());
+        for (int16_t v : value) planes = std::max(planes, std::abs((int)v));
+    }
+    const Geometry g{(int)h.tile_rows, (int)h.n_tiles, (int)h.n_blocks};
+    const Sections s = place_sections(g, (int)h.inners, (int64_t)h.stream_bytes, planes);
+    if (!out) {
+        *out_bytes = s.total;
+        return TL_OK;
+    }
+    if (*out_bytes < s.total) return fail(TL_ERR_SIZE, "out has %lld bytes, %lld needed", (long long)*out_bytes, (long long)s.total);
+    uint8_t* to = static_cast<uint8_t*>(out);
+    std::memset(to, 0, (size_t)s.total);
+    std::memcpy(to, from, (size_t)(h.off_stream + h.stream_bytes));
+    for (int y = 0; y < (int)h.columns; ++y) {
+        std::fill(value.begin(), value.end(), (int16_t)0);
+        column_values(chunkstart, stream, (int)h.n_tiles, (int)h.tile_rows, y, value.data());
+        put_codes(to + s.off_codes, y, (int)h.inners, planes, value.data());
+    }
+    h.version = TL_LAYOUT_VERSION;
+    h.off_codes = (uint64_t)s.off_codes;
+    h.code_units = (uint32_t)ceil_div(h.inners, TL_CODE_UNIT_ROWS);
+    h.code_planes = (uint32_t)planes;
+    h.total_bytes = (uint64_t)s.total;
+    std::memcpy(to, &h, sizeof(h));
     return TL_OK;
 }
 

@@ -102,6 +102,14 @@ class PackedWeight:
         if self.header.total_bytes > self.blob.size:
             raise ValueError("blob is truncated")
         self.blob = self.blob[: self.header.total_bytes]
+        if self.header.off_codes == 0:  # packed before the format carried them: made here, once
+            size = ctypes.c_int64(0)
+            L = _lib.lib()
+            _lib.check(L.tl_layout_add_codes(self.blob.ctypes.data, self.blob.size, None, ctypes.byref(size)))
+            whole = np.zeros(size.value, np.uint8)
+            _lib.check(L.tl_layout_add_codes(self.blob.ctypes.data, self.blob.size, whole.ctypes.data, ctypes.byref(size)))
+            self.blob = whole
+            self.header = _lib.LayoutHeader.from_buffer_copy(whole[:256].tobytes())
 
     @property
     def inners(self):

@@ -1,0 +1,114 @@
+"""The matrix-core kernels at the sizes where they can go wrong: edges of their tiles, stages and code units, weights
+whose entries are not ternary, activations that are not finite, blobs without codes."""
+import numpy as np
+import pytest
+import torch
+
+from tests.util import activations, ternary_weight
+
+pytestmark = pytest.mark.gpu
+
+
+def _device(w, cuda):
+    from ternaryllm_amd import ops
+    from ternaryllm_amd.packing import PackedWeight
+    return ops.DeviceWeight(PackedWeight.from_dense(w), cuda)
+
+
+# rows: the 128-row tile and the 16-row fragment; K: the 64-row stage, the four stages asked for ahead, the 256-row unit,
+# rows that are not whole 16-byte pieces; N: the 16-column block, a wave's 32 and a tile's 128 columns
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M,K,N", [(49, 1, 1), (49, 8, 16), (127, 64, 31), (128, 72, 128), (129, 192, 129), (145, 256, 113), (64, 264, 144),
+                                   (300, 320, 257), (640, 520, 300), (257, 1100, 1000), (129, 1280, 700)])
+def test_many_rows_at_the_edges(cuda, oracle, M, K, N, dtype):
+    """Integer activations: every sum is exact, whatever its order."""
+    from ternaryllm_amd import ops
+    w = ternary_weight(K, N, 0.6, M + K + N)
+    dw = _device(w, cuda)
+    x = activations(M, K, M, dtype, integer=True)
+    ref = oracle.fast_product(x.double().numpy(), w)
+    for name, xin, layout in (("rows", x.to(cuda), 0), ("k-major", x.t().contiguous().to(cuda), 1)):
+        print(f"case M={M} K={K} N={N} {dtype} {name}", flush=True)
+        y = ops.spmm(dw, xin, out_dtype=torch.float32, x_layout=layout)
+        assert np.array_equal(y.cpu().numpy().astype(np.float64), ref), name
+    if dtype == torch.float32:  # all 24 bits of an fp32 value (its three bf16 parts) pass through a column with one entry
+        rng = np.random.default_rng(M)
+        rows, one = rng.integers(0, K, N), np.zeros((K, N), np.int32)
+        one[rows, np.arange(N)] = rng.choice([-1, 1], N)
+        x = activations(M, K, M + 1, dtype)
+        y = ops.spmm(_device(one, cuda), x.to(cuda)).cpu().numpy()
+        assert np.array_equal(y, x.numpy()[:, rows] * one[rows, np.arange(N)].astype(np.float32))
+
+
+@pytest.mark.parametrize("M", [1, 5, 16, 40, 64, 200])
+def test_entries_beyond_one(cuda, M):
+    """Arrays that name a row several times make entries up to 3: the codes hold a plane for each mention."""
+    from ternaryllm_amd import ops
+    from ternaryllm_amd.packing import PackedWeight
+    rng = np.random.default_rng(5)
+    for K, N in ((100, 20), (600, 40)):
+        w = rng.integers(-3, 4, (K, N)) * (rng.random((K, N)) < 0.3)
+        neg, pos, neg_off, pos_off = [], [], np.zeros((N, 1, 2), np.int32), np.zeros((N, 1, 2), np.int32)
+        for y in range(N):
+            for rows, off, sign in ((neg, neg_off, -1), (pos, pos_off, 1)):
+                off[y, 0, 0] = len(rows)
+                for k in range(K):
+                    rows += [k] * max(0, sign * int(w[k, y]))
+                off[y, 0, 1] = len(rows)
+        pw = PackedWeight.from_tiled_csc(np.array(neg, np.int32), neg_off.reshape(-1), np.array(pos, np.int32), pos_off.reshape(-1), N, K, K)
+        pw.validate()
+        assert pw.header.code_planes == 3 and np.array_equal(pw.to_dense(), w)
+        x = activations(M, K, 6, torch.float32, integer=True)
+        print(f"case M={M} K={K}", flush=True)
+        y = ops.spmm(ops.DeviceWeight(pw, cuda), x.to(cuda))
+        assert np.array_equal(y.cpu().numpy().astype(np.float64), x.double().numpy() @ w)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M", [1, 3, 16, 33, 130])
+def test_activations_that_are_not_finite(cuda, M, dtype):
+    """A column that does not name a row is not touched by what that row holds, infinities and NaN included."""
+    from ternaryllm_amd import ops
+    K, N = 300, 50
+    w = ternary_weight(K, N, 0.9, 8)
+    x = activations(M, K, 9, dtype, integer=True)
+    x[0, 7], x[M // 2, 100], x[M - 1, 299] = float("inf"), float("-inf"), float("nan")
+    want = np.zeros((M, N))
+    xn = x.double().numpy()
+    for n in range(N):
+        rows = np.nonzero(w[:, n])[0]
+        want[:, n] = (xn[:, rows] * w[rows, n]).sum(1)
+    print(f"case M={M} {dtype}", flush=True)
+    dw = _device(w, cuda)
+    got = ops.spmm(dw, x.to(cuda), out_dtype=torch.float32).double().cpu().numpy()
+    assert np.array_equal(got, want, equal_nan=True)
+    if M > 48:
+        pairs = ops.spmm_gated(dw, x.to(cuda)).float()
+        assert torch.equal(torch.nan_to_num(pairs), torch.nan_to_num(ops.silu_mul(ops.spmm(dw, x.to(cuda)), pairs=True).float()))
+        both = ops.mlp_gate_up(dw, dw, x.to(cuda), out_dtype=torch.float32).double().cpu()
+        g = torch.from_numpy(want)
+        assert torch.allclose(both, torch.nn.functional.silu(g) * g, rtol=1e-4, atol=1e-4, equal_nan=True)
+
+
+def test_a_blob_without_codes(cuda, oracle):
+    """What an older version packed: the packed-weight object brings it up to date, and a device blob that was not is
+    multiplied by the general kernel."""
+    import ctypes
+    from ternaryllm_amd import _lib, ops
+    from ternaryllm_amd.packing import PackedWeight
+    K, N = 520, 96
+    w = ternary_weight(K, N, 0.7, 3)
+    new = PackedWeight.from_dense(w)
+    old = new.blob[:new.header.off_codes].copy()
+    h = _lib.LayoutHeader.from_buffer_copy(old[:256].tobytes())
+    h.version, h.off_codes, h.code_units, h.code_planes, h.total_bytes = 5, 0, 0, 0, old.size
+    old[:256] = np.frombuffer(bytes(h), np.uint8)
+    _lib.check(_lib.lib().tl_layout_validate(old.ctypes.data, old.size))
+    assert np.array_equal(PackedWeight(old).blob, new.blob)
+    dev = ops.DeviceWeight.__new__(ops.DeviceWeight)
+    dev.header, dev.blob = h, torch.from_numpy(old).to(cuda)
+    for M in (1, 6, 60):
+        x = activations(M, K, M, torch.float16, integer=True)
+        print(f"case M={M}", flush=True)
+        y = ops.spmm(dev, x.to(cuda), out_dtype=torch.float32)
+        assert np.array_equal(y.cpu().numpy().astype(np.float64), oracle.fast_product(x.double().numpy(), w))
