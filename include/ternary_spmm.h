@@ -317,6 +317,37 @@ int tl_rope_cache_update(const void* qkv, int dtype, int64_t batch, int heads, i
                          const void* cos_table, const void* sin_table, const int64_t* pos_dev,
                          void* q_out, void* k_cache, void* v_cache, int64_t max_seq, void* stream);
 
+/* cos and sin tables of the rotate-half rotary embedding, [count][head_dim] of `dtype` each, for the positions in
+ * `positions` (device, int64) or, with NULL, first, first + 1, ...: the angle of dimension d is
+ * position * theta^(-2 i / head_dim), i = d modulo head_dim / 2, in fp32 (TernaryLLM/TernaryAttn.py:91-93). */
+int tl_rope_table(const int64_t* positions, int64_t first, int64_t count, int head_dim, float theta, int dtype,
+                  void* cos_table, void* sin_table, void* stream);
+
+/* Rotates the keys of whole prompts and puts them where they are kept (TernaryLLM/TernaryAttn.py:93-98); with
+ * v and v_out the values are copied beside them.
+ *   k, v       device; token s of batch row b at element b * in_batch + s * in_seq, its heads side by side
+ *   tables     [seq][head_dim], those of batch row b at element b * table_batch (0: the same for all)
+ *   k_out, v_out  element (b, s, h, 0) at b * out_batch + s * out_seq + h * out_head
+ * head_dim a multiple of 16; addresses and strides whole 16-byte pieces. */
+int tl_rope_rows(const void* k, const void* v, int dtype, int64_t batch, int64_t seq, int heads, int head_dim,
+                 int64_t in_batch, int64_t in_seq, const void* cos_table, const void* sin_table, int64_t table_batch,
+                 void* k_out, void* v_out, int64_t out_batch, int64_t out_seq, int64_t out_head, void* stream);
+
+/* Elements between batch rows, tokens and heads of each operand of tl_prefill_attention, and between the rotary
+ * tables of two batch rows. */
+typedef struct tl_attention_strides {
+    int64_t q_batch, q_seq, q_head, k_batch, k_seq, k_head, v_batch, v_seq, v_head, table_batch;
+} tl_attention_strides;
+
+/* Causal softmax attention of q_len queries over kv_len >= q_len keys, query i seeing keys 0 .. i + kv_len - q_len
+ * (TernaryLLM/TernaryAttn.py:100-113 with the causal mask): fp16, head_dim 64 or 128, scores and softmax in fp32,
+ * probabilities rounded to fp16 for the product with the values.  Query head h reads key head h / (heads / kv_heads).
+ * With cos_table and sin_table ([q_len][head_dim]) the queries are rotated on the way in; the keys are taken as they
+ * are.  out [batch][q_len][heads * head_dim].  Addresses and strides whole 16-byte pieces. */
+int tl_prefill_attention(const void* q, const void* k, const void* v, const void* cos_table, const void* sin_table, int dtype,
+                         int64_t batch, int heads, int kv_heads, int head_dim, int64_t q_len, int64_t kv_len,
+                         const tl_attention_strides* strides, void* out, void* stream);
+
 /* Softmax attention of one query per (batch row, head) over cache rows [0, *pos_dev] --
  * the reference's eager matmul / softmax / matmul for q_len == 1
  * (TernaryLLM/TernaryAttn.py:100-113), scores and softmax in fp32.

@@ -89,6 +89,9 @@ SIGNATURES = {
     "tl_read_probe_workgroups": (_INT, []),
     "tl_stream_read_probe": (_INT, [_VP, _I64, _VP, _VP]),
     "tl_rope_cache_update": (_INT, [_VP, _INT, _I64, _INT, _INT, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _VP]),
+    "tl_rope_table": (_INT, [_VP, _I64, _I64, _INT, ctypes.c_float, _INT, _VP, _VP, _VP]),
+    "tl_rope_rows": (_INT, [_VP, _VP, _INT, _I64, _I64, _INT, _INT, _I64, _I64, _VP, _VP, _I64, _VP, _VP, _I64, _I64, _I64, _VP]),
+    "tl_prefill_attention": (_INT, [_VP, _VP, _VP, _VP, _VP, _INT, _I64, _INT, _INT, _INT, _I64, _I64, _I64P, _VP, _VP]),
     "tl_decode_attention": (_INT, [_VP, _VP, _VP, _INT, _I64, _INT, _INT, _I64, _VP, _VP, _I64, _VP]),
     "tl_decode_attention_split": (_INT, [_VP, _VP, _VP, _INT, _I64, _INT, _INT, _I64, _VP, _VP, _I64, _INT, _VP, _I64, _VP]),
     "tl_greedy_advance": (_INT, [_VP, _INT, _I64, _INT, _VP, _VP, _I64, _VP, _VP]),

@@ -117,11 +117,14 @@ class LlamaTernaryAttention(nn.Module):
         if past_key_value is None:
             past_key_value = kwargs.pop("past_key_values", None)
         bsz, q_len, _ = hidden_states.shape
+        dropout = self.attention_dropout if self.training else 0.0
+        qkv = None
         if self.fused_qkv and hidden_states.is_cuda:
             weight, scale = self._qkv_weight(hidden_states.device)
             nq, nkv = self.q_proj.out_features, self.k_proj.out_features
             qkv = ops.spmm(weight, hidden_states.reshape(bsz * q_len, -1), scale).view(bsz, q_len, nq + 2 * nkv)
-            q, k, v = (t.reshape(bsz, q_len, -1, self.head_dim).transpose(1, 2) for t in qkv.split((nq, nkv, nkv), dim=-1))
+            heads = [t.view(bsz, q_len, -1, self.head_dim) for t in qkv.split((nq, nkv, nkv), dim=-1)]
+            q, k, v = (t.transpose(1, 2) for t in heads)
         else:
             q = self.q_proj(hidden_states).view(bsz, q_len, -1, self.head_dim).transpose(1, 2)
             k = self.k_proj(hidden_states).view(bsz, q_len, -1, self.head_dim).transpose(1, 2)
@@ -137,8 +140,21 @@ class LlamaTernaryAttention(nn.Module):
                 past_len = int(past_key_value.get_seq_length(self.layer_idx))
             else:
                 past_len = 0
-        cos, sin = self._rotary(position_ids, position_embeddings, q_len, past_len, q.dtype, q.device)
-        q, k = apply_rope(q, cos, sin), apply_rope(k, cos, sin)
+        # causal fp16 attention without a mask: the library's kernels rotate and attend
+        native = (qkv is not None and qkv.dtype == torch.float16 and qkv.numel() > 0 and self.head_dim in (64, 128) and attention_mask is None and
+                  not output_attentions and dropout == 0.0 and (self.is_causal or q_len == 1))
+        if native and position_ids is None and position_embeddings is None:
+            cos, sin = ops.rope_table(past_len, q_len, self.head_dim, self.rope_theta, q.dtype, q.device)
+        else:
+            cos, sin = self._rotary(position_ids, position_embeddings, q_len, past_len, q.dtype, q.device)
+        native = native and all(t.dim() in (2, 3) and t.device == q.device and t.shape == cos.shape and t.shape[-2:] == (q_len, self.head_dim) and
+                                (t.dim() == 2 or t.shape[0] in (1, bsz)) and not t.requires_grad for t in (cos, sin))
+        if native:
+            tables = tuple(t if t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format) for t in (cos, sin))
+            k = torch.empty((bsz, q_len, k.shape[1], self.head_dim), dtype=k.dtype, device=k.device).transpose(1, 2)
+            ops.rope_rows(heads[1], tables, k)
+        else:
+            q, k = apply_rope(q, cos, sin), apply_rope(k, cos, sin)
         if is_tuple:
             k = torch.cat([past_key_value[0], k], dim=2)
             v = torch.cat([past_key_value[1], v], dim=2)
@@ -147,6 +163,12 @@ class LlamaTernaryAttention(nn.Module):
             k, v = past_key_value.update(k, v, self.layer_idx, {"sin": sin, "cos": cos, "cache_position": cache_position})
         elif use_cache:
             past_key_value = (k, v)
+        if native:
+            # (a cache may give back keys of another type, shape or layout)
+            if k.dtype == v.dtype == q.dtype and k.device == v.device == q.device and k.shape == v.shape and k.dim() == 4 and \
+                    k.shape[:2] == (bsz, self.num_key_value_heads) and k.shape[3] == self.head_dim and k.shape[2] >= q_len and ops.in_pieces(k, v):
+                return self.o_proj(ops.prefill_attention(heads[0], k, v, tables)), None, past_key_value
+            q = apply_rope(q, cos, sin)
         kv_len = k.shape[2]
         if self.num_key_value_groups > 1:
             k = k.repeat_interleave(self.num_key_value_groups, dim=1)
@@ -160,7 +182,6 @@ class LlamaTernaryAttention(nn.Module):
             mask = torch.ones((q_len, kv_len), dtype=torch.bool, device=q.device).tril(kv_len - q_len)
         else:
             mask = None
-        dropout = self.attention_dropout if self.training else 0.0
         if output_attentions:
             # the reference's eager form (TernaryAttn.py:101-110): scores, fp32 softmax, weights returned
             scores = torch.matmul(q, k.transpose(2, 3)) / math.sqrt(self.head_dim)

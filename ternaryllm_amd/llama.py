@@ -5,9 +5,9 @@ It stands where the reference patches a Hugging Face Llama with its ternary modu
 (ternaryLLM_GPU/TernaryLLM/TernaryLlama.py:69-75) and drives it with `generate`
 (ternaryLLM_GPU/benchmark_ternary_llama.py:81-105); the CPU twin of the same structure is
 ternaryLLM_CPU/src/LlamaModel.hpp:457-527.  Weights are random ternary matrices, drawn as the
-reference draws them; every product runs in libternary_spmm.so.  A prefill pass uses torch operators
-for normalisation, rotary embedding and attention; a single-token step uses the library's kernels
-for them (rotary + cache update, attention over the cache, residual add + RMSNorm, SiLU gate).
+reference draws them; every product runs in libternary_spmm.so, and so does what stands between the
+products (rotary + cache update, attention over the cache, residual add + RMSNorm, SiLU gate), in a
+prefill pass as in a single-token step, for the types and head sizes that the kernels are built for.
 
 The decode step has static shapes (the cache has its full length, a mask hides what is not
 written yet, position and token live in device tensors), so it can be captured once in a HIP graph
@@ -121,6 +121,9 @@ class TernaryLlamaDecoder(nn.Module):
         self._graph = None
         # single-token steps use the library's rotary / cache / attention kernels; False keeps them on torch operators
         self.native_decode = config.head_dim in (64, 128, 256) and self.max_seq_len * 4 <= 120 * 1024
+        # a pass over prompts uses the library's norm, rotary and attention kernels; False keeps them on torch operators
+        self.native_prefill = (dev.type == "cuda" and dtype == torch.float16 and config.head_dim in (64, 128) and config.num_hidden_layers > 0 and
+                               H == config.num_attention_heads * config.head_dim)
         # single-row steps fold the norms and the SiLU gate into the products' kernels; that kernel wants rows and
         # tiles of whole 16-byte pieces
         self.fused_decode = all(m._header.tile_rows % 8 == 0 and m.in_features % 8 == 0
@@ -194,6 +197,8 @@ class TernaryLlamaDecoder(nn.Module):
             raise ValueError("prompt longer than the cache")
         if self._cache is None or self._cache.shape[2] != B:
             self.allocate_cache(B)
+        if B > 0 and S > 0 and self.native_prefill:
+            return self._prefill_native(tokens)
         x = self.embed_tokens[tokens]
         pos = torch.arange(S, device=x.device)
         cos, sin = self.rope_cos[:S], self.rope_sin[:S]
@@ -205,6 +210,27 @@ class TernaryLlamaDecoder(nn.Module):
             x = self._block(layer, li, x, cos, sin, pos, attend)
         last = self.norm(x[:, -1])
         return self.lm_head(last)
+
+    def _prefill_native(self, tokens):
+        """The pass with the library's kernels around the products: residual add + RMSNorm in one, keys rotated into the
+        cache and values copied beside them in one, queries rotated inside the attention.  Seven launches a layer."""
+        c = self.config
+        B, S = tokens.shape
+        H, nh, hd, eps = c.hidden_size, c.num_attention_heads, c.head_dim, c.rms_norm_eps
+        tables = self.rope_cos[:S], self.rope_sin[:S]
+        x = self.embed_tokens[tokens].view(B * S, H)
+        _, h = ops.add_rmsnorm(x, None, self.layers[0].input_layernorm.weight, eps)
+        for li, layer in enumerate(self.layers):
+            qkv = layer.qkv_proj(h).view(B, S, 3, nh, hd)
+            kc, vc = self._cache[li, 0, :, :, :S], self._cache[li, 1, :, :, :S]
+            ops.rope_rows(qkv[:, :, 1], tables, kc, qkv[:, :, 2], vc)
+            a = ops.prefill_attention(qkv[:, :, 0], kc, vc, tables)
+            x, h = ops.add_rmsnorm(x, layer.o_proj(a.view(B * S, H)), layer.post_attention_layernorm.weight, eps)
+            y = self._mlp(layer, h)
+            if li + 1 < len(self.layers):
+                x, h = ops.add_rmsnorm(x, y, self.layers[li + 1].input_layernorm.weight, eps)
+        last = [t.view(B, S, H)[:, -1].contiguous() for t in (x, y)]
+        return self.lm_head(ops.add_rmsnorm(*last, self.norm.weight, eps)[1])
 
     # -- decode ------------------------------------------------------------------------------
     def _decode_step(self, token, pos, mask):

@@ -450,6 +450,76 @@ def rope_cache_update(qkv, cos_table, sin_table, pos, q_out, k_cache, v_cache):
     return q_out
 
 
+def rope_table(first, count, head_dim, theta, dtype, device):
+    """cos and sin of the rotate-half rotary embedding for positions first .. first + count - 1, [count, head_dim] each."""
+    cos, sin = torch.empty((2, count, head_dim), dtype=dtype, device=device).unbind(0)
+    with torch.cuda.device(device):
+        _lib.check(_lib.lib().tl_rope_table(None, first, count, head_dim, float(theta), _code(dtype, "table"), cos.data_ptr(), sin.data_ptr(),
+                                            _stream_ptr(device)))
+    return cos, sin
+
+
+def _steps(t, dims):
+    """Strides of t's dimensions `dims`, 0 where there is only one entry."""
+    return [t.stride(d) if t.shape[d] > 1 else 0 for d in dims]
+
+
+def in_pieces(*tensors):
+    """Whether the library reads these [..., head_dim] tensors as they lie: unit last stride, everything else in whole
+    16-byte pieces."""
+    return all(t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s * t.element_size() % 16 == 0 for s in _steps(t, range(t.dim() - 1)))
+               for t in tensors)
+
+
+def _table_args(tables, like, seq):
+    """(cos, sin, elements between batch rows) of [seq, head_dim] or [batch or 1, seq, head_dim] tables."""
+    cos, sin = tables
+    for t in tables:
+        if t.dtype != like.dtype or t.device != like.device or not t.is_contiguous() or t.shape[-2:] != (seq, like.shape[-1]) or \
+                (t.dim() == 3 and t.shape[0] not in (1, like.shape[0])) or t.dim() not in (2, 3) or t.shape != cos.shape:
+            raise ValueError("rotary tables must be contiguous [seq, head_dim] or [batch, seq, head_dim] of the activations' dtype")
+    return cos, sin, (_steps(cos, [0])[0] if cos.dim() == 3 else 0)
+
+
+def rope_rows(k, tables, k_out, v=None, v_out=None):
+    """k_out = k rotated and v_out = v, for k, v [batch, seq, heads, head_dim] (views whose heads lie side by side) and
+    outputs [batch, heads, seq, head_dim] of any strides of whole 16-byte pieces.  tables: (cos, sin)."""
+    B, S, heads, hd = k.shape
+    both = [k, k_out] + ([] if v is None else [v, v_out])
+    if any(t.dtype != k.dtype or t.device != k.device or t.stride(-1) != 1 for t in both) or any(t.shape != (B, heads, S, hd) for t in both[1::2]) or \
+            any(t.shape != k.shape or t.stride(2) != hd for t in both[::2]):
+        raise ValueError("k, v must be [batch, seq, heads, head_dim], the outputs [batch, heads, seq, head_dim], all of one type and device")
+    if v is not None and (v.stride() != k.stride() or v_out.stride() != k_out.stride()):
+        raise ValueError("v and v_out must have the strides of k and k_out")
+    cos, sin, table_step = _table_args(tables, k, S)
+    ob, oh, osq = _steps(k_out, (0, 1, 2))
+    with torch.cuda.device(k.device):
+        rc = _lib.lib().tl_rope_rows(k.data_ptr(), v.data_ptr() if v is not None else None, _code(k.dtype, "k"), B, S, heads, hd, *_steps(k, (0, 1)),
+                                     cos.data_ptr(), sin.data_ptr(), table_step, k_out.data_ptr(), v_out.data_ptr() if v is not None else None,
+                                     ob, osq, oh, _stream_ptr(k.device))
+    _lib.check(rc)
+
+
+def prefill_attention(q, k, v, tables=None):
+    """Causal attention of q [batch, q_len, heads, head_dim] over k, v [batch, kv_heads, kv_len, head_dim], query i seeing
+    the keys up to i + kv_len - q_len; returns [batch, q_len, heads * head_dim].  fp16, head_dim 64 or 128, strides of
+    whole 16-byte pieces.  tables: (cos, sin) by which the queries are rotated on the way in."""
+    B, S, heads, hd = q.shape
+    if k.dim() != 4 or k.shape != v.shape or k.shape[0] != B or k.shape[3] != hd:
+        raise ValueError("k and v must be [batch, kv_heads, kv_len, head_dim]")
+    if any(t.dtype != q.dtype or t.device != q.device or t.stride(-1) != 1 for t in (q, k, v)):
+        raise ValueError("q, k and v must have one dtype and device and unit last strides")
+    cos, sin, table_step = _table_args(tables, q, S) if tables is not None else (None, None, 0)
+    steps = (ctypes.c_int64 * 10)(*_steps(q, (0, 1, 2)), *_steps(k, (0, 2, 1)), *_steps(v, (0, 2, 1)), table_step)
+    out = torch.empty((B, S, heads * hd), dtype=q.dtype, device=q.device)
+    with torch.cuda.device(q.device):
+        rc = _lib.lib().tl_prefill_attention(q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr() if cos is not None else None,
+                                             sin.data_ptr() if sin is not None else None, _code(q.dtype, "q"), B, heads, k.shape[1], hd, S, k.shape[2],
+                                             steps, out.data_ptr(), _stream_ptr(q.device))
+    _lib.check(rc)
+    return out
+
+
 def _kmajor_image(rows, width, like):
     """An uninitialised K-major image [width][ld] for `rows` activation rows, ld = rows rounded up to 16: the
     layout spmm multiplies 5 to 48 rows from without a re-layout pass.  Returns (buffer, ld)."""
