@@ -65,7 +65,7 @@ int tl_version(void);
 
 /* The launchers' tuning knobs (environment variables TL_SMALL_LDS, TL_TILE_GROUP, TL_QUAD_SHARE, TL_LW,
  * TL_SPMV_SHARE, TL_SPMV_WIDE, TL_SPMV_TILES, TL_SMALL_MT, TL_SPMV_DIRECT, TL_BLOCK_SET,
- * TL_OCTET, TL_QUAD_WIDE, TL_RES16; unset = the launcher's own choice) are read once per process.  This
+ * TL_OCTET, TL_QUAD_WIDE, TL_RES16, TL_FEW; unset = the launcher's own choice) are read once per process.  This
  * reads them again -- for tests and tuning runs that change them between calls. */
 int tl_reload_options(void);
 
@@ -281,6 +281,14 @@ int tl_mlp_gate_up(const tl_layout_header* gate_header, const void* gate_blob_de
                    const void* gate_scale, const void* up_scale, int scale_dtype,
                    int activation,
                    void* workspace, int64_t workspace_bytes, void* stream);
+
+/* The same for up to 48 rows, both blobs with two-bit codes (TL_ERR_UNSUPPORTED otherwise); needs no workspace. */
+int tl_mlp_gate_up_few(const tl_layout_header* gate_header, const void* gate_blob_dev,
+                       const tl_layout_header* up_header, const void* up_blob_dev,
+                       const void* X, int x_dtype, int x_layout, int64_t ldx, int64_t M,
+                       void* H, int h_dtype, int64_t ldh,
+                       const void* gate_scale, const void* up_scale, int scale_dtype,
+                       int activation, void* stream);
 
 /* Times `iters` back-to-back tl_spmm launches on `stream` with HIP events recorded
  * on that same stream and returns the mean milliseconds per launch.  Used by the

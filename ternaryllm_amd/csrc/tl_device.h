@@ -1,6 +1,7 @@
 // What the translation units of libternary_spmm's device code share: the argument block of the kernels, the
 // device helpers every kernel family uses, and the host helpers of the launchers (knobs, device facts, checks).
 //   tl_small_m.hip  the kernels for 1 to 48 activation rows and their launchers
+//   tl_few.hip      the matrix-core kernel for up to 48 rows
 //   tl_matrix.hip   the matrix-core kernel for more than 48 rows, the image of its activations, their launcher
 //   tl_kernels.hip  the entry points, the checks in front of them, the knobs, the measurement helpers
 #pragma once
@@ -155,7 +156,7 @@ constexpr int kMaxChunkBytes = (TL_BLOCK_COLUMNS + TL_BLOCK_COLUMNS * 128) * 4; 
 // Tuning knobs (environment variables of the same names).  They are read once, at the first launch of the
 // process; tl_reload_options() reads them again.  A knob that is not set leaves the launcher's own choice.
 enum Knob { TL_SMALL_LDS, TL_TILE_GROUP, TL_QUAD_SHARE, TL_LW, TL_SPMV_SHARE, TL_SPMV_WIDE, TL_SMALL_MT, TL_SPMV_DIRECT,
-            TL_BLOCK_SET, TL_OCTET, TL_QUAD_WIDE, TL_SPMV_TILES, TL_RES16, kKnobCount };
+            TL_BLOCK_SET, TL_OCTET, TL_QUAD_WIDE, TL_SPMV_TILES, TL_RES16, TL_FEW, kKnobCount };
 int knob(Knob which, int fallback);   // tl_kernels.hip
 int compute_units();                  // of the current device, read once per device
 int check_header(const tl_layout_header* h);
@@ -180,6 +181,9 @@ inline int64_t small_kmajor_bytes(const tl_layout_header* h, int64_t M, int x_dt
 }
 int launch_small(KernelArgs a, const tl_layout_header* h, int x_dtype, void* workspace, int64_t workspace_bytes, hipStream_t st);
 
+// Whether tl_spmm_gated of these rows is served by a kernel that walks the index stream (9 to 48 fp16 rows).
+bool walk_has_gated(const KernelArgs& a, const tl_layout_header* h);
+
 // tl_matrix.hip
 // The row-major image of the activations where the kernel does not read them as they lie: two bytes a value, for fp32
 // three times two.
@@ -188,5 +192,9 @@ inline int64_t matrix_image_bytes(int64_t K, int64_t M, int x_dtype)
     return round_up(M, 256) * round_up(K, 8) * 2 * (x_dtype == TL_F16 ? 1 : 3) + 256;
 }
 int launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t workspace_bytes, bool two_weights, hipStream_t st);
+
+// tl_few.hip
+// Up to 48 rows, any layout, blobs with codes; no gated and no chained epilogue.  Two weights: silu(w0 product) * w1 product.
+int launch_matrix_few(KernelArgs a, int x_dtype, bool two_weights, hipStream_t st);
 
 }  // namespace tl

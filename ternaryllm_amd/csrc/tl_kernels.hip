@@ -27,7 +27,8 @@ int check_dtype(int d, const char* what)
 }
 
 const char* const kKnobNames[kKnobCount] = {"TL_SMALL_LDS", "TL_TILE_GROUP", "TL_QUAD_SHARE", "TL_LW", "TL_SPMV_SHARE", "TL_SPMV_WIDE",
-                                            "TL_SMALL_MT", "TL_SPMV_DIRECT", "TL_BLOCK_SET", "TL_OCTET", "TL_QUAD_WIDE", "TL_SPMV_TILES", "TL_RES16"};
+                                            "TL_SMALL_MT", "TL_SPMV_DIRECT", "TL_BLOCK_SET", "TL_OCTET", "TL_QUAD_WIDE", "TL_SPMV_TILES", "TL_RES16",
+                                            "TL_FEW"};
 struct Knobs {
     bool set[kKnobCount];
     int value[kKnobCount];
@@ -131,6 +132,29 @@ extern "C" int tl_spmm_workspace(const tl_layout_header* header, int64_t M, int 
 }
 
 namespace {
+// Whether a product is tl_few.hip's.  It costs the bytes of the codes (two bits an entry) whatever the weight; the kernels
+// that walk the index stream cost its bytes, and some of them start from a K-major image that a K-major caller has at hand.
+// us, walk / codes, 4096 -> 11008:
+//   one row         fp16 8.0 / 5.9, 5.4 / 6.1;  fp32 8.2 / 11.0, 5.4 / 11.1 (66 %, 95 % zeros): never, one row's gated and fused
+//                   products are the walk's and equal the plain one bit for bit
+//   8 rows          fp16 21.0 / 8.0, 14.8 / 8.1;  fp32 25.3 / 12.8, 18.4 / 13.0: always
+//   ... K-major     fp16 17.7 / 14.9, 11.7 / 15.1;  fp32 22.4 / 19.4, 14.6 / 19.7: by bytes (3 and 4 rows, which the walk does
+//                   not take from an image: fp16 38 / 15, 31 / 15: always)
+//   16 rows         fp16 27.6 / 10.7, 15.6 / 11.0: always;  fp32 27.3 / 18.1, 14.0 / 18.4: by bytes
+//   ... fp16 where the walk has the gated epilogue: never, so that tl_spmm_gated stays tl_spmm and the gate bit for bit
+//   48 rows         fp16 71.7 / 25.8, 43.6 / 26.1;  fp32 102 / 46, 76 / 46: always
+// A knob that names another kernel for few rows keeps the call with it.
+bool few_on_matrix_cores(const KernelArgs& a, const tl_layout_header* h, int64_t M, bool chained)
+{
+    if (M > kSmallMaxM || chained || a.gated || !a.w0.codes) return false;
+    for (Knob other : {TL_SMALL_MT, TL_OCTET, TL_QUAD_WIDE, TL_RES16, TL_SPMV_DIRECT, TL_SPMV_TILES})
+        if (knob(other, -1) >= 0) return false;
+    bool use = M > 1 && !walk_has_gated(a, h);
+    const bool fewer_bytes = (uint64_t)a.NB * a.units * a.planes * TL_CODE_UNIT_BYTES < h->stream_bytes;
+    if (use && (a.x_kmajor ? M < 3 || M > 4 : M > 8 && M <= 16 && !a.x_f16)) use = fewer_bytes;
+    return knob(TL_FEW, use ? 1 : 0) != 0;
+}
+
 // tl_spmm, or (y_layout >= 0) tl_spmm_gated with that output layout
 int spmm_call(const tl_layout_header* header, const void* blob_dev, const void* X, int x_dtype, int x_layout, int64_t ldx, int64_t M,
               void* Y, int y_dtype, int64_t ldy, int y_layout, const void* scale, int scale_dtype, void* workspace, int64_t workspace_bytes,
@@ -178,7 +202,8 @@ int spmm_call(const tl_layout_header* header, const void* blob_dev, const void* 
     a.x_f16 = x_dtype == TL_F16; a.x_kmajor = x_layout == TL_X_K_MAJOR; a.y_f16 = y_dtype == TL_F16; a.scale_f16 = scale_dtype == TL_F16;
     a.one = 1.0f;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    int rc = (M <= kSmallMaxM) ? launch_small(a, header, x_dtype, workspace, workspace_bytes, st)
+    int rc = few_on_matrix_cores(a, header, M, chain != nullptr) ? launch_matrix_few(a, x_dtype, false, st)
+             : (M <= kSmallMaxM) ? launch_small(a, header, x_dtype, workspace, workspace_bytes, st)
                                : launch_matrix_rows(a, x_dtype, workspace, workspace_bytes, false, st);
     if (rc) return rc;
     return finish_launch();
@@ -213,13 +238,15 @@ extern "C" int tl_spmm_gated(const tl_layout_header* header, const void* blob_de
     return spmm_call(header, blob_dev, X, x_dtype, x_layout, ldx, M, Y, y_dtype, ldy, y_layout, scale, scale_dtype, workspace, workspace_bytes, stream);
 }
 
-extern "C" int tl_mlp_gate_up(const tl_layout_header* gate_header, const void* gate_blob_dev,
-                              const tl_layout_header* up_header, const void* up_blob_dev,
-                              const void* X, int x_dtype, int x_layout, int64_t ldx, int64_t M,
-                              void* H, int h_dtype, int64_t ldh,
-                              const void* gate_scale, const void* up_scale, int scale_dtype,
-                              int activation,
-                              void* workspace, int64_t workspace_bytes, void* stream)
+namespace {
+// tl_mlp_gate_up, or (few) tl_mlp_gate_up_few
+int gate_up_call(bool few, const tl_layout_header* gate_header, const void* gate_blob_dev,
+                 const tl_layout_header* up_header, const void* up_blob_dev,
+                 const void* X, int x_dtype, int x_layout, int64_t ldx, int64_t M,
+                 void* H, int h_dtype, int64_t ldh,
+                 const void* gate_scale, const void* up_scale, int scale_dtype,
+                 int activation,
+                 void* workspace, int64_t workspace_bytes, void* stream)
 {
     if (int rc = check_header(gate_header)) return rc;
     if (int rc = check_header(up_header)) return rc;
@@ -230,7 +257,9 @@ extern "C" int tl_mlp_gate_up(const tl_layout_header* gate_header, const void* g
     if (!up_blob_dev || reinterpret_cast<uintptr_t>(up_blob_dev) % 256) return fail(TL_ERR_ALIGN, "up blob null or not 256-byte aligned");
     if (int rc = check_io(gate_blob_dev, X, H, x_dtype, x_layout, ldx, M, h_dtype, ldh, gate_scale, scale_dtype, gate_header)) return rc;
     if ((gate_scale == nullptr) != (up_scale == nullptr)) return fail(TL_ERR_ARG, "pass both scales or neither");
-    if (M <= kSmallMaxM) return fail(TL_ERR_UNSUPPORTED, "fused gate/up needs M > %d; use two tl_spmm calls below that", kSmallMaxM);
+    if (!few && M <= kSmallMaxM) return fail(TL_ERR_UNSUPPORTED, "fused gate/up needs M > %d; use two tl_spmm calls below that", kSmallMaxM);
+    if (few && (M > kSmallMaxM || !gate_header->off_codes || !up_header->off_codes))
+        return fail(TL_ERR_UNSUPPORTED, "fused gate/up of few rows is for M <= %d and blobs with codes", kSmallMaxM);
     KernelArgs a;
     std::memset(&a, 0, sizeof(a));
     a.w0 = weight_ptrs(gate_header, gate_blob_dev, gate_scale);
@@ -242,9 +271,35 @@ extern "C" int tl_mlp_gate_up(const tl_layout_header* gate_header, const void* g
     a.tile_rows = (int)gate_header->tile_rows;
     a.x_f16 = x_dtype == TL_F16; a.x_kmajor = x_layout == TL_X_K_MAJOR; a.y_f16 = h_dtype == TL_F16; a.scale_f16 = scale_dtype == TL_F16;
     a.one = 1.0f;
-    if (int rc = launch_matrix_rows(a, x_dtype, workspace, workspace_bytes, true, static_cast<hipStream_t>(stream))) return rc;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (int rc = few ? launch_matrix_few(a, x_dtype, true, st) : launch_matrix_rows(a, x_dtype, workspace, workspace_bytes, true, st)) return rc;
     return finish_launch();
 }
+}  // namespace
+
+extern "C" int tl_mlp_gate_up(const tl_layout_header* gate_header, const void* gate_blob_dev,
+                              const tl_layout_header* up_header, const void* up_blob_dev,
+                              const void* X, int x_dtype, int x_layout, int64_t ldx, int64_t M,
+                              void* H, int h_dtype, int64_t ldh,
+                              const void* gate_scale, const void* up_scale, int scale_dtype,
+                              int activation,
+                              void* workspace, int64_t workspace_bytes, void* stream)
+{
+    return gate_up_call(false, gate_header, gate_blob_dev, up_header, up_blob_dev, X, x_dtype, x_layout, ldx, M, H, h_dtype, ldh, gate_scale,
+                        up_scale, scale_dtype, activation, workspace, workspace_bytes, stream);
+}
+
+extern "C" int tl_mlp_gate_up_few(const tl_layout_header* gate_header, const void* gate_blob_dev,
+                                  const tl_layout_header* up_header, const void* up_blob_dev,
+                                  const void* X, int x_dtype, int x_layout, int64_t ldx, int64_t M,
+                                  void* H, int h_dtype, int64_t ldh,
+                                  const void* gate_scale, const void* up_scale, int scale_dtype,
+                                  int activation, void* stream)
+{
+    return gate_up_call(true, gate_header, gate_blob_dev, up_header, up_blob_dev, X, x_dtype, x_layout, ldx, M, H, h_dtype, ldh, gate_scale,
+                        up_scale, scale_dtype, activation, nullptr, 0, stream);
+}
+
 
 
 // Scratch of tl_spmm_noalloc: device memory that belongs to the library's code object, one copy per GPU,

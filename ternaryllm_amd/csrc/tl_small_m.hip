@@ -2533,3 +2533,12 @@ int tl::launch_small(KernelArgs a, const tl_layout_header* h, int x_dtype, void*
 {
     return small_launch(a, h, x_dtype, workspace, workspace_bytes, st);
 }
+
+bool tl::walk_has_gated(const KernelArgs& a, const tl_layout_header* h)
+{
+    if (a.M <= 8 || !a.x_f16 || a.N % 2) return false;
+    if (ceil_div(a.NB, 2) * ceil_div(a.M, 16) >= 2 * (int64_t)compute_units()) return true;  // tl_spmm_octet
+    if (a.M > 16) return false;
+    const ResShape shape = res_shape(a, h);
+    return shape.pieces != 0 && (int64_t)a.NB * shape.parts > compute_units();
+}

@@ -238,14 +238,19 @@ def spmm_chain(weight, x, scale=None, x_layout=_lib.TL_X_ROW_MAJOR, residual=Non
 
 
 def mlp_gate_up(gate, up, x, gate_scale=None, up_scale=None, out_dtype=None):
-    """h[M, N] = silu((x @ Wg) * sg) * ((x @ Wu) * su) in one pass over x (M > 48), else two products."""
+    """h[M, N] = silu((x @ Wg) * sg) * ((x @ Wu) * su) in one pass over x, or two products where no kernel does it: one
+    row (its own kernel is the faster one), weights without codes or of different tile heights, up to 48 rows whose two
+    scales are not of one kind."""
     if gate.columns != up.columns or gate.inners != up.inners:
         raise ValueError("gate and up weights must have the same shape")
     x_code = _code(x.dtype, "x")
     x, M, ldx = _x_geometry(x, gate.inners, _lib.TL_X_ROW_MAJOR)
     N = gate.columns
     out_dtype = out_dtype or x.dtype
-    if M <= 48 or gate.header.tile_rows != up.header.tile_rows:
+    alike = gate.header.tile_rows == up.header.tile_rows and gate.header.code_planes == up.header.code_planes
+    scales_alike = (gate_scale is None) == (up_scale is None) and (gate_scale is None or gate_scale.dtype == up_scale.dtype)
+    few = 2 <= M <= 48 and alike and scales_alike and gate.header.off_codes != 0 and x.device == gate.device == up.device
+    if (M <= 48 and not few) or gate.header.tile_rows != up.header.tile_rows:
         g = spmm(gate, x, gate_scale, torch.float32)
         u = spmm(up, x, up_scale, torch.float32)
         return (torch.nn.functional.silu(g) * u).to(out_dtype)
@@ -254,6 +259,14 @@ def mlp_gate_up(gate, up, x, gate_scale=None, up_scale=None, out_dtype=None):
     us, s_code2 = _scale_args(up_scale, N, x.device)
     if (gs is None) != (us is None) or (gs is not None and s_code != s_code2):
         raise ValueError("pass both scales, of one dtype, or neither")
+    if few:
+        with torch.cuda.device(x.device):
+            _lib.check(_lib.lib().tl_mlp_gate_up_few(ctypes.byref(gate.header), gate.blob.data_ptr(), ctypes.byref(up.header),
+                                                     up.blob.data_ptr(), x.data_ptr(), x_code, _lib.TL_X_ROW_MAJOR, ldx, M, h.data_ptr(),
+                                                     _code(out_dtype, "out_dtype"), h.stride(0), gs.data_ptr() if gs is not None else None,
+                                                     us.data_ptr() if us is not None else None, s_code, _lib.TL_ACT_SILU_GATE,
+                                                     _stream_ptr(x.device)))
+        return h
     ws, ws_bytes = _workspace(gate.header, M, x_code, _lib.TL_X_ROW_MAJOR, x.device)
     with torch.cuda.device(x.device):
         rc = _lib.lib().tl_mlp_gate_up(ctypes.byref(gate.header), gate.blob.data_ptr(), ctypes.byref(up.header),

@@ -1,0 +1,66 @@
+"""The matrix-core kernel for a few rows at the sizes where it can go wrong: its 16-row fragments, turns of one, two and
+four slices of 64 rows of K, more turns than waves, one and two column blocks to a workgroup, every way of reading rows."""
+import numpy as np
+import pytest
+import torch
+
+from tests.util import activations, ternary_weight
+
+pytestmark = pytest.mark.gpu
+
+
+# K: below one 16-byte piece, whole and ragged slices, 32 and 64 slices, more than 16 units; N: the 16-column block, and
+# 8200 columns are more blocks than twice the compute units
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M,K,N", [(2, 1, 1), (16, 8, 16), (3, 72, 31), (5, 1003, 77), (17, 1024, 33), (32, 2048, 16), (48, 2056, 40), (33, 4100, 50),
+                                   (9, 4352, 24), (48, 11008, 17), (16, 520, 8200), (34, 300, 8195)])
+def test_few_rows_at_the_edges(cuda, oracle, M, K, N, dtype):
+    """Integer activations: every sum is exact, whatever its order.  fp32 ones use all 24 bits where a column has one entry."""
+    from ternaryllm_amd import ops
+    from ternaryllm_amd.packing import PackedWeight
+    w = ternary_weight(K, N, 0.6, M + K + N)
+    dw = ops.DeviceWeight(PackedWeight.from_dense(w), cuda)
+    x = activations(M, K, M, dtype, integer=True)
+    ref = oracle.fast_product(x.double().numpy(), w)
+    wide = torch.zeros((M, K + 3), dtype=dtype)
+    wide[:, :K] = x
+    for name, xin, layout in (("rows", x.to(cuda), 0), ("strided rows", wide.to(cuda)[:, :K], 0), ("k-major", x.t().contiguous().to(cuda), 1)):
+        print(f"case M={M} K={K} N={N} {dtype} {name}", flush=True)
+        out = torch.full((M, N + 5), 7.0, dtype=torch.float32, device=cuda)
+        ops.spmm(dw, xin, out_dtype=torch.float32, x_layout=layout, out=out[:, :N])
+        assert np.array_equal(out[:, :N].cpu().numpy().astype(np.float64), ref), name
+        assert bool((out[:, N:] == 7.0).all()), name
+    one = np.zeros((K, N), np.int32)
+    rng = np.random.default_rng(M)
+    rows = rng.integers(0, K, N)
+    one[rows, np.arange(N)] = rng.choice([-1, 1], N)
+    x = activations(M, K, M + 1, dtype)
+    y = ops.spmm(ops.DeviceWeight(PackedWeight.from_dense(one), cuda), x.to(cuda)).cpu().numpy()
+    assert np.array_equal(y, x.numpy()[:, rows] * one[rows, np.arange(N)].astype(x.numpy().dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M", [2, 16, 31, 48])
+def test_gate_and_up_of_few_rows(cuda, M, dtype):
+    """silu(gate) * up of two weights in one launch, infinities included: a column sees only the rows that it names."""
+    from ternaryllm_amd import ops
+    from ternaryllm_amd.packing import PackedWeight
+    K, N = 1100, 83
+    wg, wu = ternary_weight(K, N, 0.8, 3), ternary_weight(K, N, 0.8, 4)
+    dg, du = (ops.DeviceWeight(PackedWeight.from_dense(w), cuda) for w in (wg, wu))
+    x = activations(M, K, 5, dtype)
+    x[M - 1, 9] = float("inf")
+    sg = (0.5 + torch.rand(N, generator=torch.Generator().manual_seed(6))).to(dtype)
+    g, u = (torch.zeros(M, N, dtype=torch.float64) for _ in range(2))
+    for n in range(N):
+        for w, out in ((wg, g), (wu, u)):
+            rows = np.nonzero(w[:, n])[0]
+            out[:, n] = (x[:, rows].double() * torch.from_numpy(w[rows, n]).double()).sum(1)
+    g, u = g * sg.double(), u * sg.double()
+    want = torch.nn.functional.silu(g) * u
+    print(f"case M={M} {dtype}", flush=True)
+    got = ops.mlp_gate_up(dg, du, x.to(cuda), sg.to(cuda), sg.to(cuda), out_dtype=torch.float32).double().cpu()
+    # K fp32 roundings of sums of magnitude sqrt(K) at most, and __expf's few units: far below 1e-4 of the result's size
+    fine = torch.isfinite(want)
+    assert torch.equal(fine, torch.isfinite(got))
+    assert float((got[fine] - want[fine]).abs().max()) <= 1e-4 * float(want[fine].abs().max())
