@@ -118,17 +118,14 @@ class LlamaTernaryAttention(nn.Module):
             past_key_value = kwargs.pop("past_key_values", None)
         bsz, q_len, _ = hidden_states.shape
         dropout = self.attention_dropout if self.training else 0.0
-        qkv = None
         if self.fused_qkv and hidden_states.is_cuda:
             weight, scale = self._qkv_weight(hidden_states.device)
             nq, nkv = self.q_proj.out_features, self.k_proj.out_features
             qkv = ops.spmm(weight, hidden_states.reshape(bsz * q_len, -1), scale).view(bsz, q_len, nq + 2 * nkv)
             heads = [t.view(bsz, q_len, -1, self.head_dim) for t in qkv.split((nq, nkv, nkv), dim=-1)]
-            q, k, v = (t.transpose(1, 2) for t in heads)
         else:
-            q = self.q_proj(hidden_states).view(bsz, q_len, -1, self.head_dim).transpose(1, 2)
-            k = self.k_proj(hidden_states).view(bsz, q_len, -1, self.head_dim).transpose(1, 2)
-            v = self.v_proj(hidden_states).view(bsz, q_len, -1, self.head_dim).transpose(1, 2)
+            heads = [p(hidden_states).view(bsz, q_len, -1, self.head_dim) for p in (self.q_proj, self.k_proj, self.v_proj)]
+        q, k, v = (t.transpose(1, 2) for t in heads)
         is_tuple = isinstance(past_key_value, (tuple, list))
         past_len = position_offset
         if past_len is None:
@@ -141,7 +138,7 @@ class LlamaTernaryAttention(nn.Module):
             else:
                 past_len = 0
         # causal fp16 attention without a mask: the library's kernels rotate and attend
-        native = (qkv is not None and qkv.dtype == torch.float16 and qkv.numel() > 0 and self.head_dim in (64, 128) and attention_mask is None and
+        native = (all(t.is_cuda and t.dtype == torch.float16 and t.numel() > 0 and not t.requires_grad for t in heads) and self.head_dim in (64, 128) and attention_mask is None and
                   not output_attentions and dropout == 0.0 and (self.is_causal or q_len == 1))
         if native and position_ids is None and position_embeddings is None:
             cos, sin = ops.rope_table(past_len, q_len, self.head_dim, self.rope_theta, q.dtype, q.device)
