@@ -73,25 +73,6 @@ enum { kPlain = 0, kPairs = 1, kTwoWeights = 2 };
 // The product of one output: from the index stream where the matrix cores' sum is not finite.
 __device__ __forceinline__ float exact_output(const KernelArgs& a, const WeightPtrs& w, int m, int n) { return walk_column(w, a.T, a.tile_rows, n, callers_x(a, m)); }
 
-// Every output of the wave's tile again, from the index stream (some activation of its rows is not finite).
-template <int MODE>
-__device__ void redo_tile(const KernelArgs& a, int m0, int rows, int n0, int cols, int lane)
-{
-    for (int e = lane; e < rows * cols; e += 64) {
-        const int m = m0 + e / cols, n = n0 + e % cols;
-        if (m >= a.M || n >= a.N || (MODE == kPairs && (n & 1))) continue;
-        float v = exact_output(a, a.w0, m, n) * load_scale(a.w0.scale, a.scale_f16, n);
-        long long at = (long long)m * a.ldy + n;
-        if constexpr (MODE == kTwoWeights) v = silu(v) * (exact_output(a, a.w1, m, n) * load_scale(a.w1.scale, a.scale_f16, n));
-        if constexpr (MODE == kPairs) {
-            const float u = exact_output(a, a.w0, m, n + 1) * load_scale(a.w0.scale, a.scale_f16, n + 1);
-            v = gate_pair(as_output(v, a.y_f16), as_output(u, a.y_f16), a.y_f16);
-            at = (long long)m * a.ldy + n / 2;
-        }
-        store_out(a.Y, a.y_f16, at, v);
-    }
-}
-
 // Bound by the matrix cores: 1024 x 4096 -> 11008 in fp16 is 92 GFLOP dense, 80 us = 1155 TFLOP/s (8192 x 2048 -> 11008:
 // 1230; a library fp16 product of that size 1090, the matrix instruction alone on trivial operands 2000).  What it took, at
 // 1024 x 12288 -> 8192: sums kept in their registers (fences around the barrier) 190 -> 161 us; operands made between the
@@ -294,21 +275,39 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
     }
 
     // ---- out ----
-    bool fine = true;
+    // A sum that is not finite is worked out again by the lane that holds it, before anything is stored: the outputs of
+    // finite rows keep their bits whatever another row of the tile holds.  (The sums that need it go into a mask that a
+    // loop takes bit by bit, so that the walk stands here once and the sums stay in registers.)
+    constexpr int OUT_FN = MODE == kTwoWeights ? FN / 2 : FN;
+    const int wave_n0 = (nb0 + wn * OUT_FN) * 16, wave_m0 = m0 + wm * FM * 16;
+    static_assert(FN * FM * 4 <= 32, "a bit for each of a lane's sums");
+    uint32_t redo = 0;
 #pragma unroll
     for (int f = 0; f < FN; ++f)
 #pragma unroll
-        for (int m = 0; m < FM; ++m) fine = fine && finite4(acc[f][m]);
-    constexpr int OUT_FN = MODE == kTwoWeights ? FN / 2 : FN;
-    const int wave_n0 = (nb0 + wn * OUT_FN) * 16, wave_m0 = m0 + wm * FM * 16;
+        for (int m = 0; m < FM; ++m) {
+            acc[f][m] *= 0.5f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const bool mine = wave_m0 + m * 16 + r16 < a.M && wave_n0 + f % OUT_FN * 16 + g * 4 + i < a.N;
+                redo |= mine && !(fabsf(acc[f][m][i]) < __builtin_huge_valf()) ? 1u << ((f * FM + m) * 4 + i) : 0u;
+            }
+        }
+    while (redo != 0) {
+        const int at = __builtin_ctz(redo), f = at / (FM * 4), m = at / 4 % FM;
+        redo &= redo - 1;
+        const float v = exact_output(a, f >= OUT_FN ? a.w1 : a.w0, wave_m0 + m * 16 + r16, wave_n0 + f % OUT_FN * 16 + g * 4 + at % 4);
+#pragma unroll
+        for (int e = 0; e < FN * FM * 4; ++e) acc[e / (FM * 4)][e / 4 % FM][e % 4] = e == at ? v : acc[e / (FM * 4)][e / 4 % FM][e % 4];
+    }
 #pragma unroll
     for (int f = 0; f < OUT_FN; ++f) {
         const int n = wave_n0 + f * 16 + g * 4;
         float s0[4], s1[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            s0[i] = 0.5f * (n + i < a.N ? load_scale(a.w0.scale, a.scale_f16, n + i) : 0.f);
-            if constexpr (MODE == kTwoWeights) s1[i] = 0.5f * (n + i < a.N ? load_scale(a.w1.scale, a.scale_f16, n + i) : 0.f);
+            s0[i] = n + i < a.N ? load_scale(a.w0.scale, a.scale_f16, n + i) : 0.f;
+            if constexpr (MODE == kTwoWeights) s1[i] = n + i < a.N ? load_scale(a.w1.scale, a.scale_f16, n + i) : 0.f;
         }
 #pragma unroll
         for (int m = 0; m < FM; ++m) {
@@ -325,7 +324,6 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
             }
         }
     }
-    if (__builtin_amdgcn_ballot_w64(!fine) != 0) redo_tile<MODE>(a, wave_m0, FM * 16, wave_n0, OUT_FN * 16, lane);
 }
 
 // Eight neighbouring activations of a row into the image: fp16 as they are, fp32 in three bf16 parts.

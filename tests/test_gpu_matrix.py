@@ -90,6 +90,21 @@ def test_activations_that_are_not_finite(cuda, M, dtype):
         assert torch.allclose(both, torch.nn.functional.silu(g) * g, rtol=1e-4, atol=1e-4, equal_nan=True)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_finite_rows_keep_their_bits_beside_rows_that_are_not(cuda, dtype):
+    """What a row holds does not show in the bits of another row's outputs."""
+    from ternaryllm_amd import ops
+    M, K, N = 150, 700, 90
+    dg, du = _device(ternary_weight(K, N, 0.5, 11), cuda), _device(ternary_weight(K, N, 0.5, 12), cuda)
+    x = activations(M, K, 13, dtype).to(cuda)
+    spoilt = x.clone()
+    spoilt[3, 5], spoilt[70, 600], spoilt[149, 0] = float("inf"), float("nan"), float("-inf")
+    keep = [m for m in range(M) if m not in (3, 70, 149)]
+    for name, call in (("plain", lambda t: ops.spmm(dg, t)), ("pairs", lambda t: ops.spmm_gated(dg, t)), ("two weights", lambda t: ops.mlp_gate_up(dg, du, t))):
+        print(f"case {name} {dtype}", flush=True)
+        assert torch.equal(call(x)[keep], call(spoilt)[keep]), name
+
+
 def test_a_blob_without_codes(cuda, oracle):
     """What an older version packed: the packed-weight object brings it up to date, and a device blob that was not is
     multiplied by the general kernel."""
