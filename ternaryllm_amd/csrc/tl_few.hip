@@ -38,8 +38,8 @@ __device__ __forceinline__ void load8(const KernelArgs& a, const XT* row, int k,
     }
 }
 
-// Eight fp32 values in three bf16 parts by truncation (tl_matrix.h).  What is not finite need not survive: any part that
-// is not finite makes the sum so, and that output is worked out again.
+// Eight fp32 values in three bf16 parts (tl_matrix.h).  What is not finite need not survive: any part that is not finite
+// makes the sum so, and that output is worked out again.
 __device__ __forceinline__ void split8(const float* v, u32x4* part)
 {
 #pragma unroll
@@ -49,7 +49,7 @@ __device__ __forceinline__ void split8(const float* v, u32x4* part)
         for (int e = 0; e < 2; ++e) {
             const float x = v[2 * i + e];
             bits[e][0] = __float_as_uint(x);
-            const float r1 = x - __uint_as_float(bits[e][0] & 0xffff0000u);
+            const float r1 = (x - __uint_as_float(bits[e][0] & 0xffff0000u)) * kLowScale;
             bits[e][1] = __float_as_uint(r1);
             bits[e][2] = __float_as_uint(r1 - __uint_as_float(bits[e][1] & 0xffff0000u));
         }
@@ -77,9 +77,8 @@ __global__ __launch_bounds__(kMaxWaves * 64) void tl_matrix_few(KernelArgs a)
     const XT* rows[FM];
 #pragma unroll
     for (int f = 0; f < FM; ++f) rows[f] = static_cast<const XT*>(a.X) + min(f * 16 + r16, a.M - 1) * a.x_sm;
-    // fp32: the leading parts, eight bits each, are summed apart from the two that follow them.  Their sums hardly round,
-    // the others' roundings are 2^-8 as large: against fp64, 3.6e-8 where one sum of all three parts had 1.1e-7 to 2.2e-7 and the walk of the
-    // index stream 0.8e-7 to 4e-7.
+    // fp32: the leading parts are summed apart from the two that follow them (against fp64, 3.6e-8 where one sum of all
+    // three parts had 1.1e-7 to 2.2e-7 and the walk of the index stream 0.8e-7 to 4e-7)
     f32x4 acc[C][FM], low[F32 ? C : 1][F32 ? FM : 1];
 #pragma unroll
     for (int c = 0; c < C; ++c)
@@ -138,7 +137,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void tl_matrix_few(KernelArgs a)
     for (int c = 0; c < C; ++c)
 #pragma unroll
         for (int f = 0; f < FM; ++f) {
-            if constexpr (F32) acc[c][f] += low[c][f];
+            if constexpr (F32) add_low(acc[c][f], low[c][f]);
             *reinterpret_cast<f32x4*>(sums + ((wave * C + c) * FM + f) * kPartFloats + lane * 4 + g * 16) = acc[c][f];
         }
     __syncthreads();

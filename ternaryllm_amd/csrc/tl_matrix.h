@@ -34,18 +34,38 @@ __device__ __forceinline__ f32x4 matrix_step(u32x4 w, u32x4 x, f32x4 acc)
     else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, w), __builtin_bit_cast(half8, x), acc, 0, 0, 0);
 }
 
-// The three bf16 numbers whose sum is v: each takes the next 8 of v's 24 significant bits, by truncation, so the sum is
-// exact (down to bf16's smallest numbers); a v that is not finite goes into the first alone.
+// An fp32 value in three bf16 parts: v = a + (b + c) / kLowScale, each part the next 8 of v's 24 significant bits, by
+// truncation.  The two low parts are scaled so that they stay in bf16's range (down to 2^-133, which the matrix
+// instruction keeps) for every v down to fp32's smallest, 2^-149: without that a v below 2^-110 lost bits (against fp64 4.4e-6
+// at 2^-116, 1.1e-3 at 2^-124; now as exact as at any magnitude).  Their products are summed apart from the leading
+// ones', which helps ordinary values too: the leading sums hardly round, and the low sums' roundings weigh 2^-8.
+// Above 2^119 the low parts overflow and make the sum infinite, and the output is worked out again.
+constexpr float kLowScale = 65536.0f;
+
+// acc + low / kLowScale, in place
+__device__ __forceinline__ void add_low(f32x4& acc, const f32x4& low)
+{
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = fmaf(low[i], 1.0f / kLowScale, acc[i]);
+}
+
+// The bit patterns of the parts, in the upper halves; a v that is not finite goes into the first alone.
 __device__ __forceinline__ void split3(float v, uint32_t* a, uint32_t* b, uint32_t* c)
 {
     const uint32_t va = __float_as_uint(v) & 0xffff0000u;
-    const float r1 = v - __uint_as_float(va);
+    const float r1 = (v - __uint_as_float(va)) * kLowScale;
     const bool fine = fabsf(v) < __builtin_huge_valf();
     const uint32_t vb = __float_as_uint(r1) & 0xffff0000u;
     const float r2 = r1 - __uint_as_float(vb);
     *a = va;
     *b = fine ? vb : 0u;
     *c = fine ? __float_as_uint(r2) & 0xffff0000u : 0u;
+}
+
+__device__ __forceinline__ bool finite4(f32x4 v)
+{
+    return fabsf(v[0]) < __builtin_huge_valf() && fabsf(v[1]) < __builtin_huge_valf() && fabsf(v[2]) < __builtin_huge_valf() &&
+           fabsf(v[3]) < __builtin_huge_valf();
 }
 
 // One output of the product from the index stream alone: x(k) of the rows that column n names, added and subtracted.

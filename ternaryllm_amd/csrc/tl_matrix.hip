@@ -172,11 +172,12 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
     const int g = lane >> 4, r16 = lane & 15;
     const uint32_t x_read = (uint32_t)((wm * FM * 16 + r16) * kStageRowBytes);
     const uint32_t swz = (uint32_t)(piece_place(r16, g) * 16);    // rows of a wave's fragments differ by multiples of 16: same place
-    f32x4 acc[FN][FM];
+    constexpr bool F32 = PARTS > 1;
+    f32x4 acc[FN][FM], low[F32 ? FN : 1][F32 ? FM : 1];           // low: the sums of the parts after the first
 #pragma unroll
     for (int f = 0; f < FN; ++f)
 #pragma unroll
-        for (int m = 0; m < FM; ++m) acc[f][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int m = 0; m < FM; ++m) acc[f][m] = low[F32 ? f : 0][F32 ? m : 0] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     // A stage is worked on in two halves of 32 rows of K, each half's activations read from LDS while the other half is
     // multiplied, across stages too: the barrier that says that the next stage has come stands between the halves.
@@ -204,13 +205,16 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
     // The products of one half with the operands of all FN column fragments.  The operand of the next fragment -- at the
     // end, of the next half's first -- is made between a fragment's products: a product keeps the matrix core busy for 16
     // clocks, and the wave can issue three vector instructions meanwhile.
-    auto products = [&](auto step_tag, const u32x4* x, auto next) {
+    auto products = [&](auto step_tag, auto first_tag, const u32x4* x, auto next) {
         constexpr int S = decltype(step_tag)::value;
 #pragma unroll
         for (int f = 0; f < FN; ++f) {
             const u32x4 now = w;
 #pragma unroll
-            for (int m = 0; m < FM; ++m) acc[f][m] = matrix_step<(PARTS > 1)>(now, x[m], acc[f][m]);
+            for (int m = 0; m < FM; ++m) {
+                f32x4& sum = decltype(first_tag)::value ? acc[f][m] : low[F32 ? f : 0][F32 ? m : 0];
+                sum = matrix_step<F32>(now, x[m], sum);
+            }
             if (f + 1 < FN) w = weight_operand<S>(codes[f + 1 < FN ? f + 1 : 0]);
             else w = next();
 #pragma unroll
@@ -220,15 +224,16 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
             }
         }
     };
-    // Stage J of unit u.  STEADY: stages t + 1 .. t + STAGES exist, so nothing needs to be asked.
-    auto turn = [&](auto j_tag, auto steady_tag, int u, int p, bool part_ends) {
+    // Stage J of part p of unit u (first: whether p is the leading part).  STEADY: stages t + 1 .. t + STAGES exist, so
+    // nothing needs to be asked.
+    auto turn = [&](auto j_tag, auto steady_tag, auto first_tag, int u, int p, bool part_ends) {
         const bool unit_ends = part_ends && p == PARTS - 1;
         constexpr int J = decltype(j_tag)::value;
         constexpr bool STEADY = decltype(steady_tag)::value;
         read_half(x1, 64);
-        if (J == 0 && p == 0 && u + 1 < all_units) issue_codes(u + 1);
+        if (J == 0 && decltype(first_tag)::value && u + 1 < all_units) issue_codes(u + 1);
         __builtin_amdgcn_sched_barrier(0);
-        products(std::integral_constant<int, 2 * J>{}, x0, [&]() { return weight_operand<2 * J + 1>(codes[0]); });
+        products(std::integral_constant<int, 2 * J>{}, first_tag, x0, [&]() { return weight_operand<2 * J + 1>(codes[0]); });
         // (without the fences the scheduler moves these products behind the barrier and pays for it with copies of the sums)
         __builtin_amdgcn_sched_barrier(0);
         u32x4 fresh[FN];
@@ -243,7 +248,7 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
         }
         __builtin_amdgcn_sched_barrier(0);
         constexpr int AFTER = J == kUnitStages - 1 ? 0 : 2 * J + 2;   // (of the unit's next stage; a part that ends starts it again)
-        products(std::integral_constant<int, 2 * J + 1>{}, x1, [&]() {
+        products(std::integral_constant<int, 2 * J + 1>{}, first_tag, x1, [&]() {
             if (unit_ends) {
 #pragma unroll
                 for (int f = 0; f < FN; ++f) codes[f] = fresh[f];
@@ -256,23 +261,20 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
     };
     constexpr std::integral_constant<int, 0> s0t; constexpr std::integral_constant<int, 1> s1t;
     constexpr std::integral_constant<int, 2> s2t; constexpr std::integral_constant<int, 3> s3t;
+    auto one_part = [&](auto steady_tag, auto first_tag, int u, int p, int stages) {
+        turn(s0t, steady_tag, first_tag, u, p, stages == 1);
+        if (stages > 1) turn(s1t, steady_tag, first_tag, u, p, stages == 2);
+        if (stages > 2) turn(s2t, steady_tag, first_tag, u, p, stages == 3);
+        if (stages > 3) turn(s3t, steady_tag, first_tag, u, p, true);
+    };
+    auto one_unit = [&](auto steady_tag, int u, int stages) {
+        one_part(steady_tag, std::true_type{}, u, 0, stages);
+        if constexpr (F32)
+            for (int p = 1; p < PARTS; ++p) one_part(steady_tag, std::false_type{}, u, p, stages);
+    };
     int u = 0;
-    for (; (u + 1) * PARTS * kUnitStages + STAGES <= total; ++u)
-        for (int p = 0; p < PARTS; ++p) {
-            turn(s0t, std::true_type{}, u, p, false);
-            turn(s1t, std::true_type{}, u, p, false);
-            turn(s2t, std::true_type{}, u, p, false);
-            turn(s3t, std::true_type{}, u, p, true);
-        }
-    for (; u < all_units; ++u) {
-        const int stages = u == all_units - 1 ? last_stages : kUnitStages;
-        for (int p = 0; p < PARTS; ++p) {
-            turn(s0t, std::false_type{}, u, p, stages == 1);
-            if (stages > 1) turn(s1t, std::false_type{}, u, p, stages == 2);
-            if (stages > 2) turn(s2t, std::false_type{}, u, p, stages == 3);
-            if (stages > 3) turn(s3t, std::false_type{}, u, p, true);
-        }
-    }
+    for (; (u + 1) * PARTS * kUnitStages + STAGES <= total; ++u) one_unit(std::true_type{}, u, kUnitStages);
+    for (; u < all_units; ++u) one_unit(std::false_type{}, u, u == all_units - 1 ? last_stages : kUnitStages);
 
     // ---- out ----
     // A sum that is not finite is worked out again by the lane that holds it, before anything is stored: the outputs of
@@ -281,24 +283,32 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
     constexpr int OUT_FN = MODE == kTwoWeights ? FN / 2 : FN;
     const int wave_n0 = (nb0 + wn * OUT_FN) * 16, wave_m0 = m0 + wm * FM * 16;
     static_assert(FN * FM * 4 <= 32, "a bit for each of a lane's sums");
-    uint32_t redo = 0;
+    bool fine = true;
+    float half = 0.5f;                                            // (the products are with +-2)
 #pragma unroll
     for (int f = 0; f < FN; ++f)
 #pragma unroll
         for (int m = 0; m < FM; ++m) {
-            acc[f][m] *= 0.5f;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const bool mine = wave_m0 + m * 16 + r16 < a.M && wave_n0 + f % OUT_FN * 16 + g * 4 + i < a.N;
-                redo |= mine && !(fabsf(acc[f][m][i]) < __builtin_huge_valf()) ? 1u << ((f * FM + m) * 4 + i) : 0u;
-            }
+            if constexpr (F32) add_low(acc[f][m], low[f][m]);
+            fine = fine && finite4(acc[f][m]);
         }
-    while (redo != 0) {
-        const int at = __builtin_ctz(redo), f = at / (FM * 4), m = at / 4 % FM;
-        redo &= redo - 1;
-        const float v = exact_output(a, f >= OUT_FN ? a.w1 : a.w0, wave_m0 + m * 16 + r16, wave_n0 + f % OUT_FN * 16 + g * 4 + at % 4);
+    if (!fine) {
+        uint32_t redo = 0;
 #pragma unroll
-        for (int e = 0; e < FN * FM * 4; ++e) acc[e / (FM * 4)][e / 4 % FM][e % 4] = e == at ? v : acc[e / (FM * 4)][e / 4 % FM][e % 4];
+        for (int e = 0; e < FN * FM * 4; ++e) {
+            const int f = e / (FM * 4), m = e / 4 % FM, i = e % 4;
+            const bool mine = wave_m0 + m * 16 + r16 < a.M && wave_n0 + f % OUT_FN * 16 + g * 4 + i < a.N;
+            redo |= mine && !(fabsf(acc[f][m][i]) < __builtin_huge_valf()) ? 1u << e : 0u;
+            acc[f][m][i] *= half;                                 // (twice what is worked out again might overflow)
+        }
+        half = 1.0f;
+        while (redo != 0) {
+            const int at = __builtin_ctz(redo), f = at / (FM * 4), m = at / 4 % FM;
+            redo &= redo - 1;
+            const float v = exact_output(a, f >= OUT_FN ? a.w1 : a.w0, wave_m0 + m * 16 + r16, wave_n0 + f % OUT_FN * 16 + g * 4 + at % 4);
+#pragma unroll
+            for (int e = 0; e < FN * FM * 4; ++e) acc[e / (FM * 4)][e / 4 % FM][e % 4] = e == at ? v : acc[e / (FM * 4)][e / 4 % FM][e % 4];
+        }
     }
 #pragma unroll
     for (int f = 0; f < OUT_FN; ++f) {
@@ -306,8 +316,8 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
         float s0[4], s1[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            s0[i] = n + i < a.N ? load_scale(a.w0.scale, a.scale_f16, n + i) : 0.f;
-            if constexpr (MODE == kTwoWeights) s1[i] = n + i < a.N ? load_scale(a.w1.scale, a.scale_f16, n + i) : 0.f;
+            s0[i] = half * (n + i < a.N ? load_scale(a.w0.scale, a.scale_f16, n + i) : 0.f);
+            if constexpr (MODE == kTwoWeights) s1[i] = half * (n + i < a.N ? load_scale(a.w1.scale, a.scale_f16, n + i) : 0.f);
         }
 #pragma unroll
         for (int m = 0; m < FM; ++m) {
@@ -430,8 +440,9 @@ int launch_tile(const KernelArgs& a, hipStream_t st)
 template <int PARTS>
 int launch_parts(const KernelArgs& a, bool two_weights, hipStream_t st)
 {
-    // 128 x 128 tiles, eight waves of 64 x 32: two workgroups share a compute unit (120 registers, 80 KB of LDS each), one of
-    // which multiplies while the other waits at a barrier or stores.  Best of the shapes tried at every size (fp16, us at
+    // 128 x 128 tiles, eight waves of 64 x 32: two workgroups share a compute unit in fp16 (114 registers, 80 KB of LDS each), one of
+    // which multiplies while the other waits at a barrier or stores (fp32, with its second set of sums, takes 188 registers:
+    // one workgroup a unit).  Best of the shapes tried at every size (fp16, us at
     // 1024 x 4096 -> 11008 / 1024 x 4096 -> 4096 / 8192 x 2048 -> 11008): 80 / 34 / 300; four waves of 64 x 64 86 / 40 / 306 or
     // 128 x 32 86 / 40 / 301; 128 x 256 tiles, eight waves of 64 x 64, one workgroup a unit 105 / 52 / 310; 256 x 192, eight of
     // 128 x 48, 84 / 72 / 370.

@@ -90,6 +90,29 @@ def test_activations_that_are_not_finite(cuda, M, dtype):
         assert torch.allclose(both, torch.nn.functional.silu(g) * g, rtol=1e-4, atol=1e-4, equal_nan=True)
 
 
+@pytest.mark.parametrize("M", [1, 4, 16, 48, 200])
+def test_activations_of_every_magnitude(cuda, M):
+    """Denormal and very large activations keep all their bits: exactly where a column has one entry, and in sums to what
+    their roundings give (2^-24 of the sum of magnitudes, once for each of the column's entries)."""
+    from ternaryllm_amd import ops
+    K, N = 520, 70
+    rng = np.random.default_rng(M)
+    rows, one = rng.integers(0, K, N), np.zeros((K, N), np.int32)
+    one[rows, np.arange(N)] = rng.choice([-1, 1], N)
+    w = ternary_weight(K, N, 0.6, 21)
+    d_one, dw = _device(one, cuda), _device(w, cuda)
+    for dtype, exponents in ((torch.float32, (-149, -140, -130, -126, -118, -110, -60, 60, 100, 115)), (torch.float16, (-24, -20, -14, 10))):
+        for e in exponents:
+            x = (activations(M, K, 22, torch.float64) * 2.0 ** e).to(dtype)
+            print(f"case M={M} {dtype} 2^{e}", flush=True)
+            y = ops.spmm(d_one, x.to(cuda)).cpu().numpy()
+            assert np.array_equal(y, x.numpy()[:, rows] * one[rows, np.arange(N)].astype(x.numpy().dtype)), e
+            xd, wd = x.double(), torch.from_numpy(w).double()
+            y = ops.spmm(dw, x.to(cuda), out_dtype=torch.float32).cpu().double()
+            bound = 2.0 ** -24 * (wd != 0).sum(0) * (xd.abs() @ wd.abs())
+            assert bool(((y - xd @ wd).abs() <= bound).all()), e
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 def test_finite_rows_keep_their_bits_beside_rows_that_are_not(cuda, dtype):
     """What a row holds does not show in the bits of another row's outputs."""
