@@ -31,6 +31,7 @@ struct WeightPtrs {
     const uint32_t* chunkstart;  // [NB * T + 1], dword offsets into stream
     const uint32_t* stream;      // chunks: 64 descriptors + runs of four 8-bit rows per dword
     const unsigned char* codes;  // two-bit codes [NB][planes][units], 1 KB each, or null
+    int planes;                  // ternary matrices that the codes hold
     const void* scale;           // per-column factor or null
 };
 
@@ -72,7 +73,7 @@ struct KernelArgs {
     const float* chain_sq_in; // [chain_sq_blocks][16] sums of squares of the rows X was made from: the product is multiplied by rsqrt(sum / K + eps), row by row
     int chain_sq_blocks;
     // matrix-core kernels
-    int units, planes;        // code units along K; ternary matrices the codes hold
+    int units, planes;        // code units along K; planes of the weight, of two weights the larger number
     const void* image;        // the activations they multiply: row-major, 16-byte pieces along K ...
     long long image_ld;       // ... elements between rows
     long long image_plane;    // ... and, for fp32 activations in three bf16 parts, between parts

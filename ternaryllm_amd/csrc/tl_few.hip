@@ -70,10 +70,14 @@ __global__ __launch_bounds__(kMaxWaves * 64) void tl_matrix_few(KernelArgs a)
     const int waves = (int)blockDim.x >> 6;
     const int g = lane >> 4, r16 = lane & 15;
     const int nb0 = (int)blockIdx.x * (TWO ? 1 : C);
-    const long long block_bytes = (long long)a.planes * a.units * TL_CODE_UNIT_BYTES;
     const unsigned char* codes[C];
+    int units[C];                                                  // that the block's weight has
 #pragma unroll
-    for (int c = 0; c < C; ++c) codes[c] = (TWO && c == 1 ? a.w1.codes : a.w0.codes) + min(TWO ? nb0 : nb0 + c, a.NB - 1) * block_bytes + lane * 16;
+    for (int c = 0; c < C; ++c) {
+        const WeightPtrs& weight = TWO && c == 1 ? a.w1 : a.w0;
+        units[c] = weight.planes * a.units;
+        codes[c] = weight.codes + min(TWO ? nb0 : nb0 + c, a.NB - 1) * ((long long)units[c] * TL_CODE_UNIT_BYTES) + lane * 16;
+    }
     const XT* rows[FM];
 #pragma unroll
     for (int f = 0; f < FM; ++f) rows[f] = static_cast<const XT*>(a.X) + min(f * 16 + r16, a.M - 1) * a.x_sm;
@@ -91,6 +95,11 @@ __global__ __launch_bounds__(kMaxWaves * 64) void tl_matrix_few(KernelArgs a)
         uint32_t w[C][4];
 #pragma unroll
         for (int c = 0; c < C; ++c) {
+            if (TWO && unit >= units[c]) {                         // (the other weight has more planes)
+#pragma unroll
+                for (int i = 0; i < Q; ++i) w[c][i] = 0u;
+                continue;
+            }
             const unsigned char* src = codes[c] + (long long)unit * TL_CODE_UNIT_BYTES + part * Q * 4;
             if constexpr (Q == 4) *reinterpret_cast<u32x4*>(w[c]) = *reinterpret_cast<const u32x4*>(src);
             else if constexpr (Q == 2) *reinterpret_cast<uint2*>(w[c]) = *reinterpret_cast<const uint2*>(src);

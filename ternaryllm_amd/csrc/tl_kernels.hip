@@ -78,6 +78,7 @@ WeightPtrs weight_ptrs(const tl_layout_header* h, const void* blob_dev, const vo
     w.chunkstart = reinterpret_cast<const uint32_t*>(b + h->off_chunkstart);
     w.stream = reinterpret_cast<const uint32_t*>(b + h->off_stream);
     w.codes = h->off_codes ? b + h->off_codes : nullptr;
+    w.planes = (int)h->code_planes;
     w.scale = scale;
     return w;
 }
@@ -198,7 +199,7 @@ int spmm_call(const tl_layout_header* header, const void* blob_dev, const void* 
     a.X = X; a.Y = Y;
     a.ldx = ldx; a.ldy = ldy;
     a.M = (int)M; a.N = (int)header->columns; a.K = (int)header->inners; a.T = (int)header->n_tiles; a.tile_rows = (int)header->tile_rows;
-    a.NB = (int)header->n_blocks; a.units = (int)header->code_units; a.planes = (int)header->code_planes;
+    a.NB = (int)header->n_blocks; a.units = (int)header->code_units; a.planes = a.w0.planes;
     a.x_f16 = x_dtype == TL_F16; a.x_kmajor = x_layout == TL_X_K_MAJOR; a.y_f16 = y_dtype == TL_F16; a.scale_f16 = scale_dtype == TL_F16;
     a.one = 1.0f;
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -251,8 +252,8 @@ int gate_up_call(bool few, const tl_layout_header* gate_header, const void* gate
     if (int rc = check_header(gate_header)) return rc;
     if (int rc = check_header(up_header)) return rc;
     if (gate_header->inners != up_header->inners || gate_header->columns != up_header->columns ||
-        gate_header->tile_rows != up_header->tile_rows || gate_header->code_planes != up_header->code_planes)
-        return fail(TL_ERR_SHAPE, "gate and up weights must share K, N, tile height and code planes");
+        gate_header->tile_rows != up_header->tile_rows)
+        return fail(TL_ERR_SHAPE, "gate and up weights must share K, N and tile height");
     if (activation != TL_ACT_SILU_GATE) return fail(TL_ERR_UNSUPPORTED, "activation code %d (only TL_ACT_SILU_GATE)", activation);
     if (!up_blob_dev || reinterpret_cast<uintptr_t>(up_blob_dev) % 256) return fail(TL_ERR_ALIGN, "up blob null or not 256-byte aligned");
     if (int rc = check_io(gate_blob_dev, X, H, x_dtype, x_layout, ldx, M, h_dtype, ldh, gate_scale, scale_dtype, gate_header)) return rc;
@@ -266,7 +267,7 @@ int gate_up_call(bool few, const tl_layout_header* gate_header, const void* gate
     a.w1 = weight_ptrs(up_header, up_blob_dev, up_scale);
     a.X = X; a.Y = H;
     a.ldx = ldx; a.ldy = ldh;
-    a.NB = (int)gate_header->n_blocks; a.units = (int)gate_header->code_units; a.planes = (int)gate_header->code_planes;
+    a.NB = (int)gate_header->n_blocks; a.units = (int)gate_header->code_units; a.planes = std::max(a.w0.planes, a.w1.planes);
     a.M = (int)M; a.N = (int)gate_header->columns; a.K = (int)gate_header->inners; a.T = (int)gate_header->n_tiles;
     a.tile_rows = (int)gate_header->tile_rows;
     a.x_f16 = x_dtype == TL_F16; a.x_kmajor = x_layout == TL_X_K_MAJOR; a.y_f16 = h_dtype == TL_F16; a.scale_f16 = scale_dtype == TL_F16;

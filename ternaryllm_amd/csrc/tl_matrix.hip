@@ -18,6 +18,7 @@ constexpr int kStageRowBytes = kStageRows * 2;       // bytes of one activation 
 // with all 64 row tiles in one group (every column tile streamed all activations through an L2), 300 / 300 / 310 with 2 / 4 / 8.
 constexpr int kRowGroup = 4;
 constexpr int kUnitStages = TL_CODE_UNIT_ROWS / kStageRows;
+__device__ __align__(16) const unsigned char kNoCodes[TL_CODE_UNIT_BYTES] = {};   // a unit of zero weights
 
 // 16 bytes per lane from `base` + offset into LDS at `lds` + 16 * lane.  (As assembly, because the compiler would wait for
 // all such loads before any read of LDS; here they are counted by hand.)
@@ -125,7 +126,6 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
     }
     const unsigned char* image = static_cast<const unsigned char*>(a.image) + (long long)m0 * a.image_ld * 2;
     const long long unit_stride = TL_CODE_UNIT_BYTES;
-    const long long block_stride = (long long)a.planes * a.units * unit_stride;
 
     const int stages_k = (a.K + kStageRows - 1) / kStageRows;     // stages of K that hold anything
     const int all_units = a.planes * a.units;
@@ -154,18 +154,24 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
     };
     const unsigned char* code_src[CL];                            // (wave-uniform)
     uint32_t code_to[CL];
+    int code_units[CL];                                           // units that the block's weight has
 #pragma unroll
     for (int i = 0; i < CL; ++i) {
         const int c = min(i * W + wave, TN / 16 - 1);             // column block of the tile
         const int owner = c / FN, f = c % FN;                     // its wave column and fragment
         const WeightPtrs& w = (MODE == kTwoWeights && f >= FN / 2) ? a.w1 : a.w0;
         const int nb = MODE == kTwoWeights ? nb0 + owner * (FN / 2) + f % (FN / 2) : nb0 + c;
-        code_src[i] = w.codes + min(nb, a.NB - 1) * block_stride;
+        code_units[i] = w.planes * a.units;
+        code_src[i] = w.codes + min(nb, a.NB - 1) * (code_units[i] * unit_stride);
         code_to[i] = lds0 + STAGES * XB + c * TL_CODE_UNIT_BYTES;
     }
     auto issue_codes = [&](int u) {
 #pragma unroll
-        for (int i = 0; i < CL; ++i) load_to_lds(code_to[i] + (u & 1) * CB, code_src[i] + u * unit_stride, (uint32_t)lane * 16);
+        for (int i = 0; i < CL; ++i) {
+            const unsigned char* src = code_src[i] + u * unit_stride;
+            if (MODE == kTwoWeights && u >= code_units[i]) src = kNoCodes;   // (the other weight has more planes)
+            load_to_lds(code_to[i] + (u & 1) * CB, src, (uint32_t)lane * 16);
+        }
     };
 
     // ---- what it reads ----

@@ -239,18 +239,18 @@ def spmm_chain(weight, x, scale=None, x_layout=_lib.TL_X_ROW_MAJOR, residual=Non
 
 def mlp_gate_up(gate, up, x, gate_scale=None, up_scale=None, out_dtype=None):
     """h[M, N] = silu((x @ Wg) * sg) * ((x @ Wu) * su) in one pass over x, or two products where no kernel does it: one
-    row (its own kernel is the faster one), weights without codes or of different tile heights, up to 48 rows whose two
-    scales are not of one kind."""
+    row (its own kernel is the faster one), weights of different tile heights, up to 48 rows of a weight without codes or
+    whose two scales are not of one kind."""
     if gate.columns != up.columns or gate.inners != up.inners:
         raise ValueError("gate and up weights must have the same shape")
     x_code = _code(x.dtype, "x")
     x, M, ldx = _x_geometry(x, gate.inners, _lib.TL_X_ROW_MAJOR)
     N = gate.columns
     out_dtype = out_dtype or x.dtype
-    alike = gate.header.tile_rows == up.header.tile_rows and gate.header.code_planes == up.header.code_planes
     scales_alike = (gate_scale is None) == (up_scale is None) and (gate_scale is None or gate_scale.dtype == up_scale.dtype)
-    few = 2 <= M <= 48 and alike and scales_alike and gate.header.off_codes != 0 and x.device == gate.device == up.device
-    if (M <= 48 and not few) or gate.header.tile_rows != up.header.tile_rows:
+    alike = gate.header.tile_rows == up.header.tile_rows
+    few = 2 <= M <= 48 and scales_alike and gate.header.off_codes != 0 and up.header.off_codes != 0 and x.device == gate.device == up.device
+    if (M <= 48 and not few) or not alike:
         g = spmm(gate, x, gate_scale, torch.float32)
         u = spmm(up, x, up_scale, torch.float32)
         return (torch.nn.functional.silu(g) * u).to(out_dtype)

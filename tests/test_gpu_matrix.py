@@ -40,22 +40,48 @@ def test_many_rows_at_the_edges(cuda, oracle, M, K, N, dtype):
         assert np.array_equal(y, x.numpy()[:, rows] * one[rows, np.arange(N)].astype(np.float32))
 
 
+def _repeated(w):
+    """The packed weight of tiled-CSC arrays that name a row |entry| times."""
+    from ternaryllm_amd.packing import PackedWeight
+    K, N = w.shape
+    neg, pos, neg_off, pos_off = [], [], np.zeros((N, 1, 2), np.int32), np.zeros((N, 1, 2), np.int32)
+    for y in range(N):
+        for rows, off, sign in ((neg, neg_off, -1), (pos, pos_off, 1)):
+            off[y, 0, 0] = len(rows)
+            for k in range(K):
+                rows += [k] * max(0, sign * int(w[k, y]))
+            off[y, 0, 1] = len(rows)
+    return PackedWeight.from_tiled_csc(np.array(neg, np.int32), neg_off.reshape(-1), np.array(pos, np.int32), pos_off.reshape(-1), N, K, K)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M", [2, 16, 48, 49, 130])
+def test_gate_and_up_of_different_planes(cuda, M, dtype):
+    """A gate that names rows three times beside an up weight that does not, and the other way round."""
+    from ternaryllm_amd import ops
+    K, N = 600, 72
+    rng = np.random.default_rng(7)
+    often, once = rng.integers(-3, 4, (K, N)) * (rng.random((K, N)) < 0.3), ternary_weight(K, N, 0.7, 8)
+    pw = _repeated(often)
+    assert pw.header.code_planes == 3
+    d_often, d_once = ops.DeviceWeight(pw, cuda), _device(once, cuda)
+    x = activations(M, K, 6, dtype, integer=True) / 16
+    for (dg, wg), (du, wu) in (((d_often, often), (d_once, once)), ((d_once, once), (d_often, often))):
+        print(f"case M={M} {dtype} gate planes {dg.header.code_planes}", flush=True)
+        got = ops.mlp_gate_up(dg, du, x.to(cuda), out_dtype=torch.float32).double().cpu()
+        want = torch.nn.functional.silu(x.double() @ torch.from_numpy(wg).double()) * (x.double() @ torch.from_numpy(wu).double())
+        # exact sums; a few units in the last place of __expf and of the division
+        assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())
+
+
 @pytest.mark.parametrize("M", [1, 5, 16, 40, 64, 200])
 def test_entries_beyond_one(cuda, M):
     """Arrays that name a row several times make entries up to 3: the codes hold a plane for each mention."""
     from ternaryllm_amd import ops
-    from ternaryllm_amd.packing import PackedWeight
     rng = np.random.default_rng(5)
     for K, N in ((100, 20), (600, 40)):
         w = rng.integers(-3, 4, (K, N)) * (rng.random((K, N)) < 0.3)
-        neg, pos, neg_off, pos_off = [], [], np.zeros((N, 1, 2), np.int32), np.zeros((N, 1, 2), np.int32)
-        for y in range(N):
-            for rows, off, sign in ((neg, neg_off, -1), (pos, pos_off, 1)):
-                off[y, 0, 0] = len(rows)
-                for k in range(K):
-                    rows += [k] * max(0, sign * int(w[k, y]))
-                off[y, 0, 1] = len(rows)
-        pw = PackedWeight.from_tiled_csc(np.array(neg, np.int32), neg_off.reshape(-1), np.array(pos, np.int32), pos_off.reshape(-1), N, K, K)
+        pw = _repeated(w)
         pw.validate()
         assert pw.header.code_planes == 3 and np.array_equal(pw.to_dense(), w)
         x = activations(M, K, 6, torch.float32, integer=True)
