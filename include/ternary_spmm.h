@@ -247,7 +247,9 @@ int tl_spmm_workspace(const tl_layout_header* header, int64_t M, int x_dtype, in
  *   Y           device, y_dtype, row-major [M][ldy]
  *   scale       device per-output-column factor of scale_dtype, or NULL (the
  *               reference has none; its result equals scale == NULL)
- *   workspace   device scratch of at least tl_spmm_workspace() bytes (may be NULL when 0)
+ *   workspace   device scratch of tl_spmm_workspace() bytes (may be NULL when 0).  For more than 48 rows less is
+ *               accepted, down to the bytes of the activations (M * K values of x_dtype): what is staged there is
+ *               then staged some rows at a time
  * Accumulation is always fp32. */
 int tl_spmm(const tl_layout_header* header, const void* blob_dev,
             const void* X, int x_dtype, int x_layout, int64_t ldx, int64_t M,
@@ -257,10 +259,11 @@ int tl_spmm(const tl_layout_header* header, const void* blob_dev,
 
 /* tl_spmm for callers that cannot allocate or pass a workspace: code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the reference.  Same
- * arguments and result as tl_spmm, minus the workspace: what tl_spmm stages there (the K-major image of the
- * activations) goes into a 32 MiB array inside the library's device code, one copy per GPU, held until
- * the process ends.  The call allocates and frees nothing.  TL_ERR_SIZE when the image would not fit
- * (e.g. 1024 x 11008 fp16 fits, 1024 x 11008 fp32 does not).  The kernels write every byte of the array
+ * arguments and result as tl_spmm, minus the workspace: what tl_spmm stages there (an image of the
+ * activations) goes into a 48 MiB array inside the library's device code, one copy per GPU, held until
+ * the process ends.  The call allocates and frees nothing.  TL_ERR_SIZE when neither the image fits (two bytes a
+ * value, for more than 48 fp32 rows six) nor the activations are 32 MiB or less: 1024 x 11008 fp16 and 2048 x 4096 fp32
+ * are taken, 1024 x 11008 fp32 is not.  The kernels write every byte of the array
  * before they read it, so nothing is cleared between calls; all calls on one GPU share the array, so
  * calls that may overlap on one GPU (different streams) race -- keep them on one stream or use tl_spmm.
  * The first call on a device looks the array's address up; make it outside graph capture. */

@@ -186,11 +186,14 @@ int launch_small(KernelArgs a, const tl_layout_header* h, int x_dtype, void* wor
 bool walk_has_gated(const KernelArgs& a, const tl_layout_header* h);
 
 // tl_matrix.hip
-// The row-major image of the activations where the kernel does not read them as they lie: two bytes a value, for fp32
-// three times two.
-inline int64_t matrix_image_bytes(int64_t K, int64_t M, int x_dtype)
+// Bytes of a row of the image of the activations, which is row-major, where the kernel does not read them as they lie: two
+// a value, for fp32 three times two.
+inline int64_t image_row_bytes(int64_t K, int x_dtype) { return round_up(K, 8) * 2 * (x_dtype == TL_F16 ? 1 : 3); }
+// The smallest workspace of such a call: the image of all rows, or, where that is more, the bytes of the activations
+// themselves -- the image is then made and multiplied some rows at a time.
+inline int64_t least_image_bytes(int64_t K, int64_t M, int x_dtype)
 {
-    return round_up(M, 256) * round_up(K, 8) * 2 * (x_dtype == TL_F16 ? 1 : 3) + 256;
+    return std::min(M * image_row_bytes(K, x_dtype), M * K * (x_dtype == TL_F16 ? 2 : 4));
 }
 int launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t workspace_bytes, bool two_weights, hipStream_t st);
 

@@ -128,7 +128,8 @@ extern "C" int tl_spmm_workspace(const tl_layout_header* header, int64_t M, int 
         *workspace_bytes = small_kmajor_bytes(header, M, x_dtype);
         return TL_OK;
     }
-    *workspace_bytes = matrix_image_bytes(header->inners, M, x_dtype);
+    // the image of all rows, in whole 256 of them, so that a caller's buffer serves nearby row counts too
+    *workspace_bytes = round_up(M, 256) * image_row_bytes(header->inners, x_dtype);
     return TL_OK;
 }
 
@@ -305,7 +306,8 @@ extern "C" int tl_mlp_gate_up_few(const tl_layout_header* gate_header, const voi
 
 // Scratch of tl_spmm_noalloc: device memory that belongs to the library's code object, one copy per GPU,
 // there from the moment the library is loaded on a device until the process ends.
-constexpr int64_t kStaticScratchBytes = 48ll << 20;  // (fp32 rows of 32 MiB are 48 MiB in three bf16 parts)
+constexpr int64_t kActivationBytes = 32ll << 20;
+constexpr int64_t kStaticScratchBytes = kActivationBytes / 2 * 3;  // fp32 rows in three bf16 parts
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 namespace {
@@ -338,8 +340,11 @@ extern "C" int tl_spmm_noalloc(const tl_layout_header* header, const void* blob_
     if (int rc = check_header(header)) return rc;
     if (int rc = check_dtype(x_dtype, "x")) return rc;
     if (M <= 0) return fail(TL_ERR_SHAPE, "M=%lld must be positive", (long long)M);
-    // what the kernels stage in the scratch: the image of the activations (none for 4 rows and fewer)
-    const int64_t need = M <= kSmallMaxM ? small_kmajor_bytes(header, M, x_dtype) : matrix_image_bytes(header->inners, M, x_dtype);
+    // what the kernels stage in the scratch: the image of the activations (none for 4 rows and fewer).  32 MiB of
+    // activations are always taken, as an image that does not fit is made some rows at a time.
+    const int64_t image = M * image_row_bytes(header->inners, x_dtype);
+    int64_t need = M <= kSmallMaxM ? small_kmajor_bytes(header, M, x_dtype) : image;
+    if (M > kSmallMaxM && image > kStaticScratchBytes && least_image_bytes(header->inners, M, x_dtype) <= kActivationBytes) need = kStaticScratchBytes;
     if (need > kStaticScratchBytes)
         return fail(TL_ERR_SIZE, "M=%lld rows of K=%u need %lld bytes of scratch; tl_spmm_noalloc has %lld (use tl_spmm with a workspace)",
                     (long long)M, header->inners, (long long)need, (long long)kStaticScratchBytes);

@@ -456,6 +456,27 @@ int launch_parts(const KernelArgs& a, bool two_weights, hipStream_t st)
     return a.gated ? launch_tile<PARTS, 2, 4, 4, 2, 4, kPairs>(a, st) : launch_tile<PARTS, 2, 4, 4, 2, 4, kPlain>(a, st);
 }
 
+// The image of a call's activations (a.image_ld and a.image_plane say how it lies).
+void make_image(const KernelArgs& a, int x_dtype, unsigned short* image, hipStream_t st)
+{
+    if (a.x_kmajor) {
+        const dim3 grid((unsigned)ceil_div(a.K, 64), (unsigned)ceil_div(a.M, 64));
+        if (x_dtype == TL_F16) hipLaunchKernelGGL(tl_x_image_k<__half>, grid, dim3(256), 0, st, a, image);
+        else hipLaunchKernelGGL(tl_x_image_k<float>, grid, dim3(256), 0, st, a, image);
+        return;
+    }
+    const int64_t pieces = ceil_div(a.K, 8);
+    const int64_t rows = std::max<int64_t>(1, ((int64_t)1 << 30) / pieces);  // of a launch, which counts its pieces in 32 bits
+    for (int64_t m = 0; m < a.M; m += rows) {
+        KernelArgs some = a;
+        some.X = static_cast<const unsigned char*>(a.X) + m * a.ldx * (x_dtype == TL_F16 ? 2 : 4);
+        some.M = (int)std::min<int64_t>(a.M - m, rows);
+        const dim3 grid((unsigned)ceil_div(pieces * some.M, 256));
+        if (x_dtype == TL_F16) hipLaunchKernelGGL(tl_x_image<__half>, grid, dim3(256), 0, st, some, image + m * a.image_ld);
+        else hipLaunchKernelGGL(tl_x_image<float>, grid, dim3(256), 0, st, some, image + m * a.image_ld);
+    }
+}
+
 }  // namespace
 
 int tl::launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t workspace_bytes, bool two_weights, hipStream_t st)
@@ -466,41 +487,34 @@ int tl::launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t w
         hipLaunchKernelGGL(tl_walk, dim3((unsigned)ceil_div(outputs, 256)), dim3(256), 0, st, a, mode);
         return TL_OK;
     }
-    // rows that lie as the kernel reads them are read where they are; any other layout, and fp32, goes through the image
-    const bool direct = x_dtype == TL_F16 && !a.x_kmajor && a.K % 8 == 0 && a.ldx % 8 == 0 && reinterpret_cast<uintptr_t>(a.X) % 16 == 0;
-    if (direct) {
-        a.image = a.X;
-        a.image_ld = a.ldx;
-    } else {
-        const int64_t need = matrix_image_bytes(a.K, a.M, x_dtype);
-        if (!workspace || workspace_bytes < need)
-            return fail(TL_ERR_SIZE, "workspace has %lld bytes, %lld needed", (long long)workspace_bytes, (long long)need);
-        if (reinterpret_cast<uintptr_t>(workspace) % 16) return fail(TL_ERR_ALIGN, "workspace must be 16-byte aligned");
-        if (a.x_kmajor && a.M > 65535 * 64) return fail(TL_ERR_SHAPE, "M=%d K-major rows are too many for one call", a.M);
-        unsigned short* image = static_cast<unsigned short*>(workspace);
-        a.image = image;
-        a.image_ld = round_up(a.K, 8);
-        a.image_plane = a.image_ld * a.M;
-        if (a.x_kmajor) {
-            const dim3 grid((unsigned)ceil_div(a.K, 64), (unsigned)ceil_div(a.M, 64));
-            if (x_dtype == TL_F16) hipLaunchKernelGGL(tl_x_image_k<__half>, grid, dim3(256), 0, st, a, image);
-            else hipLaunchKernelGGL(tl_x_image_k<float>, grid, dim3(256), 0, st, a, image);
-        } else {
-            const int64_t pieces = ceil_div(a.K, 8);
-            const int64_t rows = std::max<int64_t>(1, ((int64_t)1 << 30) / pieces);  // of a launch, which counts its pieces in 32 bits
-            for (int64_t m = 0; m < a.M; m += rows) {
-                KernelArgs some = a;
-                some.X = static_cast<const unsigned char*>(a.X) + m * a.ldx * (x_dtype == TL_F16 ? 2 : 4);
-                some.M = (int)std::min<int64_t>(a.M - m, rows);
-                const dim3 grid((unsigned)ceil_div(pieces * some.M, 256));
-                if (x_dtype == TL_F16) hipLaunchKernelGGL(tl_x_image<__half>, grid, dim3(256), 0, st, some, image + m * a.image_ld);
-                else hipLaunchKernelGGL(tl_x_image<float>, grid, dim3(256), 0, st, some, image + m * a.image_ld);
-            }
-        }
-    }
-    if (a.image_ld * 256 * 2 >= (int64_t)1 << 32)  // the kernel keeps a lane's byte offset inside a row tile in 32 bits
-        return fail(TL_ERR_ARG, "rows of %lld activations are too long for one call", (long long)a.image_ld);
     const uintptr_t y_align = a.y_f16 ? 8 : 16;
     a.vector_out = a.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(a.Y) % y_align == 0;
-    return x_dtype == TL_F16 ? launch_parts<1>(a, two_weights, st) : launch_parts<3>(a, two_weights, st);
+    // rows that lie as the kernel reads them are read where they are; any other layout, and fp32, goes through the image
+    const bool direct = x_dtype == TL_F16 && !a.x_kmajor && a.K % 8 == 0 && a.ldx % 8 == 0 && reinterpret_cast<uintptr_t>(a.X) % 16 == 0;
+    a.image_ld = direct ? a.ldx : round_up(a.K, 8);
+    if (a.image_ld * 256 * 2 >= (int64_t)1 << 32)  // the kernel keeps a lane's byte offset inside a row tile in 32 bits
+        return fail(TL_ERR_ARG, "rows of %lld activations are too long for one call", (long long)a.image_ld);
+    if (direct) {
+        a.image = a.X;
+        return launch_parts<1>(a, two_weights, st);
+    }
+    const int64_t need = least_image_bytes(a.K, a.M, x_dtype);
+    if (!workspace || workspace_bytes < need)
+        return fail(TL_ERR_SIZE, "workspace has %lld bytes, %lld needed", (long long)workspace_bytes, (long long)need);
+    if (reinterpret_cast<uintptr_t>(workspace) % 16) return fail(TL_ERR_ALIGN, "workspace must be 16-byte aligned");
+    if (a.x_kmajor && a.M > 65535 * 64) return fail(TL_ERR_SHAPE, "M=%d K-major rows are too many for one call", a.M);
+    // all rows at once where their image fits, else as many whole row tiles as do
+    int64_t rows = std::min<int64_t>(a.M, workspace_bytes / image_row_bytes(a.K, x_dtype));
+    if (rows < a.M && rows > 128) rows = rows / 128 * 128;
+    a.image = workspace;
+    for (int64_t m = 0; m < a.M; m += rows) {
+        KernelArgs some = a;
+        some.M = (int)std::min<int64_t>(a.M - m, rows);
+        some.X = static_cast<const unsigned char*>(a.X) + m * (a.x_kmajor ? 1 : a.ldx) * (x_dtype == TL_F16 ? 2 : 4);
+        some.Y = static_cast<unsigned char*>(a.Y) + m * a.ldy * (a.y_f16 ? 2 : 4);
+        some.image_plane = a.image_ld * some.M;
+        make_image(some, x_dtype, static_cast<unsigned short*>(workspace), st);
+        if (int rc = x_dtype == TL_F16 ? launch_parts<1>(some, two_weights, st) : launch_parts<3>(some, two_weights, st)) return rc;
+    }
+    return TL_OK;
 }

@@ -30,6 +30,25 @@ def _call(fn_name, dw, x, scale, ws=None):
     return y
 
 
+@pytest.mark.parametrize("M,K", [(2048, 4096), (49, 32768), (100, 40000), (300, 20000), (385, 16384), (1300001, 3), (2100000, 3)])
+def test_activations_of_up_to_32_mib(cuda, M, K):
+    """fp32, whose image is larger than the activations: whole where it fits the scratch, else some rows at a time; the
+    same with a workspace of no more than the activations' size, and nothing with less."""
+    from ternaryllm_amd import ops
+    from ternaryllm_amd.packing import PackedWeight
+    N = 24
+    dw = ops.DeviceWeight(PackedWeight.from_dense(ternary_weight(K, N, 0.7, 132)), cuda)
+    x = torch.randn((M, K), generator=torch.Generator(device=cuda).manual_seed(M), device=cuda)
+    ones = torch.ones(N, device=cuda)
+    print(f"case noalloc M={M} K={K}", flush=True)
+    want = ops.spmm(dw, x, ones)
+    assert torch.equal(_call("tl_spmm_noalloc", dw, x, ones), want)
+    ws = torch.empty(M * K * 4, dtype=torch.uint8, device=cuda)
+    assert torch.equal(_call("tl_spmm", dw, x, ones, ws), want)
+    with pytest.raises(ValueError, match="workspace"):
+        _call("tl_spmm", dw, x, ones, ws[:-16])
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 def test_noalloc_entry_point_equals_tl_spmm(cuda, oracle, dtype):
     from ternaryllm_amd import _lib, ops
