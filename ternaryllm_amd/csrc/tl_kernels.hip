@@ -350,7 +350,7 @@ extern "C" int tl_spmm_noalloc(const tl_layout_header* header, const void* blob_
                     (long long)M, header->inners, (long long)need, (long long)kStaticScratchBytes);
     void* ws = nullptr;
     if (int rc = static_scratch(&ws)) return rc;
-    return tl_spmm(header, blob_dev, X, x_dtype, x_layout, ldx, M, Y, y_dtype, ldy, scale, scale_dtype, ws, need, stream);
+    return tl_spmm(header, blob_dev, X, x_dtype, x_layout, ldx, M, Y, y_dtype, ldy, scale, scale_dtype, ws, kStaticScratchBytes, stream);
 }
 
 // Reads `pieces` 16-byte pieces and folds them: what streaming that much memory costs a launch that writes next to

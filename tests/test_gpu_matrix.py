@@ -154,6 +154,59 @@ def test_finite_rows_keep_their_bits_beside_rows_that_are_not(cuda, dtype):
         assert torch.equal(call(x)[keep], call(spoilt)[keep]), name
 
 
+def _without_codes(new, cuda):
+    """The device weight of the blob that the version before the codes would have made."""
+    from ternaryllm_amd import _lib, ops
+    old = new.blob[:new.header.off_codes].copy()
+    h = _lib.LayoutHeader.from_buffer_copy(old[:256].tobytes())
+    h.version, h.off_codes, h.code_units, h.code_planes, h.total_bytes = 5, 0, 0, 0, old.size
+    old[:256] = np.frombuffer(bytes(h), np.uint8)
+    dev = ops.DeviceWeight.__new__(ops.DeviceWeight)
+    dev.header, dev.blob = h, torch.from_numpy(old).to(cuda)
+    return dev
+
+
+def _product(dw, x, layout, M, ldx, ws):
+    """tl_spmm with just this workspace."""
+    import ctypes
+    from ternaryllm_amd import _lib
+    y = torch.full((M, dw.columns), 7.0, dtype=torch.float32, device=x.device)
+    rc = _lib.lib().tl_spmm(ctypes.byref(dw.header), dw.blob.data_ptr(), x.data_ptr(), _lib.TL_F16 if x.dtype == torch.float16 else _lib.TL_F32,
+                            layout, ldx, M, y.data_ptr(), _lib.TL_F32, dw.columns, None, _lib.TL_F32, ws.data_ptr() if ws is not None else None,
+                            ws.numel() if ws is not None else 0, ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream))
+    return rc, y
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M,K,N", [(49, 3, 5), (128, 250, 16), (129, 248, 66), (257, 600, 131), (300, 1003, 64)])
+def test_the_index_stream_alone(cuda, oracle, M, K, N, dtype):
+    """More than 48 rows of a weight without codes, in every layout, with a workspace and without."""
+    from ternaryllm_amd import ops
+    from ternaryllm_amd.packing import PackedWeight
+    w, w2 = ternary_weight(K, N, 0.6, M + K), ternary_weight(K, N, 0.7, M + N)
+    new = PackedWeight.from_dense(w)
+    dw, old, old2 = ops.DeviceWeight(new, cuda), _without_codes(new, cuda), _without_codes(PackedWeight.from_dense(w2), cuda)
+    x = activations(M, K, M, dtype, integer=True)
+    ref = oracle.fast_product(x.double().numpy(), w)
+    ld = (M + 255) // 256 * 256
+    padded = torch.full((K, ld), 9.0, dtype=dtype)
+    padded[:, :M] = x.t()
+    forms = {"rows": (x.to(cuda), 0, K), "k-major": (x.t().contiguous().to(cuda), 1, M), "k-major padded": (padded.to(cuda), 1, ld)}
+    ws = torch.empty(K * ld * 4, dtype=torch.uint8, device=cuda)
+    for name, (xd, layout, ldx) in forms.items():
+        for weight, space in ((old, None), (old, ws)):
+            print(f"case {name} {dtype} codes={weight is dw} workspace={space is not None}", flush=True)
+            rc, y = _product(weight, xd, layout, M, ldx, space)
+            assert rc == 0 and np.array_equal(y.cpu().numpy().astype(np.float64), ref)
+    xd = x.to(cuda) / 16
+    if N % 2 == 0:
+        assert torch.equal(ops.spmm_gated(old, xd), ops.silu_mul(ops.spmm(old, xd), pairs=True))
+    for g, u in ((old, old2), (dw, old2), (old, dw)):
+        got = ops.mlp_gate_up(g, u, xd, out_dtype=torch.float32).double().cpu()
+        want = torch.nn.functional.silu(xd.double().cpu() @ torch.from_numpy(w).double()) * (xd.double().cpu() @ torch.from_numpy(w2 if u is old2 else w).double())
+        assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())   # exact sums; __expf and the division
+
+
 def test_a_blob_without_codes(cuda, oracle):
     """What an older version packed: the packed-weight object brings it up to date, and a device blob that was not is
     multiplied by the general kernel."""
