@@ -409,7 +409,7 @@ __global__ __launch_bounds__(256) void tl_x_image_k(KernelArgs a, unsigned short
     }
 }
 
-// The product from the index stream alone, for blobs without codes.  A wave owns
+// The product from the index stream alone, for blobs without codes and for K-major rows without a workspace.  A wave owns
 // 64 * R rows and four columns, so indices are wave-uniform (scalar loads); R neighbouring rows of a lane are one 8-byte
 // piece.  Bound by those loads: 16 waves, 64 columns, share the pieces of a tile of K-major activations in LDS (us, 80 %
 // zeros, fp16 / fp32: 1024 x 4096 -> 11008 967 / 1259, 200 x 2048 -> 2048 143 / 87; one thread per output took 46038 / 46556
@@ -627,8 +627,8 @@ int tl::launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t w
     a.x_sm = a.x_kmajor ? 1 : a.ldx;
     a.x_sk = a.x_kmajor ? a.ldx : 1;
     const int64_t need = least_image_bytes(a.K, a.M, x_dtype);
-    // Without codes the index stream is walked.
-    if (!a.w0.codes || (two_weights && !a.w1.codes))
+    // Without codes, and for K-major rows that need no workspace, the index stream is walked.
+    if (!a.w0.codes || (two_weights && !a.w1.codes) || ((!workspace || workspace_bytes < need) && walk_reads_directly(a)))
         return x_dtype == TL_F16 ? walk_rows<__half>(a, workspace, workspace_bytes, two_weights, st)
                                  : walk_rows<float>(a, workspace, workspace_bytes, two_weights, st);
     const uintptr_t y_align = a.y_f16 ? 8 : 16;
