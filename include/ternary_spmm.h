@@ -249,7 +249,7 @@ int tl_spmm_workspace(const tl_layout_header* header, int64_t M, int x_dtype, in
  *               reference has none; its result equals scale == NULL)
  *   workspace   device scratch of tl_spmm_workspace() bytes (may be NULL when 0).  For more than 48 rows less is
  *               accepted, down to the bytes of the activations (M * K values of x_dtype): what is staged there is
- * *               then staged some rows at a time.  K-major rows whose leading dimension is a multiple of 256 (fp32 128)
+ *               then staged some rows at a time.  K-major rows whose leading dimension is a multiple of 256 (fp32 128)
  *               and holds whole 256 (128) rows, from a 16-byte aligned address, need none (they take longer without)
  * Accumulation is always fp32. */
 int tl_spmm(const tl_layout_header* header, const void* blob_dev,

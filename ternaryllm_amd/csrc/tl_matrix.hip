@@ -634,9 +634,10 @@ int tl::launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t w
     const uintptr_t y_align = a.y_f16 ? 8 : 16;
     a.vector_out = a.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(a.Y) % y_align == 0;
     // rows that lie as the kernel reads them are read where they are; any other layout, and fp32, goes through the image
-    const bool direct = x_dtype == TL_F16 && !a.x_kmajor && a.K % 8 == 0 && a.ldx % 8 == 0 && reinterpret_cast<uintptr_t>(a.X) % 16 == 0;
+    constexpr int64_t kMostLd = 1 << 24;  // (a lane's byte offset inside the 128 rows of a tile has 32 bits)
+    const bool direct = x_dtype == TL_F16 && !a.x_kmajor && a.K % 8 == 0 && a.ldx % 8 == 0 && a.ldx <= kMostLd && reinterpret_cast<uintptr_t>(a.X) % 16 == 0;
     a.image_ld = direct ? a.ldx : round_up(a.K, 8);
-    if (a.image_ld * 256 * 2 >= (int64_t)1 << 32)  // the kernel keeps a lane's byte offset inside a row tile in 32 bits
+    if (a.image_ld > kMostLd)
         return fail(TL_ERR_ARG, "rows of %lld activations are too long for one call", (long long)a.image_ld);
     if (direct) {
         a.image = a.X;
@@ -645,9 +646,9 @@ int tl::launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t w
     if (!workspace || workspace_bytes < need)
         return fail(TL_ERR_SIZE, "workspace has %lld bytes, %lld needed", (long long)workspace_bytes, (long long)need);
     if (reinterpret_cast<uintptr_t>(workspace) % 16) return fail(TL_ERR_ALIGN, "workspace must be 16-byte aligned");
-    if (a.x_kmajor && a.M > 65535 * 64) return fail(TL_ERR_SHAPE, "M=%d K-major rows are too many for one call", a.M);
-    // all rows at once where their image fits, else as many whole row tiles as do
+    // all rows at once where their image fits (and its launch's second dimension holds them), else as many whole row tiles as do
     int64_t rows = std::min<int64_t>(a.M, workspace_bytes / image_row_bytes(a.K, x_dtype));
+    if (a.x_kmajor) rows = std::min<int64_t>(rows, 65535 * 64);
     if (rows < a.M && rows > 128) rows = rows / 128 * 128;
     a.image = workspace;
     for (int64_t m = 0; m < a.M; m += rows) {

@@ -211,6 +211,23 @@ def test_the_index_stream_alone(cuda, oracle, M, K, N, dtype):
         assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())   # exact sums; __expf and the division
 
 
+@pytest.mark.parametrize("M,K,ld", [(60, 64, 1 << 23), (60, 64, (1 << 24) + 8), (4300000, 16, 0)])
+def test_rows_far_apart_and_very_many_of_them(cuda, M, K, ld):
+    """Row-major rows whose distance the kernel cannot address go through the image; K-major ones in several passes where one
+    launch's image cannot hold them (ld = 0)."""
+    from ternaryllm_amd import ops
+    N = 24
+    w = ternary_weight(K, N, 0.5, 31)
+    x = torch.randint(-8, 9, (K, M) if ld == 0 else (M, K), generator=torch.Generator(device=cuda).manual_seed(1), device=cuda).half()
+    want = (x.t() if ld == 0 else x).float() @ torch.from_numpy(w).float().to(cuda)   # exact: whole numbers
+    if ld:
+        far = torch.empty((M - 1) * ld + K, dtype=torch.float16, device=cuda).as_strided((M, K), (ld, 1))
+        far.copy_(x)
+        x = far
+    print(f"case M={M} ld={ld}", flush=True)
+    assert torch.equal(ops.spmm(_device(w, cuda), x, out_dtype=torch.float32, x_layout=1 if ld == 0 else 0), want)
+
+
 def test_a_blob_without_codes(cuda, oracle):
     """What an older version packed: the packed-weight object brings it up to date, and a device blob that was not is
     multiplied by the general kernel."""
