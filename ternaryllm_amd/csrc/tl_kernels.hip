@@ -128,8 +128,9 @@ extern "C" int tl_spmm_workspace(const tl_layout_header* header, int64_t M, int 
         *workspace_bytes = small_kmajor_bytes(header, M, x_dtype);
         return TL_OK;
     }
-    // the image of all rows, in whole 256 of them, so that a caller's buffer serves nearby row counts too
-    *workspace_bytes = round_up(M, 256) * image_row_bytes(header->inners, x_dtype);
+    // the image of all rows, in whole 256 of them, so that a caller's buffer serves nearby row counts too, and the bytes
+    // by which a buffer of any alignment may have to be moved
+    *workspace_bytes = round_up(M, 256) * image_row_bytes(header->inners, x_dtype) + 256;
     return TL_OK;
 }
 
