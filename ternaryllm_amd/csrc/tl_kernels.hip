@@ -17,6 +17,12 @@ int check_header(const tl_layout_header* h)
         h->n_blocks != (uint32_t)ceil_div(h->columns, TL_BLOCK_COLUMNS) || h->max_chunk_dwords < TL_BLOCK_COLUMNS ||
         (int64_t)h->max_chunk_dwords * 4 > kMaxChunkBytes + 16)
         return fail(TL_ERR_FORMAT, "layout header geometry is inconsistent");
+    const uint64_t code_bytes = (uint64_t)h->n_blocks * h->code_planes * h->code_units * TL_CODE_UNIT_BYTES;
+    const bool codes = h->version == TL_LAYOUT_VERSION;
+    if (codes ? h->code_planes == 0 || h->code_planes > 255 || h->code_units != (uint32_t)ceil_div(h->inners, TL_CODE_UNIT_ROWS) || h->off_codes < 256 ||
+                    h->off_codes % 16 || h->off_codes > h->total_bytes || h->total_bytes - h->off_codes < code_bytes
+              : h->code_planes != 0 || h->code_units != 0 || h->off_codes != 0)
+        return fail(TL_ERR_FORMAT, "layout header: the code section is inconsistent");
     return TL_OK;
 }
 

@@ -323,6 +323,20 @@ def test_compute_entry_points_reject_bad_arguments_before_any_launch():
     assert L.tl_last_error()
 
 
+def test_headers_whose_code_section_is_not_what_the_kernels_assume():
+    """The kernels size their reads of the codes by these fields: a header that contradicts itself is refused on the host."""
+    L = _lib.lib()
+    need = ctypes.c_int64(-1)
+    good = packing.PackedWeight.from_dense(ternary_weight(600, 40, 0.5, 2)).header
+    assert (good.code_units, good.code_planes) == (3, 1) and L.tl_spmm_workspace(ctypes.byref(good), 100, _lib.TL_F16, 0, ctypes.byref(need)) == 0
+    for change in ({"code_units": 0}, {"code_units": 4}, {"code_planes": 0}, {"code_planes": 2}, {"code_planes": 256}, {"off_codes": 0},
+                   {"off_codes": good.off_codes + 8}, {"off_codes": good.off_codes + 1024}, {"off_codes": 2 ** 64 - 1024}, {"version": 5}, {"total_bytes": good.total_bytes - 1}):
+        bad = _lib.LayoutHeader.from_buffer_copy(bytes(good))
+        for name, value in change.items():
+            setattr(bad, name, value)
+        assert L.tl_spmm_workspace(ctypes.byref(bad), 100, _lib.TL_F16, 0, ctypes.byref(need)) == -9, change   # TL_ERR_FORMAT
+
+
 def test_library_packer_on_the_hand_worked_tiles():
     """The library's merged packer against tests/golden/mcsc_hand_cases.json (outputs derived by hand from
     the reference's source)."""
