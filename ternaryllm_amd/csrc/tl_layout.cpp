@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -328,21 +329,37 @@ int pack_workers(int n_blocks)
     return std::max(1, std::min(cap / running, n_blocks));
 }
 
-// work(block) for every block, shared out among pack_workers() threads.
+// work(block) for every block, shared out among pack_workers() threads, or among as many as can be started.  Throws
+// std::bad_alloc, on the calling thread, where a work's buffers do not fit.
 template <typename Work>
 void for_each_block(int n_blocks, const Work& work)
 {
+    struct Running {
+        ~Running() { g_builds_running.fetch_sub(1); }
+    };
     const int workers = pack_workers(n_blocks);
+    const Running running;
     std::atomic<int> next{0};
+    std::atomic<bool> failed{false};
     auto take = [&]() {
-        for (int nb = next.fetch_add(1); nb < n_blocks; nb = next.fetch_add(1)) work(nb);
+        try {
+            for (int nb = next.fetch_add(1); nb < n_blocks && !failed; nb = next.fetch_add(1)) work(nb);
+        } catch (...) {
+            failed = true;
+        }
     };
     std::vector<std::thread> pool;
-    for (int i = 1; i < workers; ++i) pool.emplace_back(take);
+    pool.reserve((size_t)workers);
+    try {
+        for (int i = 1; i < workers; ++i) pool.emplace_back(take);
+    } catch (const std::exception&) {
+    }
     take();
     for (auto& th : pool) th.join();
-    g_builds_running.fetch_sub(1);
+    if (failed) throw std::bad_alloc();
 }
+
+int out_of_memory() { return fail(TL_ERR_SIZE, "not enough host memory"); }
 
 // The codes of column `y`, whose entry in row k is value[k], into their units (zero before the call).
 void put_codes(uint8_t* codes, int y, int inners, int planes, const int16_t* value)
@@ -418,7 +435,7 @@ extern "C" int tl_layout_build(const int32_t* neg_row, const int32_t* neg_off_ti
                                const int32_t* pos_row, const int32_t* pos_off_tiled,
                                int columns, int inners, int tile_k, int tile_rows,
                                void* blob, int64_t blob_bytes)
-{
+try {
     if (!neg_off_tiled || !pos_off_tiled || !blob) return fail(TL_ERR_ARG, "null pointer");
     if (columns <= 0 || inners <= 0 || tile_k <= 0) return fail(TL_ERR_SHAPE, "bad dimensions");
     Geometry g;
@@ -572,11 +589,13 @@ extern "C" int tl_layout_build(const int32_t* neg_row, const int32_t* neg_off_ti
     h.checksum = content_checksum(chunkstart, (size_t)NB * T + 1, stream, (size_t)dwords);
     std::memcpy(blob, &h, sizeof(h));
     return TL_OK;
+} catch (const std::bad_alloc&) {
+    return out_of_memory();
 }
 
 extern "C" int tl_layout_from_dense(const int32_t* w, int columns, int inners, int tile_rows,
                                     void* blob, int64_t* blob_bytes)
-{
+try {
     if (!w || !blob_bytes) return fail(TL_ERR_ARG, "null pointer");
     if (columns <= 0 || inners <= 0) return fail(TL_ERR_SHAPE, "bad dimensions");
     int64_t p = 0, n = 0;
@@ -600,12 +619,14 @@ extern "C" int tl_layout_from_dense(const int32_t* w, int columns, int inners, i
     if (*blob_bytes < need) return fail(TL_ERR_SIZE, "blob has %lld bytes, %lld needed", (long long)*blob_bytes, (long long)need);
     return tl_layout_build(neg_row.data(), neg_off.data(), pos_row.data(), pos_off.data(), columns, inners, g.tile_rows,
                            g.tile_rows, blob, *blob_bytes);
+} catch (const std::bad_alloc&) {
+    return out_of_memory();
 }
 
 extern "C" int tl_layout_from_mcsc(const void* merged_row, int index_width, int64_t n_index,
                                    const int32_t* merged_off, int columns, int inners, int tile_k,
                                    int uniformed, int tile_rows, void* blob, int64_t* blob_bytes)
-{
+try {
     if (!merged_off || !blob_bytes || (n_index > 0 && !merged_row)) return fail(TL_ERR_ARG, "null pointer");
     if (columns <= 0 || inners <= 0 || tile_k <= 0) return fail(TL_ERR_SHAPE, "bad dimensions");
     if (index_width != 2 && index_width != 4) return fail(TL_ERR_DTYPE, "index_width=%d (2 or 4 expected)", index_width);
@@ -652,10 +673,12 @@ extern "C" int tl_layout_from_mcsc(const void* merged_row, int index_width, int6
     neg_row.push_back(0);
     return tl_layout_build(neg_row.data(), neg_off.data(), pos_row.data(), pos_off.data(), columns, inners, tile_k, tile_rows,
                            blob, *blob_bytes);
+} catch (const std::bad_alloc&) {
+    return out_of_memory();
 }
 
 extern "C" int tl_layout_validate(const void* blob, int64_t blob_bytes)
-{
+try {
     if (!blob) return fail(TL_ERR_ARG, "null blob");
     if (blob_bytes < (int64_t)sizeof(tl_layout_header)) return fail(TL_ERR_FORMAT, "blob shorter than its header");
     tl_layout_header h;
@@ -742,10 +765,12 @@ extern "C" int tl_layout_validate(const void* blob, int64_t blob_bytes)
         if (bad >= 0) return fail(TL_ERR_FORMAT, "block %d: codes and index stream are not the same matrix", bad.load());
     }
     return TL_OK;
+} catch (const std::bad_alloc&) {
+    return out_of_memory();
 }
 
 extern "C" int tl_layout_add_codes(const void* blob, int64_t blob_bytes, void* out, int64_t* out_bytes)
-{
+try {
     if (!out_bytes) return fail(TL_ERR_ARG, "out_bytes is null");
     if (int rc = tl_layout_validate(blob, blob_bytes)) return rc;
     tl_layout_header h;
@@ -782,6 +807,8 @@ extern "C" int tl_layout_add_codes(const void* blob, int64_t blob_bytes, void* o
     h.total_bytes = (uint64_t)s.total;
     std::memcpy(to, &h, sizeof(h));
     return TL_OK;
+} catch (const std::bad_alloc&) {
+    return out_of_memory();
 }
 
 extern "C" int tl_layout_to_dense(const void* blob, int64_t blob_bytes, int32_t* w_out)

@@ -3,6 +3,8 @@ drop-in module surface and the error behaviour at the C boundary.  No GPU needed
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -321,6 +323,32 @@ def test_compute_entry_points_reject_bad_arguments_before_any_launch():
     assert L.tl_silu_mul(fake, 1, 1, 0, fake, 0, None) < 0
     assert L.tl_silu_mul(fake, 1, 9, 64, fake, 8, None) < 0
     assert L.tl_last_error()
+
+
+@pytest.mark.parametrize("spare,outcomes", [(7 << 20, (0,)), (0, (-8,))])
+def test_packing_without_threads_or_memory(tmp_path, spare, outcomes):
+    """Where no thread can be started (a stack takes 8 MiB) the passes go on with the threads there are; where their buffers
+    do not fit the calls return TL_ERR_SIZE.  Either way the process lives on."""
+    w = np.zeros((300000, 40), np.int32)
+    w[::50, ::3], w[3::70] = 1, -1
+    path = tmp_path / "blob.npy"
+    np.save(path, packing.PackedWeight.from_dense(w).blob)
+    script = """
+import os, resource, sys
+import numpy as np
+os.environ["TL_PACK_THREADS"] = "16"
+from ternaryllm_amd import _lib
+L = _lib.lib()
+blob = np.load(sys.argv[1])
+hard = resource.getrlimit(resource.RLIMIT_AS)[1]
+used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (used + %d, hard))
+rc = L.tl_layout_validate(blob.ctypes.data, blob.size)
+resource.setrlimit(resource.RLIMIT_AS, (hard, hard))
+print("outcome", rc, flush=True)
+""" % spare
+    run = subprocess.run([sys.executable, "-c", script, str(path)], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), capture_output=True, text=True, timeout=110)
+    assert run.returncode == 0 and int(run.stdout.split()[-1]) in outcomes, (run.returncode, run.stdout, run.stderr[-500:])
 
 
 def test_headers_whose_code_section_is_not_what_the_kernels_assume():
