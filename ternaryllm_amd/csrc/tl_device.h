@@ -30,9 +30,12 @@ __device__ __forceinline__ const_u32_ptr as_const(const uint32_t* p) { return (c
 struct WeightPtrs {
     const uint32_t* chunkstart;  // [NB * T + 1], dword offsets into stream
     const uint32_t* stream;      // chunks: 64 descriptors + runs of four 8-bit rows per dword
-    const unsigned char* codes;  // two-bit codes [NB][planes][units], 1 KB each, or null
-    int planes;                  // ternary matrices that the codes hold
     const void* scale;           // per-column factor or null
+};
+
+struct Codes {
+    const unsigned char* base;   // two-bit codes [NB][planes][units], 1 KB each, or null
+    int planes;                  // ternary matrices that they hold
 };
 
 struct KernelArgs {
@@ -51,6 +54,8 @@ struct KernelArgs {
     unsigned vpt_magic;   // small-M kernel, row-copy staging: ceil(2^32 / (tile_rows / values per vector))
     unsigned tile_magic;  // ceil(2^32 / tile_rows): k / tile_rows == (k * tile_magic) >> 32 for every k < 2^24
     long long x_sm, x_sk; // small-M kernel: element strides of the activations along M and along K
+    Codes c0;                 // matrix-core kernels: the codes of w0
+    int units, planes;        // matrix-core kernels: code units along K; planes of the weight, of two weights the larger number
     float one;  // 1.0f, passed in so that the fp16 -> fp32 accumulate stays a single mixed-precision fma
     // single-row kernel with a fused producer of its input (tl_spmv_fused)
     const void* X2;       // second summand of the residual add, or null
@@ -73,7 +78,7 @@ struct KernelArgs {
     const float* chain_sq_in; // [chain_sq_blocks][16] sums of squares of the rows X was made from: the product is multiplied by rsqrt(sum / K + eps), row by row
     int chain_sq_blocks;
     // matrix-core kernels
-    int units, planes;        // code units along K; planes of the weight, of two weights the larger number
+    Codes c1;                 // the codes of w1
     const void* image;        // the activations they multiply: row-major, 16-byte pieces along K ...
     long long image_ld;       // ... elements between rows
     long long image_plane;    // ... and, for fp32 activations in three bf16 parts, between parts
@@ -166,6 +171,10 @@ int finish_launch();
 int check_io(const void* blob_dev, const void* X, void* Y, int x_dtype, int x_layout, int64_t ldx, int64_t M, int y_dtype,
              int64_t ldy, const void* scale, int scale_dtype, const tl_layout_header* h);
 WeightPtrs weight_ptrs(const tl_layout_header* h, const void* blob_dev, const void* scale);
+inline Codes weight_codes(const tl_layout_header* h, const void* blob_dev)
+{
+    return Codes{h->off_codes ? static_cast<const unsigned char*>(blob_dev) + h->off_codes : nullptr, (int)h->code_planes};
+}
 
 template <typename KernelT>
 int raise_lds_limit(KernelT kernel, size_t bytes)

@@ -74,9 +74,9 @@ __global__ __launch_bounds__(kMaxWaves * 64) void tl_matrix_few(KernelArgs a)
     int units[C];                                                  // that the block's weight has
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        const WeightPtrs& weight = TWO && c == 1 ? a.w1 : a.w0;
+        const Codes& weight = TWO && c == 1 ? a.c1 : a.c0;
         units[c] = weight.planes * a.units;
-        codes[c] = weight.codes + min(TWO ? nb0 : nb0 + c, a.NB - 1) * ((long long)units[c] * TL_CODE_UNIT_BYTES) + lane * 16;
+        codes[c] = weight.base + min(TWO ? nb0 : nb0 + c, a.NB - 1) * ((long long)units[c] * TL_CODE_UNIT_BYTES) + lane * 16;
     }
     const XT* rows[FM];
 #pragma unroll

@@ -83,8 +83,6 @@ WeightPtrs weight_ptrs(const tl_layout_header* h, const void* blob_dev, const vo
     WeightPtrs w;
     w.chunkstart = reinterpret_cast<const uint32_t*>(b + h->off_chunkstart);
     w.stream = reinterpret_cast<const uint32_t*>(b + h->off_stream);
-    w.codes = h->off_codes ? b + h->off_codes : nullptr;
-    w.planes = (int)h->code_planes;
     w.scale = scale;
     return w;
 }
@@ -155,7 +153,7 @@ namespace {
 // A knob that names another kernel for few rows keeps the call with it.
 bool few_on_matrix_cores(const KernelArgs& a, const tl_layout_header* h, int64_t M, bool chained)
 {
-    if (M > kSmallMaxM || chained || a.gated || !a.w0.codes) return false;
+    if (M > kSmallMaxM || chained || a.gated || !a.c0.base || (M == 1 && knob(TL_FEW, 0) == 0)) return false;
     for (Knob other : {TL_SMALL_MT, TL_OCTET, TL_QUAD_WIDE, TL_RES16, TL_SPMV_DIRECT, TL_SPMV_TILES})
         if (knob(other, -1) >= 0) return false;
     bool use = M > 1 && !walk_has_gated(a, h);
@@ -207,7 +205,7 @@ int spmm_call(const tl_layout_header* header, const void* blob_dev, const void* 
     a.X = X; a.Y = Y;
     a.ldx = ldx; a.ldy = ldy;
     a.M = (int)M; a.N = (int)header->columns; a.K = (int)header->inners; a.T = (int)header->n_tiles; a.tile_rows = (int)header->tile_rows;
-    a.NB = (int)header->n_blocks; a.units = (int)header->code_units; a.planes = a.w0.planes;
+    a.NB = (int)header->n_blocks; a.c0 = weight_codes(header, blob_dev); a.units = (int)header->code_units; a.planes = a.c0.planes;
     a.x_f16 = x_dtype == TL_F16; a.x_kmajor = x_layout == TL_X_K_MAJOR; a.y_f16 = y_dtype == TL_F16; a.scale_f16 = scale_dtype == TL_F16;
     a.one = 1.0f;
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -275,7 +273,10 @@ int gate_up_call(bool few, const tl_layout_header* gate_header, const void* gate
     a.w1 = weight_ptrs(up_header, up_blob_dev, up_scale);
     a.X = X; a.Y = H;
     a.ldx = ldx; a.ldy = ldh;
-    a.NB = (int)gate_header->n_blocks; a.units = (int)gate_header->code_units; a.planes = std::max(a.w0.planes, a.w1.planes);
+    a.NB = (int)gate_header->n_blocks; a.units = (int)gate_header->code_units;
+    a.c0 = weight_codes(gate_header, gate_blob_dev);
+    a.c1 = weight_codes(up_header, up_blob_dev);
+    a.planes = std::max(a.c0.planes, a.c1.planes);
     a.M = (int)M; a.N = (int)gate_header->columns; a.K = (int)gate_header->inners; a.T = (int)gate_header->n_tiles;
     a.tile_rows = (int)gate_header->tile_rows;
     a.x_f16 = x_dtype == TL_F16; a.x_kmajor = x_layout == TL_X_K_MAJOR; a.y_f16 = h_dtype == TL_F16; a.scale_f16 = scale_dtype == TL_F16;

@@ -159,10 +159,10 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
     for (int i = 0; i < CL; ++i) {
         const int c = min(i * W + wave, TN / 16 - 1);             // column block of the tile
         const int owner = c / FN, f = c % FN;                     // its wave column and fragment
-        const WeightPtrs& w = (MODE == kTwoWeights && f >= FN / 2) ? a.w1 : a.w0;
+        const Codes& w = (MODE == kTwoWeights && f >= FN / 2) ? a.c1 : a.c0;
         const int nb = MODE == kTwoWeights ? nb0 + owner * (FN / 2) + f % (FN / 2) : nb0 + c;
         code_units[i] = w.planes * a.units;
-        code_src[i] = w.codes + min(nb, a.NB - 1) * (code_units[i] * unit_stride);
+        code_src[i] = w.base + min(nb, a.NB - 1) * (code_units[i] * unit_stride);
         code_to[i] = lds0 + STAGES * XB + c * TL_CODE_UNIT_BYTES;
     }
     auto issue_codes = [&](int u) {
@@ -628,7 +628,7 @@ int tl::launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t w
     a.x_sk = a.x_kmajor ? a.ldx : 1;
     const int64_t need = least_image_bytes(a.K, a.M, x_dtype);
     // Without codes, and for K-major rows that need no workspace, the index stream is walked.
-    if (!a.w0.codes || (two_weights && !a.w1.codes) || ((!workspace || workspace_bytes < need) && walk_reads_directly(a)))
+    if (!a.c0.base || (two_weights && !a.c1.base) || ((!workspace || workspace_bytes < need) && walk_reads_directly(a)))
         return x_dtype == TL_F16 ? walk_rows<__half>(a, workspace, workspace_bytes, two_weights, st)
                                  : walk_rows<float>(a, workspace, workspace_bytes, two_weights, st);
     const uintptr_t y_align = a.y_f16 ? 8 : 16;
