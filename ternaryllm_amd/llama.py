@@ -197,7 +197,7 @@ class TernaryLlamaDecoder(nn.Module):
             raise ValueError("prompt longer than the cache")
         if self._cache is None or self._cache.shape[2] != B:
             self.allocate_cache(B)
-        if B > 0 and S > 0 and self.native_prefill:
+        if B > 0 and S > 0 and self.native_prefill and self._norms_as_built():
             return self._prefill_native(tokens)
         x = self.embed_tokens[tokens]
         pos = torch.arange(S, device=x.device)
@@ -211,26 +211,40 @@ class TernaryLlamaDecoder(nn.Module):
         last = self.norm(x[:, -1])
         return self.lm_head(last)
 
+    def _norms_as_built(self):
+        """Whether every norm is an RMSNorm that the kernels may stand in for: no other module in its place, no hook on its
+        forward, a weight of the activations' type."""
+        module = torch.nn.modules.module
+        if module._global_forward_hooks or module._global_forward_pre_hooks:
+            return False
+        norms = [n for layer in self.layers for n in (layer.input_layernorm, layer.post_attention_layernorm)] + [self.norm]
+        return all(type(n) is RMSNorm and not n._forward_hooks and not n._forward_pre_hooks and "forward" not in n.__dict__ and
+                   n.weight.dtype == self.dtype and n.weight.is_contiguous() for n in norms)
+
     def _prefill_native(self, tokens):
         """The pass with the library's kernels around the products: residual add + RMSNorm in one, keys rotated into the
         cache and values copied beside them in one, queries rotated inside the attention.  Seven launches a layer."""
         c = self.config
         B, S = tokens.shape
-        H, nh, hd, eps = c.hidden_size, c.num_attention_heads, c.head_dim, c.rms_norm_eps
+        H, nh, hd = c.hidden_size, c.num_attention_heads, c.head_dim
+
+        def add_norm(x, y, norm):
+            return ops.add_rmsnorm(x, y, norm.weight, norm.eps)
+
         tables = self.rope_cos[:S], self.rope_sin[:S]
         x = self.embed_tokens[tokens].view(B * S, H)
-        _, h = ops.add_rmsnorm(x, None, self.layers[0].input_layernorm.weight, eps)
+        _, h = add_norm(x, None, self.layers[0].input_layernorm)
         for li, layer in enumerate(self.layers):
             qkv = layer.qkv_proj(h).view(B, S, 3, nh, hd)
             kc, vc = self._cache[li, 0, :, :, :S], self._cache[li, 1, :, :, :S]
             ops.rope_rows(qkv[:, :, 1], tables, kc, qkv[:, :, 2], vc)
             a = ops.prefill_attention(qkv[:, :, 0], kc, vc, tables)
-            x, h = ops.add_rmsnorm(x, layer.o_proj(a.view(B * S, H)), layer.post_attention_layernorm.weight, eps)
+            x, h = add_norm(x, layer.o_proj(a.view(B * S, H)), layer.post_attention_layernorm)
             y = self._mlp(layer, h)
             if li + 1 < len(self.layers):
-                x, h = ops.add_rmsnorm(x, y, self.layers[li + 1].input_layernorm.weight, eps)
+                x, h = add_norm(x, y, self.layers[li + 1].input_layernorm)
         last = [t.view(B, S, H)[:, -1].contiguous() for t in (x, y)]
-        return self.lm_head(ops.add_rmsnorm(*last, self.norm.weight, eps)[1])
+        return self.lm_head(add_norm(*last, self.norm)[1])
 
     # -- decode ------------------------------------------------------------------------------
     def _decode_step(self, token, pos, mask):

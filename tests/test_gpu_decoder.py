@@ -781,3 +781,34 @@ def test_graph_replay_equals_eager_decode(tiny, cuda):
     assert torch.equal(eager, graphed)
     assert torch.equal(eager, again)
     assert eager.shape == (3, 12) and int(eager.min()) >= 0 and int(eager.max()) < tiny.config.vocab_size
+
+
+def test_prefill_runs_norms_that_are_not_as_built(cuda):
+    """Hooks on a norm run, another module in a norm's place is used, and a norm's own eps counts, in a pass over a prompt."""
+    from ternaryllm_amd import TernaryConfig, TernaryLlamaDecoder
+    cfg = TernaryConfig(hidden_size=256, intermediate_size=512, num_hidden_layers=2, num_attention_heads=2, num_key_value_heads=2, vocab_size=300,
+                        max_position_embeddings=64, sparsity=0.7)
+    m = TernaryLlamaDecoder(cfg, seed=3, device=cuda)
+    tokens = torch.randint(0, 300, (2, 9), generator=torch.Generator().manual_seed(1)).to(cuda)
+
+    def both():
+        native = m.prefill(tokens).double()
+        m.native_prefill = False
+        plain = m.prefill(tokens).double()
+        m.native_prefill = True
+        # fp16 roundings in another order: a quarter of a percent at most over two layers
+        assert float((native - plain).norm() / plain.norm()) <= 5e-3
+        return native
+
+    as_built = both()
+    seen = []
+    handles = [n.register_forward_hook(lambda mod, args, out: seen.append(tuple(out.shape))) for n in (m.layers[1].input_layernorm, m.norm)]
+    m.prefill(tokens)
+    assert seen == [(2, 9, 256), (2, 256)]
+    for h in handles:
+        h.remove()
+    m.layers[1].post_attention_layernorm.eps = 0.5
+    assert float((both() - as_built).norm() / as_built.norm()) > 0.02
+    m.layers[1].post_attention_layernorm.eps = cfg.rms_norm_eps
+    m.layers[0].input_layernorm = torch.nn.LayerNorm(256).to(cuda, torch.float16)
+    assert float((both() - as_built).norm() / as_built.norm()) > 0.005
