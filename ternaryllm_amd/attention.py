@@ -8,6 +8,7 @@ import math
 
 import torch
 from torch import nn
+from torch.autograd import forward_ad
 
 from . import ops
 from .linear import TernaryLinear
@@ -39,6 +40,11 @@ def apply_rope(x, cos, sin):
     if cos.dim() == 2:
         cos, sin = cos[None], sin[None]
     return x * cos[:, None] + rot * sin[:, None]
+
+
+def differentiated(*tensors):
+    """Whether a derivative, backward or forward, is asked for with respect to what these tensors were made from."""
+    return any(t.requires_grad or forward_ad.unpack_dual(t).tangent is not None for t in tensors)
 
 
 class LlamaTernaryAttention(nn.Module):
@@ -127,6 +133,7 @@ class LlamaTernaryAttention(nn.Module):
             heads = [p(hidden_states).view(bsz, q_len, -1, self.head_dim) for p in (self.q_proj, self.k_proj, self.v_proj)]
         q, k, v = (t.transpose(1, 2) for t in heads)
         is_tuple = isinstance(past_key_value, (tuple, list))
+        has_past = past_key_value is not None
         past_len = position_offset
         if past_len is None:
             if is_tuple:
@@ -145,7 +152,7 @@ class LlamaTernaryAttention(nn.Module):
         else:
             cos, sin = self._rotary(position_ids, position_embeddings, q_len, past_len, q.dtype, q.device)
         native = native and all(t.dim() in (2, 3) and t.device == q.device and t.shape == cos.shape and t.shape[-2:] == (q_len, self.head_dim) and
-                                (t.dim() == 2 or t.shape[0] in (1, bsz)) and not t.requires_grad for t in (cos, sin))
+                                (t.dim() == 2 or t.shape[0] in (1, bsz)) for t in (cos, sin)) and not (position_embeddings is not None and differentiated(cos, sin))
         if native:
             tables = tuple(t if t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format) for t in (cos, sin))
             k = torch.empty((bsz, q_len, k.shape[1], self.head_dim), dtype=k.dtype, device=k.device).transpose(1, 2)
@@ -161,8 +168,8 @@ class LlamaTernaryAttention(nn.Module):
         elif use_cache:
             past_key_value = (k, v)
         if native:
-            # (a cache may give back keys of another type, shape or layout)
-            if k.dtype == v.dtype == q.dtype and k.device == v.device == q.device and k.shape == v.shape and k.dim() == 4 and \
+            # (a cache may give back keys of another type, shape or layout, or ones that are differentiated)
+            if not (has_past and differentiated(k, v)) and k.dtype == v.dtype == q.dtype and k.device == v.device == q.device and k.shape == v.shape and k.dim() == 4 and \
                     k.shape[:2] == (bsz, self.num_key_value_heads) and k.shape[3] == self.head_dim and k.shape[2] >= q_len and ops.in_pieces(k, v):
                 return self.o_proj(ops.prefill_attention(heads[0], k, v, tables)), None, past_key_value
             q = apply_rope(q, cos, sin)

@@ -581,3 +581,27 @@ def test_ternarised_float_weights(cuda):
             exact = x.double().numpy() @ wf.double().numpy()
             corr = np.corrcoef(exact.reshape(-1), ref.reshape(-1))[0, 1]
             assert corr > 0.8
+
+
+def test_attention_passes_derivatives_on_to_cached_keys_and_tables(cuda):
+    """An output projection that records gradients sees them reach the past keys and values and the rotary tables, backward
+    and forward."""
+    from torch.autograd import forward_ad
+    from ternaryllm_amd import LlamaTernaryAttention, TernaryConfig
+    H, heads, S, P = 256, 2, 5, 7
+    g = torch.Generator().manual_seed(4)
+    block = LlamaTernaryAttention(TernaryConfig(hidden_size=H, num_attention_heads=heads, num_key_value_heads=heads, sparsity=0.9), generator=g,
+                                  reference_buffers=False).to(cuda)
+    block.o_proj = torch.nn.Identity()
+    x = torch.randn((1, S, H), generator=g).half().to(cuda)
+    past = [torch.randn((1, heads, P, 128), generator=g).half().to(cuda).requires_grad_() for _ in range(2)]
+    tables = [torch.randn((1, S, 128), generator=g).half().to(cuda).requires_grad_() for _ in range(2)]
+    for inputs, call in ((past, lambda p: block(x, past_key_value=tuple(p))[0]), (tables, lambda t: block(x, position_embeddings=tuple(t))[0])):
+        for t, grad in zip(inputs, torch.autograd.grad(call(inputs).float().sum(), inputs)):
+            assert grad.shape == t.shape and bool(grad.abs().sum() > 0)
+        with torch.no_grad(), forward_ad.dual_level():
+            try:
+                out = call([forward_ad.make_dual(t.detach(), torch.ones_like(t)) for t in inputs])
+            except NotImplementedError:
+                continue   # (an attention operator of torch without forward mode says so)
+            assert forward_ad.unpack_dual(out).tangent is not None
