@@ -147,7 +147,7 @@ class LlamaTernaryAttention(nn.Module):
         # causal fp16 attention without a mask: the library's kernels rotate and attend
         native = (all(t.is_cuda and t.dtype == torch.float16 and t.numel() > 0 and not t.requires_grad for t in heads) and self.head_dim in (64, 128) and attention_mask is None and
                   not output_attentions and dropout == 0.0 and (self.is_causal or q_len == 1))
-        if native and position_ids is None and position_embeddings is None:
+        if native and position_ids is None and position_embeddings is None and isinstance(past_len, int):
             cos, sin = ops.rope_table(past_len, q_len, self.head_dim, self.rope_theta, q.dtype, q.device)
         else:
             cos, sin = self._rotary(position_ids, position_embeddings, q_len, past_len, q.dtype, q.device)

@@ -605,3 +605,17 @@ def test_attention_passes_derivatives_on_to_cached_keys_and_tables(cuda):
             except NotImplementedError:
                 continue   # (an attention operator of torch without forward mode says so)
             assert forward_ad.unpack_dual(out).tangent is not None
+
+
+def test_position_offsets_of_every_kind_of_number(cuda):
+    """position_offset as a Python, numpy or tensor integer, or as a float."""
+    import numpy as np
+    from ternaryllm_amd import LlamaTernaryAttention, TernaryConfig
+    block = LlamaTernaryAttention(TernaryConfig(hidden_size=256, num_attention_heads=2, num_key_value_heads=2, sparsity=0.9),
+                                  generator=torch.Generator().manual_seed(4), reference_buffers=False).to(cuda)
+    x = torch.randn((1, 5, 256), generator=torch.Generator().manual_seed(5)).half().to(cuda)
+    want = block(x, position_offset=3)[0].double()
+    for offset in (np.int64(3), torch.tensor(3), 3.0, torch.tensor(3, device=cuda)):
+        got = block(x, position_offset=offset)[0].double()
+        # tables rounded to fp16 from angles of a few units in the last place of fp32: the same but for ties
+        assert float((got - want).norm() / want.norm()) <= 1e-3, offset
