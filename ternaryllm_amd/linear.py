@@ -207,7 +207,7 @@ class TernaryLinear(nn.Module):
                 raise ValueError(f"packed weight is {pw.inners}x{pw.columns}, module is {self.in_features}x{self.out_features}")
             pw.validate()
             if pw.blob.size != blob.numel():  # packed by an older version: PackedWeight has brought it up to date
-                state_dict[prefix + "w_packed"] = torch.from_numpy(pw.blob)
+                state_dict[prefix + "w_packed"] = torch.from_numpy(pw.blob).to(blob.device)
             self.w_packed = torch.empty(pw.blob.size, dtype=torch.uint8, device=self.w_packed.device)
             self._header = pw.header
             self._packed_nnz = pw.nnz

@@ -211,6 +211,19 @@ def test_the_index_stream_alone(cuda, oracle, M, K, N, dtype):
         assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())   # exact sums; __expf and the division
 
 
+def test_loading_a_blob_without_codes_from_the_device(cuda):
+    """load_state_dict(assign=True) keeps the device of what it is given, also where the blob is brought up to date."""
+    from ternaryllm_amd import TernaryLinear
+    from ternaryllm_amd.packing import PackedWeight
+    K, N = 264, 40
+    new = PackedWeight.from_dense(ternary_weight(K, N, 0.6, 41))
+    module = TernaryLinear(K, N, sparsity=0.9, bias=False, reference_buffers=False).to(cuda)
+    module.load_state_dict({"w_packed": _without_codes(new, cuda).blob}, assign=True)
+    assert module.w_packed.device == cuda and np.array_equal(module.w_packed.cpu().numpy(), new.blob)
+    x = activations(60, K, 1, torch.float32, integer=True).to(cuda)
+    assert torch.equal(module(x), x @ torch.from_numpy(new.to_dense()).float().to(cuda))   # exact: whole numbers
+
+
 @pytest.mark.parametrize("M,K,ld", [(60, 64, 1 << 23), (60, 64, (1 << 24) + 8), (4300000, 16, 0)])
 def test_rows_far_apart_and_very_many_of_them(cuda, M, K, ld):
     """Row-major rows whose distance the kernel cannot address go through the image; K-major ones in several passes where one
