@@ -22,10 +22,13 @@ __device__ __align__(16) const unsigned char kNoCodes[TL_CODE_UNIT_BYTES] = {}; 
 
 // 16 bytes per lane from `base` + offset into LDS at `lds` + 16 * lane.  (As assembly, because the compiler would wait for
 // all such loads before any read of LDS; here they are counted by hand.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // (m0 is a register that the compiler reserves; named all the same, as this writes it)
 __device__ __forceinline__ void load_to_lds(uint32_t lds, const void* base, uint32_t offset)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(offset), "s"(base) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(offset), "s"(base) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 template <int N>
 __device__ __forceinline__ void wait_loads_and_barrier()
