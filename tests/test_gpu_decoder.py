@@ -65,7 +65,7 @@ def test_prefill_and_decode_match_fp32_reference(tiny, cuda):
     tokens = torch.randint(0, tiny.config.vocab_size, (B, S + extra), generator=g).to(cuda)
     ref = _reference_logits(tiny, tokens)                       # [B, S + extra, V]
     scale = ref.abs().max().item()
-    got = tiny.prefill(tokens[:, :S]).float()                   # 140 rows: the row-parallel kernel
+    got = tiny.prefill(tokens[:, :S]).float()                   # 140 rows: the matrix-core kernel
     worst = (got - ref[:, S - 1]).abs().max().item() / scale
     st = tiny._decode_state(B)
     for j in range(extra):                                      # teacher-forced single-token steps: the small-M kernel
@@ -588,7 +588,7 @@ def test_silu_gate_in_the_epilogue_of_the_gate_up_product(cuda):
     """tl_spmm_gated / tl_spmv_fused_gated on a weight whose columns are (gate, up) pairs against the product followed
     by tl_silu_mul_pairs: bit for bit -- one row (both single-row kernels, with and without a producer), 9 to 16 fp16
     rows on a wide output (row-major and as a K-major image with zeroed padding rows), more than 48 rows (the
-    row-parallel kernel), and the shapes without the epilogue, which take the two launches."""
+    matrix-core kernel), and the shapes without the epilogue, which take the two launches."""
     import ctypes
     from tests.util import knobs, ternary_weight
     from ternaryllm_amd import _lib, ops
@@ -657,20 +657,19 @@ def test_silu_gate_in_the_epilogue_of_the_gate_up_product(cuda):
     assert torch.equal(ops.spmm_gated(dw, x40, sc), ops.silu_mul(ops.spmm(dw, x40, sc), pairs=True))
     narrow = ops.DeviceWeight(PackedWeight.from_dense(ternary_weight(K, 96, 0.8, 6)), cuda)
     assert fused_rc(narrow, torch.zeros((16, K), dtype=torch.float16, device=cuda), 16) == _lib.TL_ERR_UNSUPPORTED
-    # more than 48 rows: the row-parallel kernel with the pair epilogue, whole output tiles and tiles that the matrix
-    # edge cuts, with and without K tiles shared out among the workgroups
+    # more than 48 rows: the matrix-core kernel with the pair epilogue, whole output tiles and tiles that the matrix
+    # edge cuts, contiguous rows and rows with an odd leading dimension
     sc96 = (0.5 + torch.rand(96, generator=g)).half().to(cuda)
     for dtype in (torch.float16, torch.float32):
         for M in (60, 300, 1100):
             x = torch.randn((M, K), generator=g).to(dtype).to(cuda)
             for weight, scale in ((dw, sc), (narrow, sc96)):
                 assert fused_rc(weight, x, M) == 0
-                for setting in ({}, {"TL_ROWS_SPLIT": "0"}):
-                    with knobs(**setting):
-                        got = ops.spmm_gated(weight, x, scale.to(dtype))
-                        want = ops.silu_mul(ops.spmm(weight, x, scale.to(dtype)), pairs=True)
+                for xin in (x, torch.zeros((M, K + 1), dtype=dtype, device=cuda)[:, :K].copy_(x)):
+                    got = ops.spmm_gated(weight, xin, scale.to(dtype))
+                    want = ops.silu_mul(ops.spmm(weight, xin, scale.to(dtype)), pairs=True)
                     assert got.shape == (M, weight.columns // 2)
-                    assert torch.equal(got, want), (dtype, M, weight.columns, setting)
+                    assert torch.equal(got, want), (dtype, M, weight.columns, xin.stride(0))
     image = torch.empty((dw.columns // 2, 64), dtype=torch.float16, device=cuda)
     x60 = torch.zeros((60, K), dtype=torch.float16, device=cuda)
     assert L.tl_spmm_gated(ctypes.byref(dw.header), dw.blob.data_ptr(), x60.data_ptr(), 1, 0, K, 60, image.data_ptr(), 1, 64, 1, None, 0,

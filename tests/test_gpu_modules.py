@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from tests.util import FP16_TOL, FP32_TOL, activations, knobs, max_rel_err, ternary_weight
+from tests.util import FP16_TOL, FP32_TOL, activations, max_rel_err, ternary_weight
 
 pytestmark = pytest.mark.gpu
 
@@ -459,41 +459,41 @@ def _rows_ref_mlp(x_rows, wg, wu, wd, sg, su, sd):
     return h, (h @ wd) * sd
 
 
-@pytest.mark.parametrize("split", ["0", "1"])
-def test_config3_mlp_block_at_full_size(cuda, split):
+@pytest.mark.parametrize("ld", [4096, 4097])
+def test_config3_mlp_block_at_full_size(cuda, ld):
     """BASELINE config 3 at its size: 1024 tokens, gate/up 4096 -> 11008 fused with the SiLU gate, down
-    11008 -> 4096, 80 % sparsity, fp16 activations, per-channel fp16 scales; whole output tiles and shared-out
-    K tiles (TL_ROWS_SPLIT).  Full rows of H and of Y against the float64 restatement, every row of Y against the
+    11008 -> 4096, 80 % sparsity, fp16 activations, per-channel fp16 scales; rows that are read where
+    they lie, and rows with an odd leading dimension, which go through the image.  Full rows of H and of Y against the float64 restatement, every row of Y against the
     float64 product of the H the GPU produced."""
     from ternaryllm_amd import LlamaTernaryMLP, TernaryConfig, ops
-    with knobs(TL_ROWS_SPLIT=split):
-        g = torch.Generator().manual_seed(31)
-        H, I, M = 4096, 11008, 1024
-        cfg = TernaryConfig(hidden_size=H, intermediate_size=I, sparsity=0.8)
-        sc = {"gate": ((0.5 + torch.rand(I, generator=g)) / 28.0).half(), "up": ((0.5 + torch.rand(I, generator=g)) / 28.0).half(),
-              "down": ((0.5 + torch.rand(H, generator=g)) / 47.0).half()}   # ~1 / sqrt(non-zeros per column): outputs stay O(1)
-        mlp = LlamaTernaryMLP(cfg, generator=g, scales=sc, reference_buffers=False).to(cuda)
-        x = torch.randn((M, H), generator=g).half()
-        print(f"case config 3 fused MLP, TL_ROWS_SPLIT={split}", flush=True)
-        h = ops.mlp_gate_up(mlp.gate_proj.device_weight(), mlp.up_proj.device_weight(), x.to(cuda), mlp.gate_proj.w_scale,
-                            mlp.up_proj.w_scale)
-        y = mlp(x.to(cuda).reshape(8, 128, H))
-        assert h.shape == (M, I) and h.dtype == torch.float16 and y.shape == (8, 128, H) and y.dtype == torch.float16
-        wg, wu, wd = (m.ternary_weight.numpy().astype(np.float64) for m in (mlp.gate_proj, mlp.up_proj, mlp.down_proj))
-        sg, su, sd = (sc[k].double().numpy() for k in ("gate", "up", "down"))
-        rows = [0, 255, 256, 511, 777, 1023]
-        h_ref, y_ref = _rows_ref_mlp(x[rows].double().numpy(), wg, wu, wd, sg, su, sd)
-        h_got = h[rows].double().cpu().numpy()
-        err_h = np.abs(h_got - h_ref) / np.maximum(np.abs(h_ref), np.abs(h_ref).mean())
-        print(f"  max rel err of H rows {err_h.max():.3e}", flush=True)
-        assert err_h.max() <= FP16_TOL
-        y_got = y.reshape(M, H)[rows].double().cpu().numpy()
-        err_y = np.abs(y_got - y_ref) / np.maximum(np.abs(y_ref), np.sqrt((y_ref ** 2).mean()))
-        print(f"  max rel err of Y rows (fp16 H in between) {err_y.max():.3e}", flush=True)
-        assert err_y.max() <= 1.5 * FP16_TOL   # measured 1.2e-3: the fp16 rounding of H carried through ~2200 signed adds
-        # the down projection alone, every row: float64 product of the H the GPU wrote (fp16 values, exact inputs)
-        y_all = (h.double().cpu().numpy() @ wd) * sd
-        assert max_rel_err(y.reshape(M, H).double().cpu().numpy(), y_all, h.double().cpu().numpy() * 1.0, mlp.down_proj.ternary_weight.numpy()) <= FP16_TOL
+    g = torch.Generator().manual_seed(31)
+    H, I, M = 4096, 11008, 1024
+    cfg = TernaryConfig(hidden_size=H, intermediate_size=I, sparsity=0.8)
+    sc = {"gate": ((0.5 + torch.rand(I, generator=g)) / 28.0).half(), "up": ((0.5 + torch.rand(I, generator=g)) / 28.0).half(),
+          "down": ((0.5 + torch.rand(H, generator=g)) / 47.0).half()}   # ~1 / sqrt(non-zeros per column): outputs stay O(1)
+    mlp = LlamaTernaryMLP(cfg, generator=g, scales=sc, reference_buffers=False).to(cuda)
+    x = torch.randn((M, H), generator=g).half()
+    xd = torch.zeros((M, ld), dtype=torch.float16, device=cuda)[:, :H].copy_(x)
+    print(f"case config 3 fused MLP, ld={ld}", flush=True)
+    h = ops.mlp_gate_up(mlp.gate_proj.device_weight(), mlp.up_proj.device_weight(), xd, mlp.gate_proj.w_scale,
+                        mlp.up_proj.w_scale)
+    y = mlp(xd.view(8, 128, H))
+    assert h.shape == (M, I) and h.dtype == torch.float16 and y.shape == (8, 128, H) and y.dtype == torch.float16
+    wg, wu, wd = (m.ternary_weight.numpy().astype(np.float64) for m in (mlp.gate_proj, mlp.up_proj, mlp.down_proj))
+    sg, su, sd = (sc[k].double().numpy() for k in ("gate", "up", "down"))
+    rows = [0, 255, 256, 511, 777, 1023]
+    h_ref, y_ref = _rows_ref_mlp(x[rows].double().numpy(), wg, wu, wd, sg, su, sd)
+    h_got = h[rows].double().cpu().numpy()
+    err_h = np.abs(h_got - h_ref) / np.maximum(np.abs(h_ref), np.abs(h_ref).mean())
+    print(f"  max rel err of H rows {err_h.max():.3e}", flush=True)
+    assert err_h.max() <= FP16_TOL
+    y_got = y.reshape(M, H)[rows].double().cpu().numpy()
+    err_y = np.abs(y_got - y_ref) / np.maximum(np.abs(y_ref), np.sqrt((y_ref ** 2).mean()))
+    print(f"  max rel err of Y rows (fp16 H in between) {err_y.max():.3e}", flush=True)
+    assert err_y.max() <= 1.5 * FP16_TOL   # measured 1.2e-3: the fp16 rounding of H carried through ~2200 signed adds
+    # the down projection alone, every row: float64 product of the H the GPU wrote (fp16 values, exact inputs)
+    y_all = (h.double().cpu().numpy() @ wd) * sd
+    assert max_rel_err(y.reshape(M, H).double().cpu().numpy(), y_all, h.double().cpu().numpy() * 1.0, mlp.down_proj.ternary_weight.numpy()) <= FP16_TOL
 
 
 def test_config4_attention_block_at_full_size(cuda):

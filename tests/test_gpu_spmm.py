@@ -120,9 +120,9 @@ def test_k_major_input_and_tile_heights(cuda, oracle):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("M", [49, 200, 257])
 def test_row_kernel_activation_layouts(cuda, oracle, M, dtype):
-    """Every way activations reach the row-parallel kernel: contiguous rows of whole 16-byte pieces (the 16-byte-per-lane
-    re-layout for fp16), rows with an odd leading dimension or an odd K (the element-wise re-layout), a K-major image
-    padded to the row tile (no pre-pass) and K-major with an odd leading dimension."""
+    """Every way activations reach the matrix-core kernel: contiguous rows of whole 16-byte pieces (fp16 ones are read where
+    they lie), rows with an odd leading dimension or an odd K, aligned rows further apart than K, K-major ones padded to
+    whole row tiles and K-major ones with an odd leading dimension (all through the image)."""
     from ternaryllm_amd import ops
     from ternaryllm_amd.packing import PackedWeight
     for K, N in ((520, 96), (777, 50)):
@@ -138,7 +138,7 @@ def test_row_kernel_activation_layouts(cuda, oracle, M, dtype):
         wide8 = torch.zeros((M, K + 8), dtype=dtype, device=cuda)          # aligned rows further apart than K
         wide8[:, :K] = xd
         cases["row-major, aligned stride"] = (wide8[:, :K], 0)
-        padded = torch.zeros((K, -(-M // 256) * 256), dtype=dtype, device=cuda)  # the kernel's own layout
+        padded = torch.zeros((K, -(-M // 256) * 256), dtype=dtype, device=cuda)  # aligned, whole row tiles
         padded[:, :M] = xd.t()
         cases["k-major, padded"] = (padded[:, :M], 1)
         widek = torch.zeros((K, M + 5), dtype=dtype, device=cuda)          # K-major with an odd leading dimension
@@ -177,12 +177,12 @@ def test_small_m_activation_layouts(cuda, oracle, M, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
-def test_rows_kernel_with_and_without_shared_out_tiles(cuda, oracle, dtype):
-    """The row-parallel kernel in both launch modes (one workgroup per output tile; K tiles shared out
-    among one workgroup per compute unit, partial sums added by the fix-up launch), plain and fused."""
+def test_many_rows_where_they_lie_and_through_an_image(cuda, oracle, dtype):
+    """More than 48 rows, plain and with gate and up fused: contiguous rows (fp16 of whole 16-byte pieces are read where they
+    lie) and rows with an odd leading dimension, which go through the image."""
     from ternaryllm_amd import ops
     from ternaryllm_amd.packing import PackedWeight
-    for M, K, N in ((70, 1300, 200), (520, 2100, 130), (1100, 777, 330)):
+    for M, K, N in ((70, 1304, 200), (520, 2104, 130), (1100, 777, 330)):
         wg = ternary_weight(K, N, 0.75, 51 + M)
         wu = ternary_weight(K, N, 0.75, 52 + M)
         dg, du = ops.DeviceWeight(PackedWeight.from_dense(wg), cuda), ops.DeviceWeight(PackedWeight.from_dense(wu), cuda)
@@ -193,22 +193,20 @@ def test_rows_kernel_with_and_without_shared_out_tiles(cuda, oracle, dtype):
         g = (xf.double() @ torch.from_numpy(wg).double()) * sg.double()
         u = (xf.double() @ torch.from_numpy(wu).double()) * sg.double()
         ref_fused = (torch.nn.functional.silu(g) * u).numpy()
-        fused = {}
-        for mode in ("0", "1"):
-            print(f"case M={M} K={K} N={N} dtype={dtype} split={mode}", flush=True)
-            with knobs(TL_ROWS_SPLIT=mode):
-                y = ops.spmm(dg, x.to(cuda), out_dtype=torch.float32).cpu().numpy()
-                h = ops.mlp_gate_up(dg, du, xf.to(cuda), sg.to(cuda), sg.to(cuda), out_dtype=torch.float32).cpu().numpy()
-            assert np.array_equal(y.astype(np.float64), ref), (M, K, N, mode)
+        for ld in (K, K + 1):
+            print(f"case M={M} K={K} N={N} dtype={dtype} ld={ld}", flush=True)
+            xd, xfd = (torch.zeros((M, ld), dtype=dtype, device=cuda)[:, :K].copy_(t) for t in (x, xf))
+            y = ops.spmm(dg, xd, out_dtype=torch.float32).cpu().numpy()
+            h = ops.mlp_gate_up(dg, du, xfd, sg.to(cuda), sg.to(cuda), out_dtype=torch.float32).cpu().numpy()
+            assert np.array_equal(y.astype(np.float64), ref), (M, K, N, ld)
             scale = np.abs(ref_fused).max()
-            assert np.abs(h - ref_fused).max() <= (FP16_TOL if dtype == torch.float16 else 1e-4) * scale, (M, K, N, mode)
-            fused[mode] = h
+            assert np.abs(h - ref_fused).max() <= (FP16_TOL if dtype == torch.float16 else 1e-4) * scale, (M, K, N, ld)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 def test_output_into_a_strided_buffer(cuda, oracle, dtype):
-    """`out=` as a column slice of a wider buffer: leading dimensions that allow the row kernel's whole-row
-    stores and ones that do not, for both kernels; nothing outside the slice may be touched."""
+    """`out=` as a column slice of a wider buffer: leading dimensions that allow the matrix-core kernel's
+    stores of four values and ones that do not, for both kernels; nothing outside the slice may be touched."""
     from ternaryllm_amd import ops
     from ternaryllm_amd.packing import PackedWeight
     K, N = 600, 256
@@ -249,6 +247,8 @@ def test_small_m_kernels_in_every_mode(cuda, oracle, dtype):
                                    {"TL_SMALL_MT": "16", "TL_OCTET": "1", "TL_LW": "1", "TL_TILE_GROUP": "8"},
                                    {"TL_QUAD_WIDE": "0"}, {"TL_QUAD_WIDE": "1", "TL_LW": "2"}, {"TL_QUAD_WIDE": "1", "TL_TILE_GROUP": "1"},
                                    {"TL_RES16": "1"}, {"TL_RES16": "0"}]
+        if M > 1:  # (the matrix-core kernel takes these by default)
+            extra += [dict(env, TL_FEW="0") for env in settings]
         for env in settings + extra:
             print(f"case M={M} dtype={dtype} env={env}", flush=True)
             with knobs(**env):

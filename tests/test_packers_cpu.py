@@ -162,9 +162,9 @@ def test_blob_from_merged_arrays_matches_the_oracle_walk(oracle, padding):
 
 @pytest.mark.parametrize("K,N,s,seed", [(4096, 11008, 0.8, 1237), (2048, 2048, 0.9, 3), (256, 16, 0.99, 1), (4096, 48, 0.0, 2)])
 def test_index_prefetch_stays_inside_the_blob(K, N, s, seed):
-    """The row kernel requests 192 index dwords from the start of every wave's piece of a chunk (a wave owns 4 or
-    8 neighbouring columns) and, for longer pieces, whole 64-dword groups up to 63 dwords past the piece's end:
-    the furthest byte either touches must lie inside the blob as trimmed to header.total_bytes."""
+    """The blob keeps room behind the stream for kernels that request index dwords ahead: 192 from the start of the piece
+    of a chunk that 4 or 8 neighbouring columns make, and whole 64-dword groups up to 63 dwords past its end.  The
+    furthest byte must lie inside the blob as trimmed to header.total_bytes."""
     if K * N > 1 << 24:
         rng = np.random.default_rng(seed)   # the torch generator is slow at this size
         r = rng.random((K, N), dtype=np.float32)
@@ -323,6 +323,71 @@ def test_compute_entry_points_reject_bad_arguments_before_any_launch():
     assert L.tl_silu_mul(fake, 1, 1, 0, fake, 0, None) < 0
     assert L.tl_silu_mul(fake, 1, 9, 64, fake, 8, None) < 0
     assert L.tl_last_error()
+
+
+def _old_version(new):
+    """The blob that the version before the codes would have made."""
+    old = new.blob[:new.header.off_codes].copy()
+    h = _lib.LayoutHeader.from_buffer_copy(old[:256].tobytes())
+    h.version, h.off_codes, h.code_units, h.code_planes, h.total_bytes = 5, 0, 0, 0, old.size
+    old[:256] = np.frombuffer(bytes(h), np.uint8)
+    return old
+
+
+def _decode_codes(pw):
+    """The matrix that the two-bit codes of a blob hold, from the format's description alone."""
+    h = pw.header
+    units = pw.blob[h.off_codes:h.off_codes + h.n_blocks * h.code_planes * h.code_units * 1024].view(np.uint32)
+    units = units.reshape(h.n_blocks, h.code_planes, h.code_units, 64, 4)
+    w = np.zeros((h.code_units * 256, h.n_blocks * 16), np.int32)
+    for lane in range(64):
+        for d in range(4):
+            for hh in range(2):
+                for i in range(4):
+                    for j in range(2):
+                        code = units[:, :, :, lane, d] >> (14 - 2 * (4 * hh + i) + 16 * j) & 3
+                        value = (np.where(code & 1, 1, 0) * np.where(code & 2, -1, 1)).sum(1)          # [block][unit]
+                        row = 64 * d + 32 * hh + 8 * (lane // 16) + 2 * i + j
+                        w[row::256, lane % 16::16] = value.T
+    return w[:h.inners, :h.columns], w
+
+
+@pytest.mark.parametrize("K,N", [(1, 1), (255, 16), (256, 17), (257, 40), (1000, 33)])
+def test_codes_hold_the_matrix(K, N):
+    w = ternary_weight(K, N, 0.5, K)
+    got, whole = _decode_codes(packing.PackedWeight.from_dense(w))
+    assert np.array_equal(got, w) and np.count_nonzero(whole) == np.count_nonzero(w)
+
+
+def test_codes_added_to_a_blob_of_the_version_before():
+    """tl_layout_add_codes makes what packing makes, for entries beyond one too, says how much room it takes, and refuses less."""
+    L = _lib.lib()
+    w = ternary_weight(600, 40, 0.5, 3)
+    rows, off, _ = packing.convert_to_ter_tiled_mcsc(w, 40, 600, *packing.count_nnz(w), 256, True, 8)
+    for new in (packing.PackedWeight.from_dense(w), packing.PackedWeight.from_mcsc(rows, off, 40, 600, 256)):
+        old = _old_version(new)
+        assert L.tl_layout_validate(old.ctypes.data, old.size) == 0
+        size = ctypes.c_int64(-1)
+        assert L.tl_layout_add_codes(old.ctypes.data, old.size, None, ctypes.byref(size)) == 0 and size.value == new.blob.size
+        out = np.full(size.value, 7, np.uint8)
+        assert L.tl_layout_add_codes(old.ctypes.data, old.size, out.ctypes.data, ctypes.byref(size)) == 0 and np.array_equal(out, new.blob)
+        assert np.array_equal(packing.PackedWeight(old).blob, new.blob)
+        again = np.zeros(size.value, np.uint8)
+        assert L.tl_layout_add_codes(out.ctypes.data, out.size, again.ctypes.data, ctypes.byref(size)) == 0 and np.array_equal(again, out)
+        short = ctypes.c_int64(size.value - 1)
+        assert L.tl_layout_add_codes(old.ctypes.data, old.size, out.ctypes.data, ctypes.byref(short)) == -8   # TL_ERR_SIZE
+        old[600] ^= 1
+        assert L.tl_layout_add_codes(old.ctypes.data, old.size, None, ctypes.byref(size)) == -9               # TL_ERR_FORMAT
+
+
+def test_codes_that_contradict_the_stream():
+    """Any bit of the codes that is not what the index stream says makes a blob invalid."""
+    pw = packing.PackedWeight.from_dense(ternary_weight(300, 20, 0.5, 3))
+    h = pw.header
+    for at in (0, 1023, 1024, 3000, h.total_bytes - h.off_codes - 1):
+        bad = pw.blob.copy()
+        bad[h.off_codes + at] ^= 0x40
+        assert _lib.lib().tl_layout_validate(bad.ctypes.data, bad.size) == -9, at
 
 
 @pytest.mark.parametrize("spare,outcomes", [(7 << 20, (0,)), (0, (-8,))])

@@ -57,8 +57,8 @@ def test_noalloc_entry_point_equals_tl_spmm(cuda, oracle, dtype):
     w = ternary_weight(K, N, 0.7, 131)
     dw = ops.DeviceWeight(PackedWeight.from_dense(w), cuda)
     scale = (0.5 + torch.rand(N, generator=torch.Generator().manual_seed(5))).to(dtype).to(cuda)
-    ws = torch.empty(40 << 20, dtype=torch.uint8, device=cuda)   # no room for partial sums: whole output tiles, as in the other entry point
-    # row counts of every kernel: 1 (no scratch), 16 and 40 (K-major image of a few rows), 700 and 130 (row kernel);
+    ws = torch.empty(40 << 20, dtype=torch.uint8, device=cuda)
+    # row counts of every kernel: 1, 16 and 40 (few rows), 700 and 130 (through the image of the activations);
     # each pair runs larger first, then smaller, back to back on one stream
     for sizes in ((700, 130), (40, 16), (300, 1), (16, 700)):
         for M in sizes:
