@@ -6,10 +6,11 @@ one step = one ternary SpMM of the gate projection: 8 x 128 = 1024 token rows, f
 ~N(0,1), W ternary [4096 -> 11008] at 80 % sparsity (10 % +1, 10 % -1, i.i.d., seeded), per-output
 fp16 scale ~U(0.5, 1.5), fp32 accumulation, fp16 output.  Inputs are resident in HBM before the
 timed region.  The value is algorithmic GB/s: bytes every operand must move at least once
-(index stream as stored, chunk table, X, Y, scale) divided by the step time.
+(index stream as stored, chunk table, X, Y, scale) divided by the step time.  The kernel of this step
+multiplies two-bit codes of the same weight on the matrix cores; its roofline is theirs.
 
 Prints ONE JSON line.  Besides the contract fields it carries
-  roofline      HBM roofline of the dominant kernel, timed with HIP events on the kernel's stream
+  roofline      matrix-core roofline of the dominant kernel, timed with HIP events on the kernel's stream
   cpu_baseline  the reference's CPU SIMD kernel on the same W and X, on this host's cores
   extra         the other regimes of the path (decode SpMV, small batch, fused MLP block), add-rate
                 figures, and tokens/s
@@ -24,6 +25,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E, published
+MFMA_PEAK_TFLOPS = 2500.0  # dense fp16, nominal
 VALU_PEAK_GADDS = 39321.6      # 256 CU x 64 lanes x 2.4 GHz fp32 adds/s without packed-fp32 forms
 
 
@@ -207,9 +209,10 @@ def cold_decode_leg(dev, K=4096, N=4096, sparsity=0.66, copies=48, calls=1000, M
     """Config 2 as the decoder meets it: `calls` SpMV calls, each with an x of its own, over `copies` distinct
     copies of the weight (about 300 MB, more than the last-level cache holds), captured as one HIP graph
     and replayed.  With M > 1: the same for a batch of M rows (row-major).  Beside it, under the same replay, the
-    box's own floors for a call that must stream that much memory: a launch that only READS one weight copy
-    (tl_stream_read_probe: 16 bytes per lane, one store per workgroup) and a plain device copy of it (which reads
-    and writes)."""
+    box's own floors for a call that must stream that much memory: a launch that only READS what a call needs of one
+    weight copy -- its index stream for a single row, the smaller of index stream and codes for more of them --
+    (tl_stream_read_probe: 16 bytes per lane, one store per workgroup) and a plain device copy of it
+    (which reads and writes)."""
     import torch
     from ternaryllm_amd import ops
     w, pw, dw = weight_and_packed(K, N, sparsity, 1244, dev)
@@ -232,19 +235,22 @@ def cold_decode_leg(dev, K=4096, N=4096, sparsity=0.66, copies=48, calls=1000, M
     for i in (0, calls - 1):
         ref = xs[i].double().cpu().numpy() @ w.double().numpy()
         err = max(err, float(abs(ys[i].double().cpu().numpy() - ref).max() / max(1e-9, abs(ref).max())))
-    dst = torch.empty_like(dw.blob)
+    def read_part(weight):
+        at, end = weight.header.off_codes, weight.blob.numel()
+        return weight.blob[:at] if M == 1 or at < end - at else weight.blob[at:]
+
+    dst = torch.empty_like(read_part(dw))
     nodes = min(calls, 4 * copies)
-    copy_t = graph_us_per_node(lambda i: dst.copy_(ws[i % copies].blob), nodes, 12, full=True)
+    copy_t = graph_us_per_node(lambda i: dst.copy_(read_part(ws[i % copies])), nodes, 12, full=True)
     folds = torch.empty(ops._lib.lib().tl_read_probe_workgroups(), dtype=torch.int32, device=dev)
-    whole = (dw.blob.numel() // 16) * 16
-    read_t = graph_us_per_node(lambda i: ops.stream_read_probe(ws[i % copies].blob[:whole], folds), nodes, 12, full=True)
+    read_t = graph_us_per_node(lambda i: ops.stream_read_probe(read_part(ws[i % copies]), folds), nodes, 12, full=True)
     B = pw.algorithmic_bytes(M, 2, 2)
     out = {"M": M, "K": K, "N": N, "sparsity": sparsity, "x_layout": "K-major [K][M]" if kmajor else "row-major [M][K]", "weight_copies": copies,
            "distinct_x": calls, "us_per_call_best10_mean": round(t["best10_mean"] * 1e6, 3),
            "GB_per_s": round(B / med / 1e9, 1), "pct_hbm_peak": round(100 * B / med / 1e9 / HBM_PEAK_GBS, 2),
-           "tokens_per_s": round(M / med, 1), "max_err_over_max": err, "weight_bytes": int(dw.blob.numel()),
+           "tokens_per_s": round(M / med, 1), "max_err_over_max": err, "weight_bytes": int(dw.blob.numel()), "weight_bytes_read": int(dst.numel()),
            "read_only_stream_of_one_weight_us": round(read_t["median"] * 1e6, 3),
-           "read_only_stream_GB_per_s": round(dw.blob.numel() / read_t["median"] / 1e9, 1),
+           "read_only_stream_GB_per_s": round(dst.numel() / read_t["median"] / 1e9, 1),
            "time_over_read_floor": round(med / read_t["median"], 2),
            "plain_copy_of_one_weight_us": round(copy_t["median"] * 1e6, 3), "time_over_plain_copy": round(med / copy_t["median"], 2)}
     out.update(us_fields(t))
@@ -346,9 +352,9 @@ def decode_nodes_leg(model, dev, pos_value):
     kv_bytes = 2 * c.num_attention_heads * (pos_value + 1) * c.head_dim * x.element_size()
     kv_bytes -= kv_bytes % 16
 
-    def blob(m):
-        b = m.device_weight().blob
-        return b[:(b.numel() // 16) * 16]
+    def blob(m):  # what a single-row product reads: everything in front of the codes
+        w = m.device_weight()
+        return w.blob[:w.header.off_codes]
 
     kinds = [
         ("q|k|v product, " + norm_note, lambda i: behind_norm(L[i].qkv_proj, L[i].input_layernorm),
@@ -493,10 +499,9 @@ def main():
     x = torch.randn((M, K), generator=g).to(torch.float16)
     scale = (0.5 + torch.rand(N, generator=g)).to(torch.float16)
     xd, sd = x.to(dev), scale.to(dev)
-    # row-major [M][K] activations, what TernaryLinear.forward passes: one call is the re-layout pre-pass, the row
-    # kernel and its fix-up launch
+    # row-major [M][K] activations, what TernaryLinear.forward passes: one launch of the matrix-core kernel
     wall_ms, ev_ms = time_spmm(dw, xd, sd, args.steps, args.warmup)
-    # beside it: activations already in the kernel's own layout ([K][M], M contiguous), no pre-pass
+    # beside it: K-major activations ([K][M], M contiguous), which go through the image that the kernel reads
     xk = xd.t().contiguous()
     wall_km_ms, ev_km_ms = time_spmm(dw, xk, sd, args.steps, args.warmup, x_layout=_lib.TL_X_K_MAJOR)
     y = ops.spmm(dw, xd, sd)
@@ -513,14 +518,14 @@ def main():
     # HBM bytes per call from rocprofv3's FETCH_SIZE / WRITE_SIZE (profiles/): reported only while the kernels are
     # still the ones it was recorded for
     traffic, traffic_note = None, "no traffic record"
-    tpath = os.path.join(ROOT, "profiles", "spmm_rows_c3_gate_traffic.json")
+    tpath = os.path.join(ROOT, "profiles", "matrix_rows_traffic.json")
     if os.path.exists(tpath):
         with open(tpath) as f:
             rec = json.load(f)
         if rec.get("kernel_source_sha16") == kernel_source_hash():
-            traffic, traffic_note = rec.get("hbm_bytes_per_launch"), "rocprofv3 FETCH_SIZE + WRITE_SIZE, profiles/spmm_rows_c3_gate_traffic.json"
+            traffic, traffic_note = rec.get("hbm_bytes_per_launch"), "rocprofv3 FETCH_SIZE + WRITE_SIZE, profiles/matrix_rows_traffic.json"
         else:
-            traffic_note = "profiles/spmm_rows_c3_gate_traffic.json was recorded for other kernel sources (%s)" % rec.get("kernel_source_sha16")
+            traffic_note = "profiles/matrix_rows_traffic.json was recorded for other kernel sources (%s)" % rec.get("kernel_source_sha16")
     out = {
         "metric": "ternary SpMM GB/s (% HBM peak) + tokens/s, Llama-2-7B ternary MLP shape",
         "value": round(gbs, 2), "unit": "GB/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
@@ -532,8 +537,9 @@ def main():
                    "x_layout": "row-major [M][K]", "max_rel_err": max_rel},
         "pct_hbm_peak": round(100 * gbs / HBM_PEAK_GBS, 3),
         "tokens_per_s": round(M / (wall_ms * 1e-3), 1),
-        "roofline": {"bound": "hbm", "achieved": round(B / (ev_ms * 1e-3) / 1e9, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(B / (ev_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 5), "traffic": traffic, "traffic_note": traffic_note,
+        "roofline": {"bound": "mfma", "achieved": round(2.0 * M * K * N / (ev_ms * 1e-3) / 1e12, 2), "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
+                     "frac": round(2.0 * M * K * N / (ev_ms * 1e-3) / 1e12 / MFMA_PEAK_TFLOPS, 5), "note": "dense operations; a zero weight is multiplied too",
+                     "traffic": traffic, "traffic_note": traffic_note,
                      "kernel": "tl_matrix_rows<1, 2, 4, 4, 2, 4, 0> (the one launch of a tl_spmm call on row-major activations)",
                      "kernel_ms": round(ev_ms, 5)},
     }
@@ -542,7 +548,7 @@ def main():
         "valu_add_roofline_frac": round(M * nnz / (ev_ms * 1e-3) / 1e9 / VALU_PEAK_GADDS, 4),
         "gop_equiv_per_s": round(2.0 * M * K * N / (ev_ms * 1e-3) / 1e9, 1),
         "k_major_input": {"ms_per_step": round(wall_km_ms, 5), "kernel_ms": round(ev_km_ms, 5),
-                          "note": "activations handed over as [K][M]: no re-layout pre-pass"},
+                          "note": "activations handed over as [K][M]: an image pass in front of the product"},
     }
     # the reference's own statistic (benchmark_ternary_mlp.py:51-53,98): 100 single calls timed one by one,
     # mean of the fastest 10; median and 10th percentile beside it

@@ -182,8 +182,9 @@ class PackedWeight:
         return w
 
     def algorithmic_bytes(self, M, x_bytes, y_bytes, scale_bytes=0):
-        """Bytes one product must move at least once: the stream as stored (index bytes with their
-        padding and the embedded descriptors), the chunk table, X, Y and the optional scale."""
+        """Bytes one product must move at least once where the weight is its index stream: the stream as stored (index
+        bytes with their padding and the embedded descriptors), the chunk table, X, Y and the optional scale.  (Kernels on
+        the two-bit codes read those in its place: a quarter of a byte for each of the K * N weights.)"""
         h = self.header
         table = (h.n_tiles * h.n_blocks + 1) * 4
         return int(h.stream_bytes + table + M * h.inners * x_bytes + M * h.columns * y_bytes + h.columns * scale_bytes)
