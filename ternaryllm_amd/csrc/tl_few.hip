@@ -5,7 +5,8 @@
 // activations are the matrix operand as they lie in a row, and every load of a turn (256 rows of K) is in flight before the
 // first product.  fp32 rows become three bf16 parts in registers; with 48 of them that is what takes the time.
 // us at 4096 -> 11008, 66 % zeros, walking the index stream / here: fp16 2 rows 16.6 / 6.1, 8 rows 20.8 / 7.9 (11.3 MB of
-// codes: 1.4 TB/s), 48 rows 70 / 26; fp32 8 rows 25.6 / 13.0, 48 rows 103 / 47.
+// codes: 1.4 TB/s), 48 rows 70 / 26 (at this width the rule in tl_kernels.hip leaves 9 to 48 fp16 rows to the walk); fp32 8
+// rows 25.6 / 13.0, 48 rows 103 / 47.
 #include "tl_matrix.h"
 
 using namespace tl;
@@ -39,22 +40,32 @@ __device__ __forceinline__ void load8(const KernelArgs& a, const XT* row, int k,
 }
 
 // Eight fp32 values in three bf16 parts (tl_matrix.h).  What is not finite need not survive: any part that is not finite
-// makes the sum so, and that output is worked out again.
+// makes the sum so, and that output is worked out again.  (So it is above 2^112, where a scaled value overflows here.)  A
+// part is taken off with a dot product of bf16 pairs -- one factor the part's, one zero; exact, as what is left is an
+// fp32 number, denormals included -- in the place of a mask and a subtraction, and of the scaling for the first.  us with
+// masks / so, 48 rows: 4096 -> 11008 53.2 / 46.5, 2048 -> 5504 17.0 / 15.2 (45.8 and 14.3 without the scaling); 8 rows
+// 4096 -> 11008 13.2 / 13.5 (12.0).
 __device__ __forceinline__ void split8(const float* v, u32x4* part)
 {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    auto pair = [](uint32_t lo, uint32_t hi) { return __builtin_amdgcn_perm(hi, lo, 0x07060302u); };   // the upper halves
+    // value - factor * (the lower or upper number of a pair)
+    auto less = [](float value, uint32_t two, uint32_t factors) {
+        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, two), __builtin_bit_cast(bf16x2, factors), value, false);
+    };
+    uint32_t s_lo = 0xC780u, s_hi = 0xC7800000u, o_lo = 0xBF80u, o_hi = 0xBF800000u;   // -2^16, -1 in bf16
+    // in registers: folded into the instruction, -1 in the upper half becomes an inline constant, which a pair reads otherwise
+    asm("" : "+v"(s_lo), "+v"(s_hi), "+v"(o_lo), "+v"(o_hi));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        uint32_t bits[2][3];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const float x = v[2 * i + e];
-            bits[e][0] = __float_as_uint(x);
-            const float r1 = (x - __uint_as_float(bits[e][0] & 0xffff0000u)) * kLowScale;
-            bits[e][1] = __float_as_uint(r1);
-            bits[e][2] = __float_as_uint(r1 - __uint_as_float(bits[e][1] & 0xffff0000u));
-        }
-#pragma unroll
-        for (int p = 0; p < 3; ++p) part[p][i] = __builtin_amdgcn_perm(bits[1][p], bits[0][p], 0x07060302u);  // the upper halves
+        const float lo = v[2 * i], hi = v[2 * i + 1];
+        const uint32_t a = pair(__float_as_uint(lo), __float_as_uint(hi));
+        const float lo1 = less(lo * kLowScale, a, s_lo), hi1 = less(hi * kLowScale, a, s_hi);
+        const uint32_t b = pair(__float_as_uint(lo1), __float_as_uint(hi1));
+        const float lo2 = less(lo1, b, o_lo), hi2 = less(hi1, b, o_hi);
+        part[0][i] = a;
+        part[1][i] = b;
+        part[2][i] = pair(__float_as_uint(lo2), __float_as_uint(hi2));
     }
 }
 
