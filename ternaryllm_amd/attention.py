@@ -51,8 +51,8 @@ class LlamaTernaryAttention(nn.Module):
     def __init__(self, config, layer_idx=None, *, generator=None, reference_buffers=True, fused_qkv=True):
         """fused_qkv: multiply the hidden states by ONE packed weight that holds the columns of q_proj, k_proj and
         v_proj side by side (built from the three at the first forward on a device, and again when one of them
-        changes; a fourth blob as large as the three together): one pass over the activations, one re-layout and one
-        fix-up launch instead of three of each.  q_proj, k_proj and v_proj stay what the reference has there."""
+        changes; a fourth blob as large as the three together): one launch and one pass over the activations instead
+        of three.  q_proj, k_proj and v_proj stay what the reference has there."""
         super().__init__()
         self.config = config
         self.fused_qkv = fused_qkv

@@ -141,15 +141,17 @@ extern "C" int tl_spmm_workspace(const tl_layout_header* header, int64_t M, int 
 namespace {
 // Whether a product is tl_few.hip's.  It costs the bytes of the codes (two bits an entry) whatever the weight; the kernels
 // that walk the index stream cost its bytes, and some of them start from a K-major image that a K-major caller has at hand.
-// us, walk / codes, 4096 -> 11008:
-//   one row         fp16 8.0 / 5.9, 5.4 / 6.1;  fp32 8.2 / 11.0, 5.4 / 11.1 (66 %, 95 % zeros): never, one row's gated and fused
-//                   products are the walk's and equal the plain one bit for bit
+// us, walk / codes, 4096 -> 11008 at 66 % and at 95 % zeros:
+//   one row         fp16 8.0 / 5.9, 5.4 / 6.1;  fp32 8.2 / 11.0, 5.4 / 11.1: never.  One row's gated and fused products are the
+//                   walk's and equal the plain one bit for bit; that costs the fp16 rows of dense weights.
 //   8 rows          fp16 21.0 / 8.0, 14.8 / 8.1;  fp32 25.3 / 12.8, 18.4 / 13.0: always
-//   ... K-major     fp16 17.7 / 14.9, 11.7 / 15.1;  fp32 22.4 / 19.4, 14.6 / 19.7: by bytes (3 and 4 rows, which the walk does
-//                   not take from an image: fp16 38 / 15, 31 / 15: always)
-//   16 rows         fp16 27.6 / 10.7, 15.6 / 11.0: always;  fp32 27.3 / 18.1, 14.0 / 18.4: by bytes
-//   ... fp16 where the walk has the gated epilogue: never, so that tl_spmm_gated stays tl_spmm and the gate bit for bit
-//   48 rows         fp16 71.7 / 25.8, 43.6 / 26.1;  fp32 102 / 46, 76 / 46: always
+//   16 rows         fp16 27.6 / 10.7, 15.6 / 11.0: always, but see below;  fp32 27.3 / 18.1, 14.0 / 18.4: by bytes
+//   48 rows         fp16 71.7 / 25.8, 43.6 / 26.1: always, but see below;  fp32 102 / 46, 76 / 46: always
+//   9 to 48 fp16 rows where the walk has the gated epilogue (an even N, wide -- this one is): never, so that tl_spmm_gated
+//                   stays tl_spmm and the gate bit for bit.  The price is what the two lines above say.
+//   K-major         3 and 4 rows, which the walk does not take from an image, fp16 38 / 15, 31 / 15: always;  8 rows fp16 17.7 / 14.9,
+//                   11.7 / 15.1, fp32 22.4 / 19.4, 14.6 / 19.7: by bytes, which errs where both are slow (32 fp32 rows, 95 %:
+//                   51.0 / 33.7, and the walk is taken)
 // A knob that names another kernel for few rows keeps the call with it.
 bool few_on_matrix_cores(const KernelArgs& a, const tl_layout_header* h, int64_t M, bool chained)
 {

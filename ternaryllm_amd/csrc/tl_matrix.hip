@@ -4,7 +4,8 @@
 // by direct loads (`global_load_lds_dwordx4`: no register holds them on the way), a few stages ahead; the weights' two-bit
 // codes arrive the same way, a unit of 256 rows of K ahead.  A wave turns the codes of its columns into operands in
 // registers, where they serve all of its activation rows.  tl_x_image makes the row-major, padded copy of activations that
-// come in another layout, and the three bf16 parts of fp32 ones.
+// come in another layout, and the three bf16 parts of fp32 ones.  tl_walk_rows multiplies from the index stream, for blobs
+// without codes and K-major rows without a workspace.
 #include "tl_matrix.h"
 
 using namespace tl;
@@ -13,8 +14,8 @@ namespace {
 
 constexpr int kStageRows = 64;                       // rows of K of a stage
 constexpr int kStageRowBytes = kStageRows * 2;       // bytes of one activation row in a stage
-// Row tiles whose column tiles a part of the chip works through together.  An activation tile is four times the bytes of a
-// code tile along the same K, so few row tiles against many column tiles is least traffic: 8192 x 2048 -> 11008 took 456 us
+// Row tiles whose column tiles a part of the chip works through together.  An activation tile is eight times the bytes of
+// a code tile along the same K (24 times for fp32 in three parts), so few row tiles against many column tiles is least traffic: 8192 x 2048 -> 11008 took 456 us
 // with all 64 row tiles in one group (every column tile streamed all activations through an L2), 300 / 300 / 310 with 2 / 4 / 8.
 constexpr int kRowGroup = 4;
 constexpr int kUnitStages = TL_CODE_UNIT_ROWS / kStageRows;
