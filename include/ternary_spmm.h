@@ -152,7 +152,7 @@ int tl_tiled_mcsc_to_dense(const void* merged_row, int index_width, int64_t n_in
 
 #define TL_LAYOUT_MAGIC 0x35474C54u /* "TLG5" */
 #define TL_LAYOUT_VERSION 6
-#define TL_LAYOUT_VERSION_NO_CODES 5 /* the same without the two-bit codes: still read, multiplied by a slow general kernel */
+#define TL_LAYOUT_VERSION_NO_CODES 5 /* the same without the two-bit codes: still read; any number of rows walks the index stream */
 #define TL_BLOCK_COLUMNS 16
 #define TL_CODE_UNIT_ROWS 256
 #define TL_CODE_UNIT_BYTES 1024
