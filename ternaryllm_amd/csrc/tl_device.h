@@ -43,6 +43,8 @@ struct KernelArgs {
     WeightPtrs w1;  // second weight set of the fused gate/up kernel
     const void* X;
     void* Y;
+    Codes c0;             // matrix-core kernels: the codes of w0 (among the first fields: a kernel of 3 us waits for each cache line of them)
+    int units, planes;    // matrix-core kernels: code units along K; planes of the weight, of two weights the larger number
     long long ldx, ldy;
     int M, N, K, T, tile_rows, NB;
     int x_f16, x_kmajor, y_f16, scale_f16;
@@ -54,8 +56,6 @@ struct KernelArgs {
     unsigned vpt_magic;   // small-M kernel, row-copy staging: ceil(2^32 / (tile_rows / values per vector))
     unsigned tile_magic;  // ceil(2^32 / tile_rows): k / tile_rows == (k * tile_magic) >> 32 for every k < 2^24
     long long x_sm, x_sk; // small-M kernel: element strides of the activations along M and along K
-    Codes c0;                 // matrix-core kernels: the codes of w0
-    int units, planes;        // matrix-core kernels: code units along K; planes of the weight, of two weights the larger number
     float one;  // 1.0f, passed in so that the fp16 -> fp32 accumulate stays a single mixed-precision fma
     // single-row kernel with a fused producer of its input (tl_spmv_fused)
     const void* X2;       // second summand of the residual add, or null
