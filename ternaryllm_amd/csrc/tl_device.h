@@ -82,7 +82,7 @@ struct KernelArgs {
     const void* image;        // the activations they multiply: row-major, 16-byte pieces along K ...
     long long image_ld;       // ... elements between rows
     long long image_plane;    // ... and, for fp32 activations in three bf16 parts, between parts
-    int vector_out;           // four neighbouring outputs of a row may be stored as one piece
+    int vector_out;           // whole pieces of 16 bytes of an output row may be stored (from 8-byte boundaries)
 };
 
 // rsqrt(mean square + eps) of the rows behind a chained product.  Called by the first 64 threads of a workgroup (one

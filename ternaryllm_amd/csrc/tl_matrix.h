@@ -62,12 +62,6 @@ __device__ __forceinline__ void split3(float v, uint32_t* a, uint32_t* b, uint32
     *c = fine ? __float_as_uint(r2) & 0xffff0000u : 0u;
 }
 
-__device__ __forceinline__ bool finite4(f32x4 v)
-{
-    return fabsf(v[0]) < __builtin_huge_valf() && fabsf(v[1]) < __builtin_huge_valf() && fabsf(v[2]) < __builtin_huge_valf() &&
-           fabsf(v[3]) < __builtin_huge_valf();
-}
-
 // One output of the product from the index stream alone: x(k) of the rows that column n names, added and subtracted.
 template <typename X>
 __device__ __forceinline__ float walk_column(const WeightPtrs& w, int T, int tile_rows, int n, X x)

@@ -12,6 +12,10 @@ using namespace tl;
 
 namespace {
 
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef u32x4 u32x4_out __attribute__((aligned(8)));
+typedef f32x4 f32x4_out __attribute__((aligned(8)));
+
 constexpr int kStageRows = 64;                       // rows of K of a stage
 constexpr int kStageRowBytes = kStageRows * 2;       // bytes of one activation row in a stage
 // Row tiles whose column tiles a part of the chip works through together.  An activation tile is eight times the bytes of
@@ -31,46 +35,52 @@ __device__ __forceinline__ void load_to_lds(uint32_t lds, const void* base, uint
 }
 #pragma clang diagnostic pop
 
-template <int N>
-__device__ __forceinline__ void wait_loads_and_barrier()
+// acc[i] += sum over k of w[row 8 * (i / 4) + 4 * (lane / 32) + i % 4][k] * x[column lane % 32][k], 16 values of k, eight to a lane
+template <bool BF16>
+__device__ __forceinline__ f32x16 matrix_step32(u32x4 w, u32x4 x, f32x16 acc)
 {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
+    if constexpr (BF16) return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x), acc, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, w), __builtin_bit_cast(half8, x), acc, 0, 0, 0);
+}
+
+template <int N, typename F, int... I>
+__device__ __forceinline__ void static_for(F f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F f) { static_for<N>(f, std::make_integer_sequence<int, N>{}); }
+
+// All but this wave's last N loads have come, and, where waves share what they copy, every other wave's.
+template <bool SHARED, int N>
+__device__ __forceinline__ void loads_here()
+{
+    if constexpr (SHARED) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(N) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
 }
 
 // Where an activation row's 16-byte piece p of a stage lies among the row's eight: rotated by the row so that the 16 lanes
 // the LDS serves together (rows r and r + 1 share 256 bytes, all 64 banks) find their pieces on different banks.
 __device__ __forceinline__ int piece_place(int row, int p) { return p ^ ((row >> 1) & 7); }
 
-// Four neighbouring outputs of one row, v[i] in column n + i: scale, SiLU gate of column pairs, store.
-template <bool PAIRS>
-__device__ __forceinline__ void store4(const KernelArgs& a, int m, int n, f32x4 v, const float* scale4)
+// COUNT neighbouring outputs of row m from column n on, of N: 16 bytes at a time where they lie so (vector_out), else one by one.
+template <int COUNT>
+__device__ __forceinline__ void store_piece(const KernelArgs& a, int m, int n, int N, const float* v)
 {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] *= scale4[i];
-    if constexpr (PAIRS) {
-        float o[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) o[i] = gate_pair(as_output(v[2 * i], a.y_f16), as_output(v[2 * i + 1], a.y_f16), a.y_f16);
-        const long long at = (long long)m * a.ldy + n / 2;
-        if (n < a.N) store_out(a.Y, a.y_f16, at, o[0]);
-        if (n + 2 < a.N) store_out(a.Y, a.y_f16, at + 1, o[1]);
-        return;
-    }
     const long long at = (long long)m * a.ldy + n;
-    if (n + 3 < a.N && (a.vector_out)) {
+    if (a.vector_out && n + COUNT <= N) {
         if (a.y_f16) {
-            __half h[4];
+            __align__(16) __half o[COUNT];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) h[i] = __float2half(settled(v[i]));
-            *reinterpret_cast<uint2*>(static_cast<__half*>(a.Y) + at) = *reinterpret_cast<const uint2*>(h);
+            for (int i = 0; i < COUNT; ++i) o[i] = __float2half(settled(v[i]));
+#pragma unroll
+            for (int i = 0; i < COUNT / 8; ++i) reinterpret_cast<u32x4_out*>(static_cast<__half*>(a.Y) + at)[i] = reinterpret_cast<const u32x4*>(o)[i];
         } else {
-            *reinterpret_cast<f32x4*>(static_cast<float*>(a.Y) + at) = v;
+#pragma unroll
+            for (int i = 0; i < COUNT / 4; ++i) reinterpret_cast<f32x4_out*>(static_cast<float*>(a.Y) + at)[i] = f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
         }
         return;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (n + i < a.N) store_out(a.Y, a.y_f16, at + i, v[i]);
+    for (int i = 0; i < COUNT; ++i)
+        if (n + i < N) store_out(a.Y, a.y_f16, at + i, v[i]);
 }
 
 enum { kPlain = 0, kPairs = 1, kTwoWeights = 2 };
@@ -78,29 +88,112 @@ enum { kPlain = 0, kPairs = 1, kTwoWeights = 2 };
 // The product of one output: from the index stream where the matrix cores' sum is not finite.
 __device__ __forceinline__ float exact_output(const KernelArgs& a, const WeightPtrs& w, int m, int n) { return walk_column(w, a.T, a.tile_rows, n, callers_x(a, m)); }
 
-// Bound by the matrix cores: 1024 x 4096 -> 11008 in fp16 is 92 GFLOP dense, 80 us = 1155 TFLOP/s (8192 x 2048 -> 11008:
-// 1230; a library fp16 product of that size 1090, the matrix instruction alone on trivial operands 2000).  What it took, at
-// 1024 x 12288 -> 8192: sums kept in their registers (fences around the barrier) 190 -> 161 us; operands made between the
-// products instead of in front of them 161 -> 152.  The same product by adding activation rows up, one vector lane per row
-// and non-zero, took 457 us at 80 % zeros (1024 x 4096 -> 11008), 133 at 99 %; this one takes 80 at any.
-//
-// Output tiles of (WM * FM * 16) activation rows x (WN * FN * 16) columns, one per workgroup of WM x WN waves; a wave owns
-// FM * 16 rows x FN * 16 columns.  PARTS: 1 for fp16 activations, 3 for fp32 ones in bf16 parts (all three are multiplied by
-// the same operands while a unit's codes are at hand).  STAGES of activations in LDS.
-template <int PARTS, int WM, int WN, int FM, int FN, int STAGES, int MODE>
-__global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
+// A lane's sums of FN x FM fragments (32 columns x 32 rows: 16 neighbouring columns of one row a lane) on their way out; lane_m0
+// and lane_n0: its row and first column in the first.
+// A sum that is not finite is worked out again by the lane that holds it, before anything is stored: the outputs of
+// finite rows keep their bits whatever another row of the tile holds.  (The sums that need it go into a mask that a
+// loop takes bit by bit, so that the walk stands here once and the sums stay in registers.)
+template <int FN, int FM, int MODE>
+__device__ __forceinline__ void put_out(const KernelArgs& a, f32x16 (&acc)[FN][FM], int lane_m0, int lane_n0)
 {
-    constexpr int W = WM * WN, TM = WM * FM * 16, TN = WN * FN * 16;
+    constexpr int OUT_FN = MODE == kTwoWeights ? FN / 2 : FN;
+    bool fine = true;
+    float half = 0.5f;                                            // (the products are with +-2)
+#pragma unroll
+    for (int f = 0; f < FN; ++f)
+#pragma unroll
+        for (int m = 0; m < FM; ++m)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) fine = fine && fabsf(acc[f][m][e]) < __builtin_huge_valf();
+    if (!fine) {
+        half = 1.0f;
+#pragma unroll 1
+        for (int i = 0; i < FN * FM; ++i) {
+            const int f = i / FM, m = i % FM;
+            float v[16];
+            uint32_t redo = 0;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                v[e] = acc[0][0][e];
+#pragma unroll
+                for (int o = 1; o < FN * FM; ++o) v[e] = o == i ? acc[o / FM][o % FM][e] : v[e];
+                const bool mine = lane_m0 + m * 32 < a.M && lane_n0 + f % OUT_FN * 32 + e < a.N;
+                redo |= mine && !(fabsf(v[e]) < __builtin_huge_valf()) ? 1u << e : 0u;
+                v[e] *= 0.5f;                                     // (twice what is worked out again might overflow)
+            }
+            while (redo != 0) {
+                const int at = __builtin_ctz(redo);
+                redo &= redo - 1;
+                const float y = exact_output(a, f >= OUT_FN ? a.w1 : a.w0, lane_m0 + m * 32, lane_n0 + f % OUT_FN * 32 + at);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) v[e] = e == at ? y : v[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+#pragma unroll
+                for (int o = 0; o < FN * FM; ++o) acc[o / FM][o % FM][e] = o == i ? v[e] : acc[o / FM][o % FM][e];
+        }
+    }
+#pragma unroll
+    for (int f = 0; f < OUT_FN; ++f) {
+        const int n = lane_n0 + f * 32;
+        float s0[16], s1[MODE == kTwoWeights ? 16 : 1];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            s0[i] = half * (n + i < a.N ? load_scale(a.w0.scale, a.scale_f16, n + i) : 0.f);
+            if constexpr (MODE == kTwoWeights) s1[i] = half * (n + i < a.N ? load_scale(a.w1.scale, a.scale_f16, n + i) : 0.f);
+        }
+#pragma unroll
+        for (int m = 0; m < FM; ++m) {
+            const int row = lane_m0 + m * 32;
+            if (row >= a.M || n >= a.N) continue;
+            float v[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                v[i] = acc[f][m][i] * s0[i];
+                if constexpr (MODE == kTwoWeights) v[i] = silu(v[i]) * (acc[f + FN / 2][m][i] * s1[i]);
+            }
+            if constexpr (MODE == kPairs) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] = gate_pair(as_output(v[2 * i], a.y_f16), as_output(v[2 * i + 1], a.y_f16), a.y_f16);
+                store_piece<8>(a, row, n / 2, a.N / 2, v);
+            } else {
+                store_piece<16>(a, row, n, a.N, v);
+            }
+        }
+    }
+}
+
+// Bound by the matrix cores and, at the large sizes, by the power that they draw: 8192 x 5504 -> 2048 in fp16 keeps them busy for
+// 80 % of the time at 1.88 GHz, 1290 TFLOP/s (a large library product in fp16 1197, the matrix instruction alone on such
+// operands 1710 to 1880); products of 16 x 16 x 32 instead of 32 x 32 x 16 ran 69 % of the time at 2.30 GHz, 1320.  A wave owns 64
+// columns: each fragment of activations that it reads from LDS serves two products (with 32 columns a wave the reads took
+// as many clocks as the products: 58 % busy).  us before / now: 8192 x 2048 -> 11008 gated 358 / 289, 8192 x 2048 -> 6144 194 / 169,
+// 8192 x 5504 -> 2048 161 / 143, 1024 x 4096 -> 11008 94 / 83; fp32 4096 x 4096 -> 4096 367 / 297, 200 x 2048 -> 2048 47 / 21.
+//
+// Output tiles of (WM * FM * 32) activation rows x (WN * FN * 32) columns, one per workgroup; a wave owns FM * 32 rows x
+// FN * 32 columns.  WK = 1: WM x WN waves over all of K that share what they copy.  WK > 1: one tile of a wave, whose WK waves
+// share K out by units, copy for themselves, wait for nobody and add up at the end.  PARTS: 1 for fp16 activations, 3 for fp32
+// ones in bf16 parts (a stage's three parts one after the other, with the same codes).
+template <int PARTS, int WM, int WN, int WK, int FM, int FN, int MODE>
+__global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArgs a)
+{
+    constexpr int W = WK > 1 ? 1 : WM * WN;                       // waves that work on the same rows of K, and share what is copied
+    constexpr int TM = WM * FM * 32, TN = WN * FN * 32;
+    static_assert(WK == 1 || (WM == 1 && WN == 1 && FM * FN == WK), "waves share either an output tile's rows of K or its outputs");
+    constexpr int STAGES = kUnitStages;                           // buffers of activations: a stage's place in its unit names its buffer
     constexpr int XB = TM * kStageRowBytes;                       // bytes of a stage of activations
-    constexpr int CB = (TN / 16) * TL_CODE_UNIT_BYTES;            // bytes of a unit of codes
     constexpr int XL = TM / 8 / W;                                // activation loads of a wave per stage (8 rows each)
     constexpr int CL = (TN / 16 + W - 1) / W;                     // code loads of a wave per unit
     static_assert(TM % (8 * W) == 0, "every wave loads the same number of row groups");
-    extern __shared__ __align__(16) unsigned char lds[];
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
+    extern __shared__ __align__(16) unsigned char all_lds[];
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wg_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = WK > 1 ? 0 : wg_wave, wk = WK > 1 ? wg_wave : 0;
     const int wm = wave / WN, wn = wave % WN;
+    constexpr int OWN = STAGES * XB + (TN / 16) * TL_CODE_UNIT_BYTES;   // LDS of the waves that share
+    unsigned char* lds = all_lds + wk * OWN;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
 
     // Each part of the chip (ids equal modulo 8), which has an L2 of its own, owns a contiguous run of the list of tiles; the
     // list goes through all column tiles for a few row tiles at a time.
@@ -121,40 +214,36 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
     uint32_t xrow[XL];                                            // byte offset of this lane's row from the tile's base
     const uint32_t limit = (uint32_t)((a.K + 7) / 8 * 16 - 16);          // last whole piece of a row: pieces past it meet zero weights
     const int lane_row = lane >> 3;
-    uint32_t piece[XL];
+    
+    // (rows of a lane's loads differ by 8 * W: by a multiple of 16, or, W = 1, by 8, which turns the place by half)
+    const uint32_t piece = (uint32_t)piece_place(wave * 8 + lane_row, lane & 7) * 16;
+    static_assert(W % 2 == 0 || W == 1, "a lane's pieces lie at one place, or at two in turn");
 #pragma unroll
-    for (int i = 0; i < XL; ++i) {
-        const int r = (i * W + wave) * 8 + lane_row;
-        xrow[i] = (uint32_t)(min(m0 + r, a.M - 1) - m0) * (uint32_t)(a.image_ld * 2);
-        piece[i] = (uint32_t)piece_place(r, lane & 7) * 16;
-    }
+    for (int i = 0; i < XL; ++i) xrow[i] = (uint32_t)(min(m0 + (i * W + wave) * 8 + lane_row, a.M - 1) - m0) * (uint32_t)(a.image_ld * 2);
     const unsigned char* image = static_cast<const unsigned char*>(a.image) + (long long)m0 * a.image_ld * 2;
     const long long unit_stride = TL_CODE_UNIT_BYTES;
 
     const int stages_k = (a.K + kStageRows - 1) / kStageRows;     // stages of K that hold anything
     const int all_units = a.planes * a.units;
-    // stages of unit u: the last one of the only plane may be shorter
-    const int last_stages = a.planes == 1 ? stages_k - (a.units - 1) * kUnitStages : kUnitStages;
-    const int total = PARTS * ((all_units - 1) * kUnitStages + last_stages);
+    // this wave's units, and its turns: the last stage of the only plane may end a unit early
+    const int unit0 = all_units * wk / WK, units = all_units * (wk + 1) / WK - unit0;
+    const int all_stages = a.planes == 1 ? stages_k : all_units * kUnitStages;
+    const int total = PARTS * (min((unit0 + units) * kUnitStages, all_stages) - unit0 * kUnitStages);
 
-    // load side: where the next activations to ask for lie, and the buffer they go to
-    int lu = 0, lk = 0, lp = 0, lj = 0, issued = 0;               // unit, unit within its plane, part, stage
-    uint32_t lbuf = lds0 + (uint32_t)wave * 1024;
-    auto issue_x = [&]() {
+    // load side: where the next activations to ask for lie
+    int lk = unit0 % a.units, lj = 0, lp = 0, issued = 0;                       // unit within its plane, stage, part
+    auto issue_x = [&](uint32_t buffer) {
         const uint32_t k_bytes = (uint32_t)(lk * TL_CODE_UNIT_ROWS + lj * kStageRows) * 2;
         const unsigned char* src = image + (PARTS > 1 ? (long long)lp * a.image_plane * 2 : 0ll);
+        const uint32_t at = min(k_bytes + piece, limit), at_odd = W == 1 ? min(k_bytes + (piece ^ 64u), limit) : at;
 #pragma unroll
-        for (int i = 0; i < XL; ++i) load_to_lds(lbuf + i * W * 1024, src, xrow[i] + min(k_bytes + piece[i], limit));
+        for (int i = 0; i < XL; ++i) load_to_lds(lds0 + buffer * XB + (i * W + wave) * 1024, src, xrow[i] + (i % 2 ? at_odd : at));
         ++issued;
-        lbuf = lbuf + XB >= lds0 + STAGES * XB ? lbuf - (STAGES - 1) * XB : lbuf + XB;
-        if (++lj == (lu == all_units - 1 ? last_stages : kUnitStages)) {
-            lj = 0;
-            if (++lp == PARTS) {
-                lp = 0;
-                ++lu;
-                if (++lk == a.units) lk = 0;
-            }
-        }
+        if (++lp < PARTS) return;
+        lp = 0;
+        if (++lj < kUnitStages) return;                           // (the last unit may be shorter: nothing is asked for after it)
+        lj = 0;
+        if (++lk == a.units) lk = 0;
     };
     const unsigned char* code_src[CL];                            // (wave-uniform)
     uint32_t code_to[CL];
@@ -162,9 +251,9 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
 #pragma unroll
     for (int i = 0; i < CL; ++i) {
         const int c = min(i * W + wave, TN / 16 - 1);             // column block of the tile
-        const int owner = c / FN, f = c % FN;                     // its wave column and fragment
-        const Codes& w = (MODE == kTwoWeights && f >= FN / 2) ? a.c1 : a.c0;
-        const int nb = MODE == kTwoWeights ? nb0 + owner * (FN / 2) + f % (FN / 2) : nb0 + c;
+        const int owner = c / (2 * FN), f = c % (2 * FN);         // its wave column and place there
+        const Codes& w = (MODE == kTwoWeights && f >= FN) ? a.c1 : a.c0;
+        const int nb = MODE == kTwoWeights ? nb0 + owner * FN + f % FN : nb0 + c;
         code_units[i] = w.planes * a.units;
         code_src[i] = w.base + min(nb, a.NB - 1) * (code_units[i] * unit_stride);
         code_to[i] = lds0 + STAGES * XB + c * TL_CODE_UNIT_BYTES;
@@ -172,177 +261,159 @@ __global__ __launch_bounds__(WM * WN * 64) void tl_matrix_rows(KernelArgs a)
     auto issue_codes = [&](int u) {
 #pragma unroll
         for (int i = 0; i < CL; ++i) {
-            const unsigned char* src = code_src[i] + u * unit_stride;
-            if (MODE == kTwoWeights && u >= code_units[i]) src = kNoCodes;   // (the other weight has more planes)
-            load_to_lds(code_to[i] + (u & 1) * CB, src, (uint32_t)lane * 16);
+            const unsigned char* src = code_src[i] + (unit0 + u) * unit_stride;
+            if (MODE == kTwoWeights && unit0 + u >= code_units[i]) src = kNoCodes;   // (the other weight has more planes)
+            load_to_lds(code_to[i], src, (uint32_t)lane * 16);
         }
     };
 
     // ---- what it reads ----
-    const int g = lane >> 4, r16 = lane & 15;
-    const uint32_t x_read = (uint32_t)((wm * FM * 16 + r16) * kStageRowBytes);
-    const uint32_t swz = (uint32_t)(piece_place(r16, g) * 16);    // rows of a wave's fragments differ by multiples of 16: same place
+    const int h = lane >> 5, r32 = lane & 31;
+    const uint32_t x_read = (uint32_t)((wm * FM * 32 + r32) * kStageRowBytes);
+    const uint32_t swz = (uint32_t)(piece_place(r32, h) * 16);    // rows of a wave's fragments differ by multiples of 32: same place
+    // the column of this lane's operand row: a lane's sums then are 16 neighbouring columns of one activation row
+    const int col = 16 * (r32 >> 2 & 1) + 4 * (r32 >> 3) + (r32 & 3);
+    const uint32_t c_read = (uint32_t)(STAGES * XB + (wn * FN * 2 + (col >> 4)) * TL_CODE_UNIT_BYTES + ((col & 15) + 16 * h) * 16);
     constexpr bool F32 = PARTS > 1;
-    f32x4 acc[FN][FM], low[F32 ? FN : 1][F32 ? FM : 1];           // low: the sums of the parts after the first
+    f32x16 acc[FN][FM], low[F32 ? FN : 1][F32 ? FM : 1];          // low: the sums of the parts after the first
 #pragma unroll
     for (int f = 0; f < FN; ++f)
 #pragma unroll
-        for (int m = 0; m < FM; ++m) acc[f][m] = low[F32 ? f : 0][F32 ? m : 0] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int m = 0; m < FM; ++m)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[f][m][e] = low[F32 ? f : 0][F32 ? m : 0][e] = 0.f;
 
-    // A stage is worked on in two halves of 32 rows of K, each half's activations read from LDS while the other half is
-    // multiplied, across stages too: the barrier that says that the next stage has come stands between the halves.
-    issue_codes(0);
-#pragma unroll
-    for (int s = 0; s < STAGES; ++s)
-        if (issued < total) issue_x();
-    u32x4 codes[FN], x0[FM], x1[FM];
-    uint32_t xbuf = x_read;                                       // this stage's activations
-    auto read_half = [&](u32x4* x, uint32_t half) {
-#pragma unroll
-        for (int m = 0; m < FM; ++m) x[m] = *reinterpret_cast<const u32x4*>(lds + xbuf + (swz ^ half) + m * 16 * kStageRowBytes);
+    constexpr int R = 4, AHEAD = R - 1;                           // fragments of activations in registers; read ahead
+    constexpr int STEPS = 4 * FM;                                 // of a stage: a fragment of 32 rows x 16 rows of K each
+    u32x4 x[R], codes[FN][2], w[2][FN];
+    auto read_x = [&](int buffer, int step) {                     // (constants)
+        x[step % R] = *reinterpret_cast<const u32x4*>(lds + x_read + (swz ^ (uint32_t)(step / FM * 32)) + buffer * XB + step % FM * 32 * kStageRowBytes);
     };
-    auto read_codes = [&](u32x4* c, int u) {
-        const unsigned char* cs = lds + STAGES * XB + (u & 1) * CB + (wn * FN) * TL_CODE_UNIT_BYTES + lane * 16;
+    auto read_codes = [&](int half) {
 #pragma unroll
-        for (int f = 0; f < FN; ++f) c[f] = *reinterpret_cast<const u32x4*>(cs + f * TL_CODE_UNIT_BYTES);
+        for (int f = 0; f < FN; ++f) codes[f][half] = *reinterpret_cast<const u32x4*>(lds + c_read + f * 2 * TL_CODE_UNIT_BYTES + half * 512);
     };
-    if (total >= STAGES) wait_loads_and_barrier<(STAGES - 1) * XL>();
-    else wait_loads_and_barrier<0>();
-    read_codes(codes, 0);
-    read_half(x0, 0);
+    // dword d % 4 of fragment d / 4's operand of the 16 rows of K number j of a unit (constants)
+    auto operand_dword = [&](int j, int d, u32x4* to) {
+        to[d / 4][d % 4] = (codes[d / 4][j & 1][j >> 2] << ((j >> 1 & 1) * 8 + 2 * (d % 4))) & 0xC000C000u;
+    };
+    if (WK == 1 || units > 0) issue_codes(0);
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s)
+        if (issued < total) issue_x(s);
+    if (total >= STAGES - 1) loads_here<WK == 1, (STAGES - 2) * XL>();
+    else loads_here<WK == 1, 0>();
+    read_codes(0);
+    read_codes(1);
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s) read_x(0, s);
+#pragma unroll
+    for (int d = 0; d < 4 * FN; ++d) operand_dword(0, d, w[0]);
     int t = 0;
-    u32x4 w = weight_operand<0>(codes[0]);                        // operand of the next products
-    // The products of one half with the operands of all FN column fragments.  The operand of the next fragment -- at the
-    // end, of the next half's first -- is made between a fragment's products: a product keeps the matrix core busy for 16
-    // clocks, and the wave can issue three vector instructions meanwhile.
-    auto products = [&](auto step_tag, auto first_tag, const u32x4* x, auto next) {
-        constexpr int S = decltype(step_tag)::value;
+    // Turn Q of unit u: part Q % PARTS of its stage Q / PARTS.  STEADY: turns up to t + STAGES - 1 exist.
+    constexpr int TURNS = kUnitStages * PARTS;
+    auto turn = [&](auto q_tag, auto steady_tag, int u) {
+        constexpr int Q = decltype(q_tag)::value, J = Q / PARTS, P = Q % PARTS;
+        constexpr bool STEADY = decltype(steady_tag)::value, FIRST = P == 0;
+        constexpr int PER = 4 * FN / FM;                          // operand dwords made in a step
 #pragma unroll
-        for (int f = 0; f < FN; ++f) {
-            const u32x4 now = w;
-#pragma unroll
-            for (int m = 0; m < FM; ++m) {
-                f32x4& sum = decltype(first_tag)::value ? acc[f][m] : low[F32 ? f : 0][F32 ? m : 0];
-                sum = matrix_step<F32>(now, x[m], sum);
+        for (int s = 0; s < STEPS; ++s) {
+            const int m = s % FM, k = s / FM;                     // k: 16 rows of K of the stage
+            if (s == STEPS - AHEAD) {
+                // turn t + 1's activations have come; every wave is done with turn t - 1, whose buffer takes turn t + STAGES - 1
+                if (STEADY) loads_here<WK == 1, (STAGES - 3) * XL>();
+                else if (t + 1 < total) loads_here<WK == 1, 0>();
+                if (Q == 0 && (STEADY || u + 1 < units)) issue_codes(u + 1);
+                if (STEADY || issued < total) issue_x((Q + STAGES - 1) % STAGES);
             }
-            if (f + 1 < FN) w = weight_operand<S>(codes[f + 1 < FN ? f + 1 : 0]);
-            else w = next();
+            if (s + AHEAD < STEPS) read_x(Q % STAGES, s + AHEAD);
+            else read_x((Q + 1) % STAGES, s + AHEAD - STEPS);
+            if (Q == TURNS - 1 && m == 0 && k >= 2) read_codes(k - 2);
 #pragma unroll
-            for (int m = 0; m < FM; ++m) {
+            for (int f = 0; f < FN; ++f) {
+                f32x16& sum = FIRST ? acc[f][m] : low[F32 ? f : 0][F32 ? m : 0];
+                sum = matrix_step32<F32>(w[k & 1][f], x[s % R], sum);
+            }
+            constexpr int AFTER = P < PARTS - 1 ? 4 * J : 4 * J + 4;   // the unit's 16 rows of K that follow this turn
+#pragma unroll
+            for (int i = 0; i < PER; ++i) operand_dword((k < 3 ? 4 * J + k + 1 : AFTER) % 16, m * PER + i, w[(k + 1) & 1]);
+#pragma unroll
+            for (int f = 0; f < FN; ++f) {
                 __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);               // a product,
-                __builtin_amdgcn_sched_group_barrier(0x2, FM >= 8 ? 1 : 2, 0);  // then vector instructions
+                __builtin_amdgcn_sched_group_barrier(0x2, (2 * PER + FN - 1) / FN, 0);  // then vector instructions
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
-    };
-    // Stage J of part p of unit u (first: whether p is the leading part).  STEADY: stages t + 1 .. t + STAGES exist, so
-    // nothing needs to be asked.
-    auto turn = [&](auto j_tag, auto steady_tag, auto first_tag, int u, int p, bool part_ends) {
-        const bool unit_ends = part_ends && p == PARTS - 1;
-        constexpr int J = decltype(j_tag)::value;
-        constexpr bool STEADY = decltype(steady_tag)::value;
-        read_half(x1, 64);
-        if (J == 0 && decltype(first_tag)::value && u + 1 < all_units) issue_codes(u + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        products(std::integral_constant<int, 2 * J>{}, first_tag, x0, [&]() { return weight_operand<2 * J + 1>(codes[0]); });
-        // (without the fences the scheduler moves these products behind the barrier and pays for it with copies of the sums)
-        __builtin_amdgcn_sched_barrier(0);
-        u32x4 fresh[FN];
-        if (STEADY || t + 1 < total) {
-            // after this barrier every wave has read all of stage t: its buffer takes the stage STAGES further on
-            if (STEADY || total - t >= STAGES) wait_loads_and_barrier<(STAGES - 2) * XL>();
-            else wait_loads_and_barrier<0>();
-            if (STEADY || issued < total) issue_x();
-            xbuf = xbuf + XB >= STAGES * XB ? xbuf - (STAGES - 1) * XB : xbuf + XB;
-            read_half(x0, 0);
-            if (unit_ends) read_codes(fresh, u + 1);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        constexpr int AFTER = J == kUnitStages - 1 ? 0 : 2 * J + 2;   // (of the unit's next stage; a part that ends starts it again)
-        products(std::integral_constant<int, 2 * J + 1>{}, first_tag, x1, [&]() {
-            if (unit_ends) {
-#pragma unroll
-                for (int f = 0; f < FN; ++f) codes[f] = fresh[f];
-                return weight_operand<0>(codes[0]);
-            }
-            return AFTER != 0 && part_ends ? weight_operand<0>(codes[0]) : weight_operand<AFTER>(codes[0]);
-        });
-        __builtin_amdgcn_sched_barrier(0);
         ++t;
     };
-    constexpr std::integral_constant<int, 0> s0t; constexpr std::integral_constant<int, 1> s1t;
-    constexpr std::integral_constant<int, 2> s2t; constexpr std::integral_constant<int, 3> s3t;
-    auto one_part = [&](auto steady_tag, auto first_tag, int u, int p, int stages) {
-        turn(s0t, steady_tag, first_tag, u, p, stages == 1);
-        if (stages > 1) turn(s1t, steady_tag, first_tag, u, p, stages == 2);
-        if (stages > 2) turn(s2t, steady_tag, first_tag, u, p, stages == 3);
-        if (stages > 3) turn(s3t, steady_tag, first_tag, u, p, true);
-    };
-    auto one_unit = [&](auto steady_tag, int u, int stages) {
-        one_part(steady_tag, std::true_type{}, u, 0, stages);
-        if constexpr (F32)
-            for (int p = 1; p < PARTS; ++p) one_part(steady_tag, std::false_type{}, u, p, stages);
+    auto turns = [&](auto steady_tag, int u, int count) {
+        static_for<TURNS>([&](auto q) {
+            if (decltype(steady_tag)::value || decltype(q)::value < count) turn(q, steady_tag, u);
+        });
     };
     int u = 0;
-    for (; (u + 1) * PARTS * kUnitStages + STAGES <= total; ++u) one_unit(std::true_type{}, u, kUnitStages);
-    for (; u < all_units; ++u) one_unit(std::false_type{}, u, u == all_units - 1 ? last_stages : kUnitStages);
+    for (; (u + 1) * TURNS + STAGES - 1 <= total; ++u) turns(std::true_type{}, u, TURNS);
+    for (; u < units; ++u) turns(std::false_type{}, u, min(total - u * TURNS, TURNS));
 
     // ---- out ----
-    // A sum that is not finite is worked out again by the lane that holds it, before anything is stored: the outputs of
-    // finite rows keep their bits whatever another row of the tile holds.  (The sums that need it go into a mask that a
-    // loop takes bit by bit, so that the walk stands here once and the sums stay in registers.)
     constexpr int OUT_FN = MODE == kTwoWeights ? FN / 2 : FN;
-    const int wave_n0 = (nb0 + wn * OUT_FN) * 16, wave_m0 = m0 + wm * FM * 16;
-    static_assert(FN * FM * 4 <= 32, "a bit for each of a lane's sums");
-    bool fine = true;
-    float half = 0.5f;                                            // (the products are with +-2)
+    if constexpr (WK > 1) {
+        // every wave has sums of the whole tile, of its own rows of K: they meet in LDS (a wave's in its own part, which it is
+        // done with), and wave i goes on with fragment i.  Added up in 64 bits, as many roundings in 32 would weigh.
+        constexpr int FRAGMENT = 64 * 16 * 4, PIECES = F32 ? 2 : 1;
+        static_assert(PIECES * FN * FM * FRAGMENT <= OWN, "a wave's sums fit its part of LDS");
 #pragma unroll
-    for (int f = 0; f < FN; ++f)
+        for (int i = 0; i < FN * FM; ++i)
 #pragma unroll
-        for (int m = 0; m < FM; ++m) {
-            if constexpr (F32) add_low(acc[f][m], low[f][m]);
-            fine = fine && finite4(acc[f][m]);
-        }
-    if (!fine) {
-        uint32_t redo = 0;
-#pragma unroll
-        for (int e = 0; e < FN * FM * 4; ++e) {
-            const int f = e / (FM * 4), m = e / 4 % FM, i = e % 4;
-            const bool mine = wave_m0 + m * 16 + r16 < a.M && wave_n0 + f % OUT_FN * 16 + g * 4 + i < a.N;
-            redo |= mine && !(fabsf(acc[f][m][i]) < __builtin_huge_valf()) ? 1u << e : 0u;
-            acc[f][m][i] *= half;                                 // (twice what is worked out again might overflow)
-        }
-        half = 1.0f;
-        while (redo != 0) {
-            const int at = __builtin_ctz(redo), f = at / (FM * 4), m = at / 4 % FM;
-            redo &= redo - 1;
-            const float v = exact_output(a, f >= OUT_FN ? a.w1 : a.w0, wave_m0 + m * 16 + r16, wave_n0 + f % OUT_FN * 16 + g * 4 + at % 4);
-#pragma unroll
-            for (int e = 0; e < FN * FM * 4; ++e) acc[e / (FM * 4)][e / 4 % FM][e % 4] = e == at ? v : acc[e / (FM * 4)][e / 4 % FM][e % 4];
-        }
-    }
-#pragma unroll
-    for (int f = 0; f < OUT_FN; ++f) {
-        const int n = wave_n0 + f * 16 + g * 4;
-        float s0[4], s1[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            s0[i] = half * (n + i < a.N ? load_scale(a.w0.scale, a.scale_f16, n + i) : 0.f);
-            if constexpr (MODE == kTwoWeights) s1[i] = half * (n + i < a.N ? load_scale(a.w1.scale, a.scale_f16, n + i) : 0.f);
-        }
-#pragma unroll
-        for (int m = 0; m < FM; ++m) {
-            const int row = wave_m0 + m * 16 + r16;
-            f32x4 v = acc[f][m];
-            if constexpr (MODE == kTwoWeights) {
-                const f32x4 u = acc[f + FN / 2][m];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] = silu(v[i] * s0[i]) * (u[i] * s1[i]);
-                const float one[4] = {1.f, 1.f, 1.f, 1.f};
-                if (row < a.M && n < a.N) store4<false>(a, row, n, v, one);
-            } else {
-                if (row < a.M && n < a.N) store4<MODE == kPairs>(a, row, n, v, s0);
+            for (int q = 0; q < 4; ++q) {
+                auto put = [&](int piece, const f32x16& v) {
+                    *reinterpret_cast<f32x4*>(lds + (piece * FN * FM + i) * FRAGMENT + q * 1024 + lane * 16) = f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+                };
+                put(0, acc[i / FM][i % FM]);
+                if constexpr (F32) put(1, low[i / FM][i % FM]);
             }
+        __syncthreads();
+        auto total_of = [&](int i, f32x16& v) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                std::conditional_t<F32, double, float> sum[4] = {};
+#pragma unroll
+                for (int piece = PIECES - 1; piece >= 0; --piece) {
+#pragma unroll
+                    for (int o = 0; o < WK; ++o) {
+                        const f32x4 part = *reinterpret_cast<const f32x4*>(all_lds + o * OWN + (piece * FN * FM + i) * FRAGMENT + q * 1024 + lane * 16);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) sum[e] += part[e];
+                    }
+                    if (piece == 1)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) sum[e] *= 1.0f / kLowScale;
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[4 * q + e] = (float)sum[e];
+            }
+        };
+        if constexpr (MODE == kTwoWeights) {
+            if (wk >= OUT_FN * FM) return;
+            f32x16 v[2][1];
+            total_of(wk, v[0][0]);
+            total_of(wk + OUT_FN * FM, v[1][0]);
+            put_out<2, 1, MODE>(a, v, m0 + wk % FM * 32 + r32, nb0 * 16 + wk / FM * 32 + h * 16);
+        } else {
+            f32x16 v[1][1];
+            total_of(wk, v[0][0]);
+            put_out<1, 1, MODE>(a, v, m0 + wk % FM * 32 + r32, nb0 * 16 + wk / FM * 32 + h * 16);
         }
+    } else {
+        if constexpr (F32) {
+#pragma unroll
+            for (int f = 0; f < FN; ++f)
+#pragma unroll
+                for (int m = 0; m < FM; ++m)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[f][m][e] = fmaf(low[f][m][e], 1.0f / kLowScale, acc[f][m][e]);
+        }
+        put_out<FN, FM, MODE>(a, acc, m0 + wm * FM * 32 + r32, (nb0 + wn * OUT_FN * 2) * 16 + h * 16);
     }
 }
 
@@ -573,34 +644,48 @@ int walk_rows(KernelArgs a, void* workspace, int64_t workspace_bytes, bool two_w
     return launch_walk<XT, R>(a, two_weights, st);
 }
 
-template <int PARTS, int WM, int WN, int FM, int FN, int STAGES, int MODE>
+template <int PARTS, int WM, int WN, int WK, int FM, int FN, int MODE>
 int launch_tile(const KernelArgs& a, hipStream_t st)
 {
-    constexpr int TM = WM * FM * 16, TN = WN * FN * 16, OUT_TN = MODE == kTwoWeights ? TN / 2 : TN;
-    constexpr size_t lds = (size_t)STAGES * TM * kStageRowBytes + 2 * (TN / 16) * TL_CODE_UNIT_BYTES;
+    constexpr int TM = WM * FM * 32, TN = WN * FN * 32, OUT_TN = MODE == kTwoWeights ? TN / 2 : TN;
+    constexpr size_t lds = WK * ((size_t)kUnitStages * TM * kStageRowBytes + (TN / 16) * TL_CODE_UNIT_BYTES);
     static_assert(lds <= 160 * 1024, "the stages fit a compute unit's LDS");
-    auto kernel = tl_matrix_rows<PARTS, WM, WN, FM, FN, STAGES, MODE>;
+    auto kernel = tl_matrix_rows<PARTS, WM, WN, WK, FM, FN, MODE>;
     static std::atomic<bool> raised{false};  // per instantiation; a repeated call is harmless
     if (!raised.load(std::memory_order_relaxed)) {
         if (int rc = raise_lds_limit(kernel, lds)) return rc;
         raised.store(true, std::memory_order_relaxed);
     }
     const int64_t tiles = ceil_div(a.M, TM) * ceil_div(a.N, OUT_TN);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(WM * WN * 64), lds, st, a);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(WM * WN * WK * 64), lds, st, a);
     return TL_OK;
+}
+
+// Which tile, by what the busiest compute unit has to do.  us, fp16, 128 x 256 ("tall") / 64 x 256 ("flat") / 64 x 64 with K shared out:
+//   up to two 64 x 64 tiles a unit: shared K.  64 x 4096 -> 4096 43 / 29 / 15, 512 x 4096 -> 4096 45 / 30 / 25, 1024 x 2048 -> 2048 27 / 20 / 17;
+//     past that it reads the activations too often: 200 x 4096 -> 11008 45 / 32 / 33, 1536 x 2048 -> 2048 28 / 20 / 25.  fp32 (- / flat /
+//     shared) 200 x 2048 -> 2048 - / 42 / 21, 512 x 4096 -> 4096 - / 75 / 59, 768 x 4096 -> 4096 - / 81 / 87.
+//   tall where there are two of them a unit, so that one multiplies while the other waits or stores, and where flat ones would
+//     not spread the rows better: 2048 x 4096 -> 11008 139 / 144, 8192 x 2048 -> 11008 289 / 301, 8192 x 2048 -> 2048 64 / 66, but
+//     1536 x 4096 -> 11008 129 / 117 (516 tall tiles are three for some units, 1032 flat ones five halves).  Not for fp32, whose second
+//     set of sums does not fit.
+template <int PARTS, int MODE>
+int launch_mode(const KernelArgs& a, hipStream_t st)
+{
+    const int64_t units = compute_units(), columns = (int64_t)a.N * (MODE == kTwoWeights ? 2 : 1);
+    if (ceil_div(a.M, 64) * ceil_div(columns, 64) <= 2 * units) return launch_tile<PARTS, 1, 1, 4, 2, 2, MODE>(a, st);
+    if constexpr (PARTS == 1) {
+        const int64_t tall = ceil_div(a.M, 128) * ceil_div(columns, 256), flat = ceil_div(a.M, 64) * ceil_div(columns, 256);
+        if (tall >= 2 * units && ceil_div(flat, units) >= 2 * ceil_div(tall, units)) return launch_tile<PARTS, 1, 4, 1, 4, 2, MODE>(a, st);
+    }
+    return launch_tile<PARTS, 1, 4, 1, 2, 2, MODE>(a, st);
 }
 
 template <int PARTS>
 int launch_parts(const KernelArgs& a, bool two_weights, hipStream_t st)
 {
-    // 128 x 128 tiles, eight waves of 64 x 32: two workgroups share a compute unit in fp16 (114 registers, 80 KB of LDS each), one of
-    // which multiplies while the other waits at a barrier or stores (fp32, with its second set of sums, takes 188 registers:
-    // one workgroup a unit).  Best of the shapes tried at every size (fp16, us at
-    // 1024 x 4096 -> 11008 / 1024 x 4096 -> 4096 / 8192 x 2048 -> 11008): 80 / 34 / 300; four waves of 64 x 64 86 / 40 / 306 or
-    // 128 x 32 86 / 40 / 301; 128 x 256 tiles, eight waves of 64 x 64, one workgroup a unit 105 / 52 / 310; 256 x 192, eight of
-    // 128 x 48, 84 / 72 / 370.
-    if (two_weights) return launch_tile<PARTS, 2, 4, 4, 2, 4, kTwoWeights>(a, st);
-    return a.gated ? launch_tile<PARTS, 2, 4, 4, 2, 4, kPairs>(a, st) : launch_tile<PARTS, 2, 4, 4, 2, 4, kPlain>(a, st);
+    if (two_weights) return launch_mode<PARTS, kTwoWeights>(a, st);
+    return a.gated ? launch_mode<PARTS, kPairs>(a, st) : launch_mode<PARTS, kPlain>(a, st);
 }
 
 // The image of a call's activations (a.image_ld and a.image_plane say how it lies).
@@ -635,8 +720,7 @@ int tl::launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t w
     if (!a.c0.base || (two_weights && !a.c1.base) || ((!workspace || workspace_bytes < need) && walk_reads_directly(a)))
         return x_dtype == TL_F16 ? walk_rows<__half>(a, workspace, workspace_bytes, two_weights, st)
                                  : walk_rows<float>(a, workspace, workspace_bytes, two_weights, st);
-    const uintptr_t y_align = a.y_f16 ? 8 : 16;
-    a.vector_out = a.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(a.Y) % y_align == 0;
+    a.vector_out = a.ldy % (a.y_f16 ? 4 : 2) == 0 && reinterpret_cast<uintptr_t>(a.Y) % 8 == 0;
     // rows that lie as the kernel reads them are read where they are; any other layout, and fp32, goes through the image
     constexpr int64_t kMostLd = 1 << 24;  // (a lane's byte offset inside the 128 rows of a tile has 32 bits)
     const bool direct = x_dtype == TL_F16 && !a.x_kmajor && a.K % 8 == 0 && a.ldx % 8 == 0 && a.ldx <= kMostLd && reinterpret_cast<uintptr_t>(a.X) % 16 == 0;

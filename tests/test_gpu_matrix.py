@@ -15,8 +15,8 @@ def _device(w, cuda):
     return ops.DeviceWeight(PackedWeight.from_dense(w), cuda)
 
 
-# rows: the 128-row tile and the 16-row fragment; K: the 64-row stage, the four stages asked for ahead, the 256-row unit,
-# rows that are not whole 16-byte pieces; N: the 16-column block, a wave's 32 and a tile's 128 columns
+# rows: the 64-row tile and the 32-row fragment; K: the 64-row stage, the stages asked for ahead, the 256-row unit,
+# rows that are not whole 16-byte pieces; N: the 16-column block, a wave's 64 columns
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("M,K,N", [(49, 1, 1), (49, 8, 16), (127, 64, 31), (128, 72, 128), (129, 192, 129), (145, 256, 113), (64, 264, 144),
                                    (300, 320, 257), (640, 520, 300), (257, 1100, 1000), (129, 1280, 700)])
@@ -38,6 +38,31 @@ def test_many_rows_at_the_edges(cuda, oracle, M, K, N, dtype):
         x = activations(M, K, M + 1, dtype)
         y = ops.spmm(_device(one, cuda), x.to(cuda)).cpu().numpy()
         assert np.array_equal(y, x.numpy()[:, rows] * one[rows, np.arange(N)].astype(np.float32))
+
+
+# one tile of 64 x 64 with five units and a stage shared out over four waves; tiles of 128 x 256 and of 64 x 256 with rows, columns
+# and stages left over (4093 x 4090 is 512 of the tall ones, as many as two for each compute unit)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M,K,N", [(65, 1344, 66), (200, 2048, 1032), (1030, 330, 2100), (4093, 200, 4090)])
+def test_tiles_of_every_shape(cuda, M, K, N, dtype):
+    from ternaryllm_amd import ops
+    w, w2 = ternary_weight(K, N, 0.6, M), ternary_weight(K, N, 0.7, N)
+    dw, dw2 = _device(w, cuda), _device(w2, cuda)
+    x = activations(M, K, M, dtype, integer=True).to(cuda)
+    wd, wd2 = torch.from_numpy(w).double().to(cuda), torch.from_numpy(w2).double().to(cuda)
+    scale = torch.rand(N, device=cuda).to(dtype)
+    print(f"case M={M} K={K} N={N} {dtype}", flush=True)
+    want = x.double() @ wd
+    assert torch.equal(ops.spmm(dw, x, out_dtype=torch.float32).double(), want)           # whole numbers
+    ragged = torch.full((M, N + 3), 7.0, dtype=torch.float32, device=cuda)
+    ops.spmm(dw, x, out=ragged[:, 1:N + 1], out_dtype=torch.float32)                      # rows that lie on no boundary
+    assert torch.equal(ragged[:, 1:N + 1].double(), want) and bool((ragged[:, 0] == 7).all()) and bool((ragged[:, N + 1:] == 7).all())
+    x = x / 16
+    assert torch.equal(ops.spmm_gated(dw, x, scale), ops.silu_mul(ops.spmm(dw, x, scale), pairs=True))
+    got = ops.mlp_gate_up(dw, dw2, x, scale, scale, out_dtype=torch.float32).double()
+    sd = scale.double()
+    want = torch.nn.functional.silu((x.double() @ wd) * sd) * ((x.double() @ wd2) * sd)
+    assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())              # exact sums; __expf and the division
 
 
 def _repeated(w):
