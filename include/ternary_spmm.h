@@ -486,6 +486,14 @@ int tl_spmm_chain(const tl_layout_header* header, const void* blob_dev,
                   const void* scale, int scale_dtype, const tl_chain* chain,
                   void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The same chain for 2 to 48 fp16 rows of blobs with codes, row by row: X, Y and image_out are row-major (image_ld >= N, no
+ * padding rows), the squares are [blocks][R] with R = 16, 32 or 64 for up to 16, 32 or 48 rows (rows past M are not written
+ * and not read), gated != 0 gives Y the N / 2 values silu(y[2j]) * y[2j + 1].  The product is tl_spmm's for these rows.
+ * TL_ERR_UNSUPPORTED for other types, row counts and blobs without codes. */
+int tl_spmm_chain_rows(const tl_layout_header* header, const void* blob_dev,
+                       const void* X, int x_dtype, int64_t ldx, int64_t M, void* Y, int y_dtype, int64_t ldy, int gated,
+                       const void* scale, int scale_dtype, const tl_chain* chain, void* stream);
+
 /* tl_spmv_fused with the epilogue of tl_spmm_gated: the weight's columns are (gate, up) pairs and Y holds the N / 2
  * values silu(y[2j]) * y[2j + 1].  Same arguments otherwise. */
 int tl_spmv_fused_gated(const tl_layout_header* header, const void* blob_dev, int producer,

@@ -144,23 +144,27 @@ namespace {
 // us, walk / codes, 4096 -> 11008 at 66 % and at 95 % zeros:
 //   one row         fp16 8.0 / 5.9, 5.4 / 6.1;  fp32 8.2 / 11.0, 5.4 / 11.1: never.  One row's gated and fused products are the
 //                   walk's and equal the plain one bit for bit; that costs the fp16 rows of dense weights.
-//   8 rows          fp16 21.0 / 8.0, 14.8 / 8.1;  fp32 25.3 / 12.8, 18.4 / 13.0: always
-//   16 rows         fp16 27.6 / 10.7, 15.6 / 11.0: always, but see below;  fp32 27.3 / 18.1, 14.0 / 18.4: by bytes
-//   48 rows         fp16 71.7 / 25.8, 43.6 / 26.1: always, but see below;  fp32 102 / 46, 76 / 46: always
-//   9 to 48 fp16 rows where the walk has the gated epilogue (an even N, wide -- this one is): never, so that tl_spmm_gated
-//                   stays tl_spmm and the gate bit for bit.  The price is what the two lines above say.
-//   K-major         3 and 4 rows, which the walk does not take from an image, fp16 38 / 15, 31 / 15: always;  8 rows fp16 17.7 / 14.9,
-//                   11.7 / 15.1, fp32 22.4 / 19.4, 14.6 / 19.7: by bytes, which errs where both are slow (32 fp32 rows, 95 %:
-//                   51.0 / 33.7, and the walk is taken)
+//   8 rows          fp16 20.1 / 6.7, 14.3 / 6.7;  fp32 24.3 / 13.5, 17.2 / 13.5: always
+//   16 rows         fp16 25.7 / 7.1, 14.8 / 7.1: always;  fp32 24.7 / 13.7, 13.1 / 13.7 (2048 -> 2048 at 95 % 9.8 / 5.0): by bytes
+//                   at such widths
+//   48 rows         fp16 68.9 / 15.5, 42.4 / 15.5;  fp32 100 / 41, 75 / 41: always
+//   K-major         3 and 4 rows, which the walk does not take from an image, fp16 38 / 15, 31 / 15: always;  8 rows fp16 16.9 / 15.0,
+//                   11.5 / 15.2, fp32 21.3 / 19.0, 14.6 / 19.1: by bytes;  16 fp16 rows 23.1 / 15.6, 11.9 / 15.6: where the walk would do
+//                   the gate too, from half the bytes on;  32 rows fp16 42 / 22, 23.1 / 21.8, fp32 66 / 35, 49 / 34: always at such
+//                   widths (2048 -> 2048 at 95 %: fp16 5.2 / 6.9, by bytes)
+// The gated product goes where the plain one goes, so that they are equal bit for bit.
 // A knob that names another kernel for few rows keeps the call with it.
 bool few_on_matrix_cores(const KernelArgs& a, const tl_layout_header* h, int64_t M, bool chained)
 {
-    if (M > kSmallMaxM || chained || a.gated || !a.c0.base || (M == 1 && knob(TL_FEW, 0) == 0)) return false;
+    if (M > kSmallMaxM || chained || !a.c0.base || (M == 1 && (a.gated || knob(TL_FEW, 0) == 0))) return false;
     for (Knob other : {TL_SMALL_MT, TL_OCTET, TL_QUAD_WIDE, TL_RES16, TL_SPMV_DIRECT, TL_SPMV_TILES})
         if (knob(other, -1) >= 0) return false;
-    bool use = M > 1 && !walk_has_gated(a, h);
-    const bool fewer_bytes = (uint64_t)a.NB * a.units * a.planes * TL_CODE_UNIT_BYTES < h->stream_bytes;
-    if (use && (a.x_kmajor ? M < 3 || M > 4 : M > 8 && M <= 16 && !a.x_f16)) use = fewer_bytes;
+    if (a.gated && !walk_has_gated(a, h)) return false;   // (refused there, as it is not the walk's)
+    bool use = M > 1;
+    const uint64_t code_bytes = (uint64_t)a.NB * a.units * a.planes * TL_CODE_UNIT_BYTES;
+    const bool wide = a.NB > 2 * compute_units();
+    if (use && (a.x_kmajor ? (M < 3 || M > 4) && !(wide && M > 16) : M > 8 && M <= 16 && !a.x_f16 && wide))
+        use = code_bytes < h->stream_bytes * (a.x_kmajor && walk_has_gated(a, h) ? 2 : 1);
     return knob(TL_FEW, use ? 1 : 0) != 0;
 }
 
@@ -236,6 +240,46 @@ extern "C" int tl_spmm_chain(const tl_layout_header* header, const void* blob_de
 {
     if (!chain) return fail(TL_ERR_ARG, "chain is null");
     return spmm_call(header, blob_dev, X, x_dtype, x_layout, ldx, M, Y, y_dtype, ldy, y_layout, scale, scale_dtype, workspace, workspace_bytes, stream, chain);
+}
+
+extern "C" int tl_spmm_chain_rows(const tl_layout_header* header, const void* blob_dev,
+                                  const void* X, int x_dtype, int64_t ldx, int64_t M, void* Y, int y_dtype, int64_t ldy, int gated,
+                                  const void* scale, int scale_dtype, const tl_chain* chain, void* stream)
+{
+    if (int rc = check_header(header)) return rc;
+    if (!chain) return fail(TL_ERR_ARG, "chain is null");
+    const int64_t N = header->columns;
+    if (int rc = check_io(blob_dev, X, Y, x_dtype, TL_X_ROW_MAJOR, ldx, M, y_dtype, gated ? N : ldy, scale, scale_dtype, header)) return rc;
+    if (gated && N % 2) return fail(TL_ERR_SHAPE, "N=%lld: gate and up columns come in pairs", (long long)N);
+    if (gated && ldy < N / 2) return fail(TL_ERR_SHAPE, "ldy=%lld smaller than %lld", (long long)ldy, (long long)(N / 2));
+    if (M < 2 || M > kSmallMaxM || x_dtype != TL_F16 || y_dtype != TL_F16 || !header->off_codes)
+        return fail(TL_ERR_UNSUPPORTED, "products chained row by row are for 2 to %d fp16 rows and blobs with codes", kSmallMaxM);
+    const bool out = chain->next_norm_weight || chain->image_out || chain->squares_out;
+    if (out && !(chain->next_norm_weight && chain->image_out && chain->squares_out))
+        return fail(TL_ERR_ARG, "next_norm_weight, image_out and squares_out come together");
+    if ((out || chain->residual) && gated) return fail(TL_ERR_ARG, "a gated product has no residual or image epilogue");
+    if (chain->residual && chain->residual_ld < N) return fail(TL_ERR_SHAPE, "residual_ld=%lld smaller than N", (long long)chain->residual_ld);
+    if (out && chain->image_ld < N) return fail(TL_ERR_SHAPE, "image_ld=%lld smaller than N", (long long)chain->image_ld);
+    if (chain->squares_in && chain->squares_blocks <= 0) return fail(TL_ERR_ARG, "squares_blocks must be positive");
+    for (const void* p : {chain->residual, chain->next_norm_weight, static_cast<const void*>(chain->image_out)})
+        if (reinterpret_cast<uintptr_t>(p) % 2) return fail(TL_ERR_ALIGN, "residual, next_norm_weight and image_out must be aligned to y_dtype");
+    for (const void* p : {static_cast<const void*>(chain->squares_out), static_cast<const void*>(chain->squares_in)})
+        if (reinterpret_cast<uintptr_t>(p) % 16) return fail(TL_ERR_ALIGN, "squares_out and squares_in must be 16-byte aligned");
+    KernelArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.w0 = weight_ptrs(header, blob_dev, scale);
+    a.X = X; a.Y = Y;
+    a.ldx = ldx; a.ldy = ldy;
+    a.M = (int)M; a.N = (int)N; a.K = (int)header->inners; a.T = (int)header->n_tiles; a.tile_rows = (int)header->tile_rows;
+    a.NB = (int)header->n_blocks; a.c0 = weight_codes(header, blob_dev); a.units = (int)header->code_units; a.planes = a.c0.planes;
+    a.x_f16 = a.y_f16 = 1; a.scale_f16 = scale_dtype == TL_F16;
+    a.one = 1.0f;
+    a.gated = gated != 0;
+    a.chain_res = chain->residual; a.chain_ldres = chain->residual_ld;
+    a.chain_w = chain->next_norm_weight; a.chain_image = chain->image_out; a.chain_ild = chain->image_ld; a.chain_sq_out = chain->squares_out;
+    a.chain_sq_in = chain->squares_in; a.chain_sq_blocks = chain->squares_blocks; a.eps = chain->eps;
+    if (int rc = launch_matrix_few(a, x_dtype, false, static_cast<hipStream_t>(stream))) return rc;
+    return finish_launch();
 }
 
 extern "C" int tl_spmm_gated(const tl_layout_header* header, const void* blob_dev,

@@ -34,6 +34,16 @@ __device__ __forceinline__ f32x4 matrix_step(u32x4 w, u32x4 x, f32x4 acc)
     else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, w), __builtin_bit_cast(half8, x), acc, 0, 0, 0);
 }
 
+// 16 bytes per lane from `base` + offset into LDS at `lds` + 16 * lane.  (As assembly, because the compiler would wait for
+// all such loads before any read of LDS; here they are counted by hand.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // (m0 is a register that the compiler reserves; named all the same, as this writes it)
+__device__ __forceinline__ void load_to_lds(uint32_t lds, const void* base, uint32_t offset)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(offset), "s"(base) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
 // An fp32 value in three bf16 parts: v = a + (b + c) / kLowScale, each part the next 8 of v's 24 significant bits, by
 // truncation.  The two low parts are scaled so that they stay in bf16's range (down to 2^-133, which the matrix
 // instruction keeps) for every v down to fp32's smallest, 2^-149: without that a v below 2^-110 lost bits (against fp64 4.4e-6

@@ -25,16 +25,6 @@ constexpr int kRowGroup = 4;
 constexpr int kUnitStages = TL_CODE_UNIT_ROWS / kStageRows;
 __device__ __align__(16) const unsigned char kNoCodes[TL_CODE_UNIT_BYTES] = {};   // a unit of zero weights
 
-// 16 bytes per lane from `base` + offset into LDS at `lds` + 16 * lane.  (As assembly, because the compiler would wait for
-// all such loads before any read of LDS; here they are counted by hand.)
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"  // (m0 is a register that the compiler reserves; named all the same, as this writes it)
-__device__ __forceinline__ void load_to_lds(uint32_t lds, const void* base, uint32_t offset)
-{
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(offset), "s"(base) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
 // acc[i] += sum over k of w[row 8 * (i / 4) + 4 * (lane / 32) + i % 4][k] * x[column lane % 32][k], 16 values of k, eight to a lane
 template <bool BF16>
 __device__ __forceinline__ f32x16 matrix_step32(u32x4 w, u32x4 x, f32x16 acc)

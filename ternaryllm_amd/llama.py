@@ -135,7 +135,7 @@ class TernaryLlamaDecoder(nn.Module):
         # folds their pieces.  That pays once a head's rows are many: up to about a thousand rows one workgroup per
         # head is as quick.
         self.split_attention = self.max_seq_len > 1024
-        # steps of 9 to 16 fp16 rows: the products do the residual adds and the RMSNorms around them (tl_spmm_chain);
+        # steps of 2 to 48 fp16 rows: the products do the residual adds and the RMSNorms around them (tl_spmm_chain_rows);
         # switched off by the first step whose shapes have no such kernel
         self.chain_decode = dtype == torch.float16
         # single-row steps: the o and down projections prepare the row for the norm behind them (spmv_add with
@@ -269,8 +269,6 @@ class TernaryLlamaDecoder(nn.Module):
         x = self.embed_tokens[token]
         B = x.shape[0]
         eps = c.rms_norm_eps
-        # 5 to 48 rows: the products read a K-major image, so whatever feeds one writes it in that layout
-        # (its transpose as a view) and no re-layout pass runs in front of the products
         if B == 1 and self.fused_decode:
             while self.row_chain:
                 try:
@@ -283,14 +281,16 @@ class TernaryLlamaDecoder(nn.Module):
                     else:
                         self.row_chain = False  # then without the chain
             return self._decode_step_fused(x, pos)
-        km = 5 <= B <= 48 and c.hidden_size != B and c.intermediate_size != B
-        if km and 9 <= B <= 16 and self.chain_decode:
+        if 2 <= B <= 48 and self.chain_decode:
             try:
                 return self._decode_step_chain(x, pos)
             except RuntimeError as e:
                 if "TL_ERR_UNSUPPORTED" not in str(e) or torch.cuda.is_current_stream_capturing():
                     raise
                 self.chain_decode = False
+        # 5 to 48 rows: the products that walk the index stream read a K-major image, so whatever feeds one writes it in
+        # that layout (its transpose as a view) and no re-layout pass runs in front of the products
+        km = 5 <= B <= 48 and c.hidden_size != B and c.intermediate_size != B
         _, h = ops.add_rmsnorm(x, None, self.layers[0].input_layernorm.weight, eps, kmajor=km)
         for li, layer in enumerate(self.layers):
             qkv = layer.qkv_proj(h)
@@ -305,28 +305,26 @@ class TernaryLlamaDecoder(nn.Module):
         return self.lm_head(h)
 
     def _decode_step_chain(self, x, pos):
-        """9 to 16 rows, five launches per layer, none of them elementwise: the o and down projections add the residual
+        """2 to 48 rows, five launches per layer, none of them elementwise: the o and down projections add the residual
         rows and leave the next norm's image (rows * norm weight) and sums of squares; q|k|v, gate|up (SiLU gate in
         its epilogue) and the head apply the normalisation factor to their sums.  Only the very first norm has a
-        kernel of its own."""
+        kernel of its own.  All products are tl_matrix_few's: a step of 16 rows (two layers of 2048 / 5504, 512 cached) took
+        187 us while they walked the index stream."""
         eps = self.config.rms_norm_eps
-        K_MAJOR = _lib.TL_X_K_MAJOR
-        _, h = ops.add_rmsnorm(x, None, self.layers[0].input_layernorm.weight, eps, kmajor=True)
+        _, h = ops.add_rmsnorm(x, None, self.layers[0].input_layernorm.weight, eps)
         squares = None
+
+        def product(linear, rows, **steps):
+            return ops.spmm_chain_rows(linear.device_weight(), rows, linear.w_scale, eps=eps, **steps)
+
         for li, layer in enumerate(self.layers):
-            if squares is None:
-                qkv = layer.qkv_proj(h)
-            else:
-                qkv = ops.spmm_chain(layer.qkv_proj.device_weight(), h, layer.qkv_proj.w_scale, K_MAJOR, squares_in=squares, eps=eps)
-            a = self._attend(qkv, self._cache[li, 0], self._cache[li, 1], pos, True)
-            x, h, squares = ops.spmm_chain(layer.o_proj.device_weight(), a, layer.o_proj.w_scale, K_MAJOR, residual=x,
-                                           next_norm_weight=layer.post_attention_layernorm.weight)
-            gated = ops.spmm_chain(layer.gate_up_proj.device_weight(), h, layer.gate_up_proj.w_scale, K_MAJOR, squares_in=squares, eps=eps,
-                                   gated=True, kmajor=True)
+            qkv = product(layer.qkv_proj, h, squares_in=squares)
+            a = self._attend(qkv, self._cache[li, 0], self._cache[li, 1], pos, False)
+            x, h, squares = product(layer.o_proj, a.view(x.shape), residual=x, next_norm_weight=layer.post_attention_layernorm.weight)
+            gated = product(layer.gate_up_proj, h, squares_in=squares, gated=True)
             nxt = self.layers[li + 1].input_layernorm.weight if li + 1 < len(self.layers) else self.norm.weight
-            x, h, squares = ops.spmm_chain(layer.down_proj.device_weight(), gated, layer.down_proj.w_scale, K_MAJOR, residual=x,
-                                           next_norm_weight=nxt)
-        return ops.spmm_chain(self.lm_head.device_weight(), h, self.lm_head.w_scale, K_MAJOR, squares_in=squares, eps=eps)
+            x, h, squares = product(layer.down_proj, gated, residual=x, next_norm_weight=nxt)
+        return product(self.lm_head, h, squares_in=squares)
 
     def _decode_step_fused(self, x, pos):
         """One row, five launches per layer instead of nine, none of them an elementwise kernel: q|k|v and gate|up

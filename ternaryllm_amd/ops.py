@@ -151,7 +151,7 @@ def spmm_kmajor_batch(weight, x3, scale=None):
 def spmm_gated(weight, x, scale=None, x_layout=_lib.TL_X_ROW_MAJOR, kmajor=False):
     """h[M, N / 2] with h[:, j] = silu(y[:, 2j]) * y[:, 2j + 1], y = (x @ W) * scale, for a gate | up weight whose
     columns are (gate, up) pairs.  One launch (tl_spmm_gated) where the shape's kernel has the epilogue -- one
-    aligned row, 9 to 16 fp16 rows and a wide N, or more than 48 rows -- else the product followed by
+    aligned row, 9 to 48 fp16 rows and a wide N, or more than 48 rows -- else the product followed by
     silu_mul(pairs=True); the result is the same bit for bit.  With kmajor the transpose [N / 2, M] is returned, a
     view of a K-major image."""
     if x.device != weight.device:
@@ -235,6 +235,43 @@ def spmm_chain(weight, x, scale=None, x_layout=_lib.TL_X_ROW_MAJOR, residual=Non
     if kmajor:
         y = y[:, :M]
     return (y, image[:, :M], squares) if next_norm_weight is not None else y
+
+
+def spmm_chain_rows(weight, x, scale=None, residual=None, next_norm_weight=None, squares_in=None, eps=0.0, gated=False):
+    """spmm_chain for 2 to 48 fp16 rows of a weight with codes, all row-major (tl_spmm_chain_rows): the image is an [M, N] tensor,
+    the squares are [ceil(N / 16), R] float32 with R = 16, 32 or 64 for up to 16, 32 or 48 rows.  gated: columns are (gate, up)
+    pairs, the result is [M, N / 2].  Raises RuntimeError (TL_ERR_UNSUPPORTED) for other rows, types and weights."""
+    if x.device != weight.device:
+        raise RuntimeError(f"x is on {x.device}, the weight on {weight.device}")
+    x_code = _code(x.dtype, "x")
+    xg, M, ldx = _x_geometry(x, weight.inners, _lib.TL_X_ROW_MAJOR)
+    N = weight.columns
+    R = 16 if M <= 16 else 32 if M <= 32 else 64
+    y = torch.empty((M, N // 2 if gated else N), dtype=x.dtype, device=x.device)
+    chain = _lib.Chain()
+    if residual is not None:
+        if residual.shape != (M, N) or residual.dtype != x.dtype or residual.stride(1) != 1 or residual.device != x.device:
+            raise ValueError("residual must be an [M, N] tensor of x's dtype with unit column stride")
+        chain.residual, chain.residual_ld = residual.data_ptr(), residual.stride(0)
+    image = squares = None
+    if next_norm_weight is not None:
+        if next_norm_weight.numel() != N or next_norm_weight.dtype != x.dtype or not next_norm_weight.is_contiguous() or next_norm_weight.device != x.device:
+            raise ValueError("next_norm_weight must be a contiguous [N] tensor of x's dtype")
+        image = torch.empty((M, N), dtype=x.dtype, device=x.device)
+        squares = torch.empty(((N + 15) // 16, R), dtype=torch.float32, device=x.device)
+        chain.next_norm_weight, chain.image_out, chain.image_ld, chain.squares_out = next_norm_weight.data_ptr(), image.data_ptr(), N, squares.data_ptr()
+    if squares_in is not None:
+        if squares_in.dtype != torch.float32 or squares_in.dim() != 2 or squares_in.shape[1] != R or not squares_in.is_contiguous() or \
+                squares_in.device != x.device:
+            raise ValueError(f"squares_in must be a contiguous float32 [blocks, {R}] tensor")
+        chain.squares_in, chain.squares_blocks = squares_in.data_ptr(), squares_in.shape[0]
+    chain.eps = float(eps)
+    sc, s_code = _scale_args(scale, N, x.device)
+    with torch.cuda.device(x.device):
+        _lib.check(_lib.lib().tl_spmm_chain_rows(ctypes.byref(weight.header), weight.blob.data_ptr(), xg.data_ptr(), x_code, ldx, M, y.data_ptr(), x_code,
+                                                 y.shape[1], int(gated), sc.data_ptr() if sc is not None else None, s_code, ctypes.byref(chain),
+                                                 _stream_ptr(x.device)))
+    return (y, image, squares) if next_norm_weight is not None else y
 
 
 def mlp_gate_up(gate, up, x, gate_scale=None, up_scale=None, out_dtype=None):

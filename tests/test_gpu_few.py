@@ -64,3 +64,43 @@ def test_gate_and_up_of_few_rows(cuda, M, dtype):
     fine = torch.isfinite(want)
     assert torch.equal(fine, torch.isfinite(got))
     assert float((got[fine] - want[fine]).abs().max()) <= 1e-4 * float(want[fine].abs().max())
+
+
+@pytest.mark.parametrize("M,K,N,N2", [(2, 8, 16, 2), (13, 1000, 272, 96), (16, 520, 270, 8200), (17, 2048, 43, 34), (31, 72, 4128, 40), (48, 1100, 78, 4200), (33, 5504, 2048, 64)])
+def test_chained_rows(cuda, M, K, N, N2):
+    """A product that ends a block (residual rows, the next norm's image and sums of squares) and the products behind the norm,
+    plain and gated: each step bit for bit what the separate operators give, the norm against float64."""
+    from tests.util import max_rel_err
+    from ternaryllm_amd import ops
+    from ternaryllm_amd.packing import PackedWeight
+    w1, w2 = ternary_weight(K, N, 0.7, 1), ternary_weight(N, N2, 0.7, 2)
+    d1, d2 = (ops.DeviceWeight(PackedWeight.from_dense(w), cuda) for w in (w1, w2))
+    g = torch.Generator().manual_seed(M)
+    x, res = torch.randn((M, K), generator=g).half().to(cuda), torch.randn((M, N), generator=g).half().to(cuda)
+    nw = (1 + 0.1 * torch.randn(N, generator=g)).half().to(cuda)
+    sc1, sc2 = (0.05 + 0.01 * torch.rand(N, generator=g)).half().to(cuda), (0.5 + torch.rand(N2, generator=g)).half().to(cuda)
+    print(f"case M={M} K={K} N={N} N2={N2}", flush=True)
+    y, image, squares = ops.spmm_chain_rows(d1, x, sc1, residual=res, next_norm_weight=nw)
+    assert torch.equal(y, ops.spmm(d1, x, sc1) + res)
+    assert torch.equal(image, (y.float() * nw.float()).half())
+    blocks = -(-N // 16)
+    padded = torch.zeros((M, blocks * 16), dtype=torch.float64, device=cuda)
+    padded[:, :N] = y.double().pow(2)
+    # (16 squares and 15 additions, each rounded to 2^-24)
+    assert torch.allclose(squares[:, :M].double(), padded.reshape(M, blocks, 16).sum(-1).t(), rtol=31 * 2.0 ** -24, atol=0)
+    out = ops.spmm_chain_rows(d2, image, sc2, squares_in=squares, eps=1e-5)
+    h64 = y.double() * torch.rsqrt(y.double().pow(2).mean(-1, keepdim=True) + 1e-5) * nw.double()
+    ref = (h64.cpu().numpy() @ w2.astype("float64")) * sc2.double().cpu().numpy()[None, :]
+    assert max_rel_err(out.double().cpu().numpy(), ref, h64.cpu().numpy(), w2) <= 4e-3
+    assert torch.equal(ops.spmm_chain_rows(d2, image, sc2, squares_in=squares, eps=1e-5, gated=True), ops.silu_mul(out, pairs=True))
+    assert torch.equal(ops.spmm_chain_rows(d2, image, sc2), ops.spmm(d2, image, sc2))
+    # the gated product is the plain one and the gate, rows and a K-major result with its padding rows
+    plain = ops.silu_mul(ops.spmm(d2, image, sc2), pairs=True)
+    assert torch.equal(ops.spmm_gated(d2, image, sc2), plain)
+    if 9 <= M <= 16:
+        turned = ops.spmm_gated(d2, image, sc2, kmajor=True)
+        assert torch.equal(turned.t(), plain) and not turned.as_strided((N2 // 2, 16), (16, 1))[:, M:].any()
+    x[M - 1, 7] = float("inf")          # a column that does not name the row is not touched
+    assert torch.equal(ops.spmm_chain_rows(d1, x, sc1, residual=res).isfinite(), (ops.spmm(d1, x, sc1) + res).isfinite())
+    with pytest.raises(RuntimeError, match="UNSUPPORTED"):
+        ops.spmm_chain_rows(d1, x[:1], sc1, residual=res[:1])
