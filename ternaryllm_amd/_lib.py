@@ -131,6 +131,26 @@ def lib():
 
 def check(rc):
     """Turns a negative status into ValueError (caller mistakes) or RuntimeError (launch failures)."""
+_binding = None
+
+
+def binding(workspaces):
+    """The loaded torch binding (csrc/tl_torch.cpp) over lib(); raises RuntimeError when it has not been built.  `workspaces`: the
+    scratch buffers that it may use, {(device index, stream): uint8 tensor}."""
+    global _binding
+    if _binding is None:
+        try:
+            from . import _tl_torch
+        except ImportError as e:
+            raise RuntimeError("ternaryllm_amd/_tl_torch.so is missing or does not load: build it with `python -m ternaryllm_amd.build`. "
+                               "There is no fallback path.") from e
+        address = [ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value
+                   for name in ("tl_spmm", "tl_spmm_workspace", "tl_mlp_gate_up", "tl_mlp_gate_up_few")]
+        _tl_torch.init(*address, workspaces)
+        _binding = _tl_torch
+    return _binding
+
+
     if rc == 0:
         return
     msg = lib().tl_last_error().decode("utf-8", "replace")

@@ -217,11 +217,11 @@ class TernaryLinear(nn.Module):
 
     def device_weight(self):
         """The DeviceWeight view of `w_packed` on its current device."""
-        h = self._handle
-        if h is None or h.blob.data_ptr() != self.w_packed.data_ptr():
+        h, blob = self._handle, self.w_packed
+        if h is None or (h.blob is not blob and h.blob.data_ptr() != blob.data_ptr()):
             h = ops.DeviceWeight.__new__(ops.DeviceWeight)
             h.header = self._header
-            h.blob = self.w_packed
+            h.blob = blob
             if h.blob.device.type != "cuda":
                 raise RuntimeError("TernaryLinear runs on a GPU only: call .to('cuda') first")
             self._handle = h
@@ -234,7 +234,11 @@ class TernaryLinear(nn.Module):
             raise AssertionError("Input has dim larger than 3")  # the reference asserts (TernaryLinear.py:161)
         w = self.device_weight()
         K, N = self.in_features, self.out_features
-        if input.shape[-1] == K:
+        rows = input.shape[-1] == K
+        y = ops.product(w, input, self.w_scale, not rows)
+        if y is not None:
+            return y
+        if rows:
             lead = input.shape[:-1]
             y = ops.spmm(w, input.reshape(-1, K), self.w_scale)
             return y.reshape(*lead, N)

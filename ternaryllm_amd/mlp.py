@@ -77,6 +77,11 @@ class LlamaTernaryMLP(nn.Module):
         return self._pairs[:2]
 
     def forward(self, x):
+        if not self.paired and self.hidden_act in ("silu", "swish"):
+            gate, up = self.gate_proj, self.up_proj
+            h = ops.gate_up(gate.device_weight(), up.device_weight(), x, gate.w_scale, up.w_scale)
+            if h is not None:
+                return self.down_proj(h)
         lead = x.shape[:-1]
         x2 = x.reshape(-1, self.hidden_size)
         if self.hidden_act not in ("silu", "swish"):

@@ -112,12 +112,26 @@ def _scale_args(scale, N, device):
     return scale, _code(scale.dtype, "scale")
 
 
+def _short():
+    return _lib._binding or _lib.binding(_workspaces)
+
+
+def product(weight, x, scale=None, kmajor=False):
+    """(x @ W) * scale the short way, for x [.., K] of up to three dimensions or, kmajor, [K, rows] or [1, K, rows]; returns
+    [.., N] in x's type, or None where the call is not a plain one (spmm then takes it or says what is wrong)."""
+    return _short().product(ctypes.addressof(weight.header), weight.blob, x, scale, kmajor)
+
+
 def spmm(weight, x, scale=None, out_dtype=None, x_layout=_lib.TL_X_ROW_MAJOR, out=None):
     """y[M, N] = (x @ W) * scale with fp32 accumulation.
 
     weight: DeviceWeight; x: cuda tensor [M, K] (row-major layout) or [K, M] (K-major layout),
     float32 or float16; scale: optional [N] tensor; returns a new [M, N] tensor of out_dtype
     (default: x.dtype)."""
+    if out is None and out_dtype is None and x.dim() == 2 and x_layout in (_lib.TL_X_ROW_MAJOR, _lib.TL_X_K_MAJOR):
+        y = product(weight, x, scale, x_layout == _lib.TL_X_K_MAJOR)
+        if y is not None:
+            return y
     if x.device != weight.device:
         raise RuntimeError(f"x is on {x.device}, the weight on {weight.device}")
     x_code = _code(x.dtype, "x")
@@ -274,12 +288,21 @@ def spmm_chain_rows(weight, x, scale=None, residual=None, next_norm_weight=None,
     return (y, image, squares) if next_norm_weight is not None else y
 
 
+def gate_up(gate, up, x, gate_scale=None, up_scale=None):
+    """mlp_gate_up the short way, for x [.., K] of up to three dimensions; None where the call is not a plain one or has no kernel."""
+    return _short().gate_up(ctypes.addressof(gate.header), gate.blob, ctypes.addressof(up.header), up.blob, x, gate_scale, up_scale)
+
+
 def mlp_gate_up(gate, up, x, gate_scale=None, up_scale=None, out_dtype=None):
     """h[M, N] = silu((x @ Wg) * sg) * ((x @ Wu) * su) in one pass over x, or two products where no kernel does it: one
     row (its own kernel is the faster one), weights of different tile heights, up to 48 rows of a weight without codes or
     whose two scales are not of one kind."""
     if gate.columns != up.columns or gate.inners != up.inners:
         raise ValueError("gate and up weights must have the same shape")
+    if out_dtype is None and x.dim() == 2:
+        h = gate_up(gate, up, x, gate_scale, up_scale)
+        if h is not None:
+            return h
     x_code = _code(x.dtype, "x")
     x, M, ldx = _x_geometry(x, gate.inners, _lib.TL_X_ROW_MAJOR)
     N = gate.columns

@@ -16,6 +16,8 @@ from . import _lib, ops, packing
 from .packing import convert_to_ter_csc, convert_to_ter_tiled_csc, convert_to_ter_tiled_mcsc  # noqa: F401
 
 _ATTR = "_tl_prepared"
+_LAYOUTS = {None: None, "row_major": _lib.TL_X_ROW_MAJOR, "k_major": _lib.TL_X_K_MAJOR,
+            _lib.TL_X_ROW_MAJOR: _lib.TL_X_ROW_MAJOR, _lib.TL_X_K_MAJOR: _lib.TL_X_K_MAJOR}
 
 
 def _dispatch_tile_k(inners):
@@ -91,13 +93,16 @@ def ter_spmm(X, w_tiled_merged_row_indice, w_tiled_merged_col_offset, w_col_tile
     weight = _prepared(w_tiled_merged_row_indice, w_tiled_merged_col_offset, columns, inners, uniformed)
     if X.numel() != batch_size * rows * inners:
         raise ValueError("X does not hold batch_size * rows * inners elements")
-    x3 = X.reshape(batch_size, *X.shape[-2:]) if X.dim() >= 2 else X.reshape(batch_size, rows, inners)
-    layouts = {None: None, "row_major": _lib.TL_X_ROW_MAJOR, "k_major": _lib.TL_X_K_MAJOR,
-               _lib.TL_X_ROW_MAJOR: _lib.TL_X_ROW_MAJOR, _lib.TL_X_K_MAJOR: _lib.TL_X_K_MAJOR}
-    if x_layout not in layouts:
+    x3 = X if X.dim() == 3 and X.shape[0] == batch_size else X.reshape(batch_size, *X.shape[-2:]) if X.dim() >= 2 else X.reshape(batch_size, rows, inners)
+    if x_layout not in _LAYOUTS:
         raise ValueError(f"x_layout={x_layout!r}: expected None, 'row_major' (0) or 'k_major' (1)")
-    asked = layouts[x_layout]
-    if asked != _lib.TL_X_K_MAJOR and x3.shape[-1] == inners and x3.shape[-2] == rows:
+    asked = _LAYOUTS[x_layout]
+    row_major = asked != _lib.TL_X_K_MAJOR and x3.shape[-1] == inners and x3.shape[-2] == rows
+    if row_major or (asked != _lib.TL_X_ROW_MAJOR and x3.shape[-2] == inners and x3.shape[-1] == rows):
+        y = ops.product(weight, x3, None, not row_major)
+        if y is not None:
+            return y
+    if row_major:
         return ops.spmm(weight, x3.reshape(batch_size * rows, inners)).reshape(batch_size, rows, columns)
     if asked != _lib.TL_X_ROW_MAJOR and x3.shape[-2] == inners and x3.shape[-1] == rows:
         return ops.spmm_kmajor_batch(weight, x3)
