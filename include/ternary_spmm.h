@@ -486,13 +486,17 @@ int tl_spmm_chain(const tl_layout_header* header, const void* blob_dev,
                   const void* scale, int scale_dtype, const tl_chain* chain,
                   void* workspace, int64_t workspace_bytes, void* stream);
 
-/* The same chain for 2 to 48 fp16 rows of blobs with codes, row by row: X, Y and image_out are row-major (image_ld >= N, no
- * padding rows), the squares are [blocks][R] with R = 16, 32 or 64 for up to 16, 32 or 48 rows (rows past M are not written
- * and not read), gated != 0 gives Y the N / 2 values silu(y[2j]) * y[2j + 1].  The product is tl_spmm's for these rows.
+/* The same chain for 2 and more fp16 rows of blobs with codes, row by row: X, Y and image_out are row-major (image_ld >= N, no
+ * padding rows).  Up to 48 rows the squares are [blocks][R] with R = 16, 32 or 64 for up to 16, 32 or 48 rows (rows past M are not
+ * written and not read).  More rows (X aligned to 16 bytes, K and ldx multiples of 8) leave squares_out [M][ceil(N / 32)], from
+ * which tl_row_factors makes the M factors that squares_in points to then.  gated != 0 gives Y the N / 2 values silu(y[2j]) * y[2j + 1].  The product is tl_spmm's for these rows.
  * TL_ERR_UNSUPPORTED for other types, row counts and blobs without codes. */
 int tl_spmm_chain_rows(const tl_layout_header* header, const void* blob_dev,
                        const void* X, int x_dtype, int64_t ldx, int64_t M, void* Y, int y_dtype, int64_t ldy, int gated,
                        const void* scale, int scale_dtype, const tl_chain* chain, void* stream);
+
+/* factors[r] = rsqrt((sum of squares[r][0 .. blocks)) / width + eps) for `rows` rows. */
+int tl_row_factors(const float* squares, int64_t rows, int blocks, int width, float eps, float* factors, void* stream);
 
 /* tl_spmv_fused with the epilogue of tl_spmm_gated: the weight's columns are (gate, up) pairs and Y holds the N / 2
  * values silu(y[2j]) * y[2j + 1].  Same arguments otherwise. */
@@ -524,6 +528,14 @@ int tl_spmv_attn_combine_add_norm(const tl_layout_header* header, const void* bl
                                   int splits, int head_dim, int x_dtype, const void* residual, void* Y, int y_dtype,
                                   const void* scale, int scale_dtype, const void* next_norm_weight,
                                   void* image_out, float* squares_out, void* stream);
+
+/* The start of a decode step in one launch: x[r] = table[token[r]] (negative tokens count from the end; a row of NaN where there
+ * is no such row), image[r] = x[r] * norm_weight and squares[b][r] = the sum of x[r]^2 over its values 16 b .. 16 b + 15 -- what a
+ * chained product leaves for the product behind a norm.  fp16, width a multiple of 16, all rows contiguous and 16-byte
+ * aligned; squares: float32 [width / 16][squares_rows], squares_rows >= rows, or, squares_rows == 0, [rows][ceil(width / 32)] by runs
+ * of 32 values, as more than 48 chained rows leave them. */
+int tl_embed_rows(const void* table, int dtype, int64_t vocab, int width, const int64_t* token, int64_t rows, const void* norm_weight,
+                  void* x, void* image, float* squares, int squares_rows, void* stream);
 
 /* The end of a greedy decode step in one launch: token[b] = argmax of logits[b][0 .. vocab) (the first of equal
  * values; a NaN counts as larger than any number -- torch.argmax's rule), then, when pos_dev is not NULL,

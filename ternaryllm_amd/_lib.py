@@ -96,6 +96,8 @@ SIGNATURES = {
     "tl_prefill_attention": (_INT, [_VP, _VP, _VP, _VP, _VP, _INT, _I64, _INT, _INT, _INT, _I64, _I64, _I64P, _VP, _VP]),
     "tl_decode_attention": (_INT, [_VP, _VP, _VP, _INT, _I64, _INT, _INT, _I64, _VP, _VP, _I64, _VP]),
     "tl_decode_attention_split": (_INT, [_VP, _VP, _VP, _INT, _I64, _INT, _INT, _I64, _VP, _VP, _I64, _INT, _VP, _I64, _VP]),
+    "tl_embed_rows": (_INT, [_VP, _INT, _I64, _INT, _VP, _I64, _VP, _VP, _VP, _VP, _INT, _VP]),
+    "tl_row_factors": (_INT, [_VP, _I64, _INT, _INT, ctypes.c_float, _VP, _VP]),
     "tl_greedy_advance": (_INT, [_VP, _INT, _I64, _INT, _VP, _VP, _I64, _VP, _VP]),
     "tl_decode_attention_fold": (_INT, [_VP, _VP, _VP, _VP, _VP, _VP, _INT, _I64, _INT, _INT, _I64, _VP, _VP, _I64, _INT, _VP, _I64, _VP, _VP]),
     "tl_decode_attention_rope": (_INT, [_VP, _VP, _VP, _VP, _VP, _INT, _I64, _INT, _INT, _I64, _VP, _VP, _I64, _INT, _VP, _I64, _VP]),
@@ -129,8 +131,6 @@ def lib():
     return _lib
 
 
-def check(rc):
-    """Turns a negative status into ValueError (caller mistakes) or RuntimeError (launch failures)."""
 _binding = None
 
 
@@ -151,6 +151,8 @@ def binding(workspaces):
     return _binding
 
 
+def check(rc):
+    """Turns a negative status into ValueError (caller mistakes) or RuntimeError (launch failures)."""
     if rc == 0:
         return
     msg = lib().tl_last_error().decode("utf-8", "replace")

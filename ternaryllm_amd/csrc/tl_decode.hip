@@ -858,6 +858,86 @@ extern "C" int tl_decode_attention_fold(const void* q, const void* qkv, const vo
                      pos_dev, out, out_kmajor_ld, splits, workspace, workspace_bytes, stream, arrivals);
 }
 
+// The start of a decode step: a token's row of the embedding table and what the first norm's product wants of it (the row times
+// the norm's weight, and its sums of squares).  A few KB a row: bound by the launch, 1.6 us of it in a graph, and by three trips to
+// memory in a row (token, row, stores); a lane takes 16 bytes, two lanes a block of 16.  One launch in the place of a gather (3.0 us
+// in a step of 16 rows) and a norm (3.6).
+namespace {
+__global__ __launch_bounds__(256) void tl_embed_rows_k(const __half* __restrict__ table, long long vocab, int width, const long long* __restrict__ token,
+                                                       const __half* __restrict__ norm_w, __half* __restrict__ x, __half* __restrict__ image,
+                                                       float* __restrict__ squares, int squares_rows)
+{
+    const int row = blockIdx.y, k = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 8;
+    if (k >= width) return;   // (whole pairs of lanes)
+    long long t = token[row];
+    if (t < 0) t += vocab;
+    __align__(16) __half v[8], w[8], o[8];
+    *reinterpret_cast<uint4*>(w) = *reinterpret_cast<const uint4*>(norm_w + k);
+    if (t >= 0 && t < vocab) *reinterpret_cast<uint4*>(v) = *reinterpret_cast<const uint4*>(table + t * width + k);
+    else
+        for (int i = 0; i < 8; ++i) v[i] = __float2half(__builtin_nanf(""));   // (no such row: nothing is read, and the result says so)
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float f = __half2float(v[i]);
+        sum = fmaf(f, f, sum);
+        o[i] = __float2half(f * __half2float(w[i]));
+    }
+    *reinterpret_cast<uint4*>(x + (long long)row * width + k) = *reinterpret_cast<const uint4*>(v);
+    *reinterpret_cast<uint4*>(image + (long long)row * width + k) = *reinterpret_cast<const uint4*>(o);
+    sum += lane_permuted<0xB1>(sum);   // (the neighbouring lane's)
+    if (squares_rows > 0) {
+        if (threadIdx.x % 2 == 0) squares[(long long)(k / 16) * squares_rows + row] = sum;
+        return;
+    }
+    const float next = lane_permuted<0x4E>(sum);   // (the neighbouring pair's; past the row's end it counts nothing)
+    if (threadIdx.x % 4 == 0) squares[(long long)row * ((width + 31) / 32) + k / 32] = k + 16 < width ? sum + next : sum;
+}
+}  // namespace
+
+extern "C" int tl_embed_rows(const void* table, int dtype, int64_t vocab, int width, const int64_t* token, int64_t rows, const void* norm_weight,
+                             void* x, void* image, float* squares, int squares_rows, void* stream)
+{
+    if (dtype != TL_F16) return fail(TL_ERR_UNSUPPORTED, "embedding rows are read as fp16");
+    if (!table || !token || !norm_weight || !x || !image || !squares) return fail(TL_ERR_ARG, "device pointer is null");
+    if (rows <= 0 || rows > 65535 || vocab <= 0 || width <= 0 || width % 16 || (squares_rows != 0 && squares_rows < rows))
+        return fail(TL_ERR_SHAPE, "rows=%lld (1 .. 65535, at most squares_rows=%d where that is not 0), width=%d (a multiple of 16), vocab=%lld", (long long)rows, squares_rows, width,
+                    (long long)vocab);
+    for (const void* p : {table, norm_weight, static_cast<const void*>(x), static_cast<const void*>(image)})
+        if (reinterpret_cast<uintptr_t>(p) % 16) return fail(TL_ERR_ALIGN, "table, norm_weight, x and image must be 16-byte aligned");
+    if (reinterpret_cast<uintptr_t>(token) % 8 || reinterpret_cast<uintptr_t>(squares) % 4) return fail(TL_ERR_ALIGN, "token or squares misaligned");
+    hipLaunchKernelGGL(tl_embed_rows_k, dim3((unsigned)ceil_div(width, 2048), (unsigned)rows), dim3(256), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const __half*>(table), (long long)vocab, width, reinterpret_cast<const long long*>(token),
+                       static_cast<const __half*>(norm_weight), static_cast<__half*>(x), static_cast<__half*>(image), squares, squares_rows);
+    return launched();
+}
+
+// The normalisation factors of many rows whose product left sums of squares (64 a row of 2048): 16 lanes a row.  Bound by the launch.
+namespace {
+__global__ __launch_bounds__(256) void tl_row_factors_k(const float* __restrict__ squares, long long rows, int blocks, float inv_width, float eps,
+                                                        float* __restrict__ factors)
+{
+    const long long row = (long long)blockIdx.x * 16 + threadIdx.x / 16;
+    if (row >= rows) return;   // (whole groups of 16 lanes)
+    float sum = 0.f;
+    for (int b = threadIdx.x % 16; b < blocks; b += 16) sum += squares[row * blocks + b];
+    sum += lane_permuted<0x128>(sum);   // from 8, 4, 2 and 1 lanes further on among 16, around
+    sum += lane_permuted<0x124>(sum);
+    sum += lane_permuted<0x122>(sum);
+    sum += lane_permuted<0x121>(sum);
+    if (threadIdx.x % 16 == 0) factors[row] = rsqrtf(sum * inv_width + eps);
+}
+}  // namespace
+
+extern "C" int tl_row_factors(const float* squares, int64_t rows, int blocks, int width, float eps, float* factors, void* stream)
+{
+    if (!squares || !factors) return fail(TL_ERR_ARG, "device pointer is null");
+    if (rows <= 0 || rows > (1ll << 30) || blocks <= 0 || width <= 0) return fail(TL_ERR_SHAPE, "rows, blocks and width must be positive");
+    hipLaunchKernelGGL(tl_row_factors_k, dim3((unsigned)ceil_div(rows, 16)), dim3(256), 0, static_cast<hipStream_t>(stream), squares, (long long)rows, blocks,
+                       1.0f / (float)width, eps, factors);
+    return launched();
+}
+
 extern "C" int tl_greedy_advance(const void* logits, int dtype, int64_t batch, int vocab, int64_t* token, int64_t* pos_dev, int64_t max_pos,
                                  void* mask, void* stream)
 {

@@ -77,6 +77,7 @@ struct KernelArgs {
     float* chain_sq_out;      // [NB][16]
     const float* chain_sq_in; // [chain_sq_blocks][16] sums of squares of the rows X was made from: the product is multiplied by rsqrt(sum / K + eps), row by row
     int chain_sq_blocks;
+    const float* chain_factors; // more than 48 rows: null, or [M], what the product is multiplied by, row by row (chain_sq_out is [M][ceil(N / 32)] there)
     // matrix-core kernels
     Codes c1;                 // the codes of w1
     const void* image;        // the activations they multiply: row-major, 16-byte pieces along K ...
@@ -205,6 +206,8 @@ inline int64_t least_image_bytes(int64_t K, int64_t M, int x_dtype)
     return std::min(M * image_row_bytes(K, x_dtype), M * K * (x_dtype == TL_F16 ? 2 : 4));
 }
 int launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t workspace_bytes, bool two_weights, hipStream_t st);
+// Whether rows of more than 48 are read where they lie, which products with chained steps need.
+bool matrix_reads_rows(const KernelArgs& a, int x_dtype);
 
 // tl_few.hip
 // Up to 48 rows, any layout, blobs with codes; no gated and no chained epilogue.  Two weights: silu(w0 product) * w1 product.

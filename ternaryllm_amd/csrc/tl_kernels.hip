@@ -252,15 +252,16 @@ extern "C" int tl_spmm_chain_rows(const tl_layout_header* header, const void* bl
     if (int rc = check_io(blob_dev, X, Y, x_dtype, TL_X_ROW_MAJOR, ldx, M, y_dtype, gated ? N : ldy, scale, scale_dtype, header)) return rc;
     if (gated && N % 2) return fail(TL_ERR_SHAPE, "N=%lld: gate and up columns come in pairs", (long long)N);
     if (gated && ldy < N / 2) return fail(TL_ERR_SHAPE, "ldy=%lld smaller than %lld", (long long)ldy, (long long)(N / 2));
-    if (M < 2 || M > kSmallMaxM || x_dtype != TL_F16 || y_dtype != TL_F16 || !header->off_codes)
-        return fail(TL_ERR_UNSUPPORTED, "products chained row by row are for 2 to %d fp16 rows and blobs with codes", kSmallMaxM);
+    const bool few = M <= kSmallMaxM;
+    if (M < 2 || x_dtype != TL_F16 || y_dtype != TL_F16 || !header->off_codes)
+        return fail(TL_ERR_UNSUPPORTED, "products chained row by row are for 2 and more fp16 rows and blobs with codes");
     const bool out = chain->next_norm_weight || chain->image_out || chain->squares_out;
     if (out && !(chain->next_norm_weight && chain->image_out && chain->squares_out))
         return fail(TL_ERR_ARG, "next_norm_weight, image_out and squares_out come together");
     if ((out || chain->residual) && gated) return fail(TL_ERR_ARG, "a gated product has no residual or image epilogue");
     if (chain->residual && chain->residual_ld < N) return fail(TL_ERR_SHAPE, "residual_ld=%lld smaller than N", (long long)chain->residual_ld);
     if (out && chain->image_ld < N) return fail(TL_ERR_SHAPE, "image_ld=%lld smaller than N", (long long)chain->image_ld);
-    if (chain->squares_in && chain->squares_blocks <= 0) return fail(TL_ERR_ARG, "squares_blocks must be positive");
+    if (few && chain->squares_in && chain->squares_blocks <= 0) return fail(TL_ERR_ARG, "squares_blocks must be positive");
     for (const void* p : {chain->residual, chain->next_norm_weight, static_cast<const void*>(chain->image_out)})
         if (reinterpret_cast<uintptr_t>(p) % 2) return fail(TL_ERR_ALIGN, "residual, next_norm_weight and image_out must be aligned to y_dtype");
     for (const void* p : {static_cast<const void*>(chain->squares_out), static_cast<const void*>(chain->squares_in)})
@@ -278,7 +279,13 @@ extern "C" int tl_spmm_chain_rows(const tl_layout_header* header, const void* bl
     a.chain_res = chain->residual; a.chain_ldres = chain->residual_ld;
     a.chain_w = chain->next_norm_weight; a.chain_image = chain->image_out; a.chain_ild = chain->image_ld; a.chain_sq_out = chain->squares_out;
     a.chain_sq_in = chain->squares_in; a.chain_sq_blocks = chain->squares_blocks; a.eps = chain->eps;
-    if (int rc = launch_matrix_few(a, x_dtype, false, static_cast<hipStream_t>(stream))) return rc;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (!few) {
+        if (!matrix_reads_rows(a, x_dtype)) return fail(TL_ERR_UNSUPPORTED, "more than %d chained rows are read where they lie: aligned, K and ldx multiples of 8", kSmallMaxM);
+        a.chain_factors = chain->squares_in;
+        a.chain_sq_in = nullptr;
+    }
+    if (int rc = few ? launch_matrix_few(a, x_dtype, false, st) : launch_matrix_rows(a, x_dtype, nullptr, 0, false, st)) return rc;
     return finish_launch();
 }
 

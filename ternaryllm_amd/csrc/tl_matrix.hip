@@ -73,7 +73,7 @@ __device__ __forceinline__ void store_piece(const KernelArgs& a, int m, int n, i
         if (n + i < N) store_out(a.Y, a.y_f16, at + i, v[i]);
 }
 
-enum { kPlain = 0, kPairs = 1, kTwoWeights = 2 };
+enum { kPlain = 0, kPairs = 1, kTwoWeights = 2, kSteps = 3 };   // (kSteps: with what a decoder layer does around a product)
 
 // The product of one output: from the index stream where the matrix cores' sum is not finite.
 __device__ __forceinline__ float exact_output(const KernelArgs& a, const WeightPtrs& w, int m, int n) { return walk_column(w, a.T, a.tile_rows, n, callers_x(a, m)); }
@@ -83,6 +83,48 @@ __device__ __forceinline__ float exact_output(const KernelArgs& a, const WeightP
 // A sum that is not finite is worked out again by the lane that holds it, before anything is stored: the outputs of
 // finite rows keep their bits whatever another row of the tile holds.  (The sums that need it go into a mask that a
 // loop takes bit by bit, so that the walk stands here once and the sums stay in registers.)
+// The last steps of 16 neighbouring outputs of a row (kSteps): residual row, output, the next norm's image; returns the sum of
+// the outputs' squares.  Rounded as separate operators would round.
+__device__ __forceinline__ float put_steps(const KernelArgs& a, int row, int n, float (&v)[16])
+{
+    const bool whole = a.vector_out && n + 16 <= a.N;                // (16-byte pieces of every array: the launcher has looked)
+    auto read16 = [&](const void* p, long long at, float (&to)[16]) {
+        const __half* h = static_cast<const __half*>(p) + at;
+        __align__(16) __half raw[16];
+        if (whole) {
+            reinterpret_cast<u32x4*>(raw)[0] = reinterpret_cast<const u32x4_out*>(h)[0];
+            reinterpret_cast<u32x4*>(raw)[1] = reinterpret_cast<const u32x4_out*>(h)[1];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) raw[i] = n + i < a.N ? h[i] : __half(0.f);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) to[i] = __half2float(raw[i]);
+    };
+    float other[16], sum = 0.f;
+    if (a.chain_res) {
+        read16(a.chain_res, (long long)row * a.chain_ldres + n, other);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = as_output(v[i], 1) + other[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = n + i < a.N ? as_output(v[i], 1) : 0.f;
+    store_piece<16>(a, row, n, a.N, v);
+    if (a.chain_image) {
+        read16(a.chain_w, n, other);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            sum = fmaf(v[i], v[i], sum);
+            v[i] *= other[i];
+        }
+        KernelArgs image = a;
+        image.Y = a.chain_image;
+        image.ldy = a.chain_ild;
+        store_piece<16>(image, row, n, a.N, v);
+    }
+    return sum;
+}
+
 template <int FN, int FM, int MODE>
 __device__ __forceinline__ void put_out(const KernelArgs& a, f32x16 (&acc)[FN][FM], int lane_m0, int lane_n0)
 {
@@ -136,6 +178,19 @@ __device__ __forceinline__ void put_out(const KernelArgs& a, f32x16 (&acc)[FN][F
 #pragma unroll
         for (int m = 0; m < FM; ++m) {
             const int row = lane_m0 + m * 32;
+            if constexpr (MODE == kSteps) {
+                float v[16], sum = 0.f;
+                const float factor = a.chain_factors && row < a.M ? a.chain_factors[row] : 1.0f;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[i] = acc[f][m][i] * s0[i] * factor;
+                if (row < a.M && n < a.N) sum = put_steps(a, row, n, v);
+                if (a.chain_image) {                              // (the other 16 columns of the fragment are the lane's 32 further on)
+                    const auto pair = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+                    sum = __uint_as_float(pair[0]) + __uint_as_float(pair[1]);
+                    if (threadIdx.x % 64 < 32 && row < a.M && n < a.N) a.chain_sq_out[(long long)row * ((a.N + 31) / 32) + n / 32] = sum;
+                }
+                continue;
+            }
             if (row >= a.M || n >= a.N) continue;
             float v[16];
 #pragma unroll
@@ -144,6 +199,10 @@ __device__ __forceinline__ void put_out(const KernelArgs& a, f32x16 (&acc)[FN][F
                 if constexpr (MODE == kTwoWeights) v[i] = silu(v[i]) * (acc[f + FN / 2][m][i] * s1[i]);
             }
             if constexpr (MODE == kPairs) {
+                if (a.chain_factors) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) v[i] *= a.chain_factors[row];
+                }
 #pragma unroll
                 for (int i = 0; i < 8; ++i) v[i] = gate_pair(as_output(v[2 * i], a.y_f16), as_output(v[2 * i + 1], a.y_f16), a.y_f16);
                 store_piece<8>(a, row, n / 2, a.N / 2, v);
@@ -675,6 +734,9 @@ template <int PARTS>
 int launch_parts(const KernelArgs& a, bool two_weights, hipStream_t st)
 {
     if (two_weights) return launch_mode<PARTS, kTwoWeights>(a, st);
+    if constexpr (PARTS == 1) {
+        if (!a.gated && (a.chain_res || a.chain_image || a.chain_factors)) return launch_mode<PARTS, kSteps>(a, st);
+    }
     return a.gated ? launch_mode<PARTS, kPairs>(a, st) : launch_mode<PARTS, kPlain>(a, st);
 }
 
@@ -701,6 +763,13 @@ void make_image(const KernelArgs& a, int x_dtype, unsigned short* image, hipStre
 
 }  // namespace
 
+constexpr int64_t kMostLd = 1 << 24;  // (a lane's byte offset inside the 128 rows of a tile has 32 bits)
+
+bool tl::matrix_reads_rows(const KernelArgs& a, int x_dtype)
+{
+    return x_dtype == TL_F16 && !a.x_kmajor && a.K % 8 == 0 && a.ldx % 8 == 0 && a.ldx <= kMostLd && reinterpret_cast<uintptr_t>(a.X) % 16 == 0;
+}
+
 int tl::launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t workspace_bytes, bool two_weights, hipStream_t st)
 {
     a.x_sm = a.x_kmajor ? 1 : a.ldx;
@@ -711,9 +780,11 @@ int tl::launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t w
         return x_dtype == TL_F16 ? walk_rows<__half>(a, workspace, workspace_bytes, two_weights, st)
                                  : walk_rows<float>(a, workspace, workspace_bytes, two_weights, st);
     a.vector_out = a.ldy % (a.y_f16 ? 4 : 2) == 0 && reinterpret_cast<uintptr_t>(a.Y) % 8 == 0;
+    if (a.chain_image)                                            // (the image is stored, and the residual rows read, in the same pieces)
+        a.vector_out = a.vector_out && a.chain_ild % 4 == 0 && reinterpret_cast<uintptr_t>(a.chain_image) % 8 == 0 && reinterpret_cast<uintptr_t>(a.chain_w) % 8 == 0;
+    if (a.chain_res) a.vector_out = a.vector_out && a.chain_ldres % 4 == 0 && reinterpret_cast<uintptr_t>(a.chain_res) % 8 == 0;
     // rows that lie as the kernel reads them are read where they are; any other layout, and fp32, goes through the image
-    constexpr int64_t kMostLd = 1 << 24;  // (a lane's byte offset inside the 128 rows of a tile has 32 bits)
-    const bool direct = x_dtype == TL_F16 && !a.x_kmajor && a.K % 8 == 0 && a.ldx % 8 == 0 && a.ldx <= kMostLd && reinterpret_cast<uintptr_t>(a.X) % 16 == 0;
+    const bool direct = matrix_reads_rows(a, x_dtype);
     a.image_ld = direct ? a.ldx : round_up(a.K, 8);
     if (a.image_ld > kMostLd)
         return fail(TL_ERR_ARG, "rows of %lld activations are too long for one call", (long long)a.image_ld);

@@ -221,6 +221,14 @@ class TernaryLlamaDecoder(nn.Module):
         return all(type(n) is RMSNorm and not n._forward_hooks and not n._forward_pre_hooks and "forward" not in n.__dict__ and
                    n.weight.dtype == self.dtype and n.weight.is_contiguous() for n in norms)
 
+    def _products_as_built(self):
+        """Whether no hook, replacement or forward of its own stands at a linear layer that a chained step multiplies by itself."""
+        module = torch.nn.modules.module
+        if module._global_forward_hooks or module._global_forward_pre_hooks:
+            return False
+        linears = [m for layer in self.layers for m in (layer.qkv_proj, layer.o_proj, layer.gate_up_proj, layer.down_proj)] + [self.lm_head]
+        return all(type(m) is TernaryLinear and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__ for m in linears)
+
     def _prefill_native(self, tokens):
         """The pass with the library's kernels around the products: residual add + RMSNorm in one, keys rotated into the
         cache and values copied beside them in one, queries rotated inside the attention.  Seven launches a layer."""
@@ -232,6 +240,8 @@ class TernaryLlamaDecoder(nn.Module):
             return ops.add_rmsnorm(x, y, norm.weight, norm.eps)
 
         tables = self.rope_cos[:S], self.rope_sin[:S]
+        if 48 < B * S <= 65535 and H % 16 == 0 and c.intermediate_size % 8 == 0 and tokens.dtype == torch.int64 and self._products_as_built():
+            return self._prefill_chained(tokens.contiguous(), tables)
         x = self.embed_tokens[tokens].view(B * S, H)
         _, h = add_norm(x, None, self.layers[0].input_layernorm)
         for li, layer in enumerate(self.layers):
@@ -245,6 +255,32 @@ class TernaryLlamaDecoder(nn.Module):
                 x, h = add_norm(x, y, self.layers[li + 1].input_layernorm)
         last = [t.view(B, S, H)[:, -1].contiguous() for t in (x, y)]
         return self.lm_head(add_norm(*last, self.norm)[1])
+
+    def _prefill_chained(self, tokens, tables):
+        """The layers of a pass over more than 48 tokens without kernels for the residual add and the norm: the o and down
+        projections add the residual rows and leave the next norm's image and sums of squares, and the products behind
+        the norm multiply by each row's factor.  (16 x 512 tokens of 2048: an add + norm took 35 to 52 us, four of them a pass.)"""
+        c = self.config
+        B, S = tokens.shape
+        H, nh, hd = c.hidden_size, c.num_attention_heads, c.head_dim
+        x, h, squares = ops.embed_rows(self.embed_tokens, tokens, self.layers[0].input_layernorm.weight)
+
+        def product(linear, rows, **steps):
+            return ops.spmm_chain_rows(linear.device_weight(), rows, linear.w_scale, **steps)
+
+        for li, layer in enumerate(self.layers):
+            qkv = product(layer.qkv_proj, h, squares_in=ops.row_factors(squares, H, layer.input_layernorm.eps)).view(B, S, 3, nh, hd)
+            kc, vc = self._cache[li, 0, :, :, :S], self._cache[li, 1, :, :, :S]
+            ops.rope_rows(qkv[:, :, 1], tables, kc, qkv[:, :, 2], vc)
+            a = ops.prefill_attention(qkv[:, :, 0], kc, vc, tables)
+            x, h, squares = product(layer.o_proj, a.view(B * S, H), residual=x, next_norm_weight=layer.post_attention_layernorm.weight)
+            gated = product(layer.gate_up_proj, h, squares_in=ops.row_factors(squares, H, layer.post_attention_layernorm.eps), gated=True)
+            if li + 1 == len(self.layers):
+                x = product(layer.down_proj, gated, residual=x)
+            else:
+                x, h, squares = product(layer.down_proj, gated, residual=x, next_norm_weight=self.layers[li + 1].input_layernorm.weight)
+        last = x.view(B, S, H)[:, -1].contiguous()
+        return self.lm_head(ops.add_rmsnorm(last, None, self.norm.weight, self.norm.eps)[1])
 
     # -- decode ------------------------------------------------------------------------------
     def _decode_step(self, token, pos, mask):
@@ -266,13 +302,18 @@ class TernaryLlamaDecoder(nn.Module):
         """The decode step with rotary embedding, cache update and the attention over the cache as one
         library kernel (activations stay [B, hidden] throughout)."""
         c = self.config
-        x = self.embed_tokens[token]
-        B = x.shape[0]
+        B = token.shape[0]
         eps = c.rms_norm_eps
+        chained = self.fused_decode and self.row_chain if B == 1 else B <= 48 and self.chain_decode and self._products_as_built()
+        if chained and self.dtype == torch.float16 and c.hidden_size % 16 == 0 and len(self.layers) > 0 and token.dtype == torch.int64:
+            # the tokens' rows and what the first norm's product wants of them in one launch
+            x, image, squares = ops.embed_rows(self.embed_tokens, token.contiguous(), self.layers[0].input_layernorm.weight)
+        else:
+            x, image, squares = self.embed_tokens[token], None, None
         if B == 1 and self.fused_decode:
             while self.row_chain:
                 try:
-                    return self._decode_step_fused(x, pos)
+                    return self._decode_step_fused(x, pos, image, squares)
                 except RuntimeError as e:
                     if "TL_ERR_UNSUPPORTED" not in str(e) or torch.cuda.is_current_stream_capturing():
                         raise
@@ -281,9 +322,9 @@ class TernaryLlamaDecoder(nn.Module):
                     else:
                         self.row_chain = False  # then without the chain
             return self._decode_step_fused(x, pos)
-        if 2 <= B <= 48 and self.chain_decode:
+        if B > 1 and chained:
             try:
-                return self._decode_step_chain(x, pos)
+                return self._decode_step_chain(x, pos, image, squares)
             except RuntimeError as e:
                 if "TL_ERR_UNSUPPORTED" not in str(e) or torch.cuda.is_current_stream_capturing():
                     raise
@@ -304,15 +345,15 @@ class TernaryLlamaDecoder(nn.Module):
             x, h = ops.add_rmsnorm(x, y, nxt, eps, kmajor=km)  # the residual add, and the norm the next layer (or the head) starts with
         return self.lm_head(h)
 
-    def _decode_step_chain(self, x, pos):
+    def _decode_step_chain(self, x, pos, h=None, squares=None):
         """2 to 48 rows, five launches per layer, none of them elementwise: the o and down projections add the residual
         rows and leave the next norm's image (rows * norm weight) and sums of squares; q|k|v, gate|up (SiLU gate in
-        its epilogue) and the head apply the normalisation factor to their sums.  Only the very first norm has a
-        kernel of its own.  All products are tl_matrix_few's: a step of 16 rows (two layers of 2048 / 5504, 512 cached) took
+        its epilogue) and the head apply the normalisation factor to their sums.  h and squares: the image of x and
+        its sums of squares as embed_rows left them (the very first norm has a kernel of its own without).  All products are tl_matrix_few's: a step of 16 rows (two layers of 2048 / 5504, 512 cached) took
         187 us while they walked the index stream."""
         eps = self.config.rms_norm_eps
-        _, h = ops.add_rmsnorm(x, None, self.layers[0].input_layernorm.weight, eps)
-        squares = None
+        if h is None:
+            _, h = ops.add_rmsnorm(x, None, self.layers[0].input_layernorm.weight, eps)
 
         def product(linear, rows, **steps):
             return ops.spmm_chain_rows(linear.device_weight(), rows, linear.w_scale, eps=eps, **steps)
@@ -326,7 +367,7 @@ class TernaryLlamaDecoder(nn.Module):
             x, h, squares = product(layer.down_proj, gated, residual=x, next_norm_weight=nxt)
         return product(self.lm_head, h, squares_in=squares)
 
-    def _decode_step_fused(self, x, pos):
+    def _decode_step_fused(self, x, pos, image=None, squares=None):
         """One row, five launches per layer instead of nine, none of them an elementwise kernel: q|k|v and gate|up
         normalise their input themselves (RMSNorm with the factor applied to the sums, tl_spmv_fused "rmsnorm"); the
         gate|up product applies the SiLU gate in its epilogue (columns packed as gate/up pairs); the attention rotates
@@ -342,7 +383,6 @@ class TernaryLlamaDecoder(nn.Module):
         # squares (spmv_add(..., next_norm_weight=)), and the product after the norm is the plain kernel with one
         # factor at the end ("rmsnorm_sums"): it keeps one image of the row in LDS, not two.
         chain = self.row_chain
-        image = squares = None
         for li, layer in enumerate(self.layers):
             if squares is None:
                 qkv = ops.spmv_fused(layer.qkv_proj.device_weight(), "rmsnorm", x, None, layer.input_layernorm.weight, eps, layer.qkv_proj.w_scale)

@@ -252,15 +252,16 @@ def spmm_chain(weight, x, scale=None, x_layout=_lib.TL_X_ROW_MAJOR, residual=Non
 
 
 def spmm_chain_rows(weight, x, scale=None, residual=None, next_norm_weight=None, squares_in=None, eps=0.0, gated=False):
-    """spmm_chain for 2 to 48 fp16 rows of a weight with codes, all row-major (tl_spmm_chain_rows): the image is an [M, N] tensor,
-    the squares are [ceil(N / 16), R] float32 with R = 16, 32 or 64 for up to 16, 32 or 48 rows.  gated: columns are (gate, up)
+    """spmm_chain for 2 and more fp16 rows of a weight with codes, all row-major (tl_spmm_chain_rows): the image is an [M, N] tensor,
+    the squares are [ceil(N / 16), R] float32 with R = 16, 32 or 64 for up to 16, 32 or 48 rows.  More rows leave squares
+    [M, ceil(N / 32)]; row_factors makes the [M] float32 tensor of them that is squares_in there.  gated: columns are (gate, up)
     pairs, the result is [M, N / 2].  Raises RuntimeError (TL_ERR_UNSUPPORTED) for other rows, types and weights."""
     if x.device != weight.device:
         raise RuntimeError(f"x is on {x.device}, the weight on {weight.device}")
     x_code = _code(x.dtype, "x")
     xg, M, ldx = _x_geometry(x, weight.inners, _lib.TL_X_ROW_MAJOR)
     N = weight.columns
-    R = 16 if M <= 16 else 32 if M <= 32 else 64
+    R, few = 16 if M <= 16 else 32 if M <= 32 else 64, M <= 48
     y = torch.empty((M, N // 2 if gated else N), dtype=x.dtype, device=x.device)
     chain = _lib.Chain()
     if residual is not None:
@@ -272,12 +273,12 @@ def spmm_chain_rows(weight, x, scale=None, residual=None, next_norm_weight=None,
         if next_norm_weight.numel() != N or next_norm_weight.dtype != x.dtype or not next_norm_weight.is_contiguous() or next_norm_weight.device != x.device:
             raise ValueError("next_norm_weight must be a contiguous [N] tensor of x's dtype")
         image = torch.empty((M, N), dtype=x.dtype, device=x.device)
-        squares = torch.empty(((N + 15) // 16, R), dtype=torch.float32, device=x.device)
+        squares = torch.empty(((N + 15) // 16, R) if few else (M, (N + 31) // 32), dtype=torch.float32, device=x.device)
         chain.next_norm_weight, chain.image_out, chain.image_ld, chain.squares_out = next_norm_weight.data_ptr(), image.data_ptr(), N, squares.data_ptr()
     if squares_in is not None:
-        if squares_in.dtype != torch.float32 or squares_in.dim() != 2 or squares_in.shape[1] != R or not squares_in.is_contiguous() or \
-                squares_in.device != x.device:
-            raise ValueError(f"squares_in must be a contiguous float32 [blocks, {R}] tensor")
+        fits = squares_in.dim() == 2 and squares_in.shape[1] == R if few else squares_in.shape == (M,)
+        if squares_in.dtype != torch.float32 or not fits or not squares_in.is_contiguous() or squares_in.device != x.device:
+            raise ValueError(f"squares_in must be a contiguous float32 [blocks, {R}] tensor" if few else f"squares_in must be the {M} rows' factors, float32")
         chain.squares_in, chain.squares_blocks = squares_in.data_ptr(), squares_in.shape[0]
     chain.eps = float(eps)
     sc, s_code = _scale_args(scale, N, x.device)
@@ -722,6 +723,35 @@ def decode_attention_pieces(q, k_cache, v_cache, pos, splits=None, fresh=None):
     pieces = torch.empty((B * heads, splits, hd + 4), dtype=torch.float32, device=q.device)
     _attention_call(None if fresh is not None else q, fresh, k_cache, v_cache, pos, None, 0, splits, pieces.data_ptr(), pieces.numel() * 4)
     return pieces
+
+
+def row_factors(squares, width, eps):
+    """rsqrt(mean square + eps) of rows of `width` values whose product (spmm_chain_rows, more than 48 rows) left `squares`."""
+    if squares.dtype != torch.float32 or squares.dim() != 2 or not squares.is_contiguous():
+        raise ValueError("squares must be a contiguous float32 [rows, blocks] tensor")
+    factors = torch.empty(squares.shape[0], dtype=torch.float32, device=squares.device)
+    with torch.cuda.device(squares.device):
+        _lib.check(_lib.lib().tl_row_factors(squares.data_ptr(), squares.shape[0], squares.shape[1], int(width), float(eps), factors.data_ptr(),
+                                             _stream_ptr(squares.device)))
+    return factors
+
+
+def embed_rows(table, token, norm_weight):
+    """(x, image, squares): x = table[token], image = x * norm_weight and the sums of squares of x over runs of 16 values, as
+    spmv_add(..., next_norm_weight=) leaves them for one row and spmm_chain_rows for more (tl_embed_rows).  fp16."""
+    B, width = token.numel(), table.shape[1]
+    for t in (table, norm_weight):
+        if not t.is_contiguous() or t.dtype != table.dtype or t.device != token.device:
+            raise ValueError("table and norm_weight must be contiguous, of one dtype, on the token's device")
+    if token.dtype != torch.int64 or not token.is_contiguous() or norm_weight.numel() != width or not 1 <= B <= 65535:
+        raise ValueError("token must be a contiguous int64 tensor of 1 to 65535 elements and norm_weight a row of the table's width")
+    R = 1 if B == 1 else 16 if B <= 16 else 32 if B <= 32 else 64 if B <= 48 else 0
+    x, image = torch.empty((2, B, width), dtype=table.dtype, device=table.device).unbind(0)
+    squares = torch.empty((width // 16, R) if R > 1 else (width // 16,) if R else (B, (width + 31) // 32), dtype=torch.float32, device=table.device)
+    with torch.cuda.device(table.device):
+        _lib.check(_lib.lib().tl_embed_rows(table.data_ptr(), _code(table.dtype, "table"), table.shape[0], width, token.data_ptr(), B, norm_weight.data_ptr(),
+                                            x.data_ptr(), image.data_ptr(), squares.data_ptr(), R, _stream_ptr(table.device)))
+    return x, image, squares
 
 
 def greedy_advance(logits, token, pos=None, max_pos=0, mask=None):

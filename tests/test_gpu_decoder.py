@@ -811,3 +811,37 @@ def test_prefill_runs_norms_that_are_not_as_built(cuda):
     m.layers[1].post_attention_layernorm.eps = cfg.rms_norm_eps
     m.layers[0].input_layernorm = torch.nn.LayerNorm(256).to(cuda, torch.float16)
     assert float((both() - as_built).norm() / as_built.norm()) > 0.005
+
+
+def test_chained_passes_leave_hooks_and_eps_alone(cuda):
+    """More than 48 prompt tokens and steps of two rows: hooks on a linear layer run, and a norm's own eps counts."""
+    from ternaryllm_amd import TernaryConfig, TernaryLlamaDecoder
+    cfg = TernaryConfig(hidden_size=256, intermediate_size=512, num_hidden_layers=2, num_attention_heads=2, num_key_value_heads=2, vocab_size=300,
+                        max_position_embeddings=64, sparsity=0.7)
+    m = TernaryLlamaDecoder(cfg, seed=3, device=cuda)
+    tokens = torch.randint(0, 300, (2, 40), generator=torch.Generator().manual_seed(1)).to(cuda)
+
+    def both():
+        native = m.prefill(tokens).double()
+        m.native_prefill = False
+        plain = m.prefill(tokens).double()
+        m.native_prefill = True
+        # fp16 roundings in another order: a quarter of a percent at most over two layers
+        assert float((native - plain).norm() / plain.norm()) <= 5e-3
+        return native
+
+    as_built = both()
+    m.layers[1].post_attention_layernorm.eps = 0.5
+    assert float((both() - as_built).norm() / as_built.norm()) > 0.02
+    m.layers[1].post_attention_layernorm.eps = cfg.rms_norm_eps
+    step = {"token": tokens[:, -1].clone(), "pos": torch.full((1,), 40, dtype=torch.long, device=cuda),
+            "mask": (torch.arange(64, device=cuda) <= 40)[None, None, None].clone()}
+    chained = m._decode_step(step["token"], step["pos"], step["mask"]).double()
+    seen = []
+    handles = [p.register_forward_hook(lambda mod, args, out: seen.append(tuple(out.shape))) for p in (m.layers[0].o_proj, m.layers[1].down_proj)]
+    hooked = m.prefill(tokens).double()
+    assert seen == [(80, 256)] * 2 and float((hooked - as_built).norm() / as_built.norm()) <= 5e-3
+    hooked = m._decode_step(step["token"], step["pos"], step["mask"]).double()
+    assert seen == [(80, 256)] * 2 + [(2, 256)] * 2 and float((hooked - chained).norm() / chained.norm()) <= 5e-3
+    for h in handles:
+        h.remove()

@@ -104,3 +104,25 @@ def test_chained_rows(cuda, M, K, N, N2):
     assert torch.equal(ops.spmm_chain_rows(d1, x, sc1, residual=res).isfinite(), (ops.spmm(d1, x, sc1) + res).isfinite())
     with pytest.raises(RuntimeError, match="UNSUPPORTED"):
         ops.spmm_chain_rows(d1, x[:1], sc1, residual=res[:1])
+
+
+@pytest.mark.parametrize("B,width", [(1, 16), (1, 2048), (5, 2064), (16, 4096), (17, 48), (48, 2048), (49, 48), (300, 2064)])
+def test_embedding_rows(cuda, B, width):
+    """A token's row, its image for the product behind the first norm and its sums of squares; tokens counted from the end, and
+    tokens that the table does not have."""
+    from ternaryllm_amd import ops
+    g = torch.Generator().manual_seed(B)
+    table, nw = torch.randn((37, width), generator=g).half().to(cuda), torch.rand(width, generator=g).half().to(cuda)
+    token = torch.randint(-37, 37, (B,), generator=g).to(cuda)
+    print(f"case B={B} width={width}", flush=True)
+    x, image, squares = ops.embed_rows(table, token, nw)
+    want = table[token]
+    assert torch.equal(x, want) and torch.equal(image, (want.float() * nw.float()).half())
+    run = 16 if B <= 48 else 32
+    padded = torch.zeros((B, -(-width // run) * run), dtype=torch.float64, device=cuda)
+    padded[:, :width] = want.double().pow(2)
+    got = squares.view(1, -1) if B == 1 else squares[:, :B].t() if B <= 48 else squares
+    assert torch.allclose(got.double(), padded.view(B, -1, run).sum(-1), rtol=run * 2.0 ** -24, atol=0)   # a rounding for each value
+    token[B - 1] = 37
+    x, image, squares = ops.embed_rows(table, token, nw)
+    assert bool(x[B - 1].isnan().all()) and torch.equal(x[:B - 1], want[:B - 1])

@@ -65,6 +65,42 @@ def test_tiles_of_every_shape(cuda, M, K, N, dtype):
     assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())              # exact sums; __expf and the division
 
 
+@pytest.mark.parametrize("M,K,N,N2", [(49, 8, 1, 34), (65, 1344, 66, 40), (200, 2048, 1032, 130), (1030, 336, 2100, 66), (4096, 200, 4096, 2048)])
+def test_chained_rows(cuda, M, K, N, N2):
+    """More than 48 rows: a product that adds residual rows and leaves the next norm's image and sums of squares, bit for bit as
+    separate operators do, and products that multiply by the rows' factors, plain and gated."""
+    from ternaryllm_amd import ops
+    K2 = N - N % 8
+    w1, w2 = ternary_weight(K, N, 0.7, 1), ternary_weight(max(K2, 8), N2, 0.7, 2)
+    d1, d2 = _device(w1, cuda), _device(w2, cuda)
+    g = torch.Generator(device=cuda).manual_seed(M)
+    x, res = torch.randn((M, K), generator=g, device=cuda).half(), torch.randn((M, N), generator=g, device=cuda).half()
+    nw, sc1 = (1 + 0.1 * torch.randn(N, generator=g, device=cuda)).half(), (0.05 + 0.01 * torch.rand(N, generator=g, device=cuda)).half()
+    sc2 = (0.05 + 0.01 * torch.rand(N2, generator=g, device=cuda)).half()
+    print(f"case M={M} K={K} N={N} N2={N2}", flush=True)
+    y, image, squares = ops.spmm_chain_rows(d1, x, sc1, residual=res, next_norm_weight=nw)
+    assert torch.equal(y, ops.spmm(d1, x, sc1) + res)
+    assert torch.equal(image, (y.float() * nw.float()).half())
+    blocks = -(-N // 32)
+    padded = torch.zeros((M, blocks * 32), dtype=torch.float64, device=cuda)
+    padded[:, :N] = y.double().pow(2)
+    # (32 squares and 31 additions, each rounded to 2^-24)
+    assert torch.allclose(squares.double(), padded.view(M, blocks, 32).sum(-1), rtol=63 * 2.0 ** -24, atol=0)
+    factors = ops.row_factors(squares, N, 1e-5)
+    # (the sums' roundings halved by the root, and rsqrt's own)
+    assert torch.allclose(factors.double(), torch.rsqrt(y.double().pow(2).mean(-1) + 1e-5), rtol=(64 + blocks) * 2.0 ** -24, atol=0)
+    rows = image[:, :K2].contiguous() if K2 else x
+    out = ops.spmm_chain_rows(d2, rows, sc2, squares_in=factors)
+    want = (ops.spmm(d2, rows, sc2, out_dtype=torch.float32) * factors[:, None]).half()
+    assert float((out.double() - want.double()).abs().max()) <= 2.0 ** -10 * float(want.double().abs().max())   # a unit in the last place of fp16
+    gated = ops.spmm_chain_rows(d2, rows, sc2, squares_in=factors, gated=True)
+    assert torch.equal(gated, ops.silu_mul(out, pairs=True))
+    assert torch.equal(ops.spmm_chain_rows(d2, rows, sc2, gated=True), ops.spmm_gated(d2, rows, sc2))
+    with pytest.raises(RuntimeError, match="UNSUPPORTED"):
+        wide = torch.zeros((M, K + 1), dtype=torch.float16, device=cuda)[:, :K]
+        ops.spmm_chain_rows(d1, wide, sc1, residual=res)               # rows that are not read where they lie
+
+
 def _repeated(w):
     """The packed weight of tiled-CSC arrays that name a row |entry| times."""
     from ternaryllm_amd.packing import PackedWeight
