@@ -79,6 +79,16 @@ struct PrefillAttn {
     float scale_log2;                          // 1 / sqrt(head_dim) * log2(e)
 };
 
+// f over the four lanes with the same number modulo 16, on the vector unit (16 x 512 of 16 heads took 48.4 us with shuffles, 47.6).
+template <typename F>
+__device__ __forceinline__ float with_other_rows(float v, F f)
+{
+    const auto near = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = f(__uint_as_float(near[0]), __uint_as_float(near[1]));
+    const auto far = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return f(__uint_as_float(far[0]), __uint_as_float(far[1]));
+}
+
 // Causal attention: query i of a batch row sees keys 0 .. i + (kv_len - q_len).  A workgroup of four waves owns 64 * QF
 // queries of one head, a wave QF fragments of 16; it walks the keys that its queries see in tiles of 64, one pass, with a
 // running maximum, sum and weighted sum in fp32 (rescaled when the maximum moves).
@@ -226,8 +236,7 @@ __global__ __launch_bounds__(256, 2) void tl_prefill_attn(PrefillAttn a)
                 for (int n = 0; n < 4; ++n)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) most = fmaxf(most, sc[n][f][i]);
-                most = fmaxf(most, __shfl_xor(most, 16, 64));
-                most = fmaxf(most, __shfl_xor(most, 32, 64));
+                most = with_other_rows(most, [](float x, float y) { return fmaxf(x, y); });
                 const float now = fmaxf(top[f], most);
                 const float base = now == -__builtin_huge_valf() ? 0.f : now * a.scale_log2;   // (nothing but -inf so far)
                 const float shrink = __builtin_amdgcn_exp2f(fmaf(top[f], a.scale_log2, -base));
@@ -271,8 +280,7 @@ __global__ __launch_bounds__(256, 2) void tl_prefill_attn(PrefillAttn a)
 #pragma unroll
     for (int f = 0; f < QF; ++f) {
         const int qi = wq0 + f * 16 + r16;
-        float all = sum[f] + __shfl_xor(sum[f], 16, 64);
-        all += __shfl_xor(all, 32, 64);
+        const float all = with_other_rows(sum[f], [](float x, float y) { return x + y; });
         if (qi >= a.q_len) continue;
         const float inv = 1.0f / all;
         __half* row = a.out + ((long long)b * a.q_len + qi) * a.heads * HD + h * HD + g * 4;
@@ -355,10 +363,12 @@ extern "C" int tl_prefill_attention(const void* q, const void* k, const void* v,
                   static_cast<const __half*>(sin_table), static_cast<__half*>(out), s, heads, heads / kv_heads, 0, (int)q_len, (int)kv_len, 0,
                   1.4426950408889634f / sqrtf((float)head_dim)};
     const int64_t pairs = batch * heads;
-    // 128 queries to a workgroup halve what is read from LDS per product; 64 where that leaves compute units without one.
+    // 128 queries to a workgroup halve what is read from LDS per product, and pay once there are enough of them for every compute
+    // unit to have two at a time until the end (us with 128 / 64, workgroups of 128: 16 x 512 of 16 heads, 1024: 47.6 / 59.7;
+    // 1 x 2048 of 32, 512: 81.7 / 78.9; 8 x 128 of 32, 256: 10.0 / 8.9; 4 x 1000 of 8, 256: 40.5 / 30.5).
     // (A few queries over a long past leave most of a workgroup idle and a head's keys in series; the attention block of 32 heads,
     // one query, past of 2048 / 8192 keys: 125 / 334 us, with the torch operator in its place 220 / 483.)
-    const bool tall = pairs * ceil_div(q_len, 128) >= compute_units();
+    const bool tall = pairs * ceil_div(q_len, 128) >= 3 * compute_units();
     const int64_t q_tiles = ceil_div(q_len, tall ? 128 : 64);
     if (pairs * q_tiles > INT32_MAX) return fail(TL_ERR_SHAPE, "%lld queries are more than one launch takes", (long long)(batch * q_len));
     a.bh = (int)pairs;
