@@ -540,7 +540,7 @@ def main():
         "roofline": {"bound": "mfma", "achieved": round(2.0 * M * K * N / (ev_ms * 1e-3) / 1e12, 2), "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(2.0 * M * K * N / (ev_ms * 1e-3) / 1e12 / MFMA_PEAK_TFLOPS, 5), "note": "dense operations; a zero weight is multiplied too",
                      "traffic": traffic, "traffic_note": traffic_note,
-                     "kernel": "tl_matrix_rows<1, 2, 4, 4, 2, 4, 0> (the one launch of a tl_spmm call on row-major activations)",
+                     "kernel": "tl_matrix_rows<1, 1, 4, 1, 2, 2, 0> (the one launch of a tl_spmm call on row-major activations)",
                      "kernel_ms": round(ev_ms, 5)},
     }
     extra = {

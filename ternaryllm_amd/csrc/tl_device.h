@@ -210,7 +210,7 @@ int launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t works
 bool matrix_reads_rows(const KernelArgs& a, int x_dtype);
 
 // tl_few.hip
-// Up to 48 rows, any layout, blobs with codes; no gated and no chained epilogue.  Two weights: silu(w0 product) * w1 product.
+// Up to 48 rows, any layout, blobs with codes; gated and chained steps for fp16 rows.  Two weights: silu(w0 product) * w1 product.
 int launch_matrix_few(KernelArgs a, int x_dtype, bool two_weights, hipStream_t st);
 
 }  // namespace tl
