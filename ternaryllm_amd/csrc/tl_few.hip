@@ -23,12 +23,12 @@ constexpr int kMaxWaves = 16;
 constexpr __host__ __device__ int most_waves(int C, int stage_bytes) { return C == 1 && stage_bytes <= 8192 ? kMaxWaves : kMaxWaves / 2; }
 
 
-// How rows are read: aligned 16-byte pieces (K a multiple of 8); 16 bytes at a time from any element on, but for the turn in
-// which a row ends; element by element (K-major); aligned pieces through LDS.
+// How rows are read: aligned 16-byte pieces (K a multiple of 8), as operands; through registers and LDS, 16 bytes at a time
+// from any element on; element by element (K-major); aligned pieces straight to LDS.
 enum { kRowPieces = 0, kRows = 1, kElements = 2, kStaged = 3 };
 
 // Eight activations of a row from k on.  Past K: zeros (element by element) or the row's last whole piece again (such rows
-// of K meet zero codes).  kRows: the caller has seen that k + 8 <= K.
+// of K meet zero codes).
 template <typename XT, int IN>
 __device__ __forceinline__ void load8(const KernelArgs& a, const XT* row, int k, XT* v)
 {
@@ -36,8 +36,6 @@ __device__ __forceinline__ void load8(const KernelArgs& a, const XT* row, int k,
         const u32x4* p = reinterpret_cast<const u32x4*>(row + min(k, a.K - 8));
 #pragma unroll
         for (int i = 0; i < (int)sizeof(XT) / 2; ++i) reinterpret_cast<u32x4*>(v)[i] = p[i];
-    } else if constexpr (IN == kRows) {
-        __builtin_memcpy(v, row + k, 8 * sizeof(XT));
     } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = k + i < a.K ? row[(k + i) * a.x_sk] : XT(0.f);
@@ -103,16 +101,17 @@ __device__ __forceinline__ float sum_over_lanes(float v)
     return v;
 }
 
+// (33 to 48 staged fp32 rows run with eight waves and may take the registers of sixteen.)
 // XT: activation type.  IN: how they are read.  FM: fragments of 16 rows.  C: column blocks of a workgroup (kTwo: one of each
 // weight).  Q: slices of a wave's turn.
 // LDS of a wave: its activations of a turn (kStaged), then its sums.
 template <typename XT, int IN, int FM>
-constexpr __host__ __device__ int stage_bytes(int Q) { return IN == kStaged ? Q * FM * 16 * kSliceRows * (int)sizeof(XT) : 0; }
+constexpr __host__ __device__ int stage_bytes(int Q) { return IN == kStaged || IN == kRows ? Q * FM * 16 * kSliceRows * (int)sizeof(XT) : 0; }
 template <typename XT, int IN, int FM, int C, int Q>
 constexpr __host__ __device__ int wave_floats() { return std::max(C * FM * kPartFloats, stage_bytes<XT, IN, FM>(Q) / 4); }
 
 template <typename XT, int IN, int FM, int C, int Q, int STEPS>
-__global__ __launch_bounds__(kMaxWaves * 64) void tl_matrix_few(KernelArgs a)
+__global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_waves(C, stage_bytes<XT, IN, FM>(1)) : kMaxWaves)) void tl_matrix_few(KernelArgs a)
 {
     constexpr bool F32 = sizeof(XT) == 4, TWO = STEPS == kTwo;
     constexpr int kTurnsOfUnit = TL_CODE_UNIT_ROWS / (kSliceRows * Q);
@@ -171,9 +170,10 @@ __global__ __launch_bounds__(kMaxWaves * 64) void tl_matrix_few(KernelArgs a)
     }
 
     const int turns = a.planes == 1 ? (a.K + kSliceRows * Q - 1) / (kSliceRows * Q) : a.planes * a.units * kTurnsOfUnit;
+    constexpr bool STAGED = IN == kStaged || IN == kRows;
     struct Turn {
         uint32_t w[C][4];
-        XT x[IN == kStaged ? 1 : Q * 2][FM][8] __attribute__((aligned(16)));
+        XT x[STAGED ? 1 : Q * 2][FM][8] __attribute__((aligned(16)));
     };
     // kStaged: a load takes whole slices (128 or 256 bytes) of 8 or 4 rows.  A row's pieces lie rotated so that 16 lanes that
     // read one piece of 16 rows find them on different banks.
@@ -192,6 +192,41 @@ __global__ __launch_bounds__(kMaxWaves * 64) void tl_matrix_few(KernelArgs a)
             for (int q = 0; q < Q; ++q)
                 load_to_lds(own + q * FM * BLOCK + i * 1024, a.X, row + min((uint32_t)((k0 + q * kSliceRows) * (int)sizeof(XT)) + piece, last));
         }
+    };
+    // kRows: the same through registers, 16 bytes from any element on, and element by element where a row ends.  us as operands
+    // straight from memory / so: fp16 16 rows 4095 -> 11008 26.5 / 9.3, 48 rows 67.6 / 23.0, 37 rows 1003 -> 777 8.0 / 6.2; fp32 16 rows
+    // 24.7 / 14.7, 48 rows 54.6 / 42.8, but 37 rows 1003 -> 777 7.7 / 8.8 (eight waves, whose 12 KB fill the LDS, in the place of 16).
+    [[maybe_unused]] auto stage_any = [&](int t) {
+        constexpr int E = 16 / (int)sizeof(XT), LOADS = FM * BLOCK / 1024;
+        const int k0 = t / kTurnsOfUnit % a.units * TL_CODE_UNIT_ROWS + t % kTurnsOfUnit * Q * kSliceRows;
+        const XT* x = static_cast<const XT*>(a.X);
+        u32x4 v[LOADS][Q];
+        auto read = [&](auto whole) {
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) {
+                const int r = (i * 64 + lane) / PIECES;
+                const XT* row = x + min(r, a.M - 1) * a.x_sm;
+                const int piece = (lane % PIECES ^ turned(r)) * E;
+#pragma unroll
+                for (int q = 0; q < Q; ++q) {
+                    const int k = k0 + q * kSliceRows + piece;
+                    XT e[E] __attribute__((aligned(16)));
+                    if (decltype(whole)::value || k + E <= a.K) __builtin_memcpy(e, row + k, 16);
+                    else {
+#pragma unroll
+                        for (int j = 0; j < E; ++j) e[j] = k + j < a.K ? row[k + j] : XT(0.f);
+                    }
+                    v[i][q] = *reinterpret_cast<const u32x4*>(e);
+                }
+            }
+        };
+        if (k0 + Q * kSliceRows <= a.K) read(std::true_type{});
+        else read(std::false_type{});
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i)
+#pragma unroll
+            for (int q = 0; q < Q; ++q)
+                *reinterpret_cast<u32x4*>(reinterpret_cast<unsigned char*>(sums + wave * OWN) + q * FM * BLOCK + i * 1024 + lane * 16) = v[i][q];
     };
     [[maybe_unused]] auto staged = [&](int s, int f, XT* v) {      // the eight activations of step s that are this lane's
         const unsigned char* row = reinterpret_cast<const unsigned char*>(sums + wave * OWN) + ((s >> 1) * FM + f) * BLOCK + r16 * (PIECES * 16);
@@ -218,15 +253,14 @@ __global__ __launch_bounds__(kMaxWaves * 64) void tl_matrix_few(KernelArgs a)
             asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
             return;
         }
-        const int k0 = (unit % a.units) * TL_CODE_UNIT_ROWS + part * Q * kSliceRows + g * 8;
-        auto load_x = [&](auto in) {
+        if constexpr (IN == kRows) stage_any(t);
+        else {
+            const int k0 = (unit % a.units) * TL_CODE_UNIT_ROWS + part * Q * kSliceRows + g * 8;
 #pragma unroll
             for (int s = 0; s < Q * 2; ++s)
 #pragma unroll
-                for (int f = 0; f < FM; ++f) load8<XT, decltype(in)::value>(a, rows[f], k0 + s * 32, to.x[s][f]);
-        };
-        if (IN == kRows && (unit % a.units) * TL_CODE_UNIT_ROWS + (part + 1) * Q * kSliceRows > a.K) load_x(std::integral_constant<int, kElements>{});
-        else load_x(std::integral_constant<int, IN>{});
+                for (int f = 0; f < FM; ++f) load8<XT, IN>(a, rows[f], k0 + s * 32, to.x[s][f]);
+        }
     };
     auto multiply = [&](const Turn& turn) {
 #pragma unroll
@@ -240,7 +274,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void tl_matrix_few(KernelArgs a)
 #pragma unroll
             for (int f = 0; f < FM; ++f) {
                 XT x[8] __attribute__((aligned(16)));
-                if constexpr (IN == kStaged) staged(s, f, x);
+                if constexpr (STAGED) staged(s, f, x);
                 else __builtin_memcpy(x, turn.x[s][f], sizeof(x));
                 if constexpr (F32) {
                     u32x4 p[3];
@@ -358,7 +392,7 @@ int launch_few(const KernelArgs& a, hipStream_t st)
     const int most = most_waves(C, stage_bytes<XT, IN, FM>(1));
     // a turn of four slices is one 16-byte load of codes; fewer where that would leave waves without a turn, and where the
     // turn's activations, loaded one by one, would not fit the registers
-    constexpr int kMostSlices = IN == kStaged ? std::max(1, 8192 / stage_bytes<XT, IN, FM>(1)) : IN == kRowPieces || FM == 1 ? 4 : FM == 2 ? 2 : 1;
+    constexpr int kMostSlices = stage_bytes<XT, IN, FM>(1) ? std::max(1, 8192 / stage_bytes<XT, IN, FM>(1)) : IN == kRowPieces || FM == 1 ? 4 : FM == 2 ? 2 : 1;
     const int q = std::min<int>(kMostSlices, slices >= 4 * most ? 4 : slices >= 2 * most ? 2 : 1);
     const int waves = (int)std::min<int64_t>(most, ceil_div(slices, q));
     const dim3 grid((unsigned)(STEPS == kTwo ? a.NB : ceil_div(a.NB, C))), block((unsigned)waves * 64);
@@ -366,7 +400,7 @@ int launch_few(const KernelArgs& a, hipStream_t st)
         constexpr int Q = decltype(q_tag)::value;
         const size_t lds = (size_t)waves * (wave_floats<XT, IN, FM, C, Q>() + (STEPS == kSteps ? squares_rows(FM * 16) : 0)) * sizeof(float);
         auto kernel = tl_matrix_few<XT, IN, FM, C, Q, STEPS>;
-        if (IN == kStaged) {
+        if (IN == kStaged || IN == kRows) {
             static std::atomic<bool> raised{false};  // per instantiation; a repeated call is harmless
             if (!raised.load(std::memory_order_relaxed)) {
                 if (int rc = raise_lds_limit(kernel, 160 * 1024)) return rc;
