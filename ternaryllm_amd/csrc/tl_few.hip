@@ -101,21 +101,21 @@ __device__ __forceinline__ float sum_over_lanes(float v)
     return v;
 }
 
-// (33 to 48 staged fp32 rows run with eight waves and may take the registers of sixteen.)
-// XT: activation type.  IN: how they are read.  FM: fragments of 16 rows.  C: column blocks of a workgroup (kTwo: one of each
-// weight).  Q: slices of a wave's turn.
-// LDS of a wave: its activations of a turn (kStaged), then its sums.
+// LDS of a wave: its activations of a turn (kStaged, kRows), then its sums.
 template <typename XT, int IN, int FM>
 constexpr __host__ __device__ int stage_bytes(int Q) { return IN == kStaged || IN == kRows ? Q * FM * 16 * kSliceRows * (int)sizeof(XT) : 0; }
 template <typename XT, int IN, int FM, int C, int Q>
 constexpr __host__ __device__ int wave_floats() { return std::max(C * FM * kPartFloats, stage_bytes<XT, IN, FM>(Q) / 4); }
 
+// XT: activation type.  IN: how they are read.  FM: fragments of 16 rows.  C: column blocks of a workgroup (kTwo: one of each
+// weight).  Q: slices of a wave's turn.
+// (33 to 48 staged fp32 rows run with eight waves and may take the registers of sixteen.)
 template <typename XT, int IN, int FM, int C, int Q, int STEPS>
 __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_waves(C, stage_bytes<XT, IN, FM>(1)) : kMaxWaves)) void tl_matrix_few(KernelArgs a)
 {
     constexpr bool F32 = sizeof(XT) == 4, TWO = STEPS == kTwo;
     constexpr int kTurnsOfUnit = TL_CODE_UNIT_ROWS / (kSliceRows * Q);
-        // [wave] its stage of activations (kStaged), where its sums [C][FM][kPartFloats] lie afterwards; and, kSteps, [wave][SR] sums of squares
+    // [wave] its stage of activations (kStaged, kRows), where its sums [C][FM][kPartFloats] lie afterwards; and, kSteps, [wave][SR] sums of squares
     extern __shared__ __align__(16) float sums[];
     constexpr int OWN = wave_floats<XT, IN, FM, C, Q>();
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
