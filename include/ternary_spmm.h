@@ -489,7 +489,8 @@ int tl_spmm_chain(const tl_layout_header* header, const void* blob_dev,
 /* The same chain for 2 and more fp16 rows of blobs with codes, row by row: X, Y and image_out are row-major (image_ld >= N, no
  * padding rows).  Up to 48 rows the squares are [blocks][R] with R = 16, 32 or 64 for up to 16, 32 or 48 rows (rows past M are not
  * written and not read).  More rows (X aligned to 16 bytes, K and ldx multiples of 8) leave squares_out [M][ceil(N / 32)], from
- * which tl_row_factors makes the M factors that squares_in points to then.  gated != 0 gives Y the N / 2 values silu(y[2j]) * y[2j + 1].  The product is tl_spmm's for these rows.
+ * which tl_row_factors makes the M factors that squares_in points to then.  (image_out is rounded before a row's factor: a value above 65504 / weight
+ * is infinite there, and products below fp16's normal range lose bits.)  gated != 0 gives Y the N / 2 values silu(y[2j]) * y[2j + 1].  The product is tl_spmm's for these rows.
  * TL_ERR_UNSUPPORTED for other types, row counts and blobs without codes. */
 int tl_spmm_chain_rows(const tl_layout_header* header, const void* blob_dev,
                        const void* X, int x_dtype, int64_t ldx, int64_t M, void* Y, int y_dtype, int64_t ldy, int gated,

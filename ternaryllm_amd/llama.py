@@ -231,7 +231,10 @@ class TernaryLlamaDecoder(nn.Module):
 
     def _prefill_native(self, tokens):
         """The pass with the library's kernels around the products: residual add + RMSNorm in one, keys rotated into the
-        cache and values copied beside them in one, queries rotated inside the attention.  Seven launches a layer."""
+        cache and values copied beside them in one, queries rotated inside the attention.  Seven launches a layer.
+        (The add and the norm have a kernel, which rounds a row once, behind its factor: a product that left rows times the
+        next norm's weight, 1587 us where this takes 1620 for 16 x 512 tokens of 2048 and two layers, put entries above
+        65504 / weight at infinity.  The add alone in the product's last step gains nothing.)"""
         c = self.config
         B, S = tokens.shape
         H, nh, hd = c.hidden_size, c.num_attention_heads, c.head_dim
@@ -240,8 +243,6 @@ class TernaryLlamaDecoder(nn.Module):
             return ops.add_rmsnorm(x, y, norm.weight, norm.eps)
 
         tables = self.rope_cos[:S], self.rope_sin[:S]
-        if 48 < B * S <= 65535 and H % 16 == 0 and c.intermediate_size % 8 == 0 and tokens.dtype == torch.int64 and self._products_as_built():
-            return self._prefill_chained(tokens.contiguous(), tables)
         x = self.embed_tokens[tokens].view(B * S, H)
         _, h = add_norm(x, None, self.layers[0].input_layernorm)
         for li, layer in enumerate(self.layers):
@@ -255,32 +256,6 @@ class TernaryLlamaDecoder(nn.Module):
                 x, h = add_norm(x, y, self.layers[li + 1].input_layernorm)
         last = [t.view(B, S, H)[:, -1].contiguous() for t in (x, y)]
         return self.lm_head(add_norm(*last, self.norm)[1])
-
-    def _prefill_chained(self, tokens, tables):
-        """The layers of a pass over more than 48 tokens without kernels for the residual add and the norm: the o and down
-        projections add the residual rows and leave the next norm's image and sums of squares, and the products behind
-        the norm multiply by each row's factor.  (16 x 512 tokens of 2048: an add + norm took 35 to 52 us, four of them a pass.)"""
-        c = self.config
-        B, S = tokens.shape
-        H, nh, hd = c.hidden_size, c.num_attention_heads, c.head_dim
-        x, h, squares = ops.embed_rows(self.embed_tokens, tokens, self.layers[0].input_layernorm.weight)
-
-        def product(linear, rows, **steps):
-            return ops.spmm_chain_rows(linear.device_weight(), rows, linear.w_scale, **steps)
-
-        for li, layer in enumerate(self.layers):
-            qkv = product(layer.qkv_proj, h, squares_in=ops.row_factors(squares, H, layer.input_layernorm.eps)).view(B, S, 3, nh, hd)
-            kc, vc = self._cache[li, 0, :, :, :S], self._cache[li, 1, :, :, :S]
-            ops.rope_rows(qkv[:, :, 1], tables, kc, qkv[:, :, 2], vc)
-            a = ops.prefill_attention(qkv[:, :, 0], kc, vc, tables)
-            x, h, squares = product(layer.o_proj, a.view(B * S, H), residual=x, next_norm_weight=layer.post_attention_layernorm.weight)
-            gated = product(layer.gate_up_proj, h, squares_in=ops.row_factors(squares, H, layer.post_attention_layernorm.eps), gated=True)
-            if li + 1 == len(self.layers):
-                x = product(layer.down_proj, gated, residual=x)
-            else:
-                x, h, squares = product(layer.down_proj, gated, residual=x, next_norm_weight=self.layers[li + 1].input_layernorm.weight)
-        last = x.view(B, S, H)[:, -1].contiguous()
-        return self.lm_head(ops.add_rmsnorm(last, None, self.norm.weight, self.norm.eps)[1])
 
     # -- decode ------------------------------------------------------------------------------
     def _decode_step(self, token, pos, mask):

@@ -254,7 +254,8 @@ def spmm_chain(weight, x, scale=None, x_layout=_lib.TL_X_ROW_MAJOR, residual=Non
 def spmm_chain_rows(weight, x, scale=None, residual=None, next_norm_weight=None, squares_in=None, eps=0.0, gated=False):
     """spmm_chain for 2 and more fp16 rows of a weight with codes, all row-major (tl_spmm_chain_rows): the image is an [M, N] tensor,
     the squares are [ceil(N / 16), R] float32 with R = 16, 32 or 64 for up to 16, 32 or 48 rows.  More rows leave squares
-    [M, ceil(N / 32)]; row_factors makes the [M] float32 tensor of them that is squares_in there.  gated: columns are (gate, up)
+    [M, ceil(N / 32)]; row_factors makes the [M] float32 tensor of them that is squares_in there.  (The image is rounded before the
+    rows' factors: entries above 65504 / weight are infinite there, products below 6e-5 lose bits.)  gated: columns are (gate, up)
     pairs, the result is [M, N / 2].  Raises RuntimeError (TL_ERR_UNSUPPORTED) for other rows, types and weights."""
     if x.device != weight.device:
         raise RuntimeError(f"x is on {x.device}, the weight on {weight.device}")

@@ -845,3 +845,48 @@ def test_chained_passes_leave_hooks_and_eps_alone(cuda):
     assert seen == [(80, 256)] * 2 + [(2, 256)] * 2 and float((hooked - chained).norm() / chained.norm()) <= 5e-3
     for h in handles:
         h.remove()
+
+
+def _decoder(**sizes):
+    from ternaryllm_amd import TernaryConfig, TernaryLlamaDecoder
+    cfg = TernaryConfig(**{**dict(hidden_size=256, intermediate_size=512, num_hidden_layers=2, num_attention_heads=2, num_key_value_heads=2, vocab_size=300,
+                                  max_position_embeddings=64, sparsity=0.7), **sizes})
+    return TernaryLlamaDecoder(cfg, seed=3, device="cuda")
+
+
+def _magnitudes(m, rows):
+    """Rows that leave fp16's middle: a column of 40000 in front of norm weights of 4, rows of 1e-5, norm weights of 0.01."""
+    linears = [p for layer in m.layers for p in (layer.o_proj, layer.down_proj)]
+    norms = [n for layer in m.layers for n in (layer.input_layernorm, layer.post_attention_layernorm)]
+    if rows == "large":
+        m.embed_tokens[:, 5] = 40000.0
+        for n in norms:
+            n.weight.mul_(4)
+    elif rows == "tiny":
+        m.embed_tokens.mul_(5e-4)
+        for p in linears:
+            p.w_scale.mul_(5e-4)
+    else:
+        m.embed_tokens.mul_(0.05)
+        for n in norms:
+            n.weight.mul_(0.01)
+
+
+@pytest.mark.parametrize("rows", ["large", "tiny", "small weights"])
+@pytest.mark.parametrize("B,S", [(2, 40), (7, 7), (20, 40)])
+def test_prompts_of_any_magnitude(cuda, B, S, rows):
+    """A prompt, logits and cache, against the torch operators around the products: both round in the same places and differ
+    where sums taken in another order fall on the other side of one (2^-10 of a value, on few of them).  Tokens on the CPU too."""
+    m = _decoder()
+    with torch.no_grad():
+        _magnitudes(m, rows)
+    tokens = torch.randint(0, 300, (B, S), generator=torch.Generator().manual_seed(1))
+    print(f"case B={B} S={S} {rows}", flush=True)
+    got = m.prefill(tokens.to(cuda))
+    cache = m._cache.clone()
+    assert torch.equal(m.prefill(tokens), got)
+    m.native_prefill = False
+    want = m.prefill(tokens.to(cuda))
+    assert bool(want.isfinite().all())
+    for a, b in ((got.double(), want.double()), (cache.double(), m._cache.double())):
+        assert float((a - b).norm() / b.norm()) <= 2.0 ** -10
