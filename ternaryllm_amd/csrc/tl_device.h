@@ -83,6 +83,7 @@ struct KernelArgs {
     const void* image;        // the activations they multiply: row-major, 16-byte pieces along K ...
     long long image_ld;       // ... elements between rows
     long long image_plane;    // ... and, for fp32 activations in three bf16 parts, between parts
+    int call_rows;            // of the whole call, of which a launch may have a part (M)
     int vector_out;           // whole pieces of 16 bytes of an output row may be stored (from 8-byte boundaries)
 };
 

@@ -718,13 +718,14 @@ int launch_tile(const KernelArgs& a, hipStream_t st)
 //     not spread the rows better: 2048 x 4096 -> 11008 139 / 144, 8192 x 2048 -> 11008 289 / 301, 8192 x 2048 -> 2048 64 / 66, but
 //     1536 x 4096 -> 11008 129 / 117 (516 tall tiles are three for some units, 1032 flat ones five halves).  Not for fp32, whose second
 //     set of sums does not fit.
+// The rows are the whole call's: a row's result does not depend on how many rows at a time a workspace holds.
 template <int PARTS, int MODE>
 int launch_mode(const KernelArgs& a, hipStream_t st)
 {
     const int64_t units = compute_units(), columns = (int64_t)a.N * (MODE == kTwoWeights ? 2 : 1);
-    if (ceil_div(a.M, 64) * ceil_div(columns, 64) <= 2 * units) return launch_tile<PARTS, 1, 1, 4, 2, 2, MODE>(a, st);
+    if (ceil_div(a.call_rows, 64) * ceil_div(columns, 64) <= 2 * units) return launch_tile<PARTS, 1, 1, 4, 2, 2, MODE>(a, st);
     if constexpr (PARTS == 1) {
-        const int64_t tall = ceil_div(a.M, 128) * ceil_div(columns, 256), flat = ceil_div(a.M, 64) * ceil_div(columns, 256);
+        const int64_t tall = ceil_div(a.call_rows, 128) * ceil_div(columns, 256), flat = ceil_div(a.call_rows, 64) * ceil_div(columns, 256);
         if (tall >= 2 * units && ceil_div(flat, units) >= 2 * ceil_div(tall, units)) return launch_tile<PARTS, 1, 4, 1, 4, 2, MODE>(a, st);
     }
     return launch_tile<PARTS, 1, 4, 1, 2, 2, MODE>(a, st);
@@ -772,6 +773,7 @@ bool tl::matrix_reads_rows(const KernelArgs& a, int x_dtype)
 
 int tl::launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t workspace_bytes, bool two_weights, hipStream_t st)
 {
+    a.call_rows = a.M;
     a.x_sm = a.x_kmajor ? 1 : a.ldx;
     a.x_sk = a.x_kmajor ? a.ldx : 1;
     const int64_t need = least_image_bytes(a.K, a.M, x_dtype);

@@ -272,6 +272,18 @@ def test_the_index_stream_alone(cuda, oracle, M, K, N, dtype):
         assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())   # exact sums; __expf and the division
 
 
+@pytest.mark.parametrize("M,K,N", [(2048, 4096, 2048), (1100, 1100, 2100)])
+def test_a_row_s_bits_do_not_depend_on_the_workspace(cuda, M, K, N):
+    """An image of fp32 rows that does not fit is made and multiplied some rows at a time, the last time with few (768 of 2048,
+    460 of 1100): with the tile of the whole call, whose sums are taken in one order."""
+    dw = _device(ternary_weight(K, N, 0.7, 5), cuda)
+    x = activations(M, K, 6, torch.float32).to(cuda)
+    print(f"case M={M} K={K} N={N}", flush=True)
+    rc, some = _product(dw, x, 0, M, K, torch.empty(M * K * 4, dtype=torch.uint8, device=cuda))
+    rc2, whole = _product(dw, x, 0, M, K, torch.empty(M * (K + 8) * 6, dtype=torch.uint8, device=cuda))
+    assert rc == rc2 == 0 and torch.equal(some, whole)
+
+
 def test_loading_a_blob_without_codes_from_the_device(cuda):
     """load_state_dict(assign=True) keeps the device of what it is given, also where the blob is brought up to date."""
     from ternaryllm_amd import TernaryLinear
