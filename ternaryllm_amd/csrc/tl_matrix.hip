@@ -73,6 +73,29 @@ __device__ __forceinline__ void store_piece(const KernelArgs& a, int m, int n, i
         if (n + i < N) store_out(a.Y, a.y_f16, at + i, v[i]);
 }
 
+// `factor` times the scales of 16 columns from n on, of N (past N: of the last column again; nothing of such columns is stored).
+// Read at once: a load for each column under its own condition, and a wait for each, took 2 us of a launch.
+__device__ __forceinline__ void read_scales(const void* scale, int is_f16, int n, int N, float factor, float (&s)[16])
+{
+    auto read = [&](auto type) {
+        using T = decltype(type);
+        const T* p = static_cast<const T*>(scale);
+        T raw[16];
+        if (n + 16 <= N) __builtin_memcpy(raw, p + n, sizeof(raw));
+        else {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) raw[i] = p[min(n + i, N - 1)];
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = factor * (float)raw[i];
+    };
+    if (!scale) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = factor;
+    } else if (is_f16) read(_Float16{});
+    else read(float{});
+}
+
 enum { kPlain = 0, kPairs = 1, kTwoWeights = 2, kSteps = 3 };   // (kSteps: with what a decoder layer does around a product)
 
 // The product of one output: from the index stream where the matrix cores' sum is not finite.
@@ -170,11 +193,8 @@ __device__ __forceinline__ void put_out(const KernelArgs& a, f32x16 (&acc)[FN][F
     for (int f = 0; f < OUT_FN; ++f) {
         const int n = lane_n0 + f * 32;
         float s0[16], s1[MODE == kTwoWeights ? 16 : 1];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            s0[i] = half * (n + i < a.N ? load_scale(a.w0.scale, a.scale_f16, n + i) : 0.f);
-            if constexpr (MODE == kTwoWeights) s1[i] = half * (n + i < a.N ? load_scale(a.w1.scale, a.scale_f16, n + i) : 0.f);
-        }
+        read_scales(a.w0.scale, a.scale_f16, n, a.N, half, s0);
+        if constexpr (MODE == kTwoWeights) read_scales(a.w1.scale, a.scale_f16, n, a.N, half, s1);
 #pragma unroll
         for (int m = 0; m < FM; ++m) {
             const int row = lane_m0 + m * 32;
@@ -710,22 +730,37 @@ int launch_tile(const KernelArgs& a, hipStream_t st)
     return TL_OK;
 }
 
-// Which tile, by what the busiest compute unit has to do.  us, fp16, 128 x 256 ("tall") / 64 x 256 ("flat") / 64 x 64 with K shared out:
-//   up to two 64 x 64 tiles a unit: shared K.  64 x 4096 -> 4096 43 / 29 / 15, 512 x 4096 -> 4096 45 / 30 / 25, 1024 x 2048 -> 2048 27 / 20 / 17;
-//     past that it reads the activations too often: 200 x 4096 -> 11008 45 / 32 / 33, 1536 x 2048 -> 2048 28 / 20 / 25.  fp32 (- / flat /
-//     shared) 200 x 2048 -> 2048 - / 42 / 21, 512 x 4096 -> 4096 - / 75 / 59, 768 x 4096 -> 4096 - / 81 / 87.
+// Which tile, by how many there are and by the units of 256 rows of K (a multiple of the units is shared out evenly).  us, fp16;
+// "shared": 64 x 64, K shared out among four waves; "small": 64 x 64, a wave 32 x 32; "wide": 64 x 128, a wave 64 x 32 (two weights:
+// 32 x 64); "flat": 64 x 256; "tall": 128 x 256, a wave 64 or 128 rows x 64:
+//   up to one 64 x 64 tile a compute unit: shared from four units of K on, small below, where waves would have no unit of their own.
+//     Shared / small / flat, 64 rows -> 4096: K = 256 5.3 / 3.9 / 6.2, 768 5.7 / 5.2 / 8.8, 1024 5.8 / 5.9 / 10.0, 2048 7.4 / 8.6 / 15.3; two weights
+//     (wide) 256 6.3 / 5.1 / 6.5, 512 6.5 / 6.2 / 7.9, 1024 6.8 / 8.0 / 10.5.  fp32 256 11.6 / 9.6 / 12.5, 512 12.1 / 12.1 / 16.4, 768 12.2 / 14.3 / 20.0.
+//   wide up to one of its tiles a unit, and up to two where it still gains.  Shared (which fits a unit once) / wide / flat, 512 rows
+//     -> 4096: K = 256 10.0 / 5.4 / 6.7, 1024 11.2 / 8.3 / 11.0, 4096 23.0 / 22.0 / 27.3; fp32 21.6 / 13.1 / 14.8, 25.8 / 23.1 / 28.1, 61.5 / 58.0 / 75.5.
+//     Wide / flat, 1024 rows -> 4096: 256 7.1 / 7.7, 2048 19.9 / 20.3; fp32 17.4 / 18.6, but 55.0 / 54.8, and 768 rows of 4096 81.9 / 78.4; past that
+//     1024 rows of 1024 -> 11008 28.1 / 26.8; two weights, 768 rows of 2048 -> 2048 20.0 / 17.7.
 //   tall where there are two of them a unit, so that one multiplies while the other waits or stores, and where flat ones would
-//     not spread the rows better: 2048 x 4096 -> 11008 139 / 144, 8192 x 2048 -> 11008 289 / 301, 8192 x 2048 -> 2048 64 / 66, but
-//     1536 x 4096 -> 11008 129 / 117 (516 tall tiles are three for some units, 1032 flat ones five halves).  Not for fp32, whose second
-//     set of sums does not fit.
+//     not spread the rows better: 2048 x 4096 -> 11008 141 / 150, 8192 x 2048 -> 11008 273 / 287, 8192 x 2048 -> 2048 57 / 59, but
+//     1536 x 4096 -> 11008 129 / 117, both with slower last steps (516 tall tiles are three for some units, 1032 flat ones five
+//     halves).  Not for fp32, whose second set of sums does not fit.
 // The rows are the whole call's: a row's result does not depend on how many rows at a time a workspace holds.
 template <int PARTS, int MODE>
 int launch_mode(const KernelArgs& a, hipStream_t st)
 {
-    const int64_t units = compute_units(), columns = (int64_t)a.N * (MODE == kTwoWeights ? 2 : 1);
-    if (ceil_div(a.call_rows, 64) * ceil_div(columns, 64) <= 2 * units) return launch_tile<PARTS, 1, 1, 4, 2, 2, MODE>(a, st);
+    constexpr bool TWO = MODE == kTwoWeights;
+    const int64_t units = compute_units(), columns = (int64_t)a.N * (TWO ? 2 : 1), depth = (int64_t)a.planes * a.units;
+    auto tiles = [&](int rows, int width) { return ceil_div(a.call_rows, rows) * ceil_div(columns, width); };
+    const bool one_each = tiles(64, 64) <= units;
+    if (one_each && depth > (PARTS > 1 ? 1 : TWO ? 2 : 3)) return launch_tile<PARTS, 1, 1, 4, 2, 2, MODE>(a, st);
+    if constexpr (TWO) {
+        if (tiles(64, 128) <= units) return launch_tile<PARTS, 2, 2, 1, 1, 2, MODE>(a, st);
+    } else {
+        if (one_each) return launch_tile<PARTS, 2, 2, 1, 1, 1, MODE>(a, st);
+        if (tiles(64, 128) <= (PARTS == 1 || depth <= 4 ? 2 : 1) * units) return launch_tile<PARTS, 1, 4, 1, 2, 1, MODE>(a, st);
+    }
     if constexpr (PARTS == 1) {
-        const int64_t tall = ceil_div(a.call_rows, 128) * ceil_div(columns, 256), flat = ceil_div(a.call_rows, 64) * ceil_div(columns, 256);
+        const int64_t tall = tiles(128, 256), flat = tiles(64, 256);
         if (tall >= 2 * units && ceil_div(flat, units) >= 2 * ceil_div(tall, units)) return launch_tile<PARTS, 1, 4, 1, 4, 2, MODE>(a, st);
     }
     return launch_tile<PARTS, 1, 4, 1, 2, 2, MODE>(a, st);

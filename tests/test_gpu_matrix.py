@@ -65,6 +65,14 @@ def test_tiles_of_every_shape(cuda, M, K, N, dtype):
     assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())              # exact sums; __expf and the division
 
 
+# few units of K, where one 64 x 64 tile a compute unit is four waves' own 32 x 32 (three units and, beside it, four); one and two 64 x 128
+# tiles a unit (two weights: 32 x 64 a wave); 64 x 256 ones that are not enough for 128 x 256
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M,K,N", [(65, 250, 66), (63, 264, 34), (150, 768, 98), (150, 776, 98), (520, 250, 2058), (520, 1100, 2058), (769, 330, 4090), (2110, 264, 4090)])
+def test_tiles_of_few_units(cuda, M, K, N, dtype):
+    test_tiles_of_every_shape(cuda, M, K, N, dtype)
+
+
 @pytest.mark.parametrize("M,K,N,N2", [(49, 8, 1, 34), (65, 1344, 66, 40), (200, 2048, 1032, 130), (1030, 336, 2100, 66), (4096, 200, 4096, 2048)])
 def test_chained_rows(cuda, M, K, N, N2):
     """More than 48 rows: a product that adds residual rows and leaves the next norm's image and sums of squares, bit for bit as
