@@ -490,11 +490,21 @@ int tl_spmm_chain(const tl_layout_header* header, const void* blob_dev,
  * padding rows).  Up to 48 rows the squares are [blocks][R] with R = 16, 32 or 64 for up to 16, 32 or 48 rows (rows past M are not
  * written and not read).  More rows (X aligned to 16 bytes, K and ldx multiples of 8) leave squares_out [M][ceil(N / 32)], from
  * which tl_row_factors makes the M factors that squares_in points to then.  (image_out is rounded before a row's factor: a value above 65504 / weight
- * is infinite there, and products below fp16's normal range lose bits.)  gated != 0 gives Y the N / 2 values silu(y[2j]) * y[2j + 1].  The product is tl_spmm's for these rows.
+ * is infinite there, and products below fp16's normal range lose bits.  Up to 48 rows squares_out may be asked for alone:
+ * tl_spmm_normed_rows needs no image and has no such limit.)  gated != 0 gives Y the N / 2 values silu(y[2j]) * y[2j + 1].  The product is tl_spmm's for these rows.
  * TL_ERR_UNSUPPORTED for other types, row counts and blobs without codes. */
 int tl_spmm_chain_rows(const tl_layout_header* header, const void* blob_dev,
                        const void* X, int x_dtype, int64_t ldx, int64_t M, void* Y, int y_dtype, int64_t ldy, int gated,
                        const void* scale, int scale_dtype, const tl_chain* chain, void* stream);
+
+/* The product behind a norm for 2 to 48 fp16 rows: Y = (RMSNorm(X) * W) * scale, the rows normalised on their way in --
+ * x * rsqrt(sum of squares / K + eps) * norm_weight, rounded to fp16 once, as tl_add_rmsnorm would store them.  squares:
+ * [squares_blocks][R] as tl_spmm_chain_rows and tl_embed_rows leave them.  X row-major, gated as above.  K and ldx multiples of 8,
+ * X, norm_weight and squares aligned to 16 bytes; TL_ERR_UNSUPPORTED for other types, row counts, layouts and blobs without codes. */
+int tl_spmm_normed_rows(const tl_layout_header* header, const void* blob_dev,
+                        const void* X, int x_dtype, int64_t ldx, int64_t M, void* Y, int y_dtype, int64_t ldy, int gated,
+                        const void* scale, int scale_dtype, const void* norm_weight, const float* squares, int squares_blocks, float eps,
+                        void* stream);
 
 /* factors[r] = rsqrt((sum of squares[r][0 .. blocks)) / width + eps) for `rows` rows. */
 int tl_row_factors(const float* squares, int64_t rows, int blocks, int width, float eps, float* factors, void* stream);
@@ -531,7 +541,7 @@ int tl_spmv_attn_combine_add_norm(const tl_layout_header* header, const void* bl
                                   void* image_out, float* squares_out, void* stream);
 
 /* The start of a decode step in one launch: x[r] = table[token[r]] (negative tokens count from the end; a row of NaN where there
- * is no such row), image[r] = x[r] * norm_weight and squares[b][r] = the sum of x[r]^2 over its values 16 b .. 16 b + 15 -- what a
+ * is no such row), image[r] = x[r] * norm_weight (norm_weight and image may both be NULL) and squares[b][r] = the sum of x[r]^2 over its values 16 b .. 16 b + 15 -- what a
  * chained product leaves for the product behind a norm.  fp16, width a multiple of 16, all rows contiguous and 16-byte
  * aligned; squares: float32 [width / 16][squares_rows], squares_rows >= rows, or, squares_rows == 0, [rows][ceil(width / 32)] by runs
  * of 32 values, as more than 48 chained rows leave them. */

@@ -82,6 +82,7 @@ SIGNATURES = {
     "tl_spmv_fused_gated": (_INT, [_HDRP, _VP, _INT, _VP, _VP, _VP, ctypes.c_float, _VP, _INT, _VP, _INT, _VP, _INT, _VP]),
     "tl_spmm_gated": (_INT, [_HDRP, _VP, _VP, _INT, _INT, _I64, _I64, _VP, _INT, _I64, _INT, _VP, _INT, _VP, _I64, _VP]),
     "tl_spmm_chain_rows": (_INT, [_HDRP, _VP, _VP, _INT, _I64, _I64, _VP, _INT, _I64, _INT, _VP, _INT, ctypes.POINTER(Chain), _VP]),
+    "tl_spmm_normed_rows": (_INT, [_HDRP, _VP, _VP, _INT, _I64, _I64, _VP, _INT, _I64, _INT, _VP, _INT, _VP, _VP, _INT, ctypes.c_float, _VP]),
     "tl_spmm_chain": (_INT, [_HDRP, _VP, _VP, _INT, _INT, _I64, _I64, _VP, _INT, _I64, _INT, _VP, _INT, ctypes.POINTER(Chain), _VP, _I64, _VP]),
     "tl_mlp_gate_up": (_INT, [_HDRP, _VP, _HDRP, _VP, _VP, _INT, _INT, _I64, _I64, _VP, _INT, _I64, _VP, _VP, _INT, _INT,
                               _VP, _I64, _VP]),

@@ -859,8 +859,8 @@ extern "C" int tl_decode_attention_fold(const void* q, const void* qkv, const vo
                      pos_dev, out, out_kmajor_ld, splits, workspace, workspace_bytes, stream, arrivals);
 }
 
-// The start of a decode step: a token's row of the embedding table and what the first norm's product wants of it (the row times
-// the norm's weight, and its sums of squares).  A few KB a row: bound by the launch, 1.6 us of it in a graph, and by three trips to
+// The start of a decode step: a token's row of the embedding table and what the first norm's product wants of it (its sums of
+// squares and, for one row, the row times the norm's weight).  A few KB a row: bound by the launch, 1.6 us of it in a graph, and by three trips to
 // memory in a row (token, row, stores); a lane takes 16 bytes, two lanes a block of 16.  One launch in the place of a gather (3.0 us
 // in a step of 16 rows) and a norm (3.6).
 namespace {
@@ -873,7 +873,7 @@ __global__ __launch_bounds__(256) void tl_embed_rows_k(const __half* __restrict_
     long long t = token[row];
     if (t < 0) t += vocab;
     __align__(16) __half v[8], w[8], o[8];
-    *reinterpret_cast<uint4*>(w) = *reinterpret_cast<const uint4*>(norm_w + k);
+    if (image) *reinterpret_cast<uint4*>(w) = *reinterpret_cast<const uint4*>(norm_w + k);
     if (t >= 0 && t < vocab) *reinterpret_cast<uint4*>(v) = *reinterpret_cast<const uint4*>(table + t * width + k);
     else
         for (int i = 0; i < 8; ++i) v[i] = __float2half(__builtin_nanf(""));   // (no such row: nothing is read, and the result says so)
@@ -882,10 +882,10 @@ __global__ __launch_bounds__(256) void tl_embed_rows_k(const __half* __restrict_
     for (int i = 0; i < 8; ++i) {
         const float f = __half2float(v[i]);
         sum = fmaf(f, f, sum);
-        o[i] = __float2half(f * __half2float(w[i]));
+        if (image) o[i] = __float2half(f * __half2float(w[i]));
     }
     *reinterpret_cast<uint4*>(x + (long long)row * width + k) = *reinterpret_cast<const uint4*>(v);
-    *reinterpret_cast<uint4*>(image + (long long)row * width + k) = *reinterpret_cast<const uint4*>(o);
+    if (image) *reinterpret_cast<uint4*>(image + (long long)row * width + k) = *reinterpret_cast<const uint4*>(o);
     sum += lane_permuted<0xB1>(sum);   // (the neighbouring lane's)
     if (squares_rows > 0) {
         if (threadIdx.x % 2 == 0) squares[(long long)(k / 16) * squares_rows + row] = sum;
@@ -900,7 +900,8 @@ extern "C" int tl_embed_rows(const void* table, int dtype, int64_t vocab, int wi
                              void* x, void* image, float* squares, int squares_rows, void* stream)
 {
     if (dtype != TL_F16) return fail(TL_ERR_UNSUPPORTED, "embedding rows are read as fp16");
-    if (!table || !token || !norm_weight || !x || !image || !squares) return fail(TL_ERR_ARG, "device pointer is null");
+    if (!table || !token || !x || !squares) return fail(TL_ERR_ARG, "device pointer is null");
+    if (!norm_weight != !image) return fail(TL_ERR_ARG, "norm_weight and image come together");
     if (rows <= 0 || rows > 65535 || vocab <= 0 || width <= 0 || width % 16 || (squares_rows != 0 && squares_rows < rows))
         return fail(TL_ERR_SHAPE, "rows=%lld (1 .. 65535, at most squares_rows=%d where that is not 0), width=%d (a multiple of 16), vocab=%lld", (long long)rows, squares_rows, width,
                     (long long)vocab);

@@ -72,10 +72,22 @@ __device__ __forceinline__ void split8(const float* v, u32x4* part)
     }
 }
 
-// The last steps of a call: none; one block of each of two weights, silu(gate) * up; and what a decoder layer does around a
-// product (tl_spmm_chain_rows, tl_spmm_gated), by the argument block: the rows' normalisation factors, the gate of column
-// pairs, the residual rows, the next norm's image and sums of squares.
-enum { kPlain = 0, kTwo = 1, kSteps = 2 };
+// What a call does besides the product: nothing; one block of each of two weights, silu(gate) * up; what a decoder layer does
+// around a product (tl_spmm_chain_rows, tl_spmm_gated), by the argument block: the rows' normalisation factors, the gate of column
+// pairs, the residual rows, the next norm's image and sums of squares; and the norm of the rows on their way in
+// (tl_spmm_normed_rows), with the gate by the argument block.
+enum { kPlain = 0, kTwo = 1, kSteps = 2, kNormed = 3 };
+
+// Eight activations times their row's factor times the norm's weights, in fp32, then rounded to fp16: five instructions for two
+// (v_fma_mix_f32 takes fp16 factors as they are).
+__device__ __forceinline__ u32x4 normed8(u32x4 x, float factor, u32x4 w)
+{
+    const half8 xs = __builtin_bit_cast(half8, x), ws = __builtin_bit_cast(half8, w);
+    half8 out;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) out[i] = (_Float16)__builtin_fmaf(__builtin_fmaf((float)xs[i], factor, 0.f), (float)ws[i], 0.f);
+    return __builtin_bit_cast(u32x4, out);
+}
 
 // Rows that the sums of squares of M rows have room for: a lane's four are the same in every block it reads.
 constexpr __host__ __device__ int squares_rows(int M) { return M <= 16 ? 16 : M <= 32 ? 32 : 64; }
@@ -113,9 +125,9 @@ constexpr __host__ __device__ int wave_floats() { return std::max(C * FM * kPart
 template <typename XT, int IN, int FM, int C, int Q, int STEPS>
 __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_waves(C, stage_bytes<XT, IN, FM>(1)) : kMaxWaves)) void tl_matrix_few(KernelArgs a)
 {
-    constexpr bool F32 = sizeof(XT) == 4, TWO = STEPS == kTwo;
+    constexpr bool F32 = sizeof(XT) == 4, TWO = STEPS == kTwo, NORMED = STEPS == kNormed;
     constexpr int kTurnsOfUnit = TL_CODE_UNIT_ROWS / (kSliceRows * Q);
-    // [wave] its stage of activations (kStaged, kRows), where its sums [C][FM][kPartFloats] lie afterwards; and, kSteps, [wave][SR] sums of squares
+    // [wave] its stage of activations (kStaged, kRows), where its sums [C][FM][kPartFloats] lie afterwards; and, kSteps and kNormed, [wave][SR] sums of squares
     extern __shared__ __align__(16) float sums[];
     constexpr int OWN = wave_floats<XT, IN, FM, C, Q>();
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -144,7 +156,7 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
     // What the last steps need is asked for now, for a thread's first output (its only one, mostly).  Squares lie as [block of
     // 16][SR rows], pieces of four rows.
     constexpr int SR = squares_rows(FM * 16), U = FM == 3 ? 4 : 2, COLS = TWO ? 16 : C * 16;
-    const bool pairs = STEPS == kSteps && a.gated;
+    const bool pairs = STEPS >= kSteps && a.gated;
     const int first_m = (int)threadIdx.x / (pairs ? COLS / 2 : COLS), first_col = pairs ? (int)threadIdx.x % (COLS / 2) * 2 : (int)threadIdx.x % COLS;
     const int first_n = nb0 * 16 + first_col;
     uint32_t early_scale[2] = {0u, 0u};
@@ -154,9 +166,9 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
         if (TWO) early_scale[1] = raw_value(a.w1.scale, a.scale_f16, first_n);
     }
     [[maybe_unused]] float4 squares[U];
-    const int square_pieces = STEPS == kSteps && a.chain_sq_in ? a.chain_sq_blocks * (SR / 4) : 0;
+    const int square_pieces = STEPS >= kSteps && a.chain_sq_in ? a.chain_sq_blocks * (SR / 4) : 0;
     [[maybe_unused]] uint32_t early_residual = 0, early_weight = 0;
-    if constexpr (STEPS == kSteps) {
+    if constexpr (STEPS >= kSteps) {
         const float4* pieces = reinterpret_cast<const float4*>(a.chain_sq_in);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -174,6 +186,7 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
     struct Turn {
         uint32_t w[C][4];
         XT x[STAGED ? 1 : Q * 2][FM][8] __attribute__((aligned(16)));
+        u32x4 norm[NORMED ? Q * 2 : 1];   // the norm's weights
     };
     // kStaged: a load takes whole slices (128 or 256 bytes) of 8 or 4 rows.  A row's pieces lie rotated so that 16 lanes that
     // read one piece of 16 rows find them on different banks.
@@ -248,20 +261,46 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
             else if constexpr (Q == 2) *reinterpret_cast<uint2*>(to.w[c]) = *reinterpret_cast<const uint2*>(src);
             else to.w[c][0] = *reinterpret_cast<const uint32_t*>(src);
         }
-        if constexpr (IN == kStaged) {
-            stage(t);
-            asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-            return;
+        const int k0 = (unit % a.units) * TL_CODE_UNIT_ROWS + part * Q * kSliceRows + g * 8;
+        if constexpr (NORMED) {
+#pragma unroll
+            for (int s = 0; s < Q * 2; ++s) to.norm[s] = *reinterpret_cast<const u32x4*>(static_cast<const _Float16*>(a.norm_w) + min(k0 + s * 32, a.K - 8));
         }
-        if constexpr (IN == kRows) stage_any(t);
+        if constexpr (IN == kStaged) stage(t);
+        else if constexpr (IN == kRows) stage_any(t);
         else {
-            const int k0 = (unit % a.units) * TL_CODE_UNIT_ROWS + part * Q * kSliceRows + g * 8;
 #pragma unroll
             for (int s = 0; s < Q * 2; ++s)
 #pragma unroll
                 for (int f = 0; f < FM; ++f) load8<XT, IN>(a, rows[f], k0 + s * 32, to.x[s][f]);
         }
     };
+    auto arrived = [] {
+        if constexpr (IN == kStaged) asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+    };
+    [[maybe_unused]] float* wave_squares = sums + waves * OWN;
+    auto add_squares = [&] {                                       // into wave_squares
+        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+        auto add = [&](const float4& v) { sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w; };
+#pragma unroll
+        for (int u = 0; u < U; ++u) add(squares[u]);
+        for (int i = (int)threadIdx.x + U * (int)blockDim.x; i < square_pieces; i += (int)blockDim.x) add(reinterpret_cast<const float4*>(a.chain_sq_in)[i]);
+        for (float* v : {&sum.x, &sum.y, &sum.z, &sum.w}) *v = sum_over_lanes<SR / 4, 64>(*v);   // the lanes with the same rows
+        if (lane < SR / 4) reinterpret_cast<float4*>(wave_squares + wave * SR)[lane] = sum;
+    };
+    // (All waves' sums are read at once: one after the other each is a trip to LDS.)
+    auto over_waves = [&](const float* s, int stride) {
+        constexpr int MOST = most_waves(C, stage_bytes<XT, IN, FM>(Q));
+        float part[MOST];
+#pragma unroll
+        for (int i = 0; i < MOST; ++i) part[i] = s[min(i, waves - 1) * stride];
+        std::conditional_t<F32, double, float> v = 0;  // (fp32: sixteen more roundings would be the largest part of the error)
+#pragma unroll
+        for (int i = 0; i < MOST; ++i) v += i < waves ? part[i] : 0.f;
+        return (float)v;
+    };
+    auto row_factor = [&](int m) { return rsqrtf(over_waves(wave_squares + m, SR) * (1.0f / (float)a.K) + a.eps); };
+    [[maybe_unused]] float factors[FM];                            // (kNormed: of the rows of this lane's operands)
     auto multiply = [&](const Turn& turn) {
 #pragma unroll
         for (int s = 0; s < Q * 2; ++s) {
@@ -276,6 +315,7 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
                 XT x[8] __attribute__((aligned(16)));
                 if constexpr (STAGED) staged(s, f, x);
                 else __builtin_memcpy(x, turn.x[s][f], sizeof(x));
+                if constexpr (NORMED) *reinterpret_cast<u32x4*>(x) = normed8(*reinterpret_cast<const u32x4*>(x), factors[f], turn.norm[s]);
                 if constexpr (F32) {
                     u32x4 p[3];
                     split8(x, p);
@@ -293,10 +333,26 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
             }
         }
     };
-    for (int t = wave; t < turns; t += waves) {
+    if constexpr (NORMED) {
+        // the factors are needed before the first product: what the first turn reads is on its way while they meet
         Turn turn;
-        load(t, turn);
-        multiply(turn);
+        if (wave < turns) load(wave, turn);
+        add_squares();
+        __syncthreads();
+#pragma unroll
+        for (int f = 0; f < FM; ++f) factors[f] = row_factor(f * 16 + r16);
+        for (int t = wave; t < turns; t += waves) {
+            if (t != wave) load(t, turn);
+            arrived();
+            multiply(turn);
+        }
+    } else {
+        for (int t = wave; t < turns; t += waves) {
+            Turn turn;
+            load(t, turn);
+            arrived();
+            multiply(turn);
+        }
     }
 #pragma unroll
     for (int c = 0; c < C; ++c)
@@ -305,41 +361,26 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
             if constexpr (F32) add_low(acc[c][f], low[c][f]);
             *reinterpret_cast<f32x4*>(sums + wave * OWN + (c * FM + f) * kPartFloats + lane * 4 + g * 16) = acc[c][f];
         }
-    [[maybe_unused]] float* wave_squares = sums + waves * OWN;
-    if (square_pieces) {
-        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-        auto add = [&](const float4& v) { sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w; };
-#pragma unroll
-        for (int u = 0; u < U; ++u) add(squares[u]);
-        for (int i = (int)threadIdx.x + U * (int)blockDim.x; i < square_pieces; i += (int)blockDim.x) add(reinterpret_cast<const float4*>(a.chain_sq_in)[i]);
-        for (float* v : {&sum.x, &sum.y, &sum.z, &sum.w}) *v = sum_over_lanes<SR / 4, 64>(*v);   // the lanes with the same rows
-        if (lane < SR / 4) reinterpret_cast<float4*>(wave_squares + wave * SR)[lane] = sum;
-    }
+    if (STEPS == kSteps && square_pieces) add_squares();
     __syncthreads();
 
-    // one output after the other, 16 neighbouring columns of a row to 16 neighbouring threads.  (All waves' sums are read at
-    // once: one after the other each is a trip to LDS.)
-    auto over_waves = [&](const float* s, int stride) {
-        constexpr int MOST = most_waves(C, stage_bytes<XT, IN, FM>(Q));
-        float part[MOST];
-#pragma unroll
-        for (int i = 0; i < MOST; ++i) part[i] = s[min(i, waves - 1) * stride];
-        std::conditional_t<F32, double, float> v = 0;  // (fp32: sixteen more roundings would be the largest part of the error)
-#pragma unroll
-        for (int i = 0; i < MOST; ++i) v += i < waves ? part[i] : 0.f;
-        return (float)v;
-    };
+    // one output after the other, 16 neighbouring columns of a row to 16 neighbouring threads
     auto output = [&](const WeightPtrs& w, int c, int m, int n, uint32_t early, bool first) {
         const int col = n & 15;
         float v = 0.5f * over_waves(sums + (c * FM + (m >> 4)) * kPartFloats + (col >> 2) * 80 + (m & 15) * 4 + (col & 3), OWN);
-        if (!(fabsf(v) < __builtin_huge_valf())) v = walk_column(w, a.T, a.tile_rows, n, callers_x(a, m));
+        if (!(fabsf(v) < __builtin_huge_valf())) {
+            const CallersX x = callers_x(a, m);
+            if constexpr (NORMED) {
+                const float factor = row_factor(m);
+                v = walk_column(w, a.T, a.tile_rows, n, [&](int k) { return as_output(x(k) * factor * value_of(raw_value(a.norm_w, 1, k), 1), 1); });
+            } else {
+                v = walk_column(w, a.T, a.tile_rows, n, x);
+            }
+        }
         return w.scale ? v * value_of(first ? early : raw_value(w.scale, a.scale_f16, n), a.scale_f16) : v;
     };
-    if constexpr (STEPS == kSteps) {
-        auto factor = [&](int m) {
-            if (!square_pieces) return 1.0f;
-            return rsqrtf(over_waves(wave_squares + m, SR) * (1.0f / (float)a.K) + a.eps);
-        };
+    if constexpr (STEPS >= kSteps) {
+        auto factor = [&](int m) { return NORMED || !square_pieces ? 1.0f : row_factor(m); };
         if (a.gated) {
             // column pairs; a K-major image's rows past M are zeroed
             const int rows = a.y_kld ? (int)a.y_kld : a.M;
@@ -368,7 +409,7 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
                 store_out(a.Y, 1, m * a.ldy + n, v);
                 if (a.chain_image) store_out(a.chain_image, 1, m * a.chain_ild + n, v * value_of(first ? early_weight : raw_value(a.chain_w, 1, n), 1));
             }
-            if (a.chain_image) {
+            if (a.chain_sq_out) {
                 const float square = sum_over_lanes<1, 16>(v * v);
                 if (col % 16 == 0 && n < a.N) a.chain_sq_out[(nb0 + (col >> 4)) * SR + m] = square;
             }
@@ -398,7 +439,7 @@ int launch_few(const KernelArgs& a, hipStream_t st)
     const dim3 grid((unsigned)(STEPS == kTwo ? a.NB : ceil_div(a.NB, C))), block((unsigned)waves * 64);
     auto launch = [&](auto q_tag) {
         constexpr int Q = decltype(q_tag)::value;
-        const size_t lds = (size_t)waves * (wave_floats<XT, IN, FM, C, Q>() + (STEPS == kSteps ? squares_rows(FM * 16) : 0)) * sizeof(float);
+        const size_t lds = (size_t)waves * (wave_floats<XT, IN, FM, C, Q>() + (STEPS >= kSteps ? squares_rows(FM * 16) : 0)) * sizeof(float);
         auto kernel = tl_matrix_few<XT, IN, FM, C, Q, STEPS>;
         if (IN == kStaged || IN == kRows) {
             static std::atomic<bool> raised{false};  // per instantiation; a repeated call is harmless
@@ -423,8 +464,11 @@ int launch_few_columns(const KernelArgs& a, bool two_weights, hipStream_t st)
     // compute units (fp16, us with one / two: 8 rows 4096 -> 4096 at 95 % zeros 5.2 / 5.4, 2048 -> 5504 5.2 / 4.3,
     // 4096 -> 11008 9.7 / 8.0; 48 rows 13.7 / 14.5, 13.8 / 9.2, 36 / 26).
     const bool pairs = a.NB > compute_units();
+    if constexpr (sizeof(XT) == 2 && (IN == kStaged || (IN == kRowPieces && FM == 1))) {
+        if (a.norm_w) return pairs ? launch_few<XT, IN, FM, 2, kNormed>(a, st) : launch_few<XT, IN, FM, 1, kNormed>(a, st);
+    }
     if constexpr (sizeof(XT) == 2) {
-        if (a.gated || a.chain_res || a.chain_image || a.chain_sq_in) return pairs ? launch_few<XT, IN, FM, 2, kSteps>(a, st) : launch_few<XT, IN, FM, 1, kSteps>(a, st);
+        if (a.gated || a.chain_res || a.chain_sq_out || a.chain_sq_in) return pairs ? launch_few<XT, IN, FM, 2, kSteps>(a, st) : launch_few<XT, IN, FM, 1, kSteps>(a, st);
     }
     return pairs ? launch_few<XT, IN, FM, 2, kPlain>(a, st) : launch_few<XT, IN, FM, 1, kPlain>(a, st);
 }
@@ -437,6 +481,8 @@ int launch_few_in(const KernelArgs& a, bool two_weights, hipStream_t st)
     return launch_few_columns<XT, IN, 3>(a, two_weights, st);
 }
 
+constexpr int64_t kMostStagedLd = 1 << 24;   // (a lane's byte offset inside 48 rows has 32 bits)
+
 template <typename XT>
 int launch_few_type(const KernelArgs& a, bool pieces, bool two_weights, hipStream_t st)
 {
@@ -445,7 +491,7 @@ int launch_few_type(const KernelArgs& a, bool pieces, bool two_weights, hipStrea
     // 5504 -> 2048, 11008 -> 4096): fp16 2 rows 3.2 / 3.3, 4.4 / 4.5, 6.6 / 6.5; 4 rows 3.5 / 3.4, 4.8 / 4.4, 7.4 / 6.2; 16 rows
     // 4.6 / 3.7, 7.7 / 4.7, 12.7 / 7.2; 48 rows 9.2 / 6.8, 17.7 / 8.9, 31.6 / 16.2; fp32 4 rows 5.0 / 5.7, 8.1 / 8.0, 13.1 / 14.1;
     // 8 rows 5.3 / 5.8, 9.5 / 8.3, 15.9 / 14.4; 16 rows 6.9 / 6.1, 13.0 / 8.3, 22.8 / 14.8.  (A lane's offset has 32 bits.)
-    if (pieces && a.M >= (sizeof(XT) == 2 ? 4 : 8) && a.ldx <= 1 << 24) return launch_few_in<XT, kStaged>(a, two_weights, st);
+    if (pieces && a.M >= (sizeof(XT) == 2 ? 4 : 8) && a.ldx <= kMostStagedLd) return launch_few_in<XT, kStaged>(a, two_weights, st);
     return pieces ? launch_few_in<XT, kRowPieces>(a, two_weights, st) : launch_few_in<XT, kRows>(a, two_weights, st);
 }
 
@@ -454,10 +500,12 @@ int launch_few_type(const KernelArgs& a, bool pieces, bool two_weights, hipStrea
 int tl::launch_matrix_few(KernelArgs a, int x_dtype, bool two_weights, hipStream_t st)
 {
     const int es = x_dtype == TL_F16 ? 2 : 4;
-    const bool steps = a.gated || a.chain_res || a.chain_image || a.chain_sq_in;
+    const bool steps = a.gated || a.chain_res || a.chain_sq_out || a.chain_sq_in;
     if (steps && x_dtype != TL_F16) return fail(TL_ERR_UNSUPPORTED, "the gated and chained steps of few rows are for fp16 activations");
     a.x_sm = a.x_kmajor ? 1 : a.ldx;
     a.x_sk = a.x_kmajor ? a.ldx : 1;
     const bool pieces = a.K % 8 == 0 && (a.M == 1 || (a.ldx * es) % 16 == 0) && reinterpret_cast<uintptr_t>(a.X) % 16 == 0;
+    if (a.norm_w && (!pieces || a.ldx > kMostStagedLd || reinterpret_cast<uintptr_t>(a.norm_w) % 16))
+        return fail(TL_ERR_UNSUPPORTED, "rows that are normalised on their way in, and the norm's weight, are read in aligned pieces of 16 bytes");
     return x_dtype == TL_F16 ? launch_few_type<_Float16>(a, pieces, two_weights, st) : launch_few_type<float>(a, pieces, two_weights, st);
 }

@@ -242,6 +242,33 @@ extern "C" int tl_spmm_chain(const tl_layout_header* header, const void* blob_de
     return spmm_call(header, blob_dev, X, x_dtype, x_layout, ldx, M, Y, y_dtype, ldy, y_layout, scale, scale_dtype, workspace, workspace_bytes, stream, chain);
 }
 
+namespace {
+// The argument block of a row-major product without a workspace, of checked arguments.
+KernelArgs rows_call(const tl_layout_header* h, const void* blob_dev, const void* X, int x_dtype, int64_t ldx, int64_t M, void* Y, int y_dtype, int64_t ldy,
+                     int gated, const void* scale, int scale_dtype)
+{
+    KernelArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.w0 = weight_ptrs(h, blob_dev, scale);
+    a.X = X; a.Y = Y;
+    a.ldx = ldx; a.ldy = ldy;
+    a.M = (int)M; a.N = (int)h->columns; a.K = (int)h->inners; a.T = (int)h->n_tiles; a.tile_rows = (int)h->tile_rows;
+    a.NB = (int)h->n_blocks; a.c0 = weight_codes(h, blob_dev); a.units = (int)h->code_units; a.planes = a.c0.planes;
+    a.x_f16 = x_dtype == TL_F16; a.y_f16 = y_dtype == TL_F16; a.scale_f16 = scale_dtype == TL_F16;
+    a.one = 1.0f;
+    a.gated = gated != 0;
+    return a;
+}
+
+int check_gated_rows(const tl_layout_header* h, int gated, int64_t ldy)
+{
+    const int64_t N = h->columns;
+    if (gated && N % 2) return fail(TL_ERR_SHAPE, "N=%lld: gate and up columns come in pairs", (long long)N);
+    if (gated && ldy < N / 2) return fail(TL_ERR_SHAPE, "ldy=%lld smaller than %lld", (long long)ldy, (long long)(N / 2));
+    return TL_OK;
+}
+}  // namespace
+
 extern "C" int tl_spmm_chain_rows(const tl_layout_header* header, const void* blob_dev,
                                   const void* X, int x_dtype, int64_t ldx, int64_t M, void* Y, int y_dtype, int64_t ldy, int gated,
                                   const void* scale, int scale_dtype, const tl_chain* chain, void* stream)
@@ -250,32 +277,22 @@ extern "C" int tl_spmm_chain_rows(const tl_layout_header* header, const void* bl
     if (!chain) return fail(TL_ERR_ARG, "chain is null");
     const int64_t N = header->columns;
     if (int rc = check_io(blob_dev, X, Y, x_dtype, TL_X_ROW_MAJOR, ldx, M, y_dtype, gated ? N : ldy, scale, scale_dtype, header)) return rc;
-    if (gated && N % 2) return fail(TL_ERR_SHAPE, "N=%lld: gate and up columns come in pairs", (long long)N);
-    if (gated && ldy < N / 2) return fail(TL_ERR_SHAPE, "ldy=%lld smaller than %lld", (long long)ldy, (long long)(N / 2));
+    if (int rc = check_gated_rows(header, gated, ldy)) return rc;
     const bool few = M <= kSmallMaxM;
     if (M < 2 || x_dtype != TL_F16 || y_dtype != TL_F16 || !header->off_codes)
         return fail(TL_ERR_UNSUPPORTED, "products chained row by row are for 2 and more fp16 rows and blobs with codes");
-    const bool out = chain->next_norm_weight || chain->image_out || chain->squares_out;
-    if (out && !(chain->next_norm_weight && chain->image_out && chain->squares_out))
-        return fail(TL_ERR_ARG, "next_norm_weight, image_out and squares_out come together");
+    const bool image = chain->next_norm_weight || chain->image_out, out = image || chain->squares_out;
+    if (out && !(chain->squares_out && (!image || (chain->next_norm_weight && chain->image_out)) && (few || image)))
+        return fail(TL_ERR_ARG, "next_norm_weight, image_out and squares_out come together, or squares_out alone for up to %d rows", kSmallMaxM);
     if ((out || chain->residual) && gated) return fail(TL_ERR_ARG, "a gated product has no residual or image epilogue");
     if (chain->residual && chain->residual_ld < N) return fail(TL_ERR_SHAPE, "residual_ld=%lld smaller than N", (long long)chain->residual_ld);
-    if (out && chain->image_ld < N) return fail(TL_ERR_SHAPE, "image_ld=%lld smaller than N", (long long)chain->image_ld);
+    if (image && chain->image_ld < N) return fail(TL_ERR_SHAPE, "image_ld=%lld smaller than N", (long long)chain->image_ld);
     if (few && chain->squares_in && chain->squares_blocks <= 0) return fail(TL_ERR_ARG, "squares_blocks must be positive");
     for (const void* p : {chain->residual, chain->next_norm_weight, static_cast<const void*>(chain->image_out)})
         if (reinterpret_cast<uintptr_t>(p) % 2) return fail(TL_ERR_ALIGN, "residual, next_norm_weight and image_out must be aligned to y_dtype");
     for (const void* p : {static_cast<const void*>(chain->squares_out), static_cast<const void*>(chain->squares_in)})
         if (reinterpret_cast<uintptr_t>(p) % 16) return fail(TL_ERR_ALIGN, "squares_out and squares_in must be 16-byte aligned");
-    KernelArgs a;
-    std::memset(&a, 0, sizeof(a));
-    a.w0 = weight_ptrs(header, blob_dev, scale);
-    a.X = X; a.Y = Y;
-    a.ldx = ldx; a.ldy = ldy;
-    a.M = (int)M; a.N = (int)N; a.K = (int)header->inners; a.T = (int)header->n_tiles; a.tile_rows = (int)header->tile_rows;
-    a.NB = (int)header->n_blocks; a.c0 = weight_codes(header, blob_dev); a.units = (int)header->code_units; a.planes = a.c0.planes;
-    a.x_f16 = a.y_f16 = 1; a.scale_f16 = scale_dtype == TL_F16;
-    a.one = 1.0f;
-    a.gated = gated != 0;
+    KernelArgs a = rows_call(header, blob_dev, X, x_dtype, ldx, M, Y, y_dtype, ldy, gated, scale, scale_dtype);
     a.chain_res = chain->residual; a.chain_ldres = chain->residual_ld;
     a.chain_w = chain->next_norm_weight; a.chain_image = chain->image_out; a.chain_ild = chain->image_ld; a.chain_sq_out = chain->squares_out;
     a.chain_sq_in = chain->squares_in; a.chain_sq_blocks = chain->squares_blocks; a.eps = chain->eps;
@@ -286,6 +303,25 @@ extern "C" int tl_spmm_chain_rows(const tl_layout_header* header, const void* bl
         a.chain_sq_in = nullptr;
     }
     if (int rc = few ? launch_matrix_few(a, x_dtype, false, st) : launch_matrix_rows(a, x_dtype, nullptr, 0, false, st)) return rc;
+    return finish_launch();
+}
+
+extern "C" int tl_spmm_normed_rows(const tl_layout_header* header, const void* blob_dev,
+                                   const void* X, int x_dtype, int64_t ldx, int64_t M, void* Y, int y_dtype, int64_t ldy, int gated,
+                                   const void* scale, int scale_dtype, const void* norm_weight, const float* squares, int squares_blocks, float eps,
+                                   void* stream)
+{
+    if (int rc = check_header(header)) return rc;
+    if (int rc = check_io(blob_dev, X, Y, x_dtype, TL_X_ROW_MAJOR, ldx, M, y_dtype, gated ? (int64_t)header->columns : ldy, scale, scale_dtype, header)) return rc;
+    if (int rc = check_gated_rows(header, gated, ldy)) return rc;
+    if (!norm_weight || !squares) return fail(TL_ERR_ARG, "norm_weight or squares is null");
+    if (squares_blocks <= 0) return fail(TL_ERR_ARG, "squares_blocks must be positive");
+    if (reinterpret_cast<uintptr_t>(squares) % 16) return fail(TL_ERR_ALIGN, "squares must be 16-byte aligned");
+    if (M < 2 || M > kSmallMaxM || x_dtype != TL_F16 || y_dtype != TL_F16 || !header->off_codes)
+        return fail(TL_ERR_UNSUPPORTED, "rows are normalised on their way in for 2 to %d fp16 rows and blobs with codes", kSmallMaxM);
+    KernelArgs a = rows_call(header, blob_dev, X, x_dtype, ldx, M, Y, y_dtype, ldy, gated, scale, scale_dtype);
+    a.norm_w = norm_weight; a.chain_sq_in = squares; a.chain_sq_blocks = squares_blocks; a.eps = eps;
+    if (int rc = launch_matrix_few(a, x_dtype, false, static_cast<hipStream_t>(stream))) return rc;
     return finish_launch();
 }
 

@@ -279,12 +279,16 @@ class TernaryLlamaDecoder(nn.Module):
         c = self.config
         B = token.shape[0]
         eps = c.rms_norm_eps
-        chained = self.fused_decode and self.row_chain if B == 1 else B <= 48 and self.chain_decode and self._products_as_built()
-        if chained and self.dtype == torch.float16 and c.hidden_size % 16 == 0 and len(self.layers) > 0 and token.dtype == torch.int64:
-            # the tokens' rows and what the first norm's product wants of them in one launch
-            x, image, squares = ops.embed_rows(self.embed_tokens, token.contiguous(), self.layers[0].input_layernorm.weight)
+        if B == 1:
+            chained, first = self.fused_decode and self.row_chain, self.layers[0].input_layernorm.weight if len(self.layers) else None
         else:
-            x, image, squares = self.embed_tokens[token], None, None
+            chained, first = B <= 48 and self.chain_decode and self._products_as_built() and self._norms_as_built(), None
+        x = image = squares = None
+        if chained and self._embeds_rows(token, first):
+            # the tokens' rows and what the first norm's product wants of them in one launch
+            x, image, squares = ops.embed_rows(self.embed_tokens, token.contiguous(), first)
+        else:
+            x = self.embed_tokens[token]
         if B == 1 and self.fused_decode:
             while self.row_chain:
                 try:
@@ -297,9 +301,9 @@ class TernaryLlamaDecoder(nn.Module):
                     else:
                         self.row_chain = False  # then without the chain
             return self._decode_step_fused(x, pos)
-        if B > 1 and chained:
+        if B > 1 and chained and squares is not None:
             try:
-                return self._decode_step_chain(x, pos, image, squares)
+                return self._decode_step_chain(x, pos, squares)
             except RuntimeError as e:
                 if "TL_ERR_UNSUPPORTED" not in str(e) or torch.cuda.is_current_stream_capturing():
                     raise
@@ -320,27 +324,32 @@ class TernaryLlamaDecoder(nn.Module):
             x, h = ops.add_rmsnorm(x, y, nxt, eps, kmajor=km)  # the residual add, and the norm the next layer (or the head) starts with
         return self.lm_head(h)
 
-    def _decode_step_chain(self, x, pos, h=None, squares=None):
-        """2 to 48 rows, five launches per layer, none of them elementwise: the o and down projections add the residual
-        rows and leave the next norm's image (rows * norm weight) and sums of squares; q|k|v, gate|up (SiLU gate in
-        its epilogue) and the head apply the normalisation factor to their sums.  h and squares: the image of x and
-        its sums of squares as embed_rows left them (the very first norm has a kernel of its own without).  All products are tl_matrix_few's: a step of 16 rows (two layers of 2048 / 5504, 512 cached) took
-        187 us while they walked the index stream."""
-        eps = self.config.rms_norm_eps
-        if h is None:
-            _, h = ops.add_rmsnorm(x, None, self.layers[0].input_layernorm.weight, eps)
+    def _embeds_rows(self, token, norm_weight):
+        """Whether the kernel that starts a chained step reads this table, these tokens and this norm's weight."""
+        table = self.embed_tokens
+        return (self.dtype == torch.float16 and len(self.layers) > 0 and table.shape[1] % 16 == 0 and token.dtype == torch.int64 and
+                all(t.device == token.device and t.dtype == self.dtype and t.is_contiguous() and t.data_ptr() % 16 == 0
+                    for t in (table, norm_weight) if t is not None))
 
-        def product(linear, rows, **steps):
-            return ops.spmm_chain_rows(linear.device_weight(), rows, linear.w_scale, eps=eps, **steps)
+    def _decode_step_chain(self, x, pos, squares):
+        """2 to 48 rows, five launches per layer, none of them elementwise: the o and down projections add the residual rows and
+        leave their sums of squares (as embed_rows does for the first rows); q|k|v, gate|up (SiLU gate in its epilogue) and the
+        head normalise the rows as they read them.  (While the rows times the norm's weight were made by the product in front,
+        rounded before the factor, entries above 65504 / weight became infinite.)  All products are tl_matrix_few's: a step of
+        16 rows (two layers of 2048 / 5504, 512 cached) took 169 us while they walked the index stream."""
+        def behind_norm(linear, norm, **steps):
+            return ops.spmm_normed_rows(linear.device_weight(), x, norm.weight, squares, norm.eps, linear.w_scale, **steps)
+
+        def onto_rows(linear, rows):
+            return ops.spmm_chain_rows(linear.device_weight(), rows, linear.w_scale, residual=x, squares_out=True)
 
         for li, layer in enumerate(self.layers):
-            qkv = product(layer.qkv_proj, h, squares_in=squares)
+            qkv = behind_norm(layer.qkv_proj, layer.input_layernorm)
             a = self._attend(qkv, self._cache[li, 0], self._cache[li, 1], pos, False)
-            x, h, squares = product(layer.o_proj, a.view(x.shape), residual=x, next_norm_weight=layer.post_attention_layernorm.weight)
-            gated = product(layer.gate_up_proj, h, squares_in=squares, gated=True)
-            nxt = self.layers[li + 1].input_layernorm.weight if li + 1 < len(self.layers) else self.norm.weight
-            x, h, squares = product(layer.down_proj, gated, residual=x, next_norm_weight=nxt)
-        return product(self.lm_head, h, squares_in=squares)
+            x, squares = onto_rows(layer.o_proj, a.view(x.shape))
+            gated = behind_norm(layer.gate_up_proj, layer.post_attention_layernorm, gated=True)
+            x, squares = onto_rows(layer.down_proj, gated)
+        return behind_norm(self.lm_head, self.norm)
 
     def _decode_step_fused(self, x, pos, image=None, squares=None):
         """One row, five launches per layer instead of nine, none of them an elementwise kernel: q|k|v and gate|up

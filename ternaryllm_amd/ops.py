@@ -251,12 +251,12 @@ def spmm_chain(weight, x, scale=None, x_layout=_lib.TL_X_ROW_MAJOR, residual=Non
     return (y, image[:, :M], squares) if next_norm_weight is not None else y
 
 
-def spmm_chain_rows(weight, x, scale=None, residual=None, next_norm_weight=None, squares_in=None, eps=0.0, gated=False):
+def spmm_chain_rows(weight, x, scale=None, residual=None, next_norm_weight=None, squares_in=None, eps=0.0, gated=False, squares_out=False):
     """spmm_chain for 2 and more fp16 rows of a weight with codes, all row-major (tl_spmm_chain_rows): the image is an [M, N] tensor,
     the squares are [ceil(N / 16), R] float32 with R = 16, 32 or 64 for up to 16, 32 or 48 rows.  More rows leave squares
     [M, ceil(N / 32)]; row_factors makes the [M] float32 tensor of them that is squares_in there.  (The image is rounded before the
-    rows' factors: entries above 65504 / weight are infinite there, products below 6e-5 lose bits.)  gated: columns are (gate, up)
-    pairs, the result is [M, N / 2].  Raises RuntimeError (TL_ERR_UNSUPPORTED) for other rows, types and weights."""
+    rows' factors: entries above 65504 / weight are infinite there, products below 6e-5 lose bits.)  squares_out: (y, squares)
+    without an image, for spmm_normed_rows, up to 48 rows.  gated: columns are (gate, up) pairs, the result is [M, N / 2].  Raises RuntimeError (TL_ERR_UNSUPPORTED) for other rows, types and weights."""
     if x.device != weight.device:
         raise RuntimeError(f"x is on {x.device}, the weight on {weight.device}")
     x_code = _code(x.dtype, "x")
@@ -274,8 +274,10 @@ def spmm_chain_rows(weight, x, scale=None, residual=None, next_norm_weight=None,
         if next_norm_weight.numel() != N or next_norm_weight.dtype != x.dtype or not next_norm_weight.is_contiguous() or next_norm_weight.device != x.device:
             raise ValueError("next_norm_weight must be a contiguous [N] tensor of x's dtype")
         image = torch.empty((M, N), dtype=x.dtype, device=x.device)
+        chain.next_norm_weight, chain.image_out, chain.image_ld = next_norm_weight.data_ptr(), image.data_ptr(), N
+    if image is not None or squares_out:
         squares = torch.empty(((N + 15) // 16, R) if few else (M, (N + 31) // 32), dtype=torch.float32, device=x.device)
-        chain.next_norm_weight, chain.image_out, chain.image_ld, chain.squares_out = next_norm_weight.data_ptr(), image.data_ptr(), N, squares.data_ptr()
+        chain.squares_out = squares.data_ptr()
     if squares_in is not None:
         fits = squares_in.dim() == 2 and squares_in.shape[1] == R if few else squares_in.shape == (M,)
         if squares_in.dtype != torch.float32 or not fits or not squares_in.is_contiguous() or squares_in.device != x.device:
@@ -287,7 +289,29 @@ def spmm_chain_rows(weight, x, scale=None, residual=None, next_norm_weight=None,
         _lib.check(_lib.lib().tl_spmm_chain_rows(ctypes.byref(weight.header), weight.blob.data_ptr(), xg.data_ptr(), x_code, ldx, M, y.data_ptr(), x_code,
                                                  y.shape[1], int(gated), sc.data_ptr() if sc is not None else None, s_code, ctypes.byref(chain),
                                                  _stream_ptr(x.device)))
-    return (y, image, squares) if next_norm_weight is not None else y
+    return (y, image, squares) if image is not None else (y, squares) if squares_out else y
+
+
+def spmm_normed_rows(weight, x, norm_weight, squares, eps, scale=None, gated=False):
+    """(RMSNorm(x) @ W) * scale for 2 to 48 fp16 rows whose sums of squares spmm_chain_rows or embed_rows left ([blocks, R] float32),
+    normalised on their way in and rounded as add_rmsnorm rounds (tl_spmm_normed_rows); gated: as spmm_chain_rows.  Raises
+    RuntimeError (TL_ERR_UNSUPPORTED) for other rows, types, alignments and weights."""
+    if x.device != weight.device:
+        raise RuntimeError(f"x is on {x.device}, the weight on {weight.device}")
+    x_code = _code(x.dtype, "x")
+    xg, M, ldx = _x_geometry(x, weight.inners, _lib.TL_X_ROW_MAJOR)
+    N, R = weight.columns, 16 if M <= 16 else 32 if M <= 32 else 64
+    if norm_weight.numel() != weight.inners or norm_weight.dtype != x.dtype or not norm_weight.is_contiguous() or norm_weight.device != x.device:
+        raise ValueError("norm_weight must be a contiguous [K] tensor of x's dtype")
+    if squares.dtype != torch.float32 or squares.dim() != 2 or squares.shape[1] != R or not squares.is_contiguous() or squares.device != x.device:
+        raise ValueError(f"squares must be a contiguous float32 [blocks, {R}] tensor")
+    sc, s_code = _scale_args(scale, N, x.device)
+    y = torch.empty((M, N // 2 if gated else N), dtype=x.dtype, device=x.device)
+    with torch.cuda.device(x.device):
+        _lib.check(_lib.lib().tl_spmm_normed_rows(ctypes.byref(weight.header), weight.blob.data_ptr(), xg.data_ptr(), x_code, ldx, M, y.data_ptr(), x_code,
+                                                  y.shape[1], int(gated), sc.data_ptr() if sc is not None else None, s_code, norm_weight.data_ptr(),
+                                                  squares.data_ptr(), squares.shape[0], float(eps), _stream_ptr(x.device)))
+    return y
 
 
 def gate_up(gate, up, x, gate_scale=None, up_scale=None):
@@ -737,21 +761,24 @@ def row_factors(squares, width, eps):
     return factors
 
 
-def embed_rows(table, token, norm_weight):
+def embed_rows(table, token, norm_weight=None):
     """(x, image, squares): x = table[token], image = x * norm_weight and the sums of squares of x over runs of 16 values, as
-    spmv_add(..., next_norm_weight=) leaves them for one row and spmm_chain_rows for more (tl_embed_rows).  fp16."""
+    spmv_add(..., next_norm_weight=) leaves them for one row and spmm_chain_rows for more (tl_embed_rows).  Without norm_weight
+    image is None.  fp16."""
     B, width = token.numel(), table.shape[1]
-    for t in (table, norm_weight):
+    for t in (table,) if norm_weight is None else (table, norm_weight):
         if not t.is_contiguous() or t.dtype != table.dtype or t.device != token.device:
             raise ValueError("table and norm_weight must be contiguous, of one dtype, on the token's device")
-    if token.dtype != torch.int64 or not token.is_contiguous() or norm_weight.numel() != width or not 1 <= B <= 65535:
+    if token.dtype != torch.int64 or not token.is_contiguous() or (norm_weight is not None and norm_weight.numel() != width) or not 1 <= B <= 65535:
         raise ValueError("token must be a contiguous int64 tensor of 1 to 65535 elements and norm_weight a row of the table's width")
     R = 1 if B == 1 else 16 if B <= 16 else 32 if B <= 32 else 64 if B <= 48 else 0
-    x, image = torch.empty((2, B, width), dtype=table.dtype, device=table.device).unbind(0)
+    x = torch.empty((B, width), dtype=table.dtype, device=table.device)
+    image = torch.empty_like(x) if norm_weight is not None else None
     squares = torch.empty((width // 16, R) if R > 1 else (width // 16,) if R else (B, (width + 31) // 32), dtype=torch.float32, device=table.device)
     with torch.cuda.device(table.device):
-        _lib.check(_lib.lib().tl_embed_rows(table.data_ptr(), _code(table.dtype, "table"), table.shape[0], width, token.data_ptr(), B, norm_weight.data_ptr(),
-                                            x.data_ptr(), image.data_ptr(), squares.data_ptr(), R, _stream_ptr(table.device)))
+        _lib.check(_lib.lib().tl_embed_rows(table.data_ptr(), _code(table.dtype, "table"), table.shape[0], width, token.data_ptr(), B,
+                                            norm_weight.data_ptr() if image is not None else None, x.data_ptr(),
+                                            image.data_ptr() if image is not None else None, squares.data_ptr(), R, _stream_ptr(table.device)))
     return x, image, squares
 
 

@@ -890,3 +890,27 @@ def test_prompts_of_any_magnitude(cuda, B, S, rows):
     assert bool(want.isfinite().all())
     for a, b in ((got.double(), want.double()), (cache.double(), m._cache.double())):
         assert float((a - b).norm() / b.norm()) <= 2.0 ** -10
+
+
+@pytest.mark.parametrize("rows", ["large", "tiny", "small weights"])
+@pytest.mark.parametrize("B", [2, 5, 8, 16, 17, 33, 48])
+def test_steps_of_any_magnitude(cuda, B, rows):
+    """A decode step of 2 to 48 rows, logits and cache, against the torch operators around the products.  (Differences as for
+    prompts; the sums of the attention over 12 slots are taken in another order too.)"""
+    m = _decoder()
+    with torch.no_grad():
+        _magnitudes(m, rows)
+    tokens = torch.randint(0, 300, (B, 12), generator=torch.Generator().manual_seed(B)).to(cuda)
+    print(f"case B={B} {rows}", flush=True)
+    m.prefill(tokens)
+    start = m._cache.clone()
+    step = tokens[:, 5].clone(), torch.full((1,), 12, dtype=torch.long, device=cuda), (torch.arange(64, device=cuda) <= 12)[None, None, None]
+    got = m._decode_step(*step)
+    cache = m._cache.clone()
+    assert m.chain_decode                      # (and the step was the chained one)
+    m._cache.copy_(start)
+    m.native_decode = False
+    want = m._decode_step(*step)
+    assert bool(want.isfinite().all())
+    for a, b in ((got.double(), want.double()), (cache.double(), m._cache.double())):
+        assert float((a - b).norm() / b.norm()) <= 2.0 ** -10

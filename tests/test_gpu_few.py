@@ -106,6 +106,39 @@ def test_chained_rows(cuda, M, K, N, N2):
         ops.spmm_chain_rows(d1, x[:1], sc1, residual=res[:1])
 
 
+@pytest.mark.parametrize("M,K,N", [(2, 16, 34), (3, 1104, 4200), (4, 72, 16), (13, 2048, 272), (16, 520, 8200), (17, 2064, 66), (31, 72, 4128), (33, 264, 40), (48, 5504, 2048)])
+def test_rows_normalised_on_their_way_in(cuda, M, K, N):
+    """RMSNorm and product in one against the two kernels, over magnitudes that leave fp16's middle, with a row that is not
+    finite, plain and gated; and the sums of squares without an image."""
+    from ternaryllm_amd import ops
+    from ternaryllm_amd.packing import PackedWeight
+    dw = ops.DeviceWeight(PackedWeight.from_dense(ternary_weight(K, N, 0.7, M)), cuda)
+    up = ops.DeviceWeight(PackedWeight.from_dense(ternary_weight(40, K, 0.7, 1)), cuda)
+    g = torch.Generator().manual_seed(M)
+    sc, res = (0.5 + torch.rand(N, generator=g)).half().to(cuda), torch.randn((M, K), generator=g).half().to(cuda)
+    nw = (1 + 0.1 * torch.randn(K, generator=g)).half().to(cuda)
+    few = torch.randn((M, 40), generator=g).half().to(cuda)
+    print(f"case M={M} K={K} N={N}", flush=True)
+    for rows, weights in ((1.0, 1.0), (2e-3, 0.02), (1e-5, 1.0), (1500.0, 40.0)):   # (1500: up to five times 5400, and times 40 beyond fp16)
+        r = res * rows
+        x, squares = ops.spmm_chain_rows(up, few * rows, residual=r, squares_out=True)
+        assert torch.equal(x, ops.spmm(up, few * rows) + r)
+        norm = nw * weights
+        h = ops.add_rmsnorm(x, None, norm, 1e-5)[1]
+        got, want = ops.spmm_normed_rows(dw, x, norm, squares, 1e-5, sc), ops.spmm(dw, h, sc)
+        # the squares' sum in another order moves a row by 2^-22 and few of its values across a rounding: by 2^-10 of them
+        assert float((got.double() - want.double()).norm()) <= 2.0 ** -11 * float(want.double().norm())
+        assert torch.equal(ops.spmm_normed_rows(dw, x, norm, squares, 1e-5, sc, gated=True), ops.silu_mul(got, pairs=True))
+    x[M - 1, 7] = float("inf")                  # (squares as they were: the value, not its row, is infinite)
+    got = ops.spmm_normed_rows(dw, x, norm, squares, 1e-5, sc)
+    assert torch.equal(got.isfinite(), ops.spmm(dw, x, sc * 1e-5).isfinite())
+    with pytest.raises(RuntimeError, match="UNSUPPORTED"):
+        ops.spmm_normed_rows(dw, torch.zeros((M, K + 1), dtype=torch.float16, device=cuda)[:, :K], norm, squares, 1e-5, sc)
+    if M > 8:
+        with pytest.raises(ValueError):
+            ops.spmm_normed_rows(dw, x, norm, torch.zeros((K // 16, 8), device=cuda), 1e-5, sc)
+
+
 @pytest.mark.parametrize("B,width", [(1, 16), (1, 2048), (5, 2064), (16, 4096), (17, 48), (48, 2048), (49, 48), (300, 2064)])
 def test_embedding_rows(cuda, B, width):
     """A token's row, its image for the product behind the first norm and its sums of squares; tokens counted from the end, and
