@@ -261,7 +261,7 @@ class TernaryLlamaDecoder(nn.Module):
     def _decode_step(self, token, pos, mask):
         """token: LongTensor [B]; pos: LongTensor [1] (cache slot to write); mask: bool [1, 1, 1, max_seq]
         true on slots <= pos.  Static shapes throughout.  Returns logits [B, vocab]."""
-        if self.native_decode:
+        if self.native_decode and self._norms_as_built():
             return self._decode_step_native(token, pos)
         x = self.embed_tokens[token][:, None]
         cos, sin = self.rope_cos.index_select(0, pos), self.rope_sin.index_select(0, pos)
@@ -275,14 +275,13 @@ class TernaryLlamaDecoder(nn.Module):
 
     def _decode_step_native(self, token, pos):
         """The decode step with rotary embedding, cache update and the attention over the cache as one
-        library kernel (activations stay [B, hidden] throughout)."""
+        library kernel (activations stay [B, hidden] throughout), for norms that are as built."""
         c = self.config
         B = token.shape[0]
-        eps = c.rms_norm_eps
         if B == 1:
             chained, first = self.fused_decode and self.row_chain, self.layers[0].input_layernorm.weight if len(self.layers) else None
         else:
-            chained, first = B <= 48 and self.chain_decode and self._products_as_built() and self._norms_as_built(), None
+            chained, first = B <= 48 and self.chain_decode and self._products_as_built(), None
         x = image = squares = None
         if chained and self._embeds_rows(token, first):
             # the tokens' rows and what the first norm's product wants of them in one launch
@@ -311,17 +310,20 @@ class TernaryLlamaDecoder(nn.Module):
         # 5 to 48 rows: the products that walk the index stream read a K-major image, so whatever feeds one writes it in
         # that layout (its transpose as a view) and no re-layout pass runs in front of the products
         km = 5 <= B <= 48 and c.hidden_size != B and c.intermediate_size != B
-        _, h = ops.add_rmsnorm(x, None, self.layers[0].input_layernorm.weight, eps, kmajor=km)
+
+        def add_norm(x, y, norm):
+            return ops.add_rmsnorm(x, y, norm.weight, norm.eps, kmajor=km)
+
+        _, h = add_norm(x, None, self.layers[0].input_layernorm)
         for li, layer in enumerate(self.layers):
             qkv = layer.qkv_proj(h)
             a = self._attend(qkv, self._cache[li, 0], self._cache[li, 1], pos, km)
-            x, h = ops.add_rmsnorm(x, layer.o_proj(a), layer.post_attention_layernorm.weight, eps, kmajor=km)
+            x, h = add_norm(x, layer.o_proj(a), layer.post_attention_layernorm)
             # the SiLU gate in the epilogue of the gate | up product where its kernel has one (else a launch of its own)
             gated = ops.spmm_gated(layer.gate_up_proj.device_weight(), h, layer.gate_up_proj.w_scale,
                                    x_layout=_lib.TL_X_K_MAJOR if km else _lib.TL_X_ROW_MAJOR, kmajor=km)
-            y = layer.down_proj(gated)
-            nxt = self.layers[li + 1].input_layernorm.weight if li + 1 < len(self.layers) else self.norm.weight
-            x, h = ops.add_rmsnorm(x, y, nxt, eps, kmajor=km)  # the residual add, and the norm the next layer (or the head) starts with
+            # the residual add, and the norm the next layer (or the head) starts with
+            x, h = add_norm(x, layer.down_proj(gated), self.layers[li + 1].input_layernorm if li + 1 < len(self.layers) else self.norm)
         return self.lm_head(h)
 
     def _embeds_rows(self, token, norm_weight):
@@ -360,7 +362,6 @@ class TernaryLlamaDecoder(nn.Module):
         (four with a long cache) that the o projection folds on its way in (piece_fold), or, without that, the last
         of its workgroups to finish folds them (tl_decode_attention_fold); the o and down projections add their
         result to the residual stream in their epilogue."""
-        eps = self.config.rms_norm_eps
         # x is the residual stream: every product that ends a block adds its result to it in the epilogue, and the
         # products that start one normalise it on the way in (the factor applied to their sums).  With row_chain the
         # product that ends a block also leaves the row multiplied by the next norm's weight and the sums of its
@@ -369,9 +370,9 @@ class TernaryLlamaDecoder(nn.Module):
         chain = self.row_chain
         for li, layer in enumerate(self.layers):
             if squares is None:
-                qkv = ops.spmv_fused(layer.qkv_proj.device_weight(), "rmsnorm", x, None, layer.input_layernorm.weight, eps, layer.qkv_proj.w_scale)
+                qkv = ops.spmv_fused(layer.qkv_proj.device_weight(), "rmsnorm", x, None, layer.input_layernorm.weight, layer.input_layernorm.eps, layer.qkv_proj.w_scale)
             else:
-                qkv = ops.spmv_fused(layer.qkv_proj.device_weight(), "rmsnorm_sums", image, squares, None, eps, layer.qkv_proj.w_scale)
+                qkv = ops.spmv_fused(layer.qkv_proj.device_weight(), "rmsnorm_sums", image, squares, None, layer.input_layernorm.eps, layer.qkv_proj.w_scale)
             squares = None
             caches = self._cache_of(layer, 0), self._cache_of(layer, 1)
             if self.pieces_per_head():
@@ -388,10 +389,10 @@ class TernaryLlamaDecoder(nn.Module):
                 else:
                     x = ops.spmv_add(layer.o_proj.device_weight(), att, x, layer.o_proj.w_scale)
             if squares is None:
-                gated = ops.spmv_fused(layer.gate_up_proj.device_weight(), "rmsnorm", x, None, layer.post_attention_layernorm.weight, eps,
-                                       layer.gate_up_proj.w_scale, gated=True)
+                gated = ops.spmv_fused(layer.gate_up_proj.device_weight(), "rmsnorm", x, None, layer.post_attention_layernorm.weight,
+                                       layer.post_attention_layernorm.eps, layer.gate_up_proj.w_scale, gated=True)
             else:
-                gated = ops.spmv_fused(layer.gate_up_proj.device_weight(), "rmsnorm_sums", image, squares, None, eps,
+                gated = ops.spmv_fused(layer.gate_up_proj.device_weight(), "rmsnorm_sums", image, squares, None, layer.post_attention_layernorm.eps,
                                        layer.gate_up_proj.w_scale, gated=True)
             squares = None
             if chain:
@@ -400,8 +401,8 @@ class TernaryLlamaDecoder(nn.Module):
             else:
                 x = ops.spmv_add(layer.down_proj.device_weight(), gated, x, layer.down_proj.w_scale)
         if squares is None:
-            return ops.spmv_fused(self.lm_head.device_weight(), "rmsnorm", x, None, self.norm.weight, eps, self.lm_head.w_scale)
-        return ops.spmv_fused(self.lm_head.device_weight(), "rmsnorm_sums", image, squares, None, eps, self.lm_head.w_scale)
+            return ops.spmv_fused(self.lm_head.device_weight(), "rmsnorm", x, None, self.norm.weight, self.norm.eps, self.lm_head.w_scale)
+        return ops.spmv_fused(self.lm_head.device_weight(), "rmsnorm_sums", image, squares, None, self.norm.eps, self.lm_head.w_scale)
 
     def pieces_per_head(self):
         """Pieces the attention of a single-row step leaves per head for the o projection to fold; 0: it folds them itself."""
