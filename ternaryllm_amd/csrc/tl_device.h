@@ -178,13 +178,25 @@ inline Codes weight_codes(const tl_layout_header* h, const void* blob_dev)
     return Codes{h->off_codes ? static_cast<const unsigned char*>(blob_dev) + h->off_codes : nullptr, (int)h->code_planes};
 }
 
-template <typename KernelT>
-int raise_lds_limit(KernelT kernel, size_t bytes)
-{
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    if (e != hipSuccess) return fail(TL_ERR_LAUNCH, "hipFuncSetAttribute(%zu bytes of LDS): %s", bytes, hipGetErrorString(e));
-    return TL_OK;
-}
+// More than 64 KB of dynamic LDS are asked for once per kernel and device: one of these, static, beside each kernel's launch.  (From
+// several threads at once: a repeated call is harmless.)
+class LdsLimit {
+public:
+    template <typename KernelT>
+    int raise(KernelT kernel, size_t bytes)
+    {
+        int dev = -1;
+        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;   // (not remembered then)
+        if (dev >= 0 && (done_.load(std::memory_order_relaxed) >> dev & 1)) return TL_OK;
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        if (e != hipSuccess) return fail(TL_ERR_LAUNCH, "hipFuncSetAttribute(%zu bytes of LDS): %s", bytes, hipGetErrorString(e));
+        if (dev >= 0) done_.fetch_or(1ull << dev, std::memory_order_relaxed);
+        return TL_OK;
+    }
+
+private:
+    std::atomic<uint64_t> done_{0};
+};
 
 // tl_small_m.hip
 inline int64_t small_kmajor_bytes(const tl_layout_header* h, int64_t M, int x_dtype)

@@ -442,11 +442,8 @@ int launch_few(const KernelArgs& a, hipStream_t st)
         const size_t lds = (size_t)waves * (wave_floats<XT, IN, FM, C, Q>() + (STEPS >= kSteps ? squares_rows(FM * 16) : 0)) * sizeof(float);
         auto kernel = tl_matrix_few<XT, IN, FM, C, Q, STEPS>;
         if (IN == kStaged || IN == kRows) {
-            static std::atomic<bool> raised{false};  // per instantiation; a repeated call is harmless
-            if (!raised.load(std::memory_order_relaxed)) {
-                if (int rc = raise_lds_limit(kernel, 160 * 1024)) return rc;
-                raised.store(true, std::memory_order_relaxed);
-            }
+            static LdsLimit raised;
+            if (int rc = raised.raise(kernel, 160 * 1024)) return rc;
         }
         hipLaunchKernelGGL(kernel, grid, block, lds, st, a);
         return (int)TL_OK;

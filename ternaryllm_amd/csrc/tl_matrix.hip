@@ -679,11 +679,9 @@ int launch_walk_mode(const KernelArgs& a, hipStream_t st)
     if (groups > INT32_MAX) return fail(TL_ERR_SHAPE, "%d rows are more than one launch takes", a.M);
     const size_t lds = R > 1 ? (size_t)kMaxTileRows * 512 : 0;
     auto kernel = tl_walk_rows<XT, R, MODE>;
-    static std::atomic<bool> raised{false};  // per instantiation; a repeated call is harmless
-    if (lds && !raised.load(std::memory_order_relaxed)) {
-        if (int rc = raise_lds_limit(kernel, lds)) return rc;
-        raised.store(true, std::memory_order_relaxed);
-    }
+    static LdsLimit raised;
+    if (lds)
+        if (int rc = raised.raise(kernel, lds)) return rc;
     hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(R > 1 ? 1024 : 256), lds, st, a);
     return TL_OK;
 }
@@ -720,11 +718,8 @@ int launch_tile(const KernelArgs& a, hipStream_t st)
     constexpr size_t lds = WK * ((size_t)kUnitStages * TM * kStageRowBytes + (TN / 16) * TL_CODE_UNIT_BYTES);
     static_assert(lds <= 160 * 1024, "the stages fit a compute unit's LDS");
     auto kernel = tl_matrix_rows<PARTS, WM, WN, WK, FM, FN, MODE>;
-    static std::atomic<bool> raised{false};  // per instantiation; a repeated call is harmless
-    if (!raised.load(std::memory_order_relaxed)) {
-        if (int rc = raise_lds_limit(kernel, lds)) return rc;
-        raised.store(true, std::memory_order_relaxed);
-    }
+    static LdsLimit raised;
+    if (int rc = raised.raise(kernel, lds)) return rc;
     const int64_t tiles = ceil_div(a.M, TM) * ceil_div(a.N, OUT_TN);
     hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(WM * WN * WK * 64), lds, st, a);
     return TL_OK;

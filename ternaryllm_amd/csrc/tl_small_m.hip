@@ -1924,11 +1924,8 @@ int launch_block_kernel(KernelArgs a, const tl_layout_header* h, hipStream_t st)
     const size_t lds = (size_t)a.xs_bytes + a.buf_bytes + (size_t)kMaxBlockSet * (tg + 1) * 4;
     if (lds > 160 * 1024) return fail(TL_ERR_UNSUPPORTED, "one tile of %d rows needs %zu bytes of LDS", MT, lds);
     auto kernel = tl_spmm_block<MT, XF16>;
-    static bool raised = false;  // per instantiation; a repeated or racing call is harmless
-    if (!raised) {
-        if (int rc = raise_lds_limit(kernel, 160 * 1024)) return rc;
-        raised = true;
-    }
+    static LdsLimit raised;
+    if (int rc = raised.raise(kernel, 160 * 1024)) return rc;
     hipLaunchKernelGGL(kernel, dim3(gx, gy), dim3(kBlockThreads), lds, st, a);
     return TL_OK;
 }
@@ -1972,11 +1969,8 @@ int launch_quad_kernel(KernelArgs a, const tl_layout_header* h, hipStream_t st)
     a.lpc_shift = log2_exact(groups);
     a.lw_shift = log2_exact(lw);
     auto kernel = tl_spmm_quad<MT, XF16, NT>;
-    static bool raised = false;  // per instantiation; a repeated or racing call is harmless
-    if (!raised) {
-        if (int rc = raise_lds_limit(kernel, 160 * 1024)) return rc;
-        raised = true;
-    }
+    static LdsLimit raised;
+    if (int rc = raised.raise(kernel, 160 * 1024)) return rc;
     hipLaunchKernelGGL(kernel, dim3(gx, gy), dim3(NT), lds, st, a);
     return TL_OK;
 }
@@ -2007,11 +2001,8 @@ int launch_octet_kernel(KernelArgs a, const tl_layout_header* h, hipStream_t st)
     if (lw < 1 || (lw & (lw - 1))) return fail(TL_ERR_ARG, "TL_LW=%d (a power of two expected)", lw);
     a.lpc_shift = log2_exact(groups);
     a.lw_shift = log2_exact(lw);
-    static bool raised = false;  // a repeated or racing call is harmless
-    if (!raised) {
-        if (int rc = raise_lds_limit(tl_spmm_octet, 160 * 1024)) return rc;
-        raised = true;
-    }
+    static LdsLimit raised;
+    if (int rc = raised.raise(tl_spmm_octet, 160 * 1024)) return rc;
     hipLaunchKernelGGL(tl_spmm_octet, dim3(gx, gy), dim3(kBlockThreads), lds, st, a);
     return TL_OK;
 }
@@ -2047,11 +2038,8 @@ int launch_res_np(KernelArgs a, const ResShape& shape, hipStream_t st)
     a.xs_bytes = a.T * kTileSlots * 32;
     a.tile_magic = (unsigned)(((1ull << 32) + a.tile_rows - 1) / a.tile_rows);
     auto kernel = tl_spmm_res<XF16, NP, ROWS_IN>;
-    static bool raised = false;  // per instantiation; a repeated or racing call is harmless
-    if (!raised) {
-        if (int rc = raise_lds_limit(kernel, 160 * 1024)) return rc;
-        raised = true;
-    }
+    static LdsLimit raised;
+    if (int rc = raised.raise(kernel, 160 * 1024)) return rc;
     hipLaunchKernelGGL(kernel, dim3((unsigned)shape.groups, (unsigned)shape.parts), dim3(kResWaves * 64), shape.lds, st, a);
     return TL_OK;
 }
@@ -2109,11 +2097,8 @@ int launch_spmv_direct_nt(KernelArgs a, const tl_layout_header* h, hipStream_t s
     a.lpc_shift = log2_exact(lpc);
     a.lw_shift = log2_exact(lw);
     auto kernel = tl_spmv_direct<XF16, NT, PRO>;
-    static bool raised = false;  // per instantiation; a repeated or racing call is harmless
-    if (!raised) {
-        if (int rc = raise_lds_limit(kernel, 160 * 1024)) return rc;
-        raised = true;
-    }
+    static LdsLimit raised;
+    if (int rc = raised.raise(kernel, 160 * 1024)) return rc;
     hipLaunchKernelGGL(kernel, dim3((unsigned)a.NB), dim3(NT), lds, st, a);
     return TL_OK;
 }
@@ -2145,11 +2130,8 @@ int launch_spmv_tiles_nt(KernelArgs a, const tl_layout_header* h, hipStream_t st
     if (NORM == kNormSums || a.chain_w) share = 1;
     if (lds > (size_t)(160 * 1024 / share - 1024)) return TL_ERR_UNSUPPORTED;
     auto kernel = tl_spmv_tiles<XF16, NT, NORM, EPI>;
-    static bool raised = false;  // per instantiation; a repeated or racing call is harmless
-    if (!raised) {
-        if (int rc = raise_lds_limit(kernel, 160 * 1024)) return rc;
-        raised = true;
-    }
+    static LdsLimit raised;
+    if (int rc = raised.raise(kernel, 160 * 1024)) return rc;
     hipLaunchKernelGGL(kernel, dim3((unsigned)a.NB), dim3(NT), lds, st, a);
     return TL_OK;
 }
