@@ -32,7 +32,7 @@ enum { kRowPieces = 0, kRows = 1, kElements = 2, kStaged = 3 };
 template <typename XT, int IN>
 __device__ __forceinline__ void load8(const KernelArgs& a, const XT* row, int k, XT* v)
 {
-    if constexpr (IN == kRowPieces || IN == kStaged) {
+    if constexpr (IN == kRowPieces) {
         const u32x4* p = reinterpret_cast<const u32x4*>(row + min(k, a.K - 8));
 #pragma unroll
         for (int i = 0; i < (int)sizeof(XT) / 2; ++i) reinterpret_cast<u32x4*>(v)[i] = p[i];
@@ -206,6 +206,11 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
                 load_to_lds(own + q * FM * BLOCK + i * 1024, a.X, row + min((uint32_t)((k0 + q * kSliceRows) * (int)sizeof(XT)) + piece, last));
         }
     };
+    // One lane writes what others of its wave read: a wave's LDS instructions run in order, and nothing may move across here.
+    [[maybe_unused]] auto lanes_meet = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
     // kRows: the same through registers, 16 bytes from any element on, and element by element where a row ends.  us as operands
     // straight from memory / so: fp16 16 rows 4095 -> 11008 26.5 / 9.3, 48 rows 67.6 / 23.0, 37 rows 1003 -> 777 8.0 / 6.2; fp32 16 rows
     // 24.7 / 14.7, 48 rows 54.6 / 42.8, but 37 rows 1003 -> 777 7.7 / 8.8 (eight waves, whose 12 KB fill the LDS, in the place of 16).
@@ -235,6 +240,7 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
         };
         if (k0 + Q * kSliceRows <= a.K) read(std::true_type{});
         else read(std::false_type{});
+        lanes_meet();                                              // (what was read of the turn before has been read)
 #pragma unroll
         for (int i = 0; i < LOADS; ++i)
 #pragma unroll
@@ -275,8 +281,9 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
                 for (int f = 0; f < FM; ++f) load8<XT, IN>(a, rows[f], k0 + s * 32, to.x[s][f]);
         }
     };
-    auto arrived = [] {
+    auto arrived = [&] {
         if constexpr (IN == kStaged) asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+        if constexpr (IN == kRows) lanes_meet();
     };
     [[maybe_unused]] float* wave_squares = sums + waves * OWN;
     auto add_squares = [&] {                                       // into wave_squares
