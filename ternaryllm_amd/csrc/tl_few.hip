@@ -24,11 +24,12 @@ constexpr __host__ __device__ int most_waves(int C, int stage_bytes) { return C 
 
 
 // How rows are read: aligned 16-byte pieces (K a multiple of 8), as operands; through registers and LDS, 16 bytes at a time
-// from any element on; element by element (K-major); aligned pieces straight to LDS.
-enum { kRowPieces = 0, kRows = 1, kElements = 2, kStaged = 3 };
+// from any element on; element by element (K-major); aligned pieces straight to LDS; as operands from any element on, but for the
+// turn in which a row ends.
+enum { kRowPieces = 0, kRows = 1, kElements = 2, kStaged = 3, kOperands = 4 };
 
 // Eight activations of a row from k on.  Past K: zeros (element by element) or the row's last whole piece again (such rows
-// of K meet zero codes).
+// of K meet zero codes).  kOperands: the caller has seen that k + 8 <= K.
 template <typename XT, int IN>
 __device__ __forceinline__ void load8(const KernelArgs& a, const XT* row, int k, XT* v)
 {
@@ -36,6 +37,8 @@ __device__ __forceinline__ void load8(const KernelArgs& a, const XT* row, int k,
         const u32x4* p = reinterpret_cast<const u32x4*>(row + min(k, a.K - 8));
 #pragma unroll
         for (int i = 0; i < (int)sizeof(XT) / 2; ++i) reinterpret_cast<u32x4*>(v)[i] = p[i];
+    } else if constexpr (IN == kOperands) {
+        __builtin_memcpy(v, row + k, 8 * sizeof(XT));
     } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = k + i < a.K ? row[(k + i) * a.x_sk] : XT(0.f);
@@ -275,10 +278,14 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
         if constexpr (IN == kStaged) stage(t);
         else if constexpr (IN == kRows) stage_any(t);
         else {
+            auto load_turn = [&](auto in) {
 #pragma unroll
-            for (int s = 0; s < Q * 2; ++s)
+                for (int s = 0; s < Q * 2; ++s)
 #pragma unroll
-                for (int f = 0; f < FM; ++f) load8<XT, IN>(a, rows[f], k0 + s * 32, to.x[s][f]);
+                    for (int f = 0; f < FM; ++f) load8<XT, decltype(in)::value>(a, rows[f], k0 + s * 32, to.x[s][f]);
+            };
+            if (IN == kOperands && (unit % a.units) * TL_CODE_UNIT_ROWS + (part + 1) * Q * kSliceRows > a.K) load_turn(std::integral_constant<int, kElements>{});
+            else load_turn(std::integral_constant<int, IN>{});
         }
     };
     auto arrived = [&] {
@@ -295,16 +302,23 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
         for (float* v : {&sum.x, &sum.y, &sum.z, &sum.w}) *v = sum_over_lanes<SR / 4, 64>(*v);   // the lanes with the same rows
         if (lane < SR / 4) reinterpret_cast<float4*>(wave_squares + wave * SR)[lane] = sum;
     };
-    // (All waves' sums are read at once: one after the other each is a trip to LDS.)
+    // (The waves' sums are read at once: one after the other each is a trip to LDS; and no more than there are: 37 fp32 rows of 301 ->
+    // 1024, five waves, 6.5 us with sixteen reads always, 6.1.)
     auto over_waves = [&](const float* s, int stride) {
+        auto read = [&](auto most) {
+            constexpr int MOST = decltype(most)::value;
+            float part[MOST];
+#pragma unroll
+            for (int i = 0; i < MOST; ++i) part[i] = s[min(i, waves - 1) * stride];
+            std::conditional_t<F32, double, float> v = 0;  // (fp32: sixteen more roundings would be the largest part of the error)
+#pragma unroll
+            for (int i = 0; i < MOST; ++i) v += i < waves ? part[i] : 0.f;
+            return (float)v;
+        };
         constexpr int MOST = most_waves(C, stage_bytes<XT, IN, FM>(Q));
-        float part[MOST];
-#pragma unroll
-        for (int i = 0; i < MOST; ++i) part[i] = s[min(i, waves - 1) * stride];
-        std::conditional_t<F32, double, float> v = 0;  // (fp32: sixteen more roundings would be the largest part of the error)
-#pragma unroll
-        for (int i = 0; i < MOST; ++i) v += i < waves ? part[i] : 0.f;
-        return (float)v;
+        if (waves <= 4) return read(std::integral_constant<int, 4>{});
+        if (MOST > 8 && waves <= 8) return read(std::integral_constant<int, 8>{});
+        return read(std::integral_constant<int, MOST>{});
     };
     auto row_factor = [&](int m) { return rsqrtf(over_waves(wave_squares + m, SR) * (1.0f / (float)a.K) + a.eps); };
     [[maybe_unused]] float factors[FM];                            // (kNormed: of the rows of this lane's operands)
@@ -440,7 +454,7 @@ int launch_few(const KernelArgs& a, hipStream_t st)
     const int most = most_waves(C, stage_bytes<XT, IN, FM>(1));
     // a turn of four slices is one 16-byte load of codes; fewer where that would leave waves without a turn, and where the
     // turn's activations, loaded one by one, would not fit the registers
-    constexpr int kMostSlices = stage_bytes<XT, IN, FM>(1) ? std::max(1, 8192 / stage_bytes<XT, IN, FM>(1)) : IN == kRowPieces || FM == 1 ? 4 : FM == 2 ? 2 : 1;
+    constexpr int kMostSlices = stage_bytes<XT, IN, FM>(1) ? std::max(1, 8192 / stage_bytes<XT, IN, FM>(1)) : IN == kOperands ? (FM == 3 ? 1 : 2) : IN == kRowPieces || FM == 1 ? 4 : FM == 2 ? 2 : 1;
     const int q = std::min<int>(kMostSlices, slices >= 4 * most ? 4 : slices >= 2 * most ? 2 : 1);
     const int waves = (int)std::min<int64_t>(most, ceil_div(slices, q));
     const dim3 grid((unsigned)(STEPS == kTwo ? a.NB : ceil_div(a.NB, C))), block((unsigned)waves * 64);
@@ -491,12 +505,24 @@ template <typename XT>
 int launch_few_type(const KernelArgs& a, bool pieces, bool two_weights, hipStream_t st)
 {
     if (a.x_kmajor) return launch_few_in<XT, kElements>(a, two_weights, st);
-    // Through LDS once the rows are many enough that reading them as operands costs more (us, straight / through LDS, at 2048 -> 6144,
-    // 5504 -> 2048, 11008 -> 4096): fp16 2 rows 3.2 / 3.3, 4.4 / 4.5, 6.6 / 6.5; 4 rows 3.5 / 3.4, 4.8 / 4.4, 7.4 / 6.2; 16 rows
-    // 4.6 / 3.7, 7.7 / 4.7, 12.7 / 7.2; 48 rows 9.2 / 6.8, 17.7 / 8.9, 31.6 / 16.2; fp32 4 rows 5.0 / 5.7, 8.1 / 8.0, 13.1 / 14.1;
-    // 8 rows 5.3 / 5.8, 9.5 / 8.3, 15.9 / 14.4; 16 rows 6.9 / 6.1, 13.0 / 8.3, 22.8 / 14.8.  (A lane's offset has 32 bits.)
-    if (pieces && a.M >= (sizeof(XT) == 2 ? 4 : 8) && a.ldx <= kMostStagedLd) return launch_few_in<XT, kStaged>(a, two_weights, st);
-    return pieces ? launch_few_in<XT, kRowPieces>(a, two_weights, st) : launch_few_in<XT, kRows>(a, two_weights, st);
+    // Through LDS once the rows are many enough, over a K that is long enough, that reading them as operands costs more.  us, as operands /
+    // through LDS.  Aligned, fp16: K = 1000 -> 4096 8 rows 3.11 / 3.15, 16 rows 3.35 / 3.26; 2048 -> 2048 3 rows 3.26 / 3.18, 8 rows 3.72 / 3.23;
+    // 11008 -> 4096 2 rows 6.4 / 6.4, 16 rows 12.5 / 6.8.  fp32: 8 rows 1000 -> 4096 3.78 / 3.76, 2048 -> 2048 5.03 / 4.83, 4096 -> 4096 7.4 / 6.7,
+    // 4096 -> 11008 12.5 / 12.5, but 2048 -> 6144, whose workgroups of two blocks have eight waves, 5.17 / 5.53 (12 rows 5.87 / 5.66); 6 rows
+    // 4096 -> 4096 6.7 / 6.7, 2048 -> 6144 4.9 / 5.4.
+    // On no boundary, fp16: 2 rows 1003 -> 4096 4.4 / 4.3, 16 rows 5.5 / 4.1: always LDS.  fp32: 1003 -> 4096 2 rows 4.35 / 4.45, 8 rows 4.58 / 4.51,
+    // 16 rows 5.1 / 4.7, 37 rows, whose stages fill the LDS with eight waves, 8.1 / 9.2; 2047 -> 2048 2 rows 5.6 / 5.3, 37 rows 13.3 / 13.0.
+    const int64_t depth = (int64_t)a.planes * a.K;
+    const bool wide = a.NB > compute_units();
+    if (pieces) {
+        const int enough = sizeof(XT) == 2 ? (depth > 1024 ? 4 : 9) : wide && depth < 4096 ? 12 : 8;
+        if (a.M >= enough && a.ldx <= kMostStagedLd) return launch_few_in<XT, kStaged>(a, two_weights, st);   // (a lane's offset has 32 bits)
+        return launch_few_in<XT, kRowPieces>(a, two_weights, st);
+    }
+    if constexpr (sizeof(XT) == 4) {
+        if (depth <= 1024 && (a.M < 8 || a.M > 16)) return launch_few_in<XT, kOperands>(a, two_weights, st);
+    }
+    return launch_few_in<XT, kRows>(a, two_weights, st);
 }
 
 }  // namespace

@@ -39,6 +39,30 @@ def test_few_rows_at_the_edges(cuda, oracle, M, K, N, dtype):
     assert np.array_equal(y, x.numpy()[:, rows] * one[rows, np.arange(N)].astype(x.numpy().dtype))
 
 
+# where rows go through LDS and where they are read as operands: fp16 from 4 or, up to 1024 of K, 9 rows on; fp32 from 8 or 12; on no
+# boundary fp32 rows up to 1024 of K but for 8 to 16
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M,K,N", [(2, 520, 8200), (4, 1024, 40), (7, 1032, 40), (9, 1024, 40), (11, 2048, 6150), (12, 2048, 6150), (8, 4096, 6150), (24, 1003, 8200), (37, 65, 40), (40, 1003, 4200), (7, 1025, 17)])
+def test_few_rows_of_every_path(cuda, oracle, M, K, N, dtype):
+    test_few_rows_at_the_edges(cuda, oracle, M, K, N, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M,K", [(3, 1003), (20, 301), (37, 1000), (44, 1001)])
+def test_gate_and_up_of_short_rows(cuda, M, K, dtype):
+    """silu(gate) * up of two weights over up to 1024 of K, whole numbers / 16: exact sums, then __expf and a division."""
+    from ternaryllm_amd import ops
+    from ternaryllm_amd.packing import PackedWeight
+    wg, wu = ternary_weight(K, 83, 0.8, 3), ternary_weight(K, 83, 0.8, 4)
+    dg, du = (ops.DeviceWeight(PackedWeight.from_dense(w), cuda) for w in (wg, wu))
+    x = activations(M, K, 5, dtype, integer=True).to(cuda) / 16
+    print(f"case M={M} K={K} {dtype}", flush=True)
+    got = ops.mlp_gate_up(dg, du, x, out_dtype=torch.float32).double()
+    g, u = (x.double() @ torch.from_numpy(w).double().to(cuda) for w in (wg, wu))
+    want = torch.nn.functional.silu(g) * u
+    assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("M", [2, 16, 31, 48])
 def test_gate_and_up_of_few_rows(cuda, M, dtype):
