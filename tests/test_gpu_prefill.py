@@ -43,6 +43,14 @@ def test_attention(B, heads, kv_heads, hd, S, L, rotate):
     assert (out - want).abs().max() <= 1.5 * 2.0 ** -10 * v.abs().max()
 
 
+# heads of 128 where workgroups own 128 queries (768 of them are three for each of 256 compute units): a last workgroup with two queries
+# and one with nine, more keys than queries, grouped heads
+@pytest.mark.parametrize("B,heads,kv_heads,hd,S,L", [(6, 64, 32, 128, 130, 130), (6, 64, 16, 128, 137, 200), (13, 60, 60, 128, 64, 131)])
+@pytest.mark.parametrize("rotate", [False, True])
+def test_attention_of_tall_workgroups(B, heads, kv_heads, hd, S, L, rotate):
+    test_attention(B, heads, kv_heads, hd, S, L, rotate)
+
+
 def test_attention_values_that_are_not_finite():
     """A row past the end of the keys and a key of -inf scores weigh nothing; NaN reaches the queries that see it, and only
     those outside its tile of keys are sure not to."""
