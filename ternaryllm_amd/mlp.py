@@ -77,7 +77,7 @@ class LlamaTernaryMLP(nn.Module):
         return self._pairs[:2]
 
     def forward(self, x):
-        if not self.paired and self.hidden_act in ("silu", "swish"):
+        if not self.paired and self.hidden_act in ("silu", "swish") and x.numel() != self.hidden_size:   # (one row: two products)
             gate, up = self.gate_proj, self.up_proj
             h = ops.gate_up(gate.device_weight(), up.device_weight(), x, gate.w_scale, up.w_scale)
             if h is not None:
