@@ -27,7 +27,7 @@ _VALUE_ERRORS = {-1, -2, -3, -4, -7, -8, -9}
 
 
 class Chain(ctypes.Structure):
-    """Mirror of tl_chain (the residual / RMSNorm steps a 9-16-row product may take over)."""
+    """Mirror of tl_chain (the residual / RMSNorm steps that tl_spmm_chain and tl_spmm_chain_rows take over)."""
     _fields_ = [("residual", ctypes.c_void_p), ("residual_ld", ctypes.c_int64), ("next_norm_weight", ctypes.c_void_p),
                 ("image_out", ctypes.c_void_p), ("image_ld", ctypes.c_int64), ("squares_out", ctypes.c_void_p),
                 ("squares_in", ctypes.c_void_p), ("squares_blocks", ctypes.c_int32), ("eps", ctypes.c_float)]

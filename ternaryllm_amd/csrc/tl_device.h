@@ -68,16 +68,18 @@ struct KernelArgs {
     int gated;
     const void* residual;  // single-row kernels: null, or a row of N values of Y's type: Y[n] = residual[n] + the product (rounded to that type first)
     long long y_kld;      // gated epilogue of the 16-row kernel: 0, or the leading dimension of a K-major output [N / 2][y_kld]
-    // 16-row kernels, a decoder layer without kernels for the residual add and the RMSNorm (tl_spmm_chain):
+    // A decoder layer without kernels for the residual add and the RMSNorm: the 16-row kernels (tl_spmm_chain; K-major image, squares
+    // [NB][16]), few rows on the matrix cores (tl_spmm_chain_rows; row-major image, squares [NB][16, 32 or 64]) and more (squares
+    // [M][ceil(N / 32)])
     const void* chain_res;    // [M][chain_ldres], Y's type: Y = chain_res + product
     long long chain_ldres;
-    const void* chain_w;      // [N] weight of the NEXT norm: chain_image[n][m] = Y[m][n] * chain_w[n], chain_sq_out[block][m] = sum over the block's columns of Y[m][n]^2
-    void* chain_image;        // K-major [N][chain_ild], Y's type, rows M .. chain_ild - 1 zeroed
+    const void* chain_w;      // [N] weight of the NEXT norm: chain_image = Y * chain_w, chain_sq_out = sums over a block's columns of Y^2
+    void* chain_image;        // Y's type; K-major [N][chain_ild], rows M .. chain_ild - 1 zeroed, or [M][chain_ild]
     long long chain_ild;
-    float* chain_sq_out;      // [NB][16]
-    const float* chain_sq_in; // [chain_sq_blocks][16] sums of squares of the rows X was made from: the product is multiplied by rsqrt(sum / K + eps), row by row
+    float* chain_sq_out;
+    const float* chain_sq_in; // sums of squares of the rows X was made from (with norm_w: of X's): the product is multiplied by rsqrt(sum / K + eps), row by row
     int chain_sq_blocks;
-    const float* chain_factors; // more than 48 rows: null, or [M], what the product is multiplied by, row by row (chain_sq_out is [M][ceil(N / 32)] there)
+    const float* chain_factors; // more than 48 rows: null, or [M], what the product is multiplied by, row by row
     // matrix-core kernels
     Codes c1;                 // the codes of w1
     const void* image;        // the activations they multiply: row-major, 16-byte pieces along K ...
@@ -205,7 +207,8 @@ inline int64_t small_kmajor_bytes(const tl_layout_header* h, int64_t M, int x_dt
 }
 int launch_small(KernelArgs a, const tl_layout_header* h, int x_dtype, void* workspace, int64_t workspace_bytes, hipStream_t st);
 
-// Whether tl_spmm_gated of these rows is served by a kernel that walks the index stream (9 to 48 fp16 rows).
+// Whether tl_spmm_gated has a kernel for these rows among those that walk the index stream (9 to 48 fp16 rows); with codes and
+// fewer bytes in them, the matrix cores take the call all the same (few_on_matrix_cores), and without such a kernel it is refused.
 bool walk_has_gated(const KernelArgs& a, const tl_layout_header* h);
 
 // tl_matrix.hip

@@ -101,11 +101,6 @@ enum { kPlain = 0, kPairs = 1, kTwoWeights = 2, kSteps = 3 };   // (kSteps: with
 // The product of one output: from the index stream where the matrix cores' sum is not finite.
 __device__ __forceinline__ float exact_output(const KernelArgs& a, const WeightPtrs& w, int m, int n) { return walk_column(w, a.T, a.tile_rows, n, callers_x(a, m)); }
 
-// A lane's sums of FN x FM fragments (32 columns x 32 rows: 16 neighbouring columns of one row a lane) on their way out; lane_m0
-// and lane_n0: its row and first column in the first.
-// A sum that is not finite is worked out again by the lane that holds it, before anything is stored: the outputs of
-// finite rows keep their bits whatever another row of the tile holds.  (The sums that need it go into a mask that a
-// loop takes bit by bit, so that the walk stands here once and the sums stay in registers.)
 // The last steps of 16 neighbouring outputs of a row (kSteps): residual row, output, the next norm's image; returns the sum of
 // the outputs' squares.  Rounded as separate operators would round.
 __device__ __forceinline__ float put_steps(const KernelArgs& a, int row, int n, float (&v)[16])
@@ -148,6 +143,11 @@ __device__ __forceinline__ float put_steps(const KernelArgs& a, int row, int n, 
     return sum;
 }
 
+// A lane's sums of FN x FM fragments (32 columns x 32 rows: 16 neighbouring columns of one row a lane) on their way out; lane_m0
+// and lane_n0: its row and first column in the first.
+// A sum that is not finite is worked out again by the lane that holds it, before anything is stored: the outputs of
+// finite rows keep their bits whatever another row of the tile holds.  (The sums that need it go into a mask that a
+// loop takes bit by bit, so that the walk stands here once and the sums stay in registers.)
 template <int FN, int FM, int MODE>
 __device__ __forceinline__ void put_out(const KernelArgs& a, f32x16 (&acc)[FN][FM], int lane_m0, int lane_n0)
 {
@@ -238,7 +238,7 @@ __device__ __forceinline__ void put_out(const KernelArgs& a, f32x16 (&acc)[FN][F
 // operands 1710 to 1880); products of 16 x 16 x 32 instead of 32 x 32 x 16 ran 69 % of the time at 2.30 GHz, 1320.  A wave owns 64
 // columns: each fragment of activations that it reads from LDS serves two products (with 32 columns a wave the reads took
 // as many clocks as the products: 58 % busy).  us before / now: 8192 x 2048 -> 11008 gated 358 / 289, 8192 x 2048 -> 6144 194 / 169,
-// 8192 x 5504 -> 2048 161 / 143, 1024 x 4096 -> 11008 94 / 83; fp32 4096 x 4096 -> 4096 367 / 297, 200 x 2048 -> 2048 47 / 21.
+// 8192 x 5504 -> 2048 161 / 135, 1024 x 4096 -> 11008 94 / 79; fp32 4096 x 4096 -> 4096 367 / 297, 200 x 2048 -> 2048 47 / 21.
 //
 // Output tiles of (WM * FM * 32) activation rows x (WN * FN * 32) columns, one per workgroup; a wave owns FM * 32 rows x
 // FN * 32 columns.  WK = 1: WM x WN waves over all of K that share what they copy.  WK > 1: one tile of a wave, whose WK waves
@@ -283,7 +283,7 @@ __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArg
     uint32_t xrow[XL];                                            // byte offset of this lane's row from the tile's base
     const uint32_t limit = (uint32_t)((a.K + 7) / 8 * 16 - 16);          // last whole piece of a row: pieces past it meet zero weights
     const int lane_row = lane >> 3;
-    
+
     // (rows of a lane's loads differ by 8 * W: by a multiple of 16, or, W = 1, by 8, which turns the place by half)
     const uint32_t piece = (uint32_t)piece_place(wave * 8 + lane_row, lane & 7) * 16;
     static_assert(W % 2 == 0 || W == 1, "a lane's pieces lie at one place, or at two in turn");
@@ -428,7 +428,7 @@ __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArg
     constexpr int OUT_FN = MODE == kTwoWeights ? FN / 2 : FN;
     if constexpr (WK > 1) {
         // every wave has sums of the whole tile, of its own rows of K: they meet in LDS (a wave's in its own part, which it is
-        // done with), and wave i goes on with fragment i.  Added up in 64 bits, as many roundings in 32 would weigh.
+        // done with), and wave i goes on with fragment i.  fp32 activations' are added up in 64 bits: roundings in 32 would weigh.
         constexpr int FRAGMENT = 64 * 16 * 4, PIECES = F32 ? 2 : 1;
         static_assert(PIECES * FN * FM * FRAGMENT <= OWN, "a wave's sums fit its part of LDS");
 #pragma unroll

@@ -135,7 +135,7 @@ class TernaryLlamaDecoder(nn.Module):
         # folds their pieces.  That pays once a head's rows are many: up to about a thousand rows one workgroup per
         # head is as quick.
         self.split_attention = self.max_seq_len > 1024
-        # steps of 2 to 48 fp16 rows: the products do the residual adds and the RMSNorms around them (tl_spmm_chain_rows);
+        # steps of 2 to 48 fp16 rows: the products do the residual adds and the RMSNorms around them (tl_spmm_chain_rows, tl_spmm_normed_rows);
         # switched off by the first step whose shapes have no such kernel
         self.chain_decode = dtype == torch.float16
         # single-row steps: the o and down projections prepare the row for the norm behind them (spmv_add with
