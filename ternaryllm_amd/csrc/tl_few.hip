@@ -173,11 +173,9 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
     [[maybe_unused]] uint32_t early_residual = 0, early_weight = 0;
     if constexpr (STEPS >= kSteps) {
         const float4* pieces = reinterpret_cast<const float4*>(a.chain_sq_in);
+        if (NORMED || square_pieces)
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int i = (int)threadIdx.x + u * (int)blockDim.x;
-            squares[u] = i < square_pieces ? pieces[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
+            for (int u = 0; u < U; ++u) squares[u] = pieces[min((int)threadIdx.x + u * (int)blockDim.x, square_pieces - 1)];
         if (!pairs && first_m < a.M && first_n < a.N) {
             if (a.chain_res) early_residual = raw_value(a.chain_res, 1, first_m * a.chain_ldres + first_n);
             if (a.chain_image) early_weight = raw_value(a.chain_w, 1, first_n);
@@ -295,10 +293,16 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
     [[maybe_unused]] float* wave_squares = sums + waves * OWN;
     auto add_squares = [&] {                                       // into wave_squares
         float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-        auto add = [&](const float4& v) { sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w; };
+        auto add = [&](const float4& v, bool there) {
+            sum.x += there ? v.x : 0.f; sum.y += there ? v.y : 0.f; sum.z += there ? v.z : 0.f; sum.w += there ? v.w : 0.f;
+        };
 #pragma unroll
-        for (int u = 0; u < U; ++u) add(squares[u]);
-        for (int i = (int)threadIdx.x + U * (int)blockDim.x; i < square_pieces; i += (int)blockDim.x) add(reinterpret_cast<const float4*>(a.chain_sq_in)[i]);
+        for (int u = 0; u < U; ++u) {
+            // (without this the first is added to zero, and waited for, where it is asked for: before the first turn's loads)
+            asm volatile("" : "+v"(squares[u].x), "+v"(squares[u].y), "+v"(squares[u].z), "+v"(squares[u].w));
+            add(squares[u], (int)threadIdx.x + u * (int)blockDim.x < square_pieces);
+        }
+        for (int i = (int)threadIdx.x + U * (int)blockDim.x; i < square_pieces; i += (int)blockDim.x) add(reinterpret_cast<const float4*>(a.chain_sq_in)[i], true);
         for (float* v : {&sum.x, &sum.y, &sum.z, &sum.w}) *v = sum_over_lanes<SR / 4, 64>(*v);   // the lanes with the same rows
         if (lane < SR / 4) reinterpret_cast<float4*>(wave_squares + wave * SR)[lane] = sum;
     };
@@ -355,15 +359,18 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
         }
     };
     if constexpr (NORMED) {
-        // the factors are needed before the first product: what the first turn reads is on its way while they meet
+        // the factors are needed before the first product: what the first turn reads is on its way while they meet.  (There are
+        // no more waves than turns.)
         Turn turn;
-        if (wave < turns) load(wave, turn);
+        load(wave, turn);
         add_squares();
         __syncthreads();
 #pragma unroll
         for (int f = 0; f < FM; ++f) factors[f] = row_factor(f * 16 + r16);
-        for (int t = wave; t < turns; t += waves) {
-            if (t != wave) load(t, turn);
+        arrived();
+        multiply(turn);
+        for (int t = wave + waves; t < turns; t += waves) {
+            load(t, turn);
             arrived();
             multiply(turn);
         }
