@@ -450,7 +450,8 @@ int tl_spmv_add(const tl_layout_header* header, const void* blob_dev, const void
  * TernaryLLM/TernaryLlama.py:69-75 and the Hugging Face decoder layer behind it).  Beside Y the epilogue leaves
  * image_out[n] = Y[n] * next_norm_weight[n] (y_dtype, N values) and squares_out[b] = sum of Y[n]^2 over column block b
  * (float32, ceil(N / 16) numbers): what tl_spmv_fused with TL_PRODUCER_RMSNORM_SUMS starts from, so that the product
- * after the norm neither multiplies the row nor sums its squares.  next_norm_weight: N values of y_dtype.  All three
+ * after the norm neither multiplies the row nor sums its squares.  (The image is rounded before the row's factor: an fp16 value
+ * above 65504 / weight is infinite there.)  next_norm_weight: N values of y_dtype.  All three
  * 16-byte aligned; image_out a row of its own.  TL_ERR_UNSUPPORTED where the single-row kernel with this epilogue
  * does not take the weight (call tl_spmv_add and TL_PRODUCER_RMSNORM then). */
 int tl_spmv_add_norm(const tl_layout_header* header, const void* blob_dev, const void* x, int x_dtype, const void* residual,
