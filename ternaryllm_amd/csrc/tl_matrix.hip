@@ -12,7 +12,6 @@ using namespace tl;
 
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef u32x4 u32x4_out __attribute__((aligned(8)));
 typedef f32x4 f32x4_out __attribute__((aligned(8)));
 
@@ -24,14 +23,6 @@ constexpr int kStageRowBytes = kStageRows * 2;       // bytes of one activation 
 constexpr int kRowGroup = 4;
 constexpr int kUnitStages = TL_CODE_UNIT_ROWS / kStageRows;
 __device__ __align__(16) const unsigned char kNoCodes[TL_CODE_UNIT_BYTES] = {};   // a unit of zero weights
-
-// acc[i] += sum over k of w[row 8 * (i / 4) + 4 * (lane / 32) + i % 4][k] * x[column lane % 32][k], 16 values of k, eight to a lane
-template <bool BF16>
-__device__ __forceinline__ f32x16 matrix_step32(u32x4 w, u32x4 x, f32x16 acc)
-{
-    if constexpr (BF16) return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x), acc, 0, 0, 0);
-    else return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, w), __builtin_bit_cast(half8, x), acc, 0, 0, 0);
-}
 
 template <int N, typename F, int... I>
 __device__ __forceinline__ void static_for(F f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
@@ -50,6 +41,10 @@ __device__ __forceinline__ void loads_here()
 // the LDS serves together (rows r and r + 1 share 256 bytes, all 64 banks) find their pieces on different banks.
 __device__ __forceinline__ int piece_place(int row, int p) { return p ^ ((row >> 1) & 7); }
 
+// Where column c of the 16 of a wave's column block b lies in a quarter of the block's codes: four columns to 64 bytes, turned by
+// the block, as the 16 lanes that the LDS serves together read four columns of each of four blocks, or eight of each of two.
+__device__ __forceinline__ int code_place(int c, int b) { return c ^ ((b & 3) * 4); }
+
 // COUNT neighbouring outputs of row m from column n on, of N: 16 bytes at a time where they lie so (vector_out), else one by one.
 template <int COUNT>
 __device__ __forceinline__ void store_piece(const KernelArgs& a, int m, int n, int N, const float* v)
@@ -57,11 +52,13 @@ __device__ __forceinline__ void store_piece(const KernelArgs& a, int m, int n, i
     const long long at = (long long)m * a.ldy + n;
     if (a.vector_out && n + COUNT <= N) {
         if (a.y_f16) {
+            static_assert(COUNT == 4 || COUNT % 8 == 0);
             __align__(16) __half o[COUNT];
 #pragma unroll
             for (int i = 0; i < COUNT; ++i) o[i] = __float2half(settled(v[i]));
 #pragma unroll
             for (int i = 0; i < COUNT / 8; ++i) reinterpret_cast<u32x4_out*>(static_cast<__half*>(a.Y) + at)[i] = reinterpret_cast<const u32x4*>(o)[i];
+            if constexpr (COUNT == 4) *reinterpret_cast<uint2*>(static_cast<__half*>(a.Y) + at) = *reinterpret_cast<const uint2*>(o);
         } else {
 #pragma unroll
             for (int i = 0; i < COUNT / 4; ++i) reinterpret_cast<f32x4_out*>(static_cast<float*>(a.Y) + at)[i] = f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
@@ -73,25 +70,26 @@ __device__ __forceinline__ void store_piece(const KernelArgs& a, int m, int n, i
         if (n + i < N) store_out(a.Y, a.y_f16, at + i, v[i]);
 }
 
-// `factor` times the scales of 16 columns from n on, of N (past N: of the last column again; nothing of such columns is stored).
+// `factor` times the scales of COUNT columns from n on, of N (past N: of the last column again; nothing of such columns is stored).
 // Read at once: a load for each column under its own condition, and a wait for each, took 2 us of a launch.
-__device__ __forceinline__ void read_scales(const void* scale, int is_f16, int n, int N, float factor, float (&s)[16])
+template <int COUNT>
+__device__ __forceinline__ void read_scales(const void* scale, int is_f16, int n, int N, float factor, float (&s)[COUNT])
 {
     auto read = [&](auto type) {
         using T = decltype(type);
         const T* p = static_cast<const T*>(scale);
-        T raw[16];
-        if (n + 16 <= N) __builtin_memcpy(raw, p + n, sizeof(raw));
+        T raw[COUNT];
+        if (n + COUNT <= N) __builtin_memcpy(raw, p + n, sizeof(raw));
         else {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) raw[i] = p[min(n + i, N - 1)];
+            for (int i = 0; i < COUNT; ++i) raw[i] = p[min(n + i, N - 1)];
         }
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = factor * (float)raw[i];
+        for (int i = 0; i < COUNT; ++i) s[i] = factor * (float)raw[i];
     };
     if (!scale) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = factor;
+        for (int i = 0; i < COUNT; ++i) s[i] = factor;
     } else if (is_f16) read(_Float16{});
     else read(float{});
 }
@@ -101,144 +99,154 @@ enum { kPlain = 0, kPairs = 1, kTwoWeights = 2, kSteps = 3 };   // (kSteps: with
 // The product of one output: from the index stream where the matrix cores' sum is not finite.
 __device__ __forceinline__ float exact_output(const KernelArgs& a, const WeightPtrs& w, int m, int n) { return walk_column(w, a.T, a.tile_rows, n, callers_x(a, m)); }
 
-// The last steps of 16 neighbouring outputs of a row (kSteps): residual row, output, the next norm's image; returns the sum of
+// The last steps of COUNT neighbouring outputs of a row (kSteps): residual row, output, the next norm's image; returns the sum of
 // the outputs' squares.  Rounded as separate operators would round.
-__device__ __forceinline__ float put_steps(const KernelArgs& a, int row, int n, float (&v)[16])
+template <int COUNT>
+__device__ __forceinline__ float put_steps(const KernelArgs& a, int row, int n, float (&v)[COUNT])
 {
-    const bool whole = a.vector_out && n + 16 <= a.N;                // (16-byte pieces of every array: the launcher has looked)
-    auto read16 = [&](const void* p, long long at, float (&to)[16]) {
+    const bool whole = a.vector_out && n + COUNT <= a.N;             // (16-byte pieces of every array: the launcher has looked)
+    auto read = [&](const void* p, long long at, float (&to)[COUNT]) {
         const __half* h = static_cast<const __half*>(p) + at;
-        __align__(16) __half raw[16];
+        __align__(16) __half raw[COUNT];
         if (whole) {
-            reinterpret_cast<u32x4*>(raw)[0] = reinterpret_cast<const u32x4_out*>(h)[0];
-            reinterpret_cast<u32x4*>(raw)[1] = reinterpret_cast<const u32x4_out*>(h)[1];
+#pragma unroll
+            for (int i = 0; i < COUNT / 8; ++i) reinterpret_cast<u32x4*>(raw)[i] = reinterpret_cast<const u32x4_out*>(h)[i];
         } else {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) raw[i] = n + i < a.N ? h[i] : __half(0.f);
+            for (int i = 0; i < COUNT; ++i) raw[i] = n + i < a.N ? h[i] : __half(0.f);
         }
 #pragma unroll
-        for (int i = 0; i < 16; ++i) to[i] = __half2float(raw[i]);
+        for (int i = 0; i < COUNT; ++i) to[i] = __half2float(raw[i]);
     };
-    float other[16], sum = 0.f;
+    float other[COUNT], sum = 0.f;
     if (a.chain_res) {
-        read16(a.chain_res, (long long)row * a.chain_ldres + n, other);
+        read(a.chain_res, (long long)row * a.chain_ldres + n, other);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = as_output(v[i], 1) + other[i];
+        for (int i = 0; i < COUNT; ++i) v[i] = as_output(v[i], 1) + other[i];
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = n + i < a.N ? as_output(v[i], 1) : 0.f;
-    store_piece<16>(a, row, n, a.N, v);
+    for (int i = 0; i < COUNT; ++i) v[i] = n + i < a.N ? as_output(v[i], 1) : 0.f;
+    store_piece<COUNT>(a, row, n, a.N, v);
     if (a.chain_image) {
-        read16(a.chain_w, n, other);
+        read(a.chain_w, n, other);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
+        for (int i = 0; i < COUNT; ++i) {
             sum = fmaf(v[i], v[i], sum);
             v[i] *= other[i];
         }
         KernelArgs image = a;
         image.Y = a.chain_image;
         image.ldy = a.chain_ild;
-        store_piece<16>(image, row, n, a.N, v);
+        store_piece<COUNT>(image, row, n, a.N, v);
     }
     return sum;
 }
 
-// A lane's sums of FN x FM fragments (32 columns x 32 rows: 16 neighbouring columns of one row a lane) on their way out; lane_m0
-// and lane_n0: its row and first column in the first.
+// A lane's sums of G rows on their way out: C = 4 * CF neighbouring columns of each row from each CF fragments, of one weight or of
+// two (fragments FW and on).  lane_m0 and lane_n0: its first row, of rows 16 apart, and its first column, of groups 4 * C apart.
 // A sum that is not finite is worked out again by the lane that holds it, before anything is stored: the outputs of
 // finite rows keep their bits whatever another row of the tile holds.  (The sums that need it go into a mask that a
 // loop takes bit by bit, so that the walk stands here once and the sums stay in registers.)
-template <int FN, int FM, int MODE>
-__device__ __forceinline__ void put_out(const KernelArgs& a, f32x16 (&acc)[FN][FM], int lane_m0, int lane_n0)
+template <int CF, int FW, int F, int G, int MODE>
+__device__ __forceinline__ void put_out(const KernelArgs& a, f32x4 (&acc)[F][G], int lane_m0, int lane_n0)
 {
-    constexpr int OUT_FN = MODE == kTwoWeights ? FN / 2 : FN;
+    constexpr int C = 4 * CF, GROUPS = FW / CF, ALL = F / CF * G;
+    static_assert(F == (MODE == kTwoWeights ? 2 : 1) * FW && FW % CF == 0);
     bool fine = true;
     float half = 0.5f;                                            // (the products are with +-2)
 #pragma unroll
-    for (int f = 0; f < FN; ++f)
+    for (int f = 0; f < F; ++f)
 #pragma unroll
-        for (int m = 0; m < FM; ++m)
+        for (int m = 0; m < G; ++m)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) fine = fine && fabsf(acc[f][m][e]) < __builtin_huge_valf();
+            for (int e = 0; e < 4; ++e) fine = fine && fabsf(acc[f][m][e]) < __builtin_huge_valf();
     if (!fine) {
         half = 1.0f;
 #pragma unroll 1
-        for (int i = 0; i < FN * FM; ++i) {
-            const int f = i / FM, m = i % FM;
-            float v[16];
+        for (int i = 0; i < ALL; ++i) {
+            const int group = i / G, m = i % G, n = lane_n0 + group % GROUPS * 4 * C;
+            float v[C];
             uint32_t redo = 0;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                v[e] = acc[0][0][e];
+            for (int e = 0; e < C; ++e) {
+                v[e] = acc[e / 4][0][e % 4];
 #pragma unroll
-                for (int o = 1; o < FN * FM; ++o) v[e] = o == i ? acc[o / FM][o % FM][e] : v[e];
-                const bool mine = lane_m0 + m * 32 < a.M && lane_n0 + f % OUT_FN * 32 + e < a.N;
+                for (int o = 1; o < ALL; ++o) v[e] = o == i ? acc[o / G * CF + e / 4][o % G][e % 4] : v[e];
+                const bool mine = lane_m0 + m * 16 < a.M && n + e < a.N;
                 redo |= mine && !(fabsf(v[e]) < __builtin_huge_valf()) ? 1u << e : 0u;
                 v[e] *= 0.5f;                                     // (twice what is worked out again might overflow)
             }
             while (redo != 0) {
                 const int at = __builtin_ctz(redo);
                 redo &= redo - 1;
-                const float y = exact_output(a, f >= OUT_FN ? a.w1 : a.w0, lane_m0 + m * 32, lane_n0 + f % OUT_FN * 32 + at);
+                const float y = exact_output(a, group >= GROUPS ? a.w1 : a.w0, lane_m0 + m * 16, n + at);
 #pragma unroll
-                for (int e = 0; e < 16; ++e) v[e] = e == at ? y : v[e];
+                for (int e = 0; e < C; ++e) v[e] = e == at ? y : v[e];
             }
 #pragma unroll
-            for (int e = 0; e < 16; ++e)
+            for (int e = 0; e < C; ++e)
 #pragma unroll
-                for (int o = 0; o < FN * FM; ++o) acc[o / FM][o % FM][e] = o == i ? v[e] : acc[o / FM][o % FM][e];
+                for (int o = 0; o < ALL; ++o) acc[o / G * CF + e / 4][o % G][e % 4] = o == i ? v[e] : acc[o / G * CF + e / 4][o % G][e % 4];
         }
     }
+    float s0[GROUPS][C], s1[MODE == kTwoWeights ? GROUPS : 1][C];
 #pragma unroll
-    for (int f = 0; f < OUT_FN; ++f) {
-        const int n = lane_n0 + f * 32;
-        float s0[16], s1[MODE == kTwoWeights ? 16 : 1];
-        read_scales(a.w0.scale, a.scale_f16, n, a.N, half, s0);
-        if constexpr (MODE == kTwoWeights) read_scales(a.w1.scale, a.scale_f16, n, a.N, half, s1);
+    for (int group = 0; group < GROUPS; ++group) {
+        read_scales(a.w0.scale, a.scale_f16, lane_n0 + group * 4 * C, a.N, half, s0[group]);
+        if constexpr (MODE == kTwoWeights) read_scales(a.w1.scale, a.scale_f16, lane_n0 + group * 4 * C, a.N, half, s1[group]);
+    }
 #pragma unroll
-        for (int m = 0; m < FM; ++m) {
-            const int row = lane_m0 + m * 32;
+    for (int m = 0; m < G; ++m) {
+        const int row = lane_m0 + m * 16;
+#pragma unroll
+        for (int group = 0; group < GROUPS; ++group) {
+            const int n = lane_n0 + group * 4 * C;
+            float v[C];
             if constexpr (MODE == kSteps) {
-                float v[16], sum = 0.f;
+                static_assert(C == 8, "four lanes hold 32 columns of a row");
+                float sum = 0.f;
                 const float factor = a.chain_factors && row < a.M ? a.chain_factors[row] : 1.0f;
 #pragma unroll
-                for (int i = 0; i < 16; ++i) v[i] = acc[f][m][i] * s0[i] * factor;
+                for (int i = 0; i < C; ++i) v[i] = acc[group * CF + i / 4][m][i % 4] * s0[group][i] * factor;
                 if (row < a.M && n < a.N) sum = put_steps(a, row, n, v);
-                if (a.chain_image) {                              // (the other 16 columns of the fragment are the lane's 32 further on)
-                    const auto pair = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+                if (a.chain_image) {
+                    auto pair = __builtin_amdgcn_permlane16_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
                     sum = __uint_as_float(pair[0]) + __uint_as_float(pair[1]);
-                    if (threadIdx.x % 64 < 32 && row < a.M && n < a.N) a.chain_sq_out[(long long)row * ((a.N + 31) / 32) + n / 32] = sum;
+                    pair = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+                    sum = __uint_as_float(pair[0]) + __uint_as_float(pair[1]);
+                    if (n % 32 == 0 && row < a.M && n < a.N) a.chain_sq_out[(long long)row * ((a.N + 31) / 32) + n / 32] = sum;
                 }
                 continue;
             }
             if (row >= a.M || n >= a.N) continue;
-            float v[16];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                v[i] = acc[f][m][i] * s0[i];
-                if constexpr (MODE == kTwoWeights) v[i] = silu(v[i]) * (acc[f + FN / 2][m][i] * s1[i]);
+            for (int i = 0; i < C; ++i) {
+                v[i] = acc[group * CF + i / 4][m][i % 4] * s0[group][i];
+                if constexpr (MODE == kTwoWeights) v[i] = silu(v[i]) * (acc[FW + group * CF + i / 4][m][i % 4] * s1[group][i]);
             }
             if constexpr (MODE == kPairs) {
                 if (a.chain_factors) {
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) v[i] *= a.chain_factors[row];
+                    for (int i = 0; i < C; ++i) v[i] *= a.chain_factors[row];
                 }
 #pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] = gate_pair(as_output(v[2 * i], a.y_f16), as_output(v[2 * i + 1], a.y_f16), a.y_f16);
-                store_piece<8>(a, row, n / 2, a.N / 2, v);
+                for (int i = 0; i < C / 2; ++i) v[i] = gate_pair(as_output(v[2 * i], a.y_f16), as_output(v[2 * i + 1], a.y_f16), a.y_f16);
+                store_piece<C / 2>(a, row, n / 2, a.N / 2, v);
             } else {
-                store_piece<16>(a, row, n, a.N, v);
+                store_piece<C>(a, row, n, a.N, v);
             }
         }
     }
 }
 
-// Bound by the matrix cores and, at the large sizes, by the power that they draw: 8192 x 5504 -> 2048 in fp16 keeps them busy for
-// 80 % of the time at 1.88 GHz, 1290 TFLOP/s (a large library product in fp16 1197, the matrix instruction alone on such
-// operands 1710 to 1880); products of 16 x 16 x 32 instead of 32 x 32 x 16 ran 69 % of the time at 2.30 GHz, 1320.  A wave owns 64
-// columns: each fragment of activations that it reads from LDS serves two products (with 32 columns a wave the reads took
-// as many clocks as the products: 58 % busy).  us before / now: 8192 x 2048 -> 11008 gated 358 / 289, 8192 x 2048 -> 6144 194 / 169,
-// 8192 x 5504 -> 2048 161 / 135, 1024 x 4096 -> 11008 94 / 79; fp32 4096 x 4096 -> 4096 367 / 297, 200 x 2048 -> 2048 47 / 21.
+// Bound by the matrix cores and, at the large sizes, by the power that they draw, so by the instruction: on such operands alone, and no
+// memory, 16 x 16 x 32 products run at 2200 TFLOP/s in fp16 and 2230 in bf16, 32 x 32 x 16 ones at 1750 and 1880 (with the weights as
+// the second operand 1970; at 66 % zeros).  With all that stands around them 8192 x 5504 -> 2048 runs at 1600, or 1760 without what a
+// launch costs; without making operands and reading LDS it would take 8 % less.  A wave owns 64 columns: each fragment of
+// activations that it reads from LDS serves four products.  us with 32 x 32 x 16 / now: 8192 x 2048 -> 11008 gated 281 / 250, 8192 x 2048 -> 6144
+// 156 / 140, 8192 x 5504 -> 2048 133 / 116, 1024 x 4096 -> 11008 78 / 71; fp32 4096 x 4096 -> 4096 292 / 256, 1024 x 4096 -> 4096 85 / 76.
+// A lone wave on its SIMD is bound by what it issues, of which twice as many products are more: the load side's addresses
+// are scalar and follow from the turn (fp32 1024 x 4096 -> 4096 82 us while they were worked out for every load).
 //
 // Output tiles of (WM * FM * 32) activation rows x (WN * FN * 32) columns, one per workgroup; a wave owns FM * 32 rows x
 // FN * 32 columns.  WK = 1: WM x WN waves over all of K that share what they copy.  WK > 1: one tile of a wave, whose WK waves
@@ -249,7 +257,7 @@ __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArg
 {
     constexpr int W = WK > 1 ? 1 : WM * WN;                       // waves that work on the same rows of K, and share what is copied
     constexpr int TM = WM * FM * 32, TN = WN * FN * 32;
-    static_assert(WK == 1 || (WM == 1 && WN == 1 && FM * FN == WK), "waves share either an output tile's rows of K or its outputs");
+    static_assert(WK == 1 || (WM == 1 && WN == 1 && 2 * FM <= WK), "waves share either an output tile's rows of K or its outputs");
     constexpr int STAGES = kUnitStages;                           // buffers of activations: a stage's place in its unit names its buffer
     constexpr int XB = TM * kStageRowBytes;                       // bytes of a stage of activations
     constexpr int XL = TM / 8 / W;                                // activation loads of a wave per stage (8 rows each)
@@ -284,7 +292,6 @@ __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArg
     const uint32_t limit = (uint32_t)((a.K + 7) / 8 * 16 - 16);          // last whole piece of a row: pieces past it meet zero weights
     const int lane_row = lane >> 3;
 
-    // (rows of a lane's loads differ by 8 * W: by a multiple of 16, or, W = 1, by 8, which turns the place by half)
     const uint32_t piece = (uint32_t)piece_place(wave * 8 + lane_row, lane & 7) * 16;
     static_assert(W % 2 == 0 || W == 1, "a lane's pieces lie at one place, or at two in turn");
 #pragma unroll
@@ -299,20 +306,25 @@ __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArg
     const int all_stages = a.planes == 1 ? stages_k : all_units * kUnitStages;
     const int total = PARTS * (min((unit0 + units) * kUnitStages, all_stages) - unit0 * kUnitStages);
 
-    // load side: where the next activations to ask for lie
-    int lk = unit0 % a.units, lj = 0, lp = 0, issued = 0;                       // unit within its plane, stage, part
-    auto issue_x = [&](uint32_t buffer) {
-        const uint32_t k_bytes = (uint32_t)(lk * TL_CODE_UNIT_ROWS + lj * kStageRows) * 2;
-        const unsigned char* src = image + (PARTS > 1 ? (long long)lp * a.image_plane * 2 : 0ll);
-        const uint32_t at = min(k_bytes + piece, limit), at_odd = W == 1 ? min(k_bytes + (piece ^ 64u), limit) : at;
+    // load side: the unit, within its plane, of the next activations to ask for; their stage and part follow from the turn
+    int lk = unit0 % a.units, issued = 0;
+    // (rows of a lane's loads differ by 8 * W: by a multiple of 16, or, W = 1, by 8, which turns the place by half)
+    const unsigned char* part_image[PARTS];
 #pragma unroll
-        for (int i = 0; i < XL; ++i) load_to_lds(lds0 + buffer * XB + (i * W + wave) * 1024, src, xrow[i] + (i % 2 ? at_odd : at));
+    for (int p = 0; p < PARTS; ++p) part_image[p] = image + (PARTS > 1 ? (long long)p * a.image_plane * 2 : 0ll);
+    // Turn TURN of a unit's activations.  WHOLE: all of the stage's pieces lie within K; else those past it are its last (and meet zero weights).
+    auto issue_x = [&](auto turn_tag, auto whole_tag) {
+        constexpr int TURN = decltype(turn_tag)::value, STAGE = TURN / PARTS;
+        constexpr bool WHOLE = decltype(whole_tag)::value;
+        const uint32_t k_bytes = (uint32_t)(lk * TL_CODE_UNIT_ROWS + STAGE * kStageRows) * 2;
+        const unsigned char* src = part_image[TURN % PARTS] + (WHOLE ? k_bytes : 0);
+#pragma unroll
+        for (int i = 0; i < XL; ++i) {
+            const uint32_t mine = W == 1 && i % 2 ? piece ^ 64u : piece;
+            load_to_lds(lds0 + TURN % STAGES * XB + (i * W + wave) * 1024, src, xrow[i] + (WHOLE ? mine : min(k_bytes + mine, limit)));
+        }
         ++issued;
-        if (++lp < PARTS) return;
-        lp = 0;
-        if (++lj < kUnitStages) return;                           // (the last unit may be shorter: nothing is asked for after it)
-        lj = 0;
-        if (++lk == a.units) lk = 0;
+        if (TURN == kUnitStages * PARTS - 1 && ++lk == a.units) lk = 0;   // (the last unit may be shorter: nothing is asked for after it)
     };
     const unsigned char* code_src[CL];                            // (wave-uniform)
     uint32_t code_to[CL];
@@ -332,84 +344,97 @@ __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArg
         for (int i = 0; i < CL; ++i) {
             const unsigned char* src = code_src[i] + (unit0 + u) * unit_stride;
             if (MODE == kTwoWeights && unit0 + u >= code_units[i]) src = kNoCodes;   // (the other weight has more planes)
-            load_to_lds(code_to[i], src, (uint32_t)lane * 16);
+            load_to_lds(code_to[i], src, (uint32_t)((lane & 48) + code_place(lane & 15, min(i * W + wave, TN / 16 - 1) % (MODE == kTwoWeights ? FN : 2 * FN))) * 16);
         }
     };
 
     // ---- what it reads ----
-    const int h = lane >> 5, r32 = lane & 31;
-    const uint32_t x_read = (uint32_t)((wm * FM * 32 + r32) * kStageRowBytes);
-    const uint32_t swz = (uint32_t)(piece_place(r32, h) * 16);    // rows of a wave's fragments differ by multiples of 32: same place
-    // the column of this lane's operand row: a lane's sums then are 16 neighbouring columns of one activation row
-    const int col = 16 * (r32 >> 2 & 1) + 4 * (r32 >> 3) + (r32 & 3);
-    const uint32_t c_read = (uint32_t)(STAGES * XB + (wn * FN * 2 + (col >> 4)) * TL_CODE_UNIT_BYTES + ((col & 15) + 16 * h) * 16);
+    constexpr int F = 2 * FN, G = 2 * FM;                         // fragments of 16 columns, of 16 rows
+    constexpr int FW = MODE == kTwoWeights ? FN : F;              // fragments of columns of one weight
+    const int q = lane >> 4, r16 = lane & 15;
+    const uint32_t x_read = (uint32_t)((wm * FM * 32 + r16) * kStageRowBytes);
+    const uint32_t swz = (uint32_t)(piece_place(r16, q) * 16);    // rows of a wave's fragments differ by multiples of 16: same place
+    // Fragments whose columns a lane holds side by side, so that its sums of a row are 16 bytes of output (of fp16 ones for fp16
+    // activations), and four lanes' 64.  (Where each lane held 16 columns, fp32 took 4 % longer: 4096 x 4096 -> 4096 274 us / 263.)
+    constexpr int CF = (PARTS > 1 ? 1 : 2) * (MODE == kPairs ? 2 : 1) > FW ? FW : (PARTS > 1 ? 1 : 2) * (MODE == kPairs ? 2 : 1);
+    // where the codes of this lane's row of fragment f's operand lie: column 16 * CF * (f / CF) + 4 * CF * (r16 / 4) + 4 * (f % CF) + r16 % 4
+    const int col = 4 * CF * (r16 >> 2) + (r16 & 3);
+    const uint32_t c_read = (uint32_t)(STAGES * XB + (wn * F + (col >> 4)) * TL_CODE_UNIT_BYTES + (q * 16 + code_place(col & 15, col >> 4)) * 16);
     constexpr bool F32 = PARTS > 1;
-    f32x16 acc[FN][FM], low[F32 ? FN : 1][F32 ? FM : 1];          // low: the sums of the parts after the first
+    f32x4 acc[F][G], low[F32 ? F : 1][F32 ? G : 1];               // low: the sums of the parts after the first
 #pragma unroll
-    for (int f = 0; f < FN; ++f)
+    for (int f = 0; f < F; ++f)
 #pragma unroll
-        for (int m = 0; m < FM; ++m)
+        for (int m = 0; m < G; ++m)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[f][m][e] = low[F32 ? f : 0][F32 ? m : 0][e] = 0.f;
+            for (int e = 0; e < 4; ++e) acc[f][m][e] = low[F32 ? f : 0][F32 ? m : 0][e] = 0.f;
 
     constexpr int R = 4, AHEAD = R - 1;                           // fragments of activations in registers; read ahead
-    constexpr int STEPS = 4 * FM;                                 // of a stage: a fragment of 32 rows x 16 rows of K each
-    u32x4 x[R], codes[FN][2], w[2][FN];
+    constexpr int STEPS = 2 * G;                                  // of a stage: a fragment of 16 rows x 32 rows of K each
+    u32x4 x[R], codes[F], w[2][F];
+    uint32_t last[F];                                             // the unit's last 64 rows of K, while the next unit's codes come
     auto read_x = [&](int buffer, int step) {                     // (constants)
-        x[step % R] = *reinterpret_cast<const u32x4*>(lds + x_read + (swz ^ (uint32_t)(step / FM * 32)) + buffer * XB + step % FM * 32 * kStageRowBytes);
+        x[step % R] = *reinterpret_cast<const u32x4*>(lds + x_read + (swz ^ (uint32_t)(step / G * 64)) + buffer * XB + step % G * 16 * kStageRowBytes);
     };
-    auto read_codes = [&](int half) {
+    auto read_codes = [&]() {
 #pragma unroll
-        for (int f = 0; f < FN; ++f) codes[f][half] = *reinterpret_cast<const u32x4*>(lds + c_read + f * 2 * TL_CODE_UNIT_BYTES + half * 512);
+        for (int f = 0; f < F; ++f) {
+            const int first = f % FW / CF * CF;                   // column block of the weight's fragments that stand beside f
+            codes[f] = *reinterpret_cast<const u32x4*>(lds + (c_read ^ (uint32_t)(code_place(4 * (f % CF), first) * 16)) + (first + f / FW * FN) * TL_CODE_UNIT_BYTES);
+        }
     };
-    // dword d % 4 of fragment d / 4's operand of the 16 rows of K number j of a unit (constants)
+    // dword d % 4 of fragment d / 4's operand of the 32 rows of K number j of a unit (constants)
     auto operand_dword = [&](int j, int d, u32x4* to) {
-        to[d / 4][d % 4] = (codes[d / 4][j & 1][j >> 2] << ((j >> 1 & 1) * 8 + 2 * (d % 4))) & 0xC000C000u;
+        to[d / 4][d % 4] = ((j >= 6 ? last[d / 4] : codes[d / 4][j >> 1]) << ((j & 1) * 8 + 2 * (d % 4))) & 0xC000C000u;
     };
     if (WK == 1 || units > 0) issue_codes(0);
-#pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s)
-        if (issued < total) issue_x(s);
+    static_for<STAGES - 1>([&](auto s) {
+        if (issued < total) issue_x(s, std::false_type{});
+    });
     if (total >= STAGES - 1) loads_here<WK == 1, (STAGES - 2) * XL>();
     else loads_here<WK == 1, 0>();
-    read_codes(0);
-    read_codes(1);
+    read_codes();
 #pragma unroll
     for (int s = 0; s < AHEAD; ++s) read_x(0, s);
 #pragma unroll
-    for (int d = 0; d < 4 * FN; ++d) operand_dword(0, d, w[0]);
+    for (int d = 0; d < 4 * F; ++d) operand_dword(0, d, w[0]);
     int t = 0;
-    // Turn Q of unit u: part Q % PARTS of its stage Q / PARTS.  STEADY: turns up to t + STAGES - 1 exist.
+    // Turn Q of unit u: part Q % PARTS of its stage Q / PARTS.  STEADY: turns up to t + STAGES - 1 exist, and those asked for are whole.
     constexpr int TURNS = kUnitStages * PARTS;
     auto turn = [&](auto q_tag, auto steady_tag, int u) {
         constexpr int Q = decltype(q_tag)::value, J = Q / PARTS, P = Q % PARTS;
         constexpr bool STEADY = decltype(steady_tag)::value, FIRST = P == 0;
-        constexpr int PER = 4 * FN / FM;                          // operand dwords made in a step
+        constexpr int PER = 4 * F / G;                            // operand dwords made in a step
 #pragma unroll
         for (int s = 0; s < STEPS; ++s) {
-            const int m = s % FM, k = s / FM;                     // k: 16 rows of K of the stage
+            const int m = s % G, k = s / G;                       // k: 32 rows of K of the stage
             if (s == STEPS - AHEAD) {
                 // turn t + 1's activations have come; every wave is done with turn t - 1, whose buffer takes turn t + STAGES - 1
                 if (STEADY) loads_here<WK == 1, (STAGES - 3) * XL>();
                 else if (t + 1 < total) loads_here<WK == 1, 0>();
                 if (Q == 0 && (STEADY || u + 1 < units)) issue_codes(u + 1);
-                if (STEADY || issued < total) issue_x((Q + STAGES - 1) % STAGES);
+                if (STEADY || issued < total) issue_x(std::integral_constant<int, (Q + STAGES - 1) % TURNS>{}, steady_tag);
             }
             if (s + AHEAD < STEPS) read_x(Q % STAGES, s + AHEAD);
             else read_x((Q + 1) % STAGES, s + AHEAD - STEPS);
-            if (Q == TURNS - 1 && m == 0 && k >= 2) read_codes(k - 2);
+            if (Q == TURNS - PARTS - 1 && s == STEPS / 2) {       // (what the unit's last 64 rows of K are made from)
 #pragma unroll
-            for (int f = 0; f < FN; ++f) {
-                f32x16& sum = FIRST ? acc[f][m] : low[F32 ? f : 0][F32 ? m : 0];
-                sum = matrix_step32<F32>(w[k & 1][f], x[s % R], sum);
+                for (int f = 0; f < F; ++f) last[f] = codes[f][3];
             }
-            constexpr int AFTER = P < PARTS - 1 ? 4 * J : 4 * J + 4;   // the unit's 16 rows of K that follow this turn
+            if (Q == TURNS - 1 && s == 0) read_codes();
 #pragma unroll
-            for (int i = 0; i < PER; ++i) operand_dword((k < 3 ? 4 * J + k + 1 : AFTER) % 16, m * PER + i, w[(k + 1) & 1]);
+            for (int f = 0; f < F; ++f) {
+                f32x4& sum = FIRST ? acc[f][m] : low[F32 ? f : 0][F32 ? m : 0];
+                sum = matrix_step<F32>(w[k & 1][f], x[s % R], sum);
+            }
+            if (k < 1 ? P == 0 : P == PARTS - 1) {                // (a stage's parts meet the same weights)
 #pragma unroll
-            for (int f = 0; f < FN; ++f) {
+                for (int i = 0; i < PER; ++i) operand_dword((k < 1 ? 2 * J + 1 : 2 * J + 2) % 8, m * PER + i, w[(k + 1) & 1]);
+            }
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
                 __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);               // a product,
-                __builtin_amdgcn_sched_group_barrier(0x2, (2 * PER + FN - 1) / FN, 0);  // then vector instructions
+                __builtin_amdgcn_sched_group_barrier(0x2, (2 * PER + F - 1) / F, 0);  // then vector instructions
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -421,68 +446,58 @@ __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArg
         });
     };
     int u = 0;
-    for (; (u + 1) * TURNS + STAGES - 1 <= total; ++u) turns(std::true_type{}, u, TURNS);
+    const int whole = a.planes == 1 || a.K % kStageRows == 0 ? total - (a.K % kStageRows ? PARTS : 0) : 0;   // turns before one that might end early
+    for (; (u + 1) * TURNS + STAGES - 1 <= whole; ++u) turns(std::true_type{}, u, TURNS);
     for (; u < units; ++u) turns(std::false_type{}, u, min(total - u * TURNS, TURNS));
 
     // ---- out ----
-    constexpr int OUT_FN = MODE == kTwoWeights ? FN / 2 : FN;
+    constexpr int WAVE_N = MODE == kTwoWeights ? FN * 16 : FN * 32;   // output columns of a wave
     if constexpr (WK > 1) {
         // every wave has sums of the whole tile, of its own rows of K: they meet in LDS (a wave's in its own part, which it is
-        // done with), and wave i goes on with fragment i.  fp32 activations' are added up in 64 bits: roundings in 32 would weigh.
-        constexpr int FRAGMENT = 64 * 16 * 4, PIECES = F32 ? 2 : 1;
-        static_assert(PIECES * FN * FM * FRAGMENT <= OWN, "a wave's sums fit its part of LDS");
+        // done with), and each goes on with 16 rows, or, where those are fewer than waves, with a group of their columns.  fp32
+        // activations' are added up in 64 bits: roundings in 32 would weigh.
+        constexpr int FRAGMENT = 64 * 4 * 4, PIECES = F32 ? 2 : 1;
+        static_assert(PIECES * F * G * FRAGMENT <= OWN, "a wave's sums fit its part of LDS");
 #pragma unroll
-        for (int i = 0; i < FN * FM; ++i)
+        for (int f = 0; f < F; ++f)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                auto put = [&](int piece, const f32x16& v) {
-                    *reinterpret_cast<f32x4*>(lds + (piece * FN * FM + i) * FRAGMENT + q * 1024 + lane * 16) = f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
-                };
-                put(0, acc[i / FM][i % FM]);
-                if constexpr (F32) put(1, low[i / FM][i % FM]);
+            for (int g = 0; g < G; ++g) {
+                *reinterpret_cast<f32x4*>(lds + (f * G + g) * FRAGMENT + lane * 16) = acc[f][g];
+                if constexpr (F32) *reinterpret_cast<f32x4*>(lds + (F * G + f * G + g) * FRAGMENT + lane * 16) = low[f][g];
             }
         __syncthreads();
-        auto total_of = [&](int i, f32x16& v) {
+        constexpr int MINE = G < WK ? CF : FW;                    // fragments of a weight that a wave goes on with
+        const int rows = wk % G, group = wk / G;
+        if (group >= FW / MINE) return;
+        f32x4 v[F / FW * MINE][1];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                std::conditional_t<F32, double, float> sum[4] = {};
+        for (int f = 0; f < F / FW * MINE; ++f) {
+            const int from = (f / MINE * FW + group * MINE + f % MINE) * G + rows;
+            std::conditional_t<F32, double, float> sum[4] = {};
 #pragma unroll
-                for (int piece = PIECES - 1; piece >= 0; --piece) {
+            for (int piece = PIECES - 1; piece >= 0; --piece) {
 #pragma unroll
-                    for (int o = 0; o < WK; ++o) {
-                        const f32x4 part = *reinterpret_cast<const f32x4*>(all_lds + o * OWN + (piece * FN * FM + i) * FRAGMENT + q * 1024 + lane * 16);
+                for (int o = 0; o < WK; ++o) {
+                    const f32x4 part = *reinterpret_cast<const f32x4*>(all_lds + o * OWN + (piece * F * G + from) * FRAGMENT + lane * 16);
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) sum[e] += part[e];
-                    }
-                    if (piece == 1)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) sum[e] *= 1.0f / kLowScale;
+                    for (int e = 0; e < 4; ++e) sum[e] += part[e];
                 }
+                if (piece == 1)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[4 * q + e] = (float)sum[e];
+                    for (int e = 0; e < 4; ++e) sum[e] *= 1.0f / kLowScale;
             }
-        };
-        if constexpr (MODE == kTwoWeights) {
-            if (wk >= OUT_FN * FM) return;
-            f32x16 v[2][1];
-            total_of(wk, v[0][0]);
-            total_of(wk + OUT_FN * FM, v[1][0]);
-            put_out<2, 1, MODE>(a, v, m0 + wk % FM * 32 + r32, nb0 * 16 + wk / FM * 32 + h * 16);
-        } else {
-            f32x16 v[1][1];
-            total_of(wk, v[0][0]);
-            put_out<1, 1, MODE>(a, v, m0 + wk % FM * 32 + r32, nb0 * 16 + wk / FM * 32 + h * 16);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[f][0][e] = (float)sum[e];
         }
+        put_out<CF, MINE, F / FW * MINE, 1, MODE>(a, v, m0 + rows * 16 + r16, nb0 * 16 + group * 16 * MINE + q * 4 * CF);
     } else {
         if constexpr (F32) {
 #pragma unroll
-            for (int f = 0; f < FN; ++f)
+            for (int f = 0; f < F; ++f)
 #pragma unroll
-                for (int m = 0; m < FM; ++m)
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) acc[f][m][e] = fmaf(low[f][m][e], 1.0f / kLowScale, acc[f][m][e]);
+                for (int m = 0; m < G; ++m) add_low(acc[f][m], low[f][m]);
         }
-        put_out<FN, FM, MODE>(a, acc, m0 + wm * FM * 32 + r32, (nb0 + wn * OUT_FN * 2) * 16 + h * 16);
+        put_out<CF, FW, F, G, MODE>(a, acc, m0 + wm * FM * 32 + r16, nb0 * 16 + wn * WAVE_N + q * 4 * CF);
     }
 }
 
