@@ -466,7 +466,8 @@ __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArg
                 if constexpr (F32) *reinterpret_cast<f32x4*>(lds + (F * G + f * G + g) * FRAGMENT + lane * 16) = low[f][g];
             }
         __syncthreads();
-        constexpr int MINE = G < WK ? CF : FW;                    // fragments of a weight that a wave goes on with
+        constexpr int MINE = CF > FW * G / WK ? CF : FW * G / WK; // fragments of a weight that a wave goes on with
+        static_assert(FW % MINE == 0 && FW / MINE * G <= WK, "the waves take all of the tile");
         const int rows = wk % G, group = wk / G;
         if (group >= FW / MINE) return;
         f32x4 v[F / FW * MINE][1];
@@ -741,11 +742,13 @@ int launch_tile(const KernelArgs& a, hipStream_t st)
 }
 
 // Which tile, by how many there are and by the units of 256 rows of K (a multiple of the units is shared out evenly).  us, fp16;
-// "shared": 64 x 64, K shared out among four waves; "small": 64 x 64, a wave 32 x 32; "wide": 64 x 128, a wave 64 x 32 (two weights:
-// 32 x 64); "flat": 64 x 256; "tall": 128 x 256, a wave 64 or 128 rows x 64:
-//   up to one 64 x 64 tile a compute unit: shared from four units of K on, small below, where waves would have no unit of their own.
-//     Shared / small / flat, 64 rows -> 4096: K = 256 5.3 / 3.9 / 6.2, 768 5.7 / 5.2 / 8.8, 1024 5.8 / 5.9 / 10.0, 2048 7.4 / 8.6 / 15.3; two weights
-//     (wide) 256 6.3 / 5.1 / 6.5, 512 6.5 / 6.2 / 7.9, 1024 6.8 / 8.0 / 10.5.  fp32 256 11.6 / 9.6 / 12.5, 512 12.1 / 12.1 / 16.4, 768 12.2 / 14.3 / 20.0.
+// "shared": K shared out among four waves, 32 x 32, 32 x 64 or 64 x 64; "small": 64 x 64, a wave 32 x 32; "wide": 64 x 128, a wave 64 x 32
+// (two weights: 32 x 64); "flat": 64 x 256; "tall": 128 x 256, a wave 64 or 128 rows x 64:
+//   shared up to one 64 x 64 tile a compute unit.  Bound by what a compute unit copies (some 40 bytes a clock, of which each wave's activations
+//     are most), so the smallest tile of which each compute unit has at most one, and 32 x 64 two to a unit for fp32.  32 x 32 / 32 x 64 / 64 x 64, 64 rows ->
+//     4096: K = 512 4.3 / - / 5.0, 4096 6.3 / 8.0 / 10.8, 11008 11.4 / 15.5 / 20; fp32 512 9.6 / 10.1 / 12.4, 2048 12.8 / 13.2 / 17.4, 11008 36 / 37 / 55;
+//     200 rows 2048 -> 2048 6.3 / 6.0 / 8.1, fp32 15.5 / 14.6 / 19.7.  Two 32 x 64 tiles a unit against one 64 x 64, -> 4096: fp32 200 rows of 4096 28.6 / 30.2,
+//     256 of 512 11.0 / 13.7; fp16 256 of 1024 6.5 / 6.7, but 200 of 4096 12.5 / 12.1, and 256 of 256 5.4 (small: 4.5).
 //   wide up to one of its tiles a unit, and up to two where it still gains.  Shared (which fits a unit once) / wide / flat, 512 rows
 //     -> 4096: K = 256 10.0 / 5.4 / 6.7, 1024 11.2 / 8.3 / 11.0, 4096 23.0 / 22.0 / 27.3; fp32 21.6 / 13.1 / 14.8, 25.8 / 23.1 / 28.1, 61.5 / 58.0 / 75.5.
 //     Wide / flat, 1024 rows -> 4096: 256 7.1 / 7.7, 2048 19.9 / 20.3; fp32 17.4 / 18.6, but 55.0 / 54.8, and 768 rows of 4096 81.9 / 78.4; past that
@@ -762,11 +765,17 @@ int launch_mode(const KernelArgs& a, hipStream_t st)
     const int64_t units = compute_units(), columns = (int64_t)a.N * (TWO ? 2 : 1), depth = (int64_t)a.planes * a.units;
     auto tiles = [&](int rows, int width) { return ceil_div(a.call_rows, rows) * ceil_div(columns, width); };
     const bool one_each = tiles(64, 64) <= units;
-    if (one_each && depth > (PARTS > 1 ? 1 : TWO ? 2 : 3)) return launch_tile<PARTS, 1, 1, 4, 2, 2, MODE>(a, st);
+    if (one_each) {
+        if (tiles(32, 32) <= units) return launch_tile<PARTS, 1, 1, 4, 1, 1, MODE>(a, st);
+        if (PARTS > 1 || tiles(32, 64) <= units || (depth > 3 && depth <= 8)) return launch_tile<PARTS, 1, 1, 4, 1, 2, MODE>(a, st);
+        if constexpr (PARTS == 1) {
+            if (depth > 3) return launch_tile<PARTS, 1, 1, 4, 2, 2, MODE>(a, st);
+            if constexpr (!TWO) return launch_tile<PARTS, 2, 2, 1, 1, 1, MODE>(a, st);
+        }
+    }
     if constexpr (TWO) {
         if (tiles(64, 128) <= units) return launch_tile<PARTS, 2, 2, 1, 1, 2, MODE>(a, st);
     } else {
-        if (one_each) return launch_tile<PARTS, 2, 2, 1, 1, 1, MODE>(a, st);
         if (tiles(64, 128) <= (PARTS == 1 || depth <= 4 ? 2 : 1) * units) return launch_tile<PARTS, 1, 4, 1, 2, 1, MODE>(a, st);
     }
     if constexpr (PARTS == 1) {

@@ -344,3 +344,24 @@ def test_a_blob_without_codes(cuda, oracle):
         print(f"case M={M}", flush=True)
         y = ops.spmm(dev, x.to(cuda), out_dtype=torch.float32)
         assert np.array_equal(y.cpu().numpy().astype(np.float64), oracle.fast_product(x.double().numpy(), w))
+
+
+# few tiles, whose waves share K (two compute units' worth of 64 x 64 at most): 64 x 64 of nine units and of three; 32 x 64 two to a unit;
+# 32 x 32 with rows, columns and a stage left over, and of one unit, which leaves waves without a share
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M,K,N", [(250, 2304, 4000), (250, 520, 4000), (253, 1100, 3970), (97, 1412, 1001), (49, 130, 33)])
+def test_tiles_whose_waves_share_k(cuda, M, K, N, dtype):
+    """Integer activations: every sum is exact, whatever its order; two weights and pairs against the gate of the products."""
+    from ternaryllm_amd import ops
+    N2 = N // 2 * 2
+    w, w2 = ternary_weight(K, N, 0.6, M), ternary_weight(K, N, 0.7, N)
+    dw, dw2 = _device(w, cuda), _device(w2, cuda)
+    x = activations(M, K, K, dtype, integer=True).to(cuda)
+    print(f"case M={M} K={K} N={N} {dtype}", flush=True)
+    one, two = x.double() @ torch.from_numpy(w).double().to(cuda), x.double() @ torch.from_numpy(w2).double().to(cuda)
+    assert torch.equal(ops.spmm(dw, x, out_dtype=torch.float32).double(), one)
+    x, one, two = x / 16, one / 16, two / 16
+    got, want = ops.mlp_gate_up(dw, dw2, x, out_dtype=torch.float32).double(), torch.nn.functional.silu(one) * two
+    assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())              # exact sums; __expf and the division
+    even = _device(w[:, :N2].copy(), cuda)
+    assert torch.equal(ops.spmm_gated(even, x), ops.silu_mul(ops.spmm(even, x), pairs=True))
