@@ -945,3 +945,23 @@ def test_steps_use_the_norms_as_they_are(cuda, B):
     handle.remove()
     m.layers[0].post_attention_layernorm = torch.nn.LayerNorm(256).to(cuda, torch.float16)
     assert float((both() - as_built).norm() / as_built.norm()) > 0.005
+
+
+# a wave to a row with one, two, four and eight vectors a lane, the last of them partly or not at all its own, and rows that are not
+# whole workgroups' (512 rows are two for each compute unit); a workgroup to a row where there are fewer rows, or more vectors
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,width", [(512, 8), (513, 512), (515, 520), (517, 1032), (1030, 2048), (513, 2056), (514, 4096), (5, 2048), (511, 4096), (600, 4104)])
+def test_add_rmsnorm_of_every_width(cuda, rows, width, dtype):
+    from ternaryllm_amd import ops
+    g = torch.Generator().manual_seed(rows + width)
+    x, y, w = (torch.randn(s, generator=g).to(dtype).to(cuda) for s in ((rows, width), (rows, width), (width,)))
+    for other in (y, None):
+        out, h = ops.add_rmsnorm(x, other, w, 1e-5)
+        s = x if other is None else x + other
+        if other is not None:
+            assert torch.equal(out, s)
+        want = s.double() * torch.rsqrt(s.double().square().mean(-1, keepdim=True) + 1e-5) * w.double()
+        assert torch.equal(ops.add_rmsnorm(x, other, w, 1e-5, kmajor=True)[1].t(), h)
+        # fp16: one rounding, 2^-11, and what fp32 arithmetic adds to it; fp32: a sum of squares (a lane's at most 16, then 6
+        # steps), rsqrt and two products, 2^-23 each at most
+        assert bool(((h.double() - want).abs() <= (2.0 ** -10.9 if dtype == torch.float16 else 16 * 2.0 ** -23) * want.abs() + 2.0 ** -24).all())
