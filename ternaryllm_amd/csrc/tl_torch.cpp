@@ -101,7 +101,7 @@ at::Tensor output(const at::Tensor& x, const Rows& r, int64_t N, bool kmajor)
 
 const tl_layout_header* header_at(PyObject* address) { return static_cast<const tl_layout_header*>(PyLong_AsVoidPtr(address)); }
 
-// product(header address, blob, x, scale or None, kmajor) -> tensor or None
+// product(header address, blob, x, scale or None, kmajor or None: x of K values a row is rows) -> tensor or None
 PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
     HANDLE_TH_ERRORS
@@ -111,7 +111,7 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t count)
     }
     const tl_layout_header* header = header_at(args[0]);
     const at::Tensor *blob = plain(args[1]), *x = plain(args[2]), *scale;
-    const bool kmajor = args[4] == Py_True;
+    const bool kmajor = args[4] == Py_None ? header && x && x->dim() > 0 && x->size(-1) != header->inners : args[4] == Py_True;
     Rows r;
     if (!header || !blob || !x || x->device() != blob->device() || type_code(*x) < 0 || !geometry(*x, header->inners, kmajor, &r) ||
         !scale_fits(args[3], &scale, header->columns, x->device()))

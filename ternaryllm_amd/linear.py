@@ -230,6 +230,12 @@ class TernaryLinear(nn.Module):
     def forward(self, input):
         """input: (batch, rows, K), (rows, K) or (K,) -- also (batch, K, rows) as the reference kernel
         reads it; returns (batch, rows, N) / (rows, N) / (N,) in the input dtype."""
+        # (buffers are looked up where they are kept: one row 4096 x 4096 took 4.9 us of the host through the module's attributes, 4.5)
+        w, buffers = self._handle, self._buffers
+        if w is not None and w.blob is buffers.get("w_packed"):
+            y = ops.product(w, input, buffers["w_scale"] if "w_scale" in buffers else self.w_scale, None)
+            if y is not None:
+                return y
         if input.dim() > 3:
             raise AssertionError("Input has dim larger than 3")  # the reference asserts (TernaryLinear.py:161)
         w = self.device_weight()

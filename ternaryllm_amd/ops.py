@@ -117,8 +117,8 @@ def _short():
 
 
 def product(weight, x, scale=None, kmajor=False):
-    """(x @ W) * scale the short way, for x [.., K] of up to three dimensions or, kmajor, [K, rows] or [1, K, rows]; returns
-    [.., N] in x's type, or None where the call is not a plain one (spmm then takes it or says what is wrong)."""
+    """(x @ W) * scale the short way, for x [.., K] of up to three dimensions or, kmajor, [K, rows] or [1, K, rows] (kmajor None:
+    whichever x is); returns [.., N] in x's type, or None where the call is not a plain one (spmm then takes it or says what is wrong)."""
     return _short().product(ctypes.addressof(weight.header), weight.blob, x, scale, kmajor)
 
 
