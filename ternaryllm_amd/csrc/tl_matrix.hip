@@ -250,14 +250,16 @@ __device__ __forceinline__ void put_out(const KernelArgs& a, f32x4 (&acc)[F][G],
 //
 // Output tiles of (WM * FM * 32) activation rows x (WN * FN * 32) columns, one per workgroup; a wave owns FM * 32 rows x
 // FN * 32 columns.  WK = 1: WM x WN waves over all of K that share what they copy.  WK > 1: one tile of a wave, whose WK waves
-// share K out by units, copy for themselves, wait for nobody and add up at the end.  PARTS: 1 for fp16 activations, 3 for fp32
+// share K out by units, copy for themselves, wait for nobody and add up at the end; or, WN > 1, two groups of waves that share K out
+// and whose waves share what they copy.  PARTS: 1 for fp16 activations, 3 for fp32
 // ones in bf16 parts (a stage's three parts one after the other, with the same codes).
 template <int PARTS, int WM, int WN, int WK, int FM, int FN, int MODE>
 __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArgs a)
 {
-    constexpr int W = WK > 1 ? 1 : WM * WN;                       // waves that work on the same rows of K, and share what is copied
+    constexpr int W = WM * WN;                                    // waves that work on the same rows of K, and share what is copied
+    constexpr bool SHARED = W > 1;
     constexpr int TM = WM * FM * 32, TN = WN * FN * 32;
-    static_assert(WK == 1 || (WM == 1 && WN == 1 && 2 * FM <= WK), "waves share either an output tile's rows of K or its outputs");
+    static_assert(WK == 1 || (W == 1 && 2 * FM <= WK) || (WM == 1 && WK == 2), "how the sums of waves that share out K meet");
     constexpr int STAGES = kUnitStages;                           // buffers of activations: a stage's place in its unit names its buffer
     constexpr int XB = TM * kStageRowBytes;                       // bytes of a stage of activations
     constexpr int XL = TM / 8 / W;                                // activation loads of a wave per stage (8 rows each)
@@ -266,7 +268,7 @@ __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArg
     extern __shared__ __align__(16) unsigned char all_lds[];
     const int lane = threadIdx.x & 63;
     const int wg_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wave = WK > 1 ? 0 : wg_wave, wk = WK > 1 ? wg_wave : 0;
+    const int wave = wg_wave % W, wk = wg_wave / W;
     const int wm = wave / WN, wn = wave % WN;
     constexpr int OWN = STAGES * XB + (TN / 16) * TL_CODE_UNIT_BYTES;   // LDS of the waves that share
     unsigned char* lds = all_lds + wk * OWN;
@@ -304,7 +306,8 @@ __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArg
     // this wave's units, and its turns: the last stage of the only plane may end a unit early
     const int unit0 = all_units * wk / WK, units = all_units * (wk + 1) / WK - unit0;
     const int all_stages = a.planes == 1 ? stages_k : all_units * kUnitStages;
-    const int total = PARTS * (min((unit0 + units) * kUnitStages, all_stages) - unit0 * kUnitStages);
+    auto turns_of = [&](int first, int count) { return PARTS * (min((first + count) * kUnitStages, all_stages) - first * kUnitStages); };
+    const int total = turns_of(unit0, units);
 
     // load side: the unit, within its plane, of the next activations to ask for; their stage and part follow from the turn
     int lk = unit0 % a.units, issued = 0;
@@ -387,12 +390,12 @@ __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArg
     auto operand_dword = [&](int j, int d, u32x4* to) {
         to[d / 4][d % 4] = ((j >= 6 ? last[d / 4] : codes[d / 4][j >> 1]) << ((j & 1) * 8 + 2 * (d % 4))) & 0xC000C000u;
     };
-    if (WK == 1 || units > 0) issue_codes(0);
+    if (units > 0) issue_codes(0);
     static_for<STAGES - 1>([&](auto s) {
         if (issued < total) issue_x(s, std::false_type{});
     });
-    if (total >= STAGES - 1) loads_here<WK == 1, (STAGES - 2) * XL>();
-    else loads_here<WK == 1, 0>();
+    if (total >= STAGES - 1) loads_here<SHARED, (STAGES - 2) * XL>();
+    else loads_here<SHARED, 0>();
     read_codes();
 #pragma unroll
     for (int s = 0; s < AHEAD; ++s) read_x(0, s);
@@ -410,8 +413,8 @@ __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArg
             const int m = s % G, k = s / G;                       // k: 32 rows of K of the stage
             if (s == STEPS - AHEAD) {
                 // turn t + 1's activations have come; every wave is done with turn t - 1, whose buffer takes turn t + STAGES - 1
-                if (STEADY) loads_here<WK == 1, (STAGES - 3) * XL>();
-                else if (t + 1 < total) loads_here<WK == 1, 0>();
+                if (STEADY) loads_here<SHARED, (STAGES - 3) * XL>();
+                else if (t + 1 < total) loads_here<SHARED, 0>();
                 if (Q == 0 && (STEADY || u + 1 < units)) issue_codes(u + 1);
                 if (STEADY || issued < total) issue_x(std::integral_constant<int, (Q + STAGES - 1) % TURNS>{}, steady_tag);
             }
@@ -450,9 +453,53 @@ __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArg
     for (; (u + 1) * TURNS + STAGES - 1 <= whole; ++u) turns(std::true_type{}, u, TURNS);
     for (; u < units; ++u) turns(std::false_type{}, u, min(total - u * TURNS, TURNS));
 
+    // (waves that meet at barriers take as many of them: a group whose share of K is shorter waits for the longest)
+    if constexpr (SHARED && WK > 1) {
+        int most = 0;
+#pragma unroll
+        for (int o = 0; o < WK; ++o) most = max(most, turns_of(all_units * o / WK, all_units * (o + 1) / WK - all_units * o / WK));
+        for (int i = max(total, 1); i < most; ++i) __builtin_amdgcn_s_barrier();
+    }
+
     // ---- out ----
     constexpr int WAVE_N = MODE == kTwoWeights ? FN * 16 : FN * 32;   // output columns of a wave
-    if constexpr (WK > 1) {
+    if constexpr (SHARED && WK > 1) {
+        // A wave and the other group's wave of the same outputs give each other half of their sums, by rows, through LDS (all of the
+        // workgroup's, which every wave is done with); fp32 activations' are added up in 64 bits.
+        constexpr int FRAGMENT = 64 * 4 * 4, HALF = G / 2, GIVEN = (F32 ? 2 : 1) * F * HALF * FRAGMENT;
+        f32x4 v[F][HALF], v_low[F32 ? F : 1][F32 ? HALF : 1];
+        unsigned char* mine = all_lds + wg_wave * GIVEN + lane * 16;
+        const unsigned char* other = all_lds + ((1 - wk) * W + wave) * GIVEN + lane * 16;
+        __syncthreads();
+#pragma unroll
+        for (int f = 0; f < F; ++f)
+#pragma unroll
+            for (int g = 0; g < HALF; ++g) {
+                v[f][g] = wk ? acc[f][HALF + g] : acc[f][g];
+                *reinterpret_cast<f32x4*>(mine + (f * HALF + g) * FRAGMENT) = wk ? acc[f][g] : acc[f][HALF + g];
+                if constexpr (F32) {
+                    v_low[f][g] = wk ? low[f][HALF + g] : low[f][g];
+                    *reinterpret_cast<f32x4*>(mine + (F * HALF + f * HALF + g) * FRAGMENT) = wk ? low[f][g] : low[f][HALF + g];
+                }
+            }
+        __syncthreads();
+#pragma unroll
+        for (int f = 0; f < F; ++f)
+#pragma unroll
+            for (int g = 0; g < HALF; ++g) {
+                const f32x4 high = *reinterpret_cast<const f32x4*>(other + (f * HALF + g) * FRAGMENT);
+                if constexpr (F32) {
+                    const f32x4 rest = *reinterpret_cast<const f32x4*>(other + (F * HALF + f * HALF + g) * FRAGMENT);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        v[f][g][e] = (float)(((double)v_low[f][g][e] + rest[e]) * (1.0 / kLowScale) + ((double)v[f][g][e] + high[e]));
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[f][g][e] += high[e];
+                }
+            }
+        put_out<CF, FW, F, HALF, MODE>(a, v, m0 + wk * HALF * 16 + r16, nb0 * 16 + wn * WAVE_N + q * 4 * CF);
+    } else if constexpr (WK > 1) {
         // every wave has sums of the whole tile, of its own rows of K: they meet in LDS (a wave's in its own part, which it is
         // done with), and each goes on with 16 rows, or, where those are fewer than waves, with a group of their columns.  fp32
         // activations' are added up in 64 bits: roundings in 32 would weigh.
@@ -731,7 +778,9 @@ template <int PARTS, int WM, int WN, int WK, int FM, int FN, int MODE>
 int launch_tile(const KernelArgs& a, hipStream_t st)
 {
     constexpr int TM = WM * FM * 32, TN = WN * FN * 32, OUT_TN = MODE == kTwoWeights ? TN / 2 : TN;
-    constexpr size_t lds = WK * ((size_t)kUnitStages * TM * kStageRowBytes + (TN / 16) * TL_CODE_UNIT_BYTES);
+    constexpr size_t copied = WK * ((size_t)kUnitStages * TM * kStageRowBytes + (TN / 16) * TL_CODE_UNIT_BYTES);
+    constexpr size_t given = WK > 1 && WN > 1 ? (size_t)TM * TN * sizeof(float) * (PARTS > 1 ? 2 : 1) : 0;   // half of each group's sums
+    constexpr size_t lds = copied > given ? copied : given;
     static_assert(lds <= 160 * 1024, "the stages fit a compute unit's LDS");
     auto kernel = tl_matrix_rows<PARTS, WM, WN, WK, FM, FN, MODE>;
     static LdsLimit raised;
@@ -751,8 +800,11 @@ int launch_tile(const KernelArgs& a, hipStream_t st)
 //     256 of 512 11.0 / 13.7; fp16 256 of 1024 6.5 / 6.7, but 200 of 4096 12.5 / 12.1, and 256 of 256 5.4 (small: 4.5).
 //   wide up to one of its tiles a unit, and up to two where it still gains.  Shared (which fits a unit once) / wide / flat, 512 rows
 //     -> 4096: K = 256 10.0 / 5.4 / 6.7, 1024 11.2 / 8.3 / 11.0, 4096 23.0 / 22.0 / 27.3; fp32 21.6 / 13.1 / 14.8, 25.8 / 23.1 / 28.1, 61.5 / 58.0 / 75.5.
-//     Wide / flat, 1024 rows -> 4096: 256 7.1 / 7.7, 2048 19.9 / 20.3; fp32 17.4 / 18.6, but 55.0 / 54.8, and 768 rows of 4096 81.9 / 78.4; past that
-//     1024 rows of 1024 -> 11008 28.1 / 26.8; two weights, 768 rows of 2048 -> 2048 20.0 / 17.7.
+//     Wide / flat, 1024 rows -> 4096: 256 7.1 / 7.7, 2048 19.9 / 20.3; fp32 17.4 / 18.6; past that 1024 rows of 1024 -> 11008 28.1 / 26.8; two weights, 768
+//     rows of 2048 -> 2048 20.0 / 17.7.
+//   "groups": 64 x 256 for eight waves, two for each 64 columns, which share K out, while such tiles are one a unit and K is long: with flat ones a unit has four
+//     waves, one on each SIMD.  Wide / groups, 1024 rows -> 4096: 512 8.0 / 9.3, 1024 12.0 / 12.4, 4096 28.8 / 27.3, 11008 73.5 / 65; fp32 512 19.2 / 21.3, 1024 29.7 / 30.7;
+//     flat / groups, fp32, 4096: 76.0 / 71.3, 768 rows 73.3 / 68.1.
 //   tall where there are two of them a unit, so that one multiplies while the other waits or stores, and where flat ones would
 //     not spread the rows better: 2048 x 4096 -> 11008 141 / 150, 8192 x 2048 -> 11008 273 / 287, 8192 x 2048 -> 2048 57 / 59, but
 //     1536 x 4096 -> 11008 129 / 117, both with slower last steps (516 tall tiles are three for some units, 1032 flat ones five
@@ -776,7 +828,11 @@ int launch_mode(const KernelArgs& a, hipStream_t st)
     if constexpr (TWO) {
         if (tiles(64, 128) <= units) return launch_tile<PARTS, 2, 2, 1, 1, 2, MODE>(a, st);
     } else {
-        if (tiles(64, 128) <= (PARTS == 1 || depth <= 4 ? 2 : 1) * units) return launch_tile<PARTS, 1, 4, 1, 2, 1, MODE>(a, st);
+        if (tiles(64, 128) <= units) return launch_tile<PARTS, 1, 4, 1, 2, 1, MODE>(a, st);
+    }
+    if (tiles(64, 256) <= units && depth > (PARTS > 1 ? 4 : 8)) return launch_tile<PARTS, 1, 4, 2, 2, 2, MODE>(a, st);
+    if constexpr (!TWO) {
+        if (tiles(64, 128) <= 2 * units) return launch_tile<PARTS, 1, 4, 1, 2, 1, MODE>(a, st);
     }
     if constexpr (PARTS == 1) {
         const int64_t tall = tiles(128, 256), flat = tiles(64, 256);

@@ -365,3 +365,11 @@ def test_tiles_whose_waves_share_k(cuda, M, K, N, dtype):
     assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())              # exact sums; __expf and the division
     even = _device(w[:, :N2].copy(), cuda)
     assert torch.equal(ops.spmm_gated(even, x), ops.silu_mul(ops.spmm(even, x), pairs=True))
+
+
+# two groups of four waves that share K: eleven units (five and six) and a last one of one stage or of eight rows, for one weight and, at
+# half the rows, for two
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M,K,N", [(900, 2568, 4090), (500, 2616, 4090), (1000, 2816, 3850)])
+def test_groups_of_waves_that_share_k(cuda, M, K, N, dtype):
+    test_tiles_whose_waves_share_k(cuda, M, K, N, dtype)
