@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "tl_common.h"
+#include "tl_silu.h"
 
 namespace tl {
 
@@ -136,14 +137,12 @@ __device__ __forceinline__ void store_out(void* Y, int is_f16, long long off, fl
     else static_cast<float*>(Y)[off] = v;
 }
 
-__device__ __forceinline__ float silu(float g) { return g / (1.0f + __expf(-g)); }
-
 // v as a stored output of the call's type would read back
 __device__ __forceinline__ float as_output(float v, int is_f16) { return is_f16 ? __half2float(__float2half(settled(v))) : v; }
 
 // silu(g) * u for a product's outputs g, u (already rounded to the output type), with the roundings of the separate
 // operator: the SiLU is rounded to the type before the product.
-__device__ __forceinline__ float gate_pair(float g, float u, int is_f16) { return as_output(g / (1.0f + __expf(-g)), is_f16) * u; }
+__device__ __forceinline__ float gate_pair(float g, float u, int is_f16) { return as_output(silu(g, is_f16), is_f16) * u; }
 
 // One output of a single-row product on its way out: plain, or added to the residual row as a separate add of the
 // stored product would add it.
