@@ -19,7 +19,8 @@ constexpr int kStageRows = 64;                       // rows of K of a stage
 constexpr int kStageRowBytes = kStageRows * 2;       // bytes of one activation row in a stage
 // Row tiles whose column tiles a part of the chip works through together.  An activation tile is eight times the bytes of
 // a code tile along the same K (24 times for fp32 in three parts), so few row tiles against many column tiles is least traffic: 8192 x 2048 -> 11008 took 456 us
-// with all 64 row tiles in one group (every column tile streamed all activations through an L2), 300 / 300 / 310 with 2 / 4 / 8.
+// with all 64 row tiles in one group (every column tile streamed all activations through an L2), 300 / 300 / 310 with 2 / 4 / 8 (gated, as
+// it is now, 246 / 247 / 249 and 255 with 16).
 constexpr int kRowGroup = 4;
 constexpr int kUnitStages = TL_CODE_UNIT_ROWS / kStageRows;
 __device__ __align__(16) const unsigned char kNoCodes[TL_CODE_UNIT_BYTES] = {};   // a unit of zero weights
@@ -243,8 +244,8 @@ __device__ __forceinline__ void put_out(const KernelArgs& a, f32x4 (&acc)[F][G],
 // memory, 16 x 16 x 32 products run at 2200 TFLOP/s in fp16 and 2230 in bf16, 32 x 32 x 16 ones at 1750 and 1880 (with the weights as
 // the second operand 1970; at 66 % zeros).  With all that stands around them 8192 x 5504 -> 2048 runs at 1600, or 1760 without what a
 // launch costs; without making operands and reading LDS it would take 8 % less.  A wave owns 64 columns: each fragment of
-// activations that it reads from LDS serves four products.  us with 32 x 32 x 16 / now: 8192 x 2048 -> 11008 gated 281 / 250, 8192 x 2048 -> 6144
-// 156 / 140, 8192 x 5504 -> 2048 133 / 116, 1024 x 4096 -> 11008 78 / 71; fp32 4096 x 4096 -> 4096 292 / 256, 1024 x 4096 -> 4096 85 / 76.
+// activations that it reads from LDS serves four products.  us with 32 x 32 x 16 / now: 8192 x 2048 -> 11008 gated 281 / 247, 8192 x 2048 -> 6144
+// 156 / 140, 8192 x 5504 -> 2048 133 / 116, 1024 x 4096 -> 11008 78 / 71; fp32 4096 x 4096 -> 4096 292 / 250, 1024 x 4096 -> 4096 85 / 71.
 // A lone wave on its SIMD is bound by what it issues, of which twice as many products are more: the load side's addresses
 // are scalar and follow from the turn (fp32 1024 x 4096 -> 4096 82 us while they were worked out for every load).
 //
@@ -449,7 +450,8 @@ __global__ __launch_bounds__(WM * WN * WK * 64, 2) void tl_matrix_rows(KernelArg
         });
     };
     int u = 0;
-    const int whole = a.planes == 1 || a.K % kStageRows == 0 ? total - (a.K % kStageRows ? PARTS : 0) : 0;   // turns before one that might end early
+    // turns before one that might reach past K: the last stage, or, of several planes, those that fill up every plane's last unit
+    const int whole = a.planes == 1 ? total - (a.K % kStageRows ? PARTS : 0) : a.K % TL_CODE_UNIT_ROWS == 0 ? total : 0;
     for (; (u + 1) * TURNS + STAGES - 1 <= whole; ++u) turns(std::true_type{}, u, TURNS);
     for (; u < units; ++u) turns(std::false_type{}, u, min(total - u * TURNS, TURNS));
 
@@ -806,9 +808,9 @@ int launch_tile(const KernelArgs& a, hipStream_t st)
 //     waves, one on each SIMD.  Wide / groups, 1024 rows -> 4096: 512 8.0 / 9.3, 1024 12.0 / 12.4, 4096 28.8 / 27.3, 11008 73.5 / 65; fp32 512 19.2 / 21.3, 1024 29.7 / 30.7;
 //     flat / groups, fp32, 4096: 76.0 / 71.3, 768 rows 73.3 / 68.1.
 //   tall where there are two of them a unit, so that one multiplies while the other waits or stores, and where flat ones would
-//     not spread the rows better: 2048 x 4096 -> 11008 141 / 150, 8192 x 2048 -> 11008 273 / 287, 8192 x 2048 -> 2048 57 / 59, but
-//     1536 x 4096 -> 11008 129 / 117, both with slower last steps (516 tall tiles are three for some units, 1032 flat ones five
-//     halves).  Not for fp32, whose second set of sums does not fit.
+//     not spread the rows better.  Tall / flat: 2048 x 4096 -> 11008 121 / 125, 8192 x 2048 -> 11008 gated 247 / 255, 8192 x 5504 -> 2048 115 / 122, but
+//     1024 x 4096 -> 11008 76 / 69 (344 tall tiles are two for some units, 688 flat ones five halves).  Not for fp32, whose second
+//     set of sums does not fit.
 // The rows are the whole call's: a row's result does not depend on how many rows at a time a workspace holds.
 template <int PARTS, int MODE>
 int launch_mode(const KernelArgs& a, hipStream_t st)

@@ -40,7 +40,7 @@ def test_many_rows_at_the_edges(cuda, oracle, M, K, N, dtype):
         assert np.array_equal(y, x.numpy()[:, rows] * one[rows, np.arange(N)].astype(np.float32))
 
 
-# one tile of 64 x 64 with five units and a stage shared out over four waves; tiles of 128 x 256 and of 64 x 256 with rows, columns
+# tiles of 32 x 32 with five units and a stage shared out over four waves; tiles of 128 x 256 and of 64 x 256 with rows, columns
 # and stages left over (4093 x 4090 is 512 of the tall ones, as many as two for each compute unit)
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("M,K,N", [(65, 1344, 66), (200, 2048, 1032), (1030, 330, 2100), (4093, 200, 4090)])
@@ -65,7 +65,7 @@ def test_tiles_of_every_shape(cuda, M, K, N, dtype):
     assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())              # exact sums; __expf and the division
 
 
-# few units of K, where one 64 x 64 tile a compute unit is four waves' own 32 x 32 (three units and, beside it, four); one and two 64 x 128
+# few units of K, of which four waves' 32 x 32 tiles leave some without a share (one, two, three and, beside it, four); one and two 64 x 128
 # tiles a unit (two weights: 32 x 64 a wave); 64 x 256 ones that are not enough for 128 x 256
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("M,K,N", [(65, 250, 66), (63, 264, 34), (150, 768, 98), (150, 776, 98), (520, 250, 2058), (520, 1100, 2058), (769, 330, 4090), (2110, 264, 4090)])
@@ -373,3 +373,16 @@ def test_tiles_whose_waves_share_k(cuda, M, K, N, dtype):
 @pytest.mark.parametrize("M,K,N", [(900, 2568, 4090), (500, 2616, 4090), (1000, 2816, 3850)])
 def test_groups_of_waves_that_share_k(cuda, M, K, N, dtype):
     test_tiles_whose_waves_share_k(cuda, M, K, N, dtype)
+
+
+# planes of rows that are named again, where K is whole stages of 64 rows but not whole units of 256 (the stages that fill up a plane's last
+# unit lie past K), and where it is both
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M,K", [(60, 192), (130, 1088), (130, 1024)])
+def test_entries_beyond_one_of_whole_stages(cuda, M, K, dtype):
+    from ternaryllm_amd import ops
+    rng = np.random.default_rng(K)
+    w = rng.integers(-3, 4, (K, 40)) * (rng.random((K, 40)) < 0.3)
+    x = activations(M, K, 6, dtype, integer=True)
+    y = ops.spmm(ops.DeviceWeight(_repeated(w), cuda), x.to(cuda), out_dtype=torch.float32)
+    assert np.array_equal(y.cpu().numpy().astype(np.float64), x.double().numpy() @ w)
