@@ -346,8 +346,8 @@ def test_a_blob_without_codes(cuda, oracle):
         assert np.array_equal(y.cpu().numpy().astype(np.float64), oracle.fast_product(x.double().numpy(), w))
 
 
-# few tiles, whose waves share K (two compute units' worth of 64 x 64 at most): 64 x 64 of nine units and of three; 32 x 64 two to a unit;
-# 32 x 32 with rows, columns and a stage left over, and of one unit, which leaves waves without a share
+# few tiles (one of 64 x 64 a compute unit at most), whose waves share K: 64 x 64 of nine units, and of three, which they own parts of;
+# 32 x 64 two to a compute unit; 32 x 32 with rows, columns and a stage left over, and of one unit, which leaves waves without a share
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("M,K,N", [(250, 2304, 4000), (250, 520, 4000), (253, 1100, 3970), (97, 1412, 1001), (49, 130, 33)])
 def test_tiles_whose_waves_share_k(cuda, M, K, N, dtype):
