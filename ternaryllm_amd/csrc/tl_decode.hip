@@ -585,7 +585,7 @@ __global__ __launch_bounds__(256) void tl_silu_mul_k(const T* __restrict__ gu, T
     // gate and up of column c: side by side halves of the row, or (pairs) neighbours 2c, 2c + 1
     const T* row = gu + (size_t)r * 2 * width;
     const float g = to_f(pairs ? row[2 * c] : row[c]), u = to_f(pairs ? row[2 * c + 1] : row[width + c]);
-    out[i] = from_f<T>(to_f(from_f<T>(silu(g, sizeof(T) == 2))) * u);  // the SiLU is rounded to T before the product, as two separate operators would
+    out[i] = from_f<T>(to_f(from_f<T>(silu(g))) * u);  // the SiLU is rounded to T before the product, as two separate operators would
 }
 
 // The end of a greedy decode step as one launch: token[b] = index of the largest of row b's logits (the first of equal

@@ -142,7 +142,7 @@ __device__ __forceinline__ float as_output(float v, int is_f16) { return is_f16 
 
 // silu(g) * u for a product's outputs g, u (already rounded to the output type), with the roundings of the separate
 // operator: the SiLU is rounded to the type before the product.
-__device__ __forceinline__ float gate_pair(float g, float u, int is_f16) { return as_output(silu(g, is_f16), is_f16) * u; }
+__device__ __forceinline__ float gate_pair(float g, float u, int is_f16) { return as_output(silu(g), is_f16) * u; }
 
 // One output of a single-row product on its way out: plain, or added to the residual row as a separate add of the
 // stored product would add it.

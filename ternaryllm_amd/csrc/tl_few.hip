@@ -449,7 +449,7 @@ __global__ __launch_bounds__(64 * (stage_bytes<XT, IN, FM>(1) > 8192 ? most_wave
         if (n >= a.N) continue;
         const bool first = e == (int)threadIdx.x;
         float v = output(a.w0, col >> 4, m, n, early_scale[0], first);
-        if constexpr (TWO) v = silu(v, a.y_f16) * output(a.w1, 1, m, n, early_scale[1], first);
+        if constexpr (TWO) v = silu(v) * output(a.w1, 1, m, n, early_scale[1], first);
         store_out(a.Y, a.y_f16, m * a.ldy + n, v);
     }
 }

@@ -223,7 +223,7 @@ __device__ __forceinline__ void put_out(const KernelArgs& a, f32x4 (&acc)[F][G],
 #pragma unroll
             for (int i = 0; i < C; ++i) {
                 v[i] = acc[group * CF + i / 4][m][i % 4] * s0[group][i];
-                if constexpr (MODE == kTwoWeights) v[i] = silu(v[i], a.y_f16) * (acc[FW + group * CF + i / 4][m][i % 4] * s1[group][i]);
+                if constexpr (MODE == kTwoWeights) v[i] = silu(v[i]) * (acc[FW + group * CF + i / 4][m][i % 4] * s1[group][i]);
             }
             if constexpr (MODE == kPairs) {
                 if (a.chain_factors) {
@@ -698,7 +698,7 @@ __global__ __launch_bounds__(R > 1 ? 1024 : 256) void tl_walk_rows(KernelArgs a)
         for (int j = 0; j < R; ++j) {
             if (m0 + j >= a.M) break;
             float v = acc[0][c][j] * s0;
-            if constexpr (MODE == kTwoWeights) v = silu(v, a.y_f16) * (acc[1][c][j] * s1);
+            if constexpr (MODE == kTwoWeights) v = silu(v) * (acc[1][c][j] * s1);
             if constexpr (MODE == kPairs) v = gate_pair(as_output(v, a.y_f16), as_output(acc[0][c + 1][j] * s1, a.y_f16), a.y_f16);
             store_out(a.Y, a.y_f16, (long long)(m0 + j) * a.ldy + (MODE == kPairs ? n / 2 : n), v);
         }

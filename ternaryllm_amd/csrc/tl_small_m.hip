@@ -1337,7 +1337,7 @@ __global__ __launch_bounds__(NT) void tl_spmv_direct(KernelArgs a)
 #pragma unroll
             for (int e = 0; e < VE; ++e) {
                 const float gf = (float)g[e];
-                o[e] = XT(round_to_x<XF16>(silu(gf, XF16)) * (float)u[e]);
+                o[e] = XT(round_to_x<XF16>(silu(gf)) * (float)u[e]);
             }
         } else if constexpr (PRO == kProAttnCombine) {
             const int hd = a.pro_hd, sp = a.pro_splits;

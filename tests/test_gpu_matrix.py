@@ -386,3 +386,19 @@ def test_entries_beyond_one_of_whole_stages(cuda, M, K, dtype):
     x = activations(M, K, 6, dtype, integer=True)
     y = ops.spmm(ops.DeviceWeight(_repeated(w), cuda), x.to(cuda), out_dtype=torch.float32)
     assert np.array_equal(y.cpu().numpy().astype(np.float64), x.double().numpy() @ w)
+
+
+# few rows and many
+@pytest.mark.parametrize("M,N", [(32, 11008), (1024, 4096)])
+def test_a_gate_rounded_to_fp16_is_the_fp32_gate_rounded(cuda, M, N):
+    """The SiLU in front of an fp16 result is the fp32 one, a division's quotient: an approximate one shows where the product with the up
+    column is near a tie (a unit of fp32 moves one in some 10^4 results by one of fp16)."""
+    from ternaryllm_amd import ops
+    K = 64
+    g = torch.Generator(device=cuda).manual_seed(M)
+    dg, du = _device(ternary_weight(K, N, 0.5, 51), cuda), _device(ternary_weight(K, N, 0.5, 52), cuda)
+    x = torch.randn((M, K), generator=g, device=cuda).half()
+    scale = 0.1 + 0.3 * torch.rand(N, generator=g, device=cuda)
+    print(f"case M={M}", flush=True)
+    full = ops.mlp_gate_up(dg, du, x, scale, scale, out_dtype=torch.float32)
+    assert torch.equal(ops.mlp_gate_up(dg, du, x, scale, scale, out_dtype=torch.float16), full.half())
