@@ -524,20 +524,26 @@ __global__ __launch_bounds__(256) void tl_add_rmsnorm_rows(const T* __restrict__
         for (int k = 0; k < NV; ++k) yv[k] = *reinterpret_cast<const uint4*>(y + row + (size_t)min(lane + k * 64, nvec - 1) * VE);
 #pragma unroll
     for (int k = 0; k < NV; ++k) wv[k] = *reinterpret_cast<const uint4*>(weight + (size_t)min(lane + k * 64, nvec - 1) * VE);
-    float ss = 0.f;
+    float sums[NV];   // a vector's squares each, then of pairs: one sum over a lane's up to 64 would round as often
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         T* xe = reinterpret_cast<T*>(&xv[k]);
         const T* ye = reinterpret_cast<const T*>(&yv[k]);
         const bool live = lane + k * 64 < nvec;
+        sums[k] = 0.f;
 #pragma unroll
         for (int e = 0; e < VE; ++e) {
             if (y) xe[e] = from_f<T>(to_f(xe[e]) + to_f(ye[e]));
             const float v = to_f(xe[e]);
-            if (live) ss = fmaf(v, v, ss);
+            if (live) sums[k] = fmaf(v, v, sums[k]);
         }
         if (live && x_out) *reinterpret_cast<uint4*>(x_out + row + (size_t)(lane + k * 64) * VE) = xv[k];
     }
+#pragma unroll
+    for (int n = NV / 2; n > 0; n /= 2)
+#pragma unroll
+        for (int k = 0; k < n; ++k) sums[k] += sums[k + n];
+    float ss = sums[0];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
     const float inv = rsqrtf(ss / (float)width + eps);

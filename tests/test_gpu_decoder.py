@@ -962,6 +962,22 @@ def test_add_rmsnorm_of_every_width(cuda, rows, width, dtype):
             assert torch.equal(out, s)
         want = s.double() * torch.rsqrt(s.double().square().mean(-1, keepdim=True) + 1e-5) * w.double()
         assert torch.equal(ops.add_rmsnorm(x, other, w, 1e-5, kmajor=True)[1].t(), h)
-        # fp16: one rounding, 2^-11, and what fp32 arithmetic adds to it; fp32: a sum of squares (a lane's at most 16, then 6
-        # steps), rsqrt and two products, 2^-23 each at most
+        # fp16: one rounding, 2^-11, and what fp32 arithmetic adds to it; fp32, in units of 2^-24: a sum of squares (a thread's at most 12, 14
+        # steps among a workgroup's, the division and eps: 28, halved by the root), 2 for rsqrt and one for each of two products
         assert bool(((h.double() - want).abs() <= (2.0 ** -10.9 if dtype == torch.float16 else 16 * 2.0 ** -23) * want.abs() + 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("rows,width", [(512, 2048), (513, 1024), (515, 512), (5, 2048)])
+def test_add_rmsnorm_adds_squares_up_in_short_runs(cuda, rows, width):
+    """fp32 rows whose small squares a running sum of one would lose one after the other: a 1 at the head of each of the first 64 vectors of four,
+    and everywhere else just less than 2^-12, whose square is less than half a unit of 1."""
+    from ternaryllm_amd import ops
+    x = torch.full((rows, width), 2.0 ** -12 * (1 - 2.0 ** -7), device=cuda)
+    x[:, 0:256:4] = 1.0
+    w = torch.ones(width, device=cuda)
+    print(f"case {rows} x {width}", flush=True)
+    h = ops.add_rmsnorm(x, None, w, 1e-12)[1].double()
+    want = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + 1e-12)
+    # in units of 2^-24: a vector's sum may lose its three others (3 and a rounding), then three and six steps, the division and eps, halved
+    # by the root; rsqrt 2; two products.  (One sum over a lane's 32 squares loses 31: 15 of these.)
+    assert float(((h - want) / want).abs().max()) <= (15 / 2 + 4) * 2.0 ** -24
