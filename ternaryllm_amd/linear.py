@@ -232,26 +232,26 @@ class TernaryLinear(nn.Module):
         reads it; returns (batch, rows, N) / (rows, N) / (N,) in the input dtype."""
         # (buffers are looked up where they are kept: one row 4096 x 4096 took 4.9 us of the host through the module's attributes, 4.5)
         w, buffers = self._handle, self._buffers
-        if w is not None and w.blob is buffers.get("w_packed"):
-            y = ops.product(w, input, buffers["w_scale"] if "w_scale" in buffers else self.w_scale, None)
-            if y is not None:
-                return y
-        if input.dim() > 3:
-            raise AssertionError("Input has dim larger than 3")  # the reference asserts (TernaryLinear.py:161)
-        w = self.device_weight()
-        K, N = self.in_features, self.out_features
-        rows = input.shape[-1] == K
-        y = ops.product(w, input, self.w_scale, not rows)
+        if w is None or w.blob is not buffers.get("w_packed"):
+            if input.dim() > 3:
+                raise AssertionError("Input has dim larger than 3")  # the reference asserts (TernaryLinear.py:161)
+            w = self.device_weight()
+        scale = buffers["w_scale"] if "w_scale" in buffers else self.w_scale
+        y = ops.product(w, input, scale, None)
         if y is not None:
             return y
+        if input.dim() > 3:
+            raise AssertionError("Input has dim larger than 3")
+        K, N = self.in_features, self.out_features
+        rows = input.shape[-1] == K
         if rows:
             lead = input.shape[:-1]
-            y = ops.spmm(w, input.reshape(-1, K), self.w_scale)
+            y = ops.spmm(w, input.reshape(-1, K), scale)
             return y.reshape(*lead, N)
         if input.dim() >= 2 and input.shape[-2] == K:  # K-major activations
             if input.dim() == 2:
-                return ops.spmm(w, input, self.w_scale, x_layout=1)
-            return ops.spmm_kmajor_batch(w, input, self.w_scale)
+                return ops.spmm(w, input, scale, x_layout=1)
+            return ops.spmm_kmajor_batch(w, input, scale)
         raise ValueError(f"input of shape {tuple(input.shape)} does not match in_features={K}")
 
     def extra_repr(self):

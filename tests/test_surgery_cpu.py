@@ -1,4 +1,5 @@
 """Model surgery on a toy module tree with Llama's layer names (no GPU, no transformers)."""
+import pytest
 import torch
 from torch import nn
 
@@ -94,3 +95,33 @@ def test_ternarize_threshold_and_from_weights():
     approx = mod.ternary_weight.float() * mod.w_scale[None, :]
     err = (approx - ref_w.t()).norm() / ref_w.norm()
     assert err < 0.6                                                          # a ternary fit of uniform weights, not noise
+
+
+@pytest.mark.parametrize("shape,call", [((2, 3, 96), "spmm"), ((5, 96), "spmm"), ((96,), "spmm"), ((96, 5), "spmm"), ((2, 96, 5), "spmm_kmajor_batch")])
+@pytest.mark.parametrize("fresh", [False, True])
+def test_a_call_that_is_not_plain_asks_the_short_way_once(monkeypatch, shape, call, fresh):
+    """What the short way refuses, or has no scratch for, goes on to the general path at once, with the module's handle there and without."""
+    from ternaryllm_amd import ops
+    module = TernaryLinear(96, 32, sparsity=0.5, bias=False, scale=torch.ones(32), reference_buffers=False)
+    handle = ops.DeviceWeight.from_blob_tensor(module.w_packed)
+    asked, taken = [], []
+    monkeypatch.setattr(ops, "product", lambda w, x, scale=None, kmajor=False: asked.append((w, x, scale, kmajor)))
+
+    def general(name):
+        def spmm(w, x, scale=None, **kw):
+            taken.append((name, w, scale))
+            rows = x.shape[0] * x.shape[2] if name != "spmm" else x.shape[1] if kw.get("x_layout") else x.shape[0]
+            return torch.zeros(rows, 32)
+        return spmm
+
+    monkeypatch.setattr(ops, "spmm", general("spmm"))
+    monkeypatch.setattr(ops, "spmm_kmajor_batch", general("spmm_kmajor_batch"))
+    if fresh:
+        monkeypatch.setattr(module, "device_weight", lambda: handle)
+    else:
+        module._handle = handle
+    module(torch.zeros(shape))
+    assert len(asked) == 1 and asked[0][0] is handle and asked[0][2] is module.w_scale
+    assert taken == [(call, handle, module.w_scale)]
+    with pytest.raises(AssertionError, match="dim larger than 3"):
+        module(torch.zeros(1, 1, 2, 96))
