@@ -472,6 +472,13 @@ __global__ __launch_bounds__(256) void tl_read_probe(const u32x4* __restrict__ s
     if (threadIdx.x == 0) out[blockIdx.x] = part[0] ^ part[1] ^ part[2] ^ part[3];
 }
 
+extern "C" int tl_matrix_tile(int64_t M, int columns, int inners, int planes, int x_dtype, int two_weights, int units)
+{
+    if (int rc = check_dtype(x_dtype, "x_dtype")) return rc;
+    if (M < 1 || columns < 1 || inners < 1 || planes < 1 || units < 1) return fail(TL_ERR_SHAPE, "sizes must be positive");
+    return matrix_tile(M, columns, (int64_t)planes * ceil_div(inners, TL_CODE_UNIT_ROWS), x_dtype == TL_F32, two_weights != 0, units);
+}
+
 extern "C" int tl_read_probe_workgroups(void) { return 8 * compute_units(); }
 
 extern "C" int tl_stream_read_probe(const void* src, int64_t bytes, void* out, void* stream)

@@ -792,55 +792,73 @@ int launch_tile(const KernelArgs& a, hipStream_t st)
     return TL_OK;
 }
 
-// Which tile, by how many there are and by the units of 256 rows of K (a multiple of the units is shared out evenly).  us, fp16;
-// "shared": K shared out among four waves, 32 x 32, 32 x 64 or 64 x 64; "small": 64 x 64, a wave 32 x 32; "wide": 64 x 128, a wave 64 x 32
-// (two weights: 32 x 64); "flat": 64 x 256; "tall": 128 x 256, a wave 64 or 128 rows x 64:
-//   shared up to one 64 x 64 tile a compute unit.  Bound by what a compute unit copies (some 40 bytes a clock, of which each wave's activations
-//     are most), so the smallest tile of which each compute unit has at most one, and 32 x 64 two to a unit for fp32.  32 x 32 / 32 x 64 / 64 x 64, 64 rows ->
-//     4096: K = 512 4.3 / - / 5.0, 4096 6.3 / 8.0 / 10.8, 11008 11.4 / 15.5 / 20; fp32 512 9.6 / 10.1 / 12.4, 2048 12.8 / 13.2 / 17.4, 11008 36 / 37 / 55;
-//     200 rows 2048 -> 2048 6.3 / 6.0 / 8.1, fp32 15.5 / 14.6 / 19.7.  Two 32 x 64 tiles a unit against one 64 x 64, -> 4096: fp32 200 rows of 4096 28.6 / 30.2,
-//     256 of 512 11.0 / 13.7; fp16 256 of 1024 6.5 / 6.7, but 200 of 4096 12.5 / 12.1, and 256 of 256 5.4 (small: 4.5).
-//   wide up to one of its tiles a unit, and up to two where it still gains.  Shared (which fits a unit once) / wide / flat, 512 rows
-//     -> 4096: K = 256 10.0 / 5.4 / 6.7, 1024 11.2 / 8.3 / 11.0, 4096 23.0 / 22.0 / 27.3; fp32 21.6 / 13.1 / 14.8, 25.8 / 23.1 / 28.1, 61.5 / 58.0 / 75.5.
-//     Wide / flat, 1024 rows -> 4096: 256 7.1 / 7.7, 2048 19.9 / 20.3; fp32 17.4 / 18.6; past that 1024 rows of 1024 -> 11008 28.1 / 26.8; two weights, 768
+}  // namespace
+
+// Which tile, by how many there are and by the units of 256 rows of K (a multiple of the units is shared out evenly).  us, fp16, graphs of
+// a call (`tl_spmm`, `tl_mlp_gate_up`), both sides of a line in turn:
+//   "shared", K shared out among four waves, up to one 64 x 64 tile a compute unit.  Bound by what a compute unit copies (some 40 bytes a clock, of
+//     which each wave's activations are most), so the smallest tile of which each compute unit has at most one, and 32 x 64 two to a unit for fp32.
+//     32 x 32 / 32 x 64 / 64 x 64, 64 rows -> 4096: K = 512 4.1 / 4.6 / 5.8, 4096 6.6 / 8.1 / 10.6; fp32 512 9.4 / 10.3 / 12.0, 4096 17.7 / 19.0 / 24.6.  Two
+//     32 x 64 tiles a unit / one 64 x 64, 256 rows -> 4096: 1024 6.3 / 6.4, 1536 7.4 / 8.0, 2048 8.1 / 8.2, 4096 11.5 / 11.2; fp32 1024 13.7 / 14.5, 2048
+//     19.1 / 20.9; two weights, 128 rows -> 4096: 512 5.6 / 6.0, 768 6.3 / 6.2, 1536 7.8 / 7.8, 2048 8.4 / 8.1, 4096 11.7 / 10.9.
+//   "small", 64 x 64, a wave 32 x 32, where K is one unit, of which three waves that share it have none, and for fp16 up to three where shared ones are two
+//     to a unit.  32 x 64 / small, 128 rows -> 4096: K = 64 3.9 / 3.6, 256 4.7 / 4.2, but 512 4.7 / 4.8; 256 rows 256 5.3 / 4.3, 768 6.1 / 5.8, 1024 6.3 / 6.5; fp32,
+//     128 rows 64 7.0 / 6.4, 256 10.0 / 9.6, 512 10.6 / 12.2; 256 rows 64 7.8 / 6.8, 256 10.8 / 10.2, 512 11.6 / 13.0.  (32 x 32, one to a unit, are as fast:
+//     64 rows 64 3.6 / 3.5, 256 4.0 / 4.1.)  Two weights, 128 rows -> 4096, 32 x 64 / wide: 256 5.5 / 5.3, 512 5.6 / 6.4, 768 6.3 / 7.4.
+//   "wide", 64 x 128, a wave 64 x 32 (two weights: 32 x 64), up to one of its tiles a unit, and up to two where it still gains.  Shared (which fits a unit once) /
+//     wide / flat, 512 rows -> 4096: K = 256 10.0 / 5.4 / 6.7, 1024 11.2 / 8.3 / 11.0, 4096 23.0 / 22.0 / 27.3; fp32 21.6 / 13.1 / 14.8, 25.8 / 23.1 / 28.1, 61.5 /
+//     58.0 / 75.5.  Wide / flat, 1024 rows -> 4096: 256 7.1 / 7.7, 2048 19.9 / 20.3; fp32 17.4 / 18.6; past that 1024 rows of 1024 -> 11008 28.1 / 26.8; two weights, 768
 //     rows of 2048 -> 2048 20.0 / 17.7.
-//   "groups": 64 x 256 for eight waves, two for each 64 columns, which share K out, while such tiles are one a unit and K is long: with flat ones a unit has four
-//     waves, one on each SIMD.  Wide / groups, 1024 rows -> 4096: 512 8.0 / 9.3, 1024 12.0 / 12.4, 4096 28.8 / 27.3, 11008 73.5 / 65; fp32 512 19.2 / 21.3, 1024 29.7 / 30.7;
+//   "groups", 64 x 256 for eight waves, two for each 64 columns, which share K out, while such tiles are one a unit and K is long: with flat ones a unit has
+//     four waves, one on each SIMD.  Wide / groups, 1024 rows -> 4096: 512 8.0 / 9.3, 1024 12.0 / 12.4, 4096 28.8 / 27.3, 11008 73.5 / 65; fp32 512 19.2 / 21.3, 1024 29.7 / 30.7;
 //     flat / groups, fp32, 4096: 76.0 / 71.3, 768 rows 73.3 / 68.1.
-//   tall where there are two of them a unit, so that one multiplies while the other waits or stores, and where flat ones would
-//     not spread the rows better.  Tall / flat: 2048 x 4096 -> 11008 121 / 125, 8192 x 2048 -> 11008 gated 247 / 255, 8192 x 5504 -> 2048 115 / 122, but
-//     1024 x 4096 -> 11008 76 / 69 (344 tall tiles are two for some units, 688 flat ones five halves).  Not for fp32, whose second
+//   "tall", 128 x 256, a wave 128 rows x 64, where there are two of them a unit, so that one multiplies while the other waits or stores, and where flat ones
+//     (64 x 256) would not spread the rows better.  Tall / flat: 2048 x 4096 -> 11008 121 / 125, 8192 x 2048 -> 11008 gated 247 / 255, 8192 x 5504 -> 2048 115 / 122,
+//     but 1024 x 4096 -> 11008 76 / 69 (344 tall tiles are two for some units, 688 flat ones five halves).  Not for fp32, whose second
 //     set of sums does not fit.
+MatrixTile tl::matrix_tile(int64_t rows, int64_t columns, int64_t depth, bool f32, bool two, int64_t units)
+{
+    auto tiles = [&](int height, int width) { return ceil_div(rows, height) * ceil_div(columns * (two ? 2 : 1), width); };
+    if (tiles(64, 64) <= units) {
+        const bool one_each = tiles(32, 64) <= units;
+        if (tiles(32, 32) <= units) return kShared32x32;
+        if (!two && depth <= (f32 || one_each ? 1 : 3)) return kSmall;
+        if (f32 || one_each || (depth > 1 && depth <= (two ? 6 : 8))) return kShared32x64;
+        if (depth > 1) return kShared64x64;
+    }
+    if (tiles(64, 128) <= units) return kWide;
+    if (tiles(64, 256) <= units && depth > (f32 ? 4 : 8)) return kGroups;
+    if (!two && tiles(64, 128) <= 2 * units) return kWide;
+    if (!f32 && tiles(128, 256) >= 2 * units && ceil_div(tiles(64, 256), units) >= 2 * ceil_div(tiles(128, 256), units)) return kTall;
+    return kFlat;
+}
+
+namespace {
+
 // The rows are the whole call's: a row's result does not depend on how many rows at a time a workspace holds.
 template <int PARTS, int MODE>
 int launch_mode(const KernelArgs& a, hipStream_t st)
 {
-    constexpr bool TWO = MODE == kTwoWeights;
-    const int64_t units = compute_units(), columns = (int64_t)a.N * (TWO ? 2 : 1), depth = (int64_t)a.planes * a.units;
-    auto tiles = [&](int rows, int width) { return ceil_div(a.call_rows, rows) * ceil_div(columns, width); };
-    const bool one_each = tiles(64, 64) <= units;
-    if (one_each) {
-        if (tiles(32, 32) <= units) return launch_tile<PARTS, 1, 1, 4, 1, 1, MODE>(a, st);
-        if (PARTS > 1 || tiles(32, 64) <= units || (depth > 3 && depth <= 8)) return launch_tile<PARTS, 1, 1, 4, 1, 2, MODE>(a, st);
-        if constexpr (PARTS == 1) {
-            if (depth > 3) return launch_tile<PARTS, 1, 1, 4, 2, 2, MODE>(a, st);
-            if constexpr (!TWO) return launch_tile<PARTS, 2, 2, 1, 1, 1, MODE>(a, st);
-        }
+    constexpr bool TWO = MODE == kTwoWeights, F32 = PARTS > 1;
+    switch (matrix_tile(a.call_rows, a.N, (int64_t)a.planes * a.units, F32, TWO, compute_units())) {
+    case kShared32x32: return launch_tile<PARTS, 1, 1, 4, 1, 1, MODE>(a, st);
+    case kShared32x64: return launch_tile<PARTS, 1, 1, 4, 1, 2, MODE>(a, st);
+    case kShared64x64:
+        if constexpr (!F32) return launch_tile<PARTS, 1, 1, 4, 2, 2, MODE>(a, st);
+        break;
+    case kSmall:
+        if constexpr (!TWO) return launch_tile<PARTS, 2, 2, 1, 1, 1, MODE>(a, st);
+        break;
+    case kWide:
+        if constexpr (TWO) return launch_tile<PARTS, 2, 2, 1, 1, 2, MODE>(a, st);
+        else return launch_tile<PARTS, 1, 4, 1, 2, 1, MODE>(a, st);
+    case kGroups: return launch_tile<PARTS, 1, 4, 2, 2, 2, MODE>(a, st);
+    case kFlat: return launch_tile<PARTS, 1, 4, 1, 2, 2, MODE>(a, st);
+    case kTall:
+        if constexpr (!F32) return launch_tile<PARTS, 1, 4, 1, 4, 2, MODE>(a, st);
+        break;
     }
-    if constexpr (TWO) {
-        if (tiles(64, 128) <= units) return launch_tile<PARTS, 2, 2, 1, 1, 2, MODE>(a, st);
-    } else {
-        if (tiles(64, 128) <= units) return launch_tile<PARTS, 1, 4, 1, 2, 1, MODE>(a, st);
-    }
-    if (tiles(64, 256) <= units && depth > (PARTS > 1 ? 4 : 8)) return launch_tile<PARTS, 1, 4, 2, 2, 2, MODE>(a, st);
-    if constexpr (!TWO) {
-        if (tiles(64, 128) <= 2 * units) return launch_tile<PARTS, 1, 4, 1, 2, 1, MODE>(a, st);
-    }
-    if constexpr (PARTS == 1) {
-        const int64_t tall = tiles(128, 256), flat = tiles(64, 256);
-        if (tall >= 2 * units && ceil_div(flat, units) >= 2 * ceil_div(tall, units)) return launch_tile<PARTS, 1, 4, 1, 4, 2, MODE>(a, st);
-    }
-    return launch_tile<PARTS, 1, 4, 1, 2, 2, MODE>(a, st);
+    return fail(TL_ERR_UNSUPPORTED, "no such tile");
 }
 
 template <int PARTS>

@@ -347,9 +347,10 @@ def test_a_blob_without_codes(cuda, oracle):
 
 
 # few tiles (one of 64 x 64 a compute unit at most), whose waves share K: 64 x 64 of nine units, and of three, which they own parts of;
-# 32 x 64 two to a compute unit; 32 x 32 with rows, columns and a stage left over, and of one unit, which leaves waves without a share
+# 32 x 64 two to a compute unit; 32 x 32 with rows, columns and a stage left over, and of one unit, which leaves waves without a share; of one unit,
+# 64 x 64 that share nothing; two weights of three units, 32 x 64
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
-@pytest.mark.parametrize("M,K,N", [(250, 2304, 4000), (250, 520, 4000), (253, 1100, 3970), (97, 1412, 1001), (49, 130, 33)])
+@pytest.mark.parametrize("M,K,N", [(250, 2304, 4000), (250, 520, 4000), (253, 1100, 3970), (97, 1412, 1001), (49, 130, 33), (130, 250, 4000), (130, 600, 2000)])
 def test_tiles_whose_waves_share_k(cuda, M, K, N, dtype):
     """Integer activations: every sum is exact, whatever its order; two weights and pairs against the gate of the products."""
     from ternaryllm_amd import ops

@@ -1,0 +1,50 @@
+"""Which tile a product of more than 48 rows takes on a device of 256 compute units (no GPU: the rule alone)."""
+import pytest
+
+from ternaryllm_amd import _lib
+
+TILES = ["shared 32x32", "shared 32x64", "shared 64x64", "small", "wide", "groups", "flat", "tall"]   # in the order of tl_matrix_tile's results
+
+
+def tile_of(M, K, N, dtype, two=False, planes=1, units=256):
+    rc = _lib.lib().tl_matrix_tile(M, N, K, planes, _lib.TL_F32 if dtype == "fp32" else _lib.TL_F16, int(two), units)
+    _lib.check(min(rc, 0))
+    return TILES[rc]
+
+
+# The sides of each line at which both tiles were timed: the tile that was the faster one there (us, the faster / the other).
+@pytest.mark.parametrize("M,K,N,dtype,two,tile", [
+    (64, 64, 4096, "fp16", False, "shared 32x32"),      # 3.6 / 3.6 small
+    (64, 4096, 4096, "fp16", False, "shared 32x32"),    # 6.6 / 8.1 shared 32x64
+    (128, 64, 4096, "fp16", False, "small"),            # 3.6 / 3.9 shared 32x64
+    (128, 256, 4096, "fp16", False, "small"),           # 4.2 / 4.7 shared 32x64
+    (200, 256, 2048, "fp16", False, "small"),           # 4.1 / 4.7 shared 32x64
+    (128, 512, 4096, "fp16", False, "shared 32x64"),    # 4.7 / 4.8 small
+    (256, 256, 4096, "fp16", False, "small"),           # 4.3 / 5.3 shared 32x64
+    (256, 768, 4096, "fp16", False, "small"),           # 5.8 / 6.1 shared 32x64
+    (256, 1024, 4096, "fp16", False, "shared 32x64"),   # 6.3 / 6.4 shared 64x64
+    (256, 2048, 4096, "fp16", False, "shared 32x64"),   # 8.1 / 8.2 shared 64x64
+    (256, 4096, 4096, "fp16", False, "shared 64x64"),   # 11.2 / 11.5 shared 32x64
+    (64, 256, 4096, "fp32", False, "shared 32x32"),     # 9.1 / 9.5 small
+    (128, 64, 4096, "fp32", False, "small"),            # 6.4 / 7.0 shared 32x64
+    (256, 64, 4096, "fp32", False, "small"),            # 6.8 / 7.8 shared 32x64
+    (256, 256, 4096, "fp32", False, "small"),           # 10.2 / 10.8 shared 32x64
+    (256, 512, 4096, "fp32", False, "shared 32x64"),    # 11.6 / 13.0 small
+    (256, 2048, 4096, "fp32", False, "shared 32x64"),   # 19.1 / 20.9 shared 64x64
+    (128, 256, 4096, "fp16", True, "wide"),             # 5.3 / 5.5 shared 32x64
+    (128, 512, 4096, "fp16", True, "shared 32x64"),     # 5.6 / 6.4 wide
+    (256, 768, 2048, "fp16", True, "shared 32x64"),     # 6.4 / 7.5 wide
+    (128, 1536, 4096, "fp16", True, "shared 32x64"),    # 7.8 / 7.8 shared 64x64
+    (128, 2048, 4096, "fp16", True, "shared 64x64"),    # 8.1 / 8.4 shared 32x64
+    (128, 4096, 4096, "fp16", True, "shared 64x64"),    # 10.9 / 11.7 shared 32x64
+    (128, 768, 4096, "fp32", True, "shared 32x64"),     # 12.1 / 12.7 shared 64x64
+])
+def test_few_tiles_take_the_faster_one(M, K, N, dtype, two, tile):
+    assert tile_of(M, K, N, dtype, two) == tile
+
+
+def test_planes_count_as_units_and_other_devices_have_their_own_lines():
+    assert tile_of(128, 256, 4096, "fp16", planes=2) == tile_of(128, 512, 4096, "fp16") == "shared 32x64"
+    assert tile_of(128, 256, 2048, "fp16", units=64) == tile_of(256, 256, 4096, "fp16")
+    for bad in ((0, 8, 8, 1, 0, 0, 256), (64, 8, 8, 1, 2, 0, 256), (64, 8, 8, 0, 0, 0, 256), (64, 8, 8, 1, 0, 0, 0)):
+        assert _lib.lib().tl_matrix_tile(*bad) < 0
