@@ -307,7 +307,7 @@ int tl_spmm_time(const tl_layout_header* header, const void* blob_dev,
 /* Measurement helper with no counterpart in the reference: which tile a product of more than 48 rows takes on a device of
  * `units` compute units, for fp16 or fp32 activations, one weight or two (tl_mlp_gate_up).  Launches nothing and asks no
  * device.  Returns, of a workgroup's rows x columns, 0 to 2 where four waves share K: 32 x 32, 32 x 64, 64 x 64; 3 64 x 64,
- * 4 64 x 128, 5 64 x 256 by two groups of waves that share K, 6 64 x 256, 7 128 x 256; or a negative TL_ERR_*. */
+ * 4 64 x 128; 5 64 x 128, 6 64 x 256 by two groups of waves that share K; 7 64 x 256, 8 128 x 256; or a negative TL_ERR_*. */
 int tl_matrix_tile(int64_t M, int columns, int inners, int planes, int x_dtype, int two_weights, int units);
 
 /* Measurement helper with no counterpart in the reference: one launch that only READS `bytes` bytes

@@ -223,7 +223,7 @@ inline int64_t least_image_bytes(int64_t K, int64_t M, int x_dtype)
 int launch_matrix_rows(KernelArgs a, int x_dtype, void* workspace, int64_t workspace_bytes, bool two_weights, hipStream_t st);
 // The tiles of tl_matrix_rows, and which of them a call takes: columns of one weight (two: of each), depth in units of 256 rows of K, planes
 // counted, units of the device.
-enum MatrixTile { kShared32x32, kShared32x64, kShared64x64, kSmall, kWide, kGroups, kFlat, kTall };
+enum MatrixTile { kShared32x32, kShared32x64, kShared64x64, kSmall, kWide, kHalves, kGroups, kFlat, kTall };
 MatrixTile matrix_tile(int64_t rows, int64_t columns, int64_t depth, bool f32, bool two, int64_t units);
 // Whether rows of more than 48 are read where they lie, which products with chained steps need.
 bool matrix_reads_rows(const KernelArgs& a, int x_dtype);

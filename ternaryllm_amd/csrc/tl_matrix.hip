@@ -805,13 +805,18 @@ int launch_tile(const KernelArgs& a, hipStream_t st)
 //     to a unit.  32 x 64 / small, 128 rows -> 4096: K = 64 3.9 / 3.6, 256 4.7 / 4.2, but 512 4.7 / 4.8; 256 rows 256 5.3 / 4.3, 768 6.1 / 5.8, 1024 6.3 / 6.5; fp32,
 //     128 rows 64 7.0 / 6.4, 256 10.0 / 9.6, 512 10.6 / 12.2; 256 rows 64 7.8 / 6.8, 256 10.8 / 10.2, 512 11.6 / 13.0.  (32 x 32, one to a unit, are as fast:
 //     64 rows 64 3.6 / 3.5, 256 4.0 / 4.1.)  Two weights, 128 rows -> 4096, 32 x 64 / wide: 256 5.5 / 5.3, 512 5.6 / 6.4, 768 6.3 / 7.4.
-//   "wide", 64 x 128, a wave 64 x 32 (two weights: 32 x 64), up to one of its tiles a unit, and up to two where it still gains.  Shared (which fits a unit once) /
-//     wide / flat, 512 rows -> 4096: K = 256 10.0 / 5.4 / 6.7, 1024 11.2 / 8.3 / 11.0, 4096 23.0 / 22.0 / 27.3; fp32 21.6 / 13.1 / 14.8, 25.8 / 23.1 / 28.1, 61.5 /
-//     58.0 / 75.5.  Wide / flat, 1024 rows -> 4096: 256 7.1 / 7.7, 2048 19.9 / 20.3; fp32 17.4 / 18.6; past that 1024 rows of 1024 -> 11008 28.1 / 26.8; two weights, 768
-//     rows of 2048 -> 2048 20.0 / 17.7.
+//   "wide", 64 x 128, a wave 64 x 32 (two weights: 32 x 64), up to three a unit; two weights of fp16 rows up to eight units of K only; one weight
+//     of fp16 rows up to three units of K as many as fit the units at once, four each.  Shared (which fits a unit once) / wide / flat, 512 rows -> 4096: K = 256 10.0 / 5.4 / 6.7, 1024
+//     11.2 / 8.3 / 11.0, 4096 23.0 / 22.0 / 27.3; fp32 21.6 / 13.1 / 14.8, 25.8 / 23.1 / 28.1, 61.5 / 58.0 / 75.5.  Wide / flat, two or three a unit: 1024 rows -> 5504 256
+//     8.0 / 9.1, 1024 13.3 / 15.7, 5504 49.1 / 55.6; two weights, 768 rows -> 4096 256 8.5 / 8.9, 1536 20.0 / 20.3, 2048 25.0 / 25.1, 5504 59.4 / 57.2.  Four, 2048 rows -> 4096:
+//     256 9.6 / 9.8, 512 11.7 / 12.2, 768 13.8 / 14.3, 1024 16.5 / 16.6; more, 1024 rows of 256 -> 11008 12.1 / 11.8.
+//   "halves", 64 x 128 for four waves, two for each 64 columns, which share K out, for two weights in the place of wide ones that are one a unit, from four
+//     units of K on: a wave's 64 columns meet each fragment of activations four times, as it makes half the operands a product, and twice as much is
+//     asked for ahead.  Wide / halves, 512 rows -> 2048: 768 7.7 / 8.3, 1024 8.8 / 8.2, 2048 13.1 / 11.3, 5504 29.5 / 23.1; fp32 768 17.7 / 19.8, 1024 20.7 / 19.8, 5504 68.2 / 58.0.
 //   "groups", 64 x 256 for eight waves, two for each 64 columns, which share K out, while such tiles are one a unit and K is long: with flat ones a unit has
-//     four waves, one on each SIMD.  Wide / groups, 1024 rows -> 4096: 512 8.0 / 9.3, 1024 12.0 / 12.4, 4096 28.8 / 27.3, 11008 73.5 / 65; fp32 512 19.2 / 21.3, 1024 29.7 / 30.7;
-//     flat / groups, fp32, 4096: 76.0 / 71.3, 768 rows 73.3 / 68.1.
+//     four waves, one on each SIMD.  Wide / groups, 1024 rows -> 4096: 1024 10.3 / 11.2, 2816 20.6 / 20.5, 4096 28.1 / 26.8, 5504 37.0 / 34.7; 768 rows 2816 19.0 / 19.7, 4096
+//     25.5 / 25.1; fp32, 1024 rows 1536 38.0 / 38.7, 2048 46.2 / 46.6, 4096 79.1 / 73.0; 768 rows 1536 36.1 / 36.4, 2048 43.9 / 43.3.  Two weights, wide / flat / groups, 512 rows -> 4096: 256
+//     6.9 / 7.2 / 7.8, 768 10.2 / 10.2 / 10.2, 1024 11.8 / 11.7 / 11.1, 2048 18.4 / 17.4 / 15.9.
 //   "tall", 128 x 256, a wave 128 rows x 64, where there are two of them a unit, so that one multiplies while the other waits or stores, and where flat ones
 //     (64 x 256) would not spread the rows better.  Tall / flat: 2048 x 4096 -> 11008 121 / 125, 8192 x 2048 -> 11008 gated 247 / 255, 8192 x 5504 -> 2048 115 / 122,
 //     but 1024 x 4096 -> 11008 76 / 69 (344 tall tiles are two for some units, 688 flat ones five halves).  Not for fp32, whose second
@@ -826,9 +831,11 @@ MatrixTile tl::matrix_tile(int64_t rows, int64_t columns, int64_t depth, bool f3
         if (f32 || one_each || (depth > 1 && depth <= (two ? 6 : 8))) return kShared32x64;
         if (depth > 1) return kShared64x64;
     }
-    if (tiles(64, 128) <= units) return kWide;
-    if (tiles(64, 256) <= units && depth > (f32 ? 4 : 8)) return kGroups;
-    if (!two && tiles(64, 128) <= 2 * units) return kWide;
+    const int64_t wide = tiles(64, 128);
+    if (wide <= units) return two && depth > 3 ? kHalves : kWide;
+    if (tiles(64, 256) <= units && depth > (f32 ? two ? 4 : 6 : two ? 3 : 12)) return kGroups;
+    if (wide <= 3 * units && (f32 || !two || depth <= 8)) return kWide;
+    if (wide <= 4 * units && !f32 && !two && depth <= 3) return kWide;
     if (!f32 && tiles(128, 256) >= 2 * units && ceil_div(tiles(64, 256), units) >= 2 * ceil_div(tiles(128, 256), units)) return kTall;
     return kFlat;
 }
@@ -852,6 +859,9 @@ int launch_mode(const KernelArgs& a, hipStream_t st)
     case kWide:
         if constexpr (TWO) return launch_tile<PARTS, 2, 2, 1, 1, 2, MODE>(a, st);
         else return launch_tile<PARTS, 1, 4, 1, 2, 1, MODE>(a, st);
+    case kHalves:
+        if constexpr (TWO) return launch_tile<PARTS, 1, 2, 2, 2, 2, MODE>(a, st);
+        break;
     case kGroups: return launch_tile<PARTS, 1, 4, 2, 2, 2, MODE>(a, st);
     case kFlat: return launch_tile<PARTS, 1, 4, 1, 2, 2, MODE>(a, st);
     case kTall:

@@ -368,10 +368,10 @@ def test_tiles_whose_waves_share_k(cuda, M, K, N, dtype):
     assert torch.equal(ops.spmm_gated(even, x), ops.silu_mul(ops.spmm(even, x), pairs=True))
 
 
-# two groups of four waves that share K: eleven units (five and six) and a last one of one stage or of eight rows, for one weight and, at
-# half the rows, for two
+# two groups of four waves that share K: eleven units (five and six), fp16 fourteen, and a last one of one stage or of eight rows, for one weight
+# and, at half the rows, for two; two groups of two waves, for two weights: the same and five units
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
-@pytest.mark.parametrize("M,K,N", [(900, 2568, 4090), (500, 2616, 4090), (1000, 2816, 3850)])
+@pytest.mark.parametrize("M,K,N", [(900, 2568, 4090), (500, 2616, 4090), (1000, 2816, 3850), (900, 3336, 4090), (500, 2616, 2040), (450, 1032, 2000)])
 def test_groups_of_waves_that_share_k(cuda, M, K, N, dtype):
     test_tiles_whose_waves_share_k(cuda, M, K, N, dtype)
 

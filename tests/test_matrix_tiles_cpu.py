@@ -3,7 +3,7 @@ import pytest
 
 from ternaryllm_amd import _lib
 
-TILES = ["shared 32x32", "shared 32x64", "shared 64x64", "small", "wide", "groups", "flat", "tall"]   # in the order of tl_matrix_tile's results
+TILES = ["shared 32x32", "shared 32x64", "shared 64x64", "small", "wide", "halves", "groups", "flat", "tall"]   # in the order of tl_matrix_tile's results
 
 
 def tile_of(M, K, N, dtype, two=False, planes=1, units=256):
@@ -40,6 +40,34 @@ def tile_of(M, K, N, dtype, two=False, planes=1, units=256):
     (128, 768, 4096, "fp32", True, "shared 32x64"),     # 12.1 / 12.7 shared 64x64
 ])
 def test_few_tiles_take_the_faster_one(M, K, N, dtype, two, tile):
+    assert tile_of(M, K, N, dtype, two) == tile
+
+
+@pytest.mark.parametrize("M,K,N,dtype,two,tile", [
+    (512, 5504, 4096, "fp16", False, "wide"),           # one tile a unit: as it was
+    (1024, 1024, 5504, "fp16", False, "wide"),          # 13.3 / 15.7 flat
+    (768, 512, 5504, "fp16", False, "wide"),            # 9.3 / 11.1 flat
+    (768, 5504, 5504, "fp16", False, "wide"),           # 45.6 / 54.1 flat
+    (2048, 512, 4096, "fp16", False, "wide"),           # 11.7 / 12.2 flat
+    (1024, 256, 11008, "fp16", False, "flat"),          # 11.8 / 12.1 wide
+    (1024, 2816, 4096, "fp16", False, "wide"),          # 20.6 / 20.5 groups
+    (768, 2816, 4096, "fp16", False, "wide"),           # 19.0 / 19.7 groups
+    (1024, 4096, 4096, "fp16", False, "groups"),        # 26.8 / 28.1 wide
+    (1024, 1536, 4096, "fp32", False, "wide"),          # 38.0 / 38.7 groups
+    (768, 2048, 4096, "fp32", False, "groups"),         # 43.3 / 43.9 wide
+    (1024, 4096, 4096, "fp32", False, "groups"),        # 73.0 / 79.1 wide
+    (512, 768, 2048, "fp16", True, "wide"),             # 7.7 / 8.3 halves
+    (512, 1024, 2048, "fp16", True, "halves"),          # 8.2 / 8.8 wide
+    (512, 2048, 2048, "fp16", True, "halves"),          # 11.3 / 13.1 wide
+    (512, 768, 2048, "fp32", True, "wide"),             # 17.7 / 19.8 halves
+    (512, 1024, 2048, "fp32", True, "halves"),          # 19.8 / 20.7 wide
+    (512, 256, 4096, "fp16", True, "wide"),             # 6.9 / 7.2 flat
+    (512, 1024, 4096, "fp16", True, "groups"),          # 11.1 / 11.7 flat
+    (768, 2048, 2048, "fp16", True, "groups"),          # 15.5 / 17.2 flat
+    (768, 1536, 4096, "fp16", True, "wide"),            # 20.0 / 20.3 flat
+    (768, 5504, 4096, "fp16", True, "flat"),            # 57.2 / 59.4 wide
+])
+def test_more_tiles_take_the_faster_one(M, K, N, dtype, two, tile):
     assert tile_of(M, K, N, dtype, two) == tile
 
 
