@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+from tests.test_matrix_tiles_cpu import SIZES
 from tests.util import activations, ternary_weight
 
 pytestmark = pytest.mark.gpu
@@ -387,6 +388,99 @@ def test_entries_beyond_one_of_whole_stages(cuda, M, K, dtype):
     x = activations(M, K, 6, dtype, integer=True)
     y = ops.spmm(ops.DeviceWeight(_repeated(w), cuda), x.to(cuda), out_dtype=torch.float32)
     assert np.array_equal(y.cpu().numpy().astype(np.float64), x.double().numpy() @ w)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_nothing_past_k_is_read_for_entries_beyond_one(cuda, dtype):
+    """What lies behind a row's K values -- for fp16 rows read where they are the gap to the next row, in the fp32 rows' image the next row's
+    head -- shows in no bit: NaN there would meet zero weights, and the sum be worked out again in another order."""
+    from ternaryllm_amd import ops
+    M, K, ld, N = 130, 1088, 1344, 40
+    rng = np.random.default_rng(K)
+    w = rng.integers(-3, 4, (K, N)) * (rng.random((K, N)) < 0.3)
+    dw = ops.DeviceWeight(_repeated(w), cuda)
+    values = activations(M, K, 6, dtype).to(cuda)
+    rows = torch.zeros((M + 1, ld), dtype=dtype, device=cuda)
+    rows[:M, :K] = values
+    print(f"case {dtype}", flush=True)
+    want = ops.spmm(dw, rows[:M, :K], out_dtype=torch.float32)
+    assert bool(want.isfinite().all())
+    rows[:, K:] = float("nan")
+    assert torch.equal(ops.spmm(dw, rows[:M, :K], out_dtype=torch.float32), want)
+    spoilt = values.clone()
+    spoilt[1::2, :192] = float("nan")
+    assert torch.equal(ops.spmm(dw, spoilt, out_dtype=torch.float32)[0::2], want[0::2])
+
+
+def _of_every_tile(two):
+    return [pytest.param(dtype, tile, *size, id=f"{kind}-{tile}") for kind, dtype in (("fp16", torch.float16), ("fp32", torch.float32)) for tile, size in SIZES[kind, two].items()]
+
+
+def _spoilt_rows(M):
+    """Rows in each fragment of 16 of a tile's first 128, at its edges and between (groups of waves exchange half of a tile's fragments), and the last."""
+    return [m for m in (0, 15, 21, 40, 63, 70, 90, 101, 127) if m < M - 1] + [M - 1]
+
+
+@pytest.mark.parametrize("dtype,tile,M,K,N", _of_every_tile(False))
+def test_sums_that_are_not_finite_on_every_tile(cuda, dtype, tile, M, K, N):
+    """One infinity or NaN a row, at rows of K of every stage's parts: outputs that name it have it, all others are exact (whole numbers); gated
+    outputs are the gate of those; and with other activations, rows without one keep their bits."""
+    from ternaryllm_amd import ops
+    w = ternary_weight(K, N, 0.6, M)
+    dw, wd = _device(w, cuda), torch.from_numpy(w).double().to(cuda)
+    x = activations(M, K, K, dtype, integer=True).to(cuda)
+    want = x.double() @ wd
+    spoilt, rows = x.clone(), _spoilt_rows(M)
+    for i, m in enumerate(rows):
+        k, v = (i * 37 + i * K // len(rows)) % K, (float("inf"), float("nan"), float("-inf"))[i % 3]
+        want[m] += torch.where(wd[k] != 0, v * wd[k], 0.0) - x[m, k].double() * wd[k]
+        spoilt[m, k] = v
+    print(f"case {tile} M={M} K={K} N={N} {dtype}", flush=True)
+    got = ops.spmm(dw, spoilt, out_dtype=torch.float32).double()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0, 1e30, -1e30), want.nan_to_num(7.0, 1e30, -1e30))
+    pairs, both = ops.spmm_gated(dw, spoilt), ops.silu_mul(ops.spmm(dw, spoilt), pairs=True)
+    assert torch.equal(pairs.isnan(), both.isnan()) and torch.equal(pairs.nan_to_num(7.0), both.nan_to_num(7.0))
+    keep = torch.ones(M, dtype=torch.bool, device=cuda)
+    keep[rows] = False
+    x = activations(M, K, 13, dtype).to(cuda)
+    beside = torch.where(spoilt.isfinite(), x, spoilt)
+    assert torch.equal(ops.spmm(dw, x)[keep], ops.spmm(dw, beside)[keep])
+    assert torch.equal(ops.spmm_gated(dw, x)[keep], ops.spmm_gated(dw, beside)[keep])
+
+
+@pytest.mark.parametrize("dtype,tile,M,K,N", _of_every_tile(True))
+def test_two_weights_sums_that_are_not_finite_on_every_tile(cuda, dtype, tile, M, K, N):
+    from ternaryllm_amd import ops
+    wg, wu = ternary_weight(K, N, 0.6, M), ternary_weight(K, N, 0.7, N)
+    dg, du = _device(wg, cuda), _device(wu, cuda)
+    x = (activations(M, K, K, dtype, integer=True) / 16).to(cuda)
+    spoilt, rows, products = x.clone(), _spoilt_rows(M), []
+    for i, m in enumerate(rows):
+        spoilt[m, (i * 37 + i * K // len(rows)) % K] = (float("inf"), float("nan"), float("-inf"))[i % 3]
+    for w in (wg, wu):
+        wd = torch.from_numpy(w).double().to(cuda)
+        y = torch.where(spoilt.isfinite(), x, 0).double() @ wd
+        for i, m in enumerate(rows):
+            k = (i * 37 + i * K // len(rows)) % K
+            y[m] += torch.where(wd[k] != 0, spoilt[m, k].double() * wd[k], 0.0)
+        products.append(y)
+    print(f"case {tile} M={M} K={K} N={N} {dtype}", flush=True)
+    want = products[0] / (1 + torch.exp(-products[0])) * products[1]
+    got = ops.mlp_gate_up(dg, du, spoilt, out_dtype=torch.float32).double()
+    assert torch.equal(got.isnan(), want.isnan())
+    got, want = got.nan_to_num(0.0, 1e30, -1e30), want.nan_to_num(0.0, 1e30, -1e30)
+    largest = float(want[want.abs() < 1e29].abs().max())
+    assert float((got - want).abs().max()) <= 1e-5 * largest                  # exact sums; __expf and the division (infinities are equal)
+    keep = torch.ones(M, dtype=torch.bool, device=cuda)
+    keep[rows] = False
+    x = activations(M, K, 13, dtype).to(cuda)
+    beside = torch.where(spoilt.isfinite(), x, spoilt)
+    assert torch.equal(ops.mlp_gate_up(dg, du, x)[keep], ops.mlp_gate_up(dg, du, beside)[keep])
+
+
+@pytest.mark.parametrize("tile", list(SIZES["fp16", False]))
+def test_chained_rows_on_every_tile(cuda, tile):
+    test_chained_rows(cuda, *SIZES["fp16", False][tile], 66)
 
 
 # few rows and many

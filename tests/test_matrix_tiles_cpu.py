@@ -76,3 +76,27 @@ def test_planes_count_as_units_and_other_devices_have_their_own_lines():
     assert tile_of(128, 256, 2048, "fp16", units=64) == tile_of(256, 256, 4096, "fp16")
     for bad in ((0, 8, 8, 1, 0, 0, 256), (64, 8, 8, 1, 2, 0, 256), (64, 8, 8, 0, 0, 0, 256), (64, 8, 8, 1, 0, 0, 0)):
         assert _lib.lib().tl_matrix_tile(*bad) < 0
+
+
+# For each kind of call (rows, two weights) a size at which it takes each of its tiles, with rows, columns and a stage of K left over: what the
+# GPU tests that have to reach every tile run (columns are even, K whole 16-byte pieces, for gated and chained calls).
+SIZES = {
+    ("fp16", False): {"shared 32x32": (97, 1408, 1002), "shared 32x64": (253, 1104, 3970), "shared 64x64": (250, 2312, 4002), "small": (130, 248, 4002),
+                      "wide": (520, 1096, 2058), "groups": (900, 3336, 4090), "flat": (2110, 264, 4090), "tall": (4093, 200, 4090)},
+    ("fp32", False): {"shared 32x32": (97, 1408, 1002), "shared 32x64": (253, 1104, 3970), "small": (130, 248, 4002),
+                      "wide": (520, 1096, 2058), "groups": (900, 2568, 4090), "flat": (2110, 264, 4090)},
+    ("fp16", True): {"shared 32x32": (97, 1408, 1002), "shared 32x64": (200, 2056, 1034), "shared 64x64": (150, 2312, 2050), "wide": (520, 248, 2058),
+                     "halves": (450, 1032, 2002), "groups": (500, 2616, 4090), "flat": (850, 2312, 4090), "tall": (4093, 200, 4090)},
+    ("fp32", True): {"shared 32x32": (97, 1408, 1002), "shared 32x64": (200, 2056, 1034), "wide": (520, 248, 2058),
+                     "halves": (450, 1032, 2002), "groups": (500, 2616, 4090), "flat": (1100, 264, 4090)},
+}
+
+
+@pytest.mark.parametrize("kind", list(SIZES))
+def test_every_tile_has_a_size(kind):
+    """A line that moves takes no tile out of the tests unnoticed; and no tile is reached that has none."""
+    for tile, (M, K, N) in SIZES[kind].items():
+        assert tile_of(M, K, N, *kind) == tile and N % 2 == 0 and K % 8 == 0
+    reached = {tile_of(M, K, N, *kind) for M in (49, 97, 128, 250, 520, 900, 1100, 2110, 8192) for K in (8, 256, 512, 1024, 2048, 4096, 11008)
+               for N in (8, 512, 1024, 2048, 4096, 11008)}
+    assert reached == set(SIZES[kind])
