@@ -63,6 +63,9 @@ def weight_and_packed(K, N, sparsity, seed, device):
     return _packed[key]
 
 
+KERNEL_SOURCES = ("tl_matrix.hip", "tl_matrix.h", "tl_device.h", "tl_silu.h", "tl_layout.cpp", "tl_common.h")
+
+
 def kernel_source_hash():
     """sha256 over the sources the headline's kernel and its launcher are built from (the matrix-core
     kernel's translation unit, what it shares with the others, the blob builder, the shared constants): a traffic
@@ -70,7 +73,7 @@ def kernel_source_hash():
     import hashlib
     h = hashlib.sha256()
     csrc = os.path.join(ROOT, "ternaryllm_amd", "csrc")
-    for name in ("tl_matrix.hip", "tl_matrix.h", "tl_device.h", "tl_layout.cpp", "tl_common.h"):
+    for name in KERNEL_SOURCES:
         with open(os.path.join(csrc, name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()[:16]

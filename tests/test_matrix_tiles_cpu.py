@@ -100,3 +100,20 @@ def test_every_tile_has_a_size(kind):
     reached = {tile_of(M, K, N, *kind) for M in (49, 97, 128, 250, 520, 900, 1100, 2110, 8192) for K in (8, 256, 512, 1024, 2048, 4096, 11008)
                for N in (8, 512, 1024, 2048, 4096, 11008)}
     assert reached == set(SIZES[kind])
+
+
+def test_the_traffic_record_s_hash_covers_what_the_kernel_includes():
+    import os
+    import re
+
+    import bench
+    csrc = os.path.join(bench.ROOT, "ternaryllm_amd", "csrc")
+    seen, todo = set(), ["tl_matrix.hip", "tl_layout.cpp"]
+    while todo:
+        name = todo.pop()
+        if name in seen or not os.path.exists(os.path.join(csrc, name)):
+            continue                                                 # (the interface's header is not of the kernel's own)
+        seen.add(name)
+        with open(os.path.join(csrc, name)) as f:
+            todo += re.findall(r'#include "(.*?)"', f.read())
+    assert seen == set(bench.KERNEL_SOURCES)
