@@ -213,14 +213,14 @@ __global__ __launch_bounds__(256, 2) void tl_prefill_attn(PrefillAttn a)
         if (t * KT <= wq0 + 16 * QF - 1 + offset) {               // (a tile of which the wave's queries see nothing is skipped)
             f32x4 sc[4][QF];
 #pragma unroll
-            for (int s = 0; s < KS; ++s)                          // (outermost: a product waits for its sum's last one, four steps of keys before)
+            for (int i = 0; i < 4 * KS; ++i) {
+                // heads of 128: the four steps of keys in turn, so that a product waits for its sum's last one three products before; of 64, whose
+                // sums have two, one step after the other (2 x 4096 tokens, 16 heads: 123.7 us in turn, 108.3 so; of 128 183.5 / 184.7)
+                const int s = HD == 128 ? i / 4 : i % KS, n = HD == 128 ? i % 4 : i / KS, key = n * 16 + r16;
+                const u32x4 kx = *reinterpret_cast<const u32x4*>(ks + key * HD * 2 + key_place(key, s * 4 + g) * 16);
 #pragma unroll
-                for (int n = 0; n < 4; ++n) {
-                    const int key = n * 16 + r16;
-                    const u32x4 kx = *reinterpret_cast<const u32x4*>(ks + key * HD * 2 + key_place(key, s * 4 + g) * 16);
-#pragma unroll
-                    for (int f = 0; f < QF; ++f) sc[n][f] = matrix_step<false>(kx, qx[f][s], s == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sc[n][f]);
-                }
+                for (int f = 0; f < QF; ++f) sc[n][f] = matrix_step<false>(kx, qx[f][s], s == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sc[n][f]);
+            }
             if (t * KT + KT - 1 > wq0 + offset) {                 // some query of the wave does not see all of the tile
 #pragma unroll
                 for (int f = 0; f < QF; ++f) {
