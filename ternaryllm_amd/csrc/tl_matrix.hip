@@ -20,7 +20,7 @@ constexpr int kStageRowBytes = kStageRows * 2;       // bytes of one activation 
 // Row tiles whose column tiles a part of the chip works through together.  An activation tile is eight times the bytes of
 // a code tile along the same K (24 times for fp32 in three parts), so few row tiles against many column tiles is least traffic: 8192 x 2048 -> 11008 took 456 us
 // with all 64 row tiles in one group (every column tile streamed all activations through an L2), 300 / 300 / 310 with 2 / 4 / 8 (gated, as
-// it is now, 246 / 247 / 249 and 255 with 16).
+// it is now, 248 / 247 / 248 and 254 with 16).
 constexpr int kRowGroup = 4;
 constexpr int kUnitStages = TL_CODE_UNIT_ROWS / kStageRows;
 __device__ __align__(16) const unsigned char kNoCodes[TL_CODE_UNIT_BYTES] = {};   // a unit of zero weights
@@ -244,8 +244,9 @@ __device__ __forceinline__ void put_out(const KernelArgs& a, f32x4 (&acc)[F][G],
 // memory, 16 x 16 x 32 products run at 2200 TFLOP/s in fp16 and 2230 in bf16, 32 x 32 x 16 ones at 1750 and 1880 (with the weights as
 // the second operand 1970; at 66 % zeros).  With all that stands around them 8192 x 5504 -> 2048 runs at 1600, or 1760 without what a
 // launch costs; without making operands and reading LDS it would take 8 % less.  A wave owns 64 columns: each fragment of
-// activations that it reads from LDS serves four products.  us with 32 x 32 x 16 / now: 8192 x 2048 -> 11008 gated 281 / 247, 8192 x 2048 -> 6144
-// 156 / 140, 8192 x 5504 -> 2048 133 / 116, 1024 x 4096 -> 11008 78 / 71; fp32 4096 x 4096 -> 4096 292 / 250, 1024 x 4096 -> 4096 85 / 71.
+// activations that it reads from LDS serves four products.  us with 32 x 32 x 16 / now: 8192 x 2048 -> 11008 gated 280 / 247, 8192 x 2048 -> 6144
+// 152 / 136, 8192 x 5504 -> 2048 133 / 115, 1024 x 4096 -> 11008 76 / 69; fp32 4096 x 4096 -> 4096 301 / 257, 1024 x 4096 -> 4096 88 / 74 (one run; by a tenth
+// more or less on other cards).
 // A lone wave on its SIMD is bound by what it issues, of which twice as many products are more: the load side's addresses
 // are scalar and follow from the turn (fp32 1024 x 4096 -> 4096 82 us while they were worked out for every load).
 //
@@ -818,8 +819,8 @@ int launch_tile(const KernelArgs& a, hipStream_t st)
 //     25.5 / 25.1; fp32, 1024 rows 1536 38.0 / 38.7, 2048 46.2 / 46.6, 4096 79.1 / 73.0; 768 rows 1536 36.1 / 36.4, 2048 43.9 / 43.3.  Two weights, wide / flat / groups, 512 rows -> 4096: 256
 //     6.9 / 7.2 / 7.8, 768 10.2 / 10.2 / 10.2, 1024 11.8 / 11.7 / 11.1, 2048 18.4 / 17.4 / 15.9.
 //   "tall", 128 x 256, a wave 128 rows x 64, where there are two of them a unit, so that one multiplies while the other waits or stores, and where flat ones
-//     (64 x 256) would not spread the rows better.  Tall / flat: 2048 x 4096 -> 11008 121 / 125, 8192 x 2048 -> 11008 gated 247 / 255, 8192 x 5504 -> 2048 115 / 122,
-//     but 1024 x 4096 -> 11008 76 / 69 (344 tall tiles are two for some units, 688 flat ones five halves).  Not for fp32, whose second
+//     (64 x 256) would not spread the rows better.  Tall / flat: 2048 x 4096 -> 11008 122 / 128, 8192 x 2048 -> 11008 gated 244 / 253, 8192 x 5504 -> 2048 114 / 120,
+//     but 1024 x 4096 -> 11008 80 / 68 (344 tall tiles are two for some units, 688 flat ones five halves).  Not for fp32, whose second
 //     set of sums does not fit.
 MatrixTile tl::matrix_tile(int64_t rows, int64_t columns, int64_t depth, bool f32, bool two, int64_t units)
 {

@@ -233,8 +233,8 @@ class TernaryLlamaDecoder(nn.Module):
         """The pass with the library's kernels around the products: residual add + RMSNorm in one, keys rotated into the
         cache and values copied beside them in one, queries rotated inside the attention.  Seven launches a layer.
         (The add and the norm have a kernel, which rounds a row once, behind its factor: a product that left rows times the
-        next norm's weight, 1587 us where this takes 1620 for 16 x 512 tokens of 2048 and two layers, put entries above
-        65504 / weight at infinity.  The add alone in the product's last step gains nothing.)"""
+        next norm's weight made the pass 2 % faster, and put entries above 65504 / weight at infinity.  The add alone in the
+        product's last step gains nothing.)"""
         c = self.config
         B, S = tokens.shape
         H, nh, hd = c.hidden_size, c.num_attention_heads, c.head_dim
