@@ -811,9 +811,12 @@ int launch_tile(const KernelArgs& a, hipStream_t st)
 //     11.2 / 8.3 / 11.0, 4096 23.0 / 22.0 / 27.3; fp32 21.6 / 13.1 / 14.8, 25.8 / 23.1 / 28.1, 61.5 / 58.0 / 75.5.  Wide / flat, two or three a unit: 1024 rows -> 5504 256
 //     8.0 / 9.1, 1024 13.3 / 15.7, 5504 49.1 / 55.6; two weights, 768 rows -> 4096 256 8.5 / 8.9, 1536 20.0 / 20.3, 2048 25.0 / 25.1, 5504 59.4 / 57.2.  Four, 2048 rows -> 4096:
 //     256 9.6 / 9.8, 512 11.7 / 12.2, 768 13.8 / 14.3, 1024 16.5 / 16.6; more, 1024 rows of 256 -> 11008 12.1 / 11.8.
-//   "halves", 64 x 128 for four waves, two for each 64 columns, which share K out, for two weights in the place of wide ones that are one a unit, from four
+//   "halves", 64 x 128 for four waves, two for each 64 columns, which share K out, in the place of wide ones that are one a unit, for two weights from four
 //     units of K on: a wave's 64 columns meet each fragment of activations four times, as it makes half the operands a product, and twice as much is
 //     asked for ahead.  Wide / halves, 512 rows -> 2048: 768 7.7 / 8.3, 1024 8.8 / 8.2, 2048 13.1 / 11.3, 5504 29.5 / 23.1; fp32 768 17.7 / 19.8, 1024 20.7 / 19.8, 5504 68.2 / 58.0.
+//     One weight, fp16 rows, from eight units on where the groups' shares are alike, and past twelve at all: wide ones had become up to 6 % slower with products
+//     of 16 x 16 x 32 (with those before / wide / halves, 640 rows -> 2048: 1536 9.1 / 9.5 / 9.5, 2048 11.3 / 11.7 / 11.4, 2304 12.2 / 12.6 / 13.1, 2560 13.1 / 13.5 / 13.0, 2816
+//     14.1 / 14.5 / 14.7, 3328 16.3 / 17.3 / 16.7, 4096 20.3 / 20.9 / 18.1, 8192 36.8 / 36.0 / 29.4; 512 rows -> 4096: 1536 9.9 / 9.8 / 9.8, 2048 12.2 / 11.9 / 11.7, 5504 26.5 / 26.3 / 23.0).
 //   "groups", 64 x 256 for eight waves, two for each 64 columns, which share K out, while such tiles are one a unit and K is long: with flat ones a unit has
 //     four waves, one on each SIMD.  Wide / groups, 1024 rows -> 4096: 1024 10.3 / 11.2, 2816 20.6 / 20.5, 4096 28.1 / 26.8, 5504 37.0 / 34.7; 768 rows 2816 19.0 / 19.7, 4096
 //     25.5 / 25.1; fp32, 1024 rows 1536 38.0 / 38.7, 2048 46.2 / 46.6, 4096 79.1 / 73.0; 768 rows 1536 36.1 / 36.4, 2048 43.9 / 43.3.  Two weights, wide / flat / groups, 512 rows -> 4096: 256
@@ -833,7 +836,7 @@ MatrixTile tl::matrix_tile(int64_t rows, int64_t columns, int64_t depth, bool f3
         if (depth > 1) return kShared64x64;
     }
     const int64_t wide = tiles(64, 128);
-    if (wide <= units) return two && depth > 3 ? kHalves : kWide;
+    if (wide <= units) return (two ? depth > 3 : !f32 && (depth > 12 || (depth >= 8 && depth % 2 == 0))) ? kHalves : kWide;
     if (tiles(64, 256) <= units && depth > (f32 ? two ? 4 : 6 : two ? 3 : 12)) return kGroups;
     if (wide <= 3 * units && (f32 || !two || depth <= 8)) return kWide;
     if (wide <= 4 * units && !f32 && !two && depth <= 3) return kWide;
@@ -861,7 +864,7 @@ int launch_mode(const KernelArgs& a, hipStream_t st)
         if constexpr (TWO) return launch_tile<PARTS, 2, 2, 1, 1, 2, MODE>(a, st);
         else return launch_tile<PARTS, 1, 4, 1, 2, 1, MODE>(a, st);
     case kHalves:
-        if constexpr (TWO) return launch_tile<PARTS, 1, 2, 2, 2, 2, MODE>(a, st);
+        if constexpr (TWO || !F32) return launch_tile<PARTS, 1, 2, 2, 2, 2, MODE>(a, st);
         break;
     case kGroups: return launch_tile<PARTS, 1, 4, 2, 2, 2, MODE>(a, st);
     case kFlat: return launch_tile<PARTS, 1, 4, 1, 2, 2, MODE>(a, st);

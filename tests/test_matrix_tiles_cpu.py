@@ -44,7 +44,13 @@ def test_few_tiles_take_the_faster_one(M, K, N, dtype, two, tile):
 
 
 @pytest.mark.parametrize("M,K,N,dtype,two,tile", [
-    (512, 5504, 4096, "fp16", False, "wide"),           # one tile a unit: as it was
+    (512, 1536, 4096, "fp16", False, "wide"),           # 9.8 / 9.8 halves
+    (640, 1792, 2048, "fp16", False, "wide"),           # 10.8 / 11.6 halves
+    (640, 2048, 2048, "fp16", False, "halves"),         # 11.4 / 11.7 wide
+    (640, 2816, 2048, "fp16", False, "wide"),           # 14.5 / 14.7 halves
+    (640, 3072, 2048, "fp16", False, "halves"),         # 14.6 / 15.7 wide
+    (640, 3328, 2048, "fp16", False, "halves"),         # 16.7 / 17.3 wide
+    (512, 5504, 4096, "fp16", False, "halves"),         # 23.0 / 26.3 wide
     (1024, 1024, 5504, "fp16", False, "wide"),          # 13.3 / 15.7 flat
     (768, 512, 5504, "fp16", False, "wide"),            # 9.3 / 11.1 flat
     (768, 5504, 5504, "fp16", False, "wide"),           # 45.6 / 54.1 flat
@@ -82,7 +88,7 @@ def test_planes_count_as_units_and_other_devices_have_their_own_lines():
 # GPU tests that have to reach every tile run (columns are even, K whole 16-byte pieces, for gated and chained calls).
 SIZES = {
     ("fp16", False): {"shared 32x32": (97, 1408, 1002), "shared 32x64": (253, 1104, 3970), "shared 64x64": (250, 2312, 4002), "small": (130, 248, 4002),
-                      "wide": (520, 1096, 2058), "groups": (900, 3336, 4090), "flat": (2110, 264, 4090), "tall": (4093, 200, 4090)},
+                      "wide": (520, 1096, 2058), "halves": (450, 2040, 4002), "groups": (900, 3336, 4090), "flat": (2110, 264, 4090), "tall": (4093, 200, 4090)},
     ("fp32", False): {"shared 32x32": (97, 1408, 1002), "shared 32x64": (253, 1104, 3970), "small": (130, 248, 4002),
                       "wide": (520, 1096, 2058), "groups": (900, 2568, 4090), "flat": (2110, 264, 4090)},
     ("fp16", True): {"shared 32x32": (97, 1408, 1002), "shared 32x64": (200, 2056, 1034), "shared 64x64": (150, 2312, 2050), "wide": (520, 248, 2058),
